@@ -155,6 +155,9 @@ int k3q_unpack_int4(const void* in, int64_t outer, int64_t packed_len, int64_t i
 #define K3Q_GEMM_EXACT_EPILOGUE 1
 #define K3Q_GEMM_ROUND_ACC_BF16 2
 int64_t k3q_gemm_i8_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* room for the partials of a K split of the tile kernel alone: the workspace of a call whose
+ * operand needs no copy (b_layout 2, or b_layout 1 with K % 128 == 0), at any M */
+int64_t k3q_gemm_i8_split_bytes(int64_t M, int64_t N, int64_t K);
 int k3q_prepack_kernel_i8(const int8_t* kernel, int64_t K, int64_t N, int8_t* prepacked,
                           void* stream);
 int k3q_gemm_i8(const int8_t* a, const int8_t* b, int b_layout, int64_t M, int64_t N, int64_t K,
@@ -496,9 +499,11 @@ int k3q_embedding_lookup(const void* ids, int ids_dtype, int64_t count, const in
  * (k3q_dense_i8_w8s_supported says; K3Q_ERR_SHAPE otherwise).
  *
  * k3q_gemm_i8_w8s is the same kernel for rows that are already quantised (a: int8 [M, K],
- * a_scale: bfloat16 [M], as k3q_absmax_quantize writes them): every workgroup re-quantising
+ * a_scale: [M] of scale_dtype, as k3q_absmax_quantize writes them): every workgroup re-quantising
  * all of x costs more than a quantizer launch from about 16 K values of x on, and layers that
- * share their input quantise it once.  Same shapes, same bits.
+ * share their input quantise it once.  kernel_scale, bias and y have scale_dtype, bfloat16 (the same
+ * bits) or float32 (acc / (a_scale * kernel_scale) + bias, a rounding each).  Takes any K % 64 == 0 and
+ * any N while the rows fit LDS (k3q_gemm_i8_w8s_supported).
  */
 int64_t k3q_w8s_shadow_bytes(int64_t K, int64_t N);
 int k3q_w8s_pack(const int8_t* w, int64_t K, int64_t N, void* shadow, void* stream);
@@ -506,6 +511,7 @@ int k3q_dense_i8_w8s_supported(int64_t M, int64_t K, int64_t N);
 int k3q_dense_i8_w8s(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
                      const void* kernel_scale, const void* bias, int64_t bias_stride, float epsilon,
                      float range_lo, float range_hi, void* y, void* stream);
+int k3q_gemm_i8_w8s_supported(int64_t M, int64_t K, int64_t N);
 int k3q_gemm_i8_w8s(const int8_t* a, const void* a_scale, int scale_dtype, int64_t M, int64_t K, int64_t N,
                     const void* shadow, const void* kernel_scale, const void* bias, int64_t bias_stride,
                     void* y, void* stream);

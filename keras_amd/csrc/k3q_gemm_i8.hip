@@ -947,6 +947,10 @@ extern "C" int64_t k3q_gemm_i8_workspace_bytes(int64_t M, int64_t N, int64_t K) 
     return (N * K + 15) / 16 * 16 + split_workspace_bytes(M, N, K);
 }
 
+extern "C" int64_t k3q_gemm_i8_split_bytes(int64_t M, int64_t N, int64_t K) {
+    return K > 0 && N > 0 ? split_workspace_bytes(M, N, K) : 0;
+}
+
 extern "C" int k3q_prepack_kernel_i8(const int8_t* kernel, int64_t K, int64_t N, int8_t* prepacked,
                                      void* stream) {
     if (K <= 0 || N <= 0) return K3Q_ERR_SHAPE;

@@ -30,11 +30,11 @@ constexpr int kResident8 = 256;  // workgroups the chip holds at once (one per C
 struct W8sParams {
     const uint16_t* x;      // [M, K] bfloat16 (quantised in the kernel), or
     const int8_t* xq;       // [M, K] int8 with
-    const uint16_t* xs;     // [M] bfloat16 scales (already quantised rows)
+    const void* xs;         // T [M] scales (already quantised rows)
     const v4i* w;           // strip-linear copy
-    const uint16_t* scale;  // [N] bfloat16 kernel scale
-    const uint16_t* bias;   // [N] or [M, N] bfloat16, or null
-    uint16_t* y;            // [M, N] bfloat16
+    const void* scale;      // T [N] kernel scale; T is bfloat16, or float32 (kernels built with kF32)
+    const void* bias;       // T [N] or [M, N], or null
+    void* y;                // T [M, N]
     int64_t bias_stride;    // 0: one row for all, N: a row per row of x
     int M, K, N;
     int units;              // K / 64
@@ -58,17 +58,29 @@ __device__ __forceinline__ float descale_exact_bf16(int acc, float sa, float sb,
     return r;
 }
 
+// The same in float32: acc / (sa * sb) (+ bias), one rounding each.
+__device__ __forceinline__ float descale_exact_f32(int acc, float sa, float sb, float bv, bool has_bias) {
+    float r = (float)acc / (sb * sa);
+    if (has_bias) r = r + bv;
+    return r;
+}
+
 // kNP: 16-byte pieces of x a thread keeps in registers between the row maxima and the
 // quantisation (0: it reads them twice); -1: the rows arrive quantised (p.xq, p.xs).
 // kPre (kNP > 0 only): the rows are transformed before they are quantised (p.pre_kind): rms_norm with
 // a gain, the bits of k3q_rmsnorm, or multiplied by silu of a second input, the bits of k3q_silu_mul.
-template <int kSW, int kD, int kNP, bool kPre = false>
+// kF32 (kNP < 0 only): scales, bias and result are float32.
+// kTail (kNP < 0 only): the units are no whole number of blocks of kD, or fewer blocks than waves (K = 1600
+// is 25 units): the rows of x in LDS are zero past K, and a unit past the last one reads the last one.
+template <int kSW, int kD, int kNP, bool kPre = false, bool kF32 = false, bool kTail = false>
 __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int block, const int n_blocks) {
     extern __shared__ __attribute__((aligned(16))) char w8s_lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int q = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = p.M, K = p.K;
-    const int pitch = K + 16;
+    static_assert(kNP < 0 || !(kF32 || kTail), "float32 results and ragged K: rows that arrive quantised");
+    const int blocks = kTail ? (p.units + kD - 1) / kD : p.units / kD;
+    const int pitch = (kTail ? blocks * kD * 64 : K) + 16;
     // LDS: x rows as int8 | row maxima (uint bits) | row scales | reduction buffers
     char* xs = w8s_lds;
     u32* rowmax = (u32*)(w8s_lds + ((M * pitch + 255) & ~255));
@@ -78,7 +90,6 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
     const int red_one = kQ * kSW * mq * 16 * 4;  // ints per buffer
 
     // ---- this wave's slice of the units: blocks of kD units, the first waves take one more ----
-    const int blocks = p.units / kD;
     const int per = blocks / kQ, extra = blocks - per * kQ;
     const int b0 = q * per + (q < extra ? q : extra);
     const int my_units = (per + (q < extra ? 1 : 0)) * kD;
@@ -103,7 +114,8 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
     auto at_cursor = [&]() {
         const int g2 = place(lg < last_group ? lg : last_group);  // past the end: a valid address, never used
 #pragma unroll
-        for (int t = 0; t < kSW; ++t) nb[t] = p.w + ((int64_t)(g2 * kSW + t) * p.units + lu) * 64 + lane;
+        for (int t = 0; t < kSW; ++t)
+            nb[t] = p.w + ((int64_t)(g2 * kSW + t) * p.units + (kTail && lu >= p.units ? p.units - 1 : lu)) * 64 + lane;
     };
     auto advance = [&]() {
         lu += kD;
@@ -116,7 +128,10 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
     v4i W[kD][kSW];
     auto refill = [&](int d) {
 #pragma unroll
-        for (int t = 0; t < kSW; ++t) W[d][t] = __builtin_nontemporal_load(nb[t] + d * 64);
+        for (int t = 0; t < kSW; ++t) {
+            const int dd = kTail ? (lu + d < p.units ? d : lu < p.units ? p.units - 1 - lu : 0) : d;
+            W[d][t] = __builtin_nontemporal_load(nb[t] + dd * 64);
+        }
     };
     at_cursor();
     // Every wave's first x requests go out before any wave's weight requests: a compute unit's
@@ -162,7 +177,14 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
             copy_load(base);
             copy_store(base);
         }
-        if (tid < M) sa[tid] = bf16_bits_to_f32(p.xs[tid]);
+        if (kTail) {  // the columns past K of every row: zeros add nothing, whatever weights they meet
+            const int tail = (blocks * kD * 64 - K) >> 4;
+            for (int i = tid; i < M * tail; i += kT) {
+                const int row = i / tail;
+                *(v4u*)(xs + row * pitch + K + (i - row * tail) * 16) = v4u{0u, 0u, 0u, 0u};
+            }
+        }
+        if (tid < M) sa[tid] = raw_to_f32<!kF32>(load_raw<!kF32>(p.xs, tid));
     } else {
         // row maxima, scales, int8 rows: abs_max_quantize of the rows inside the workgroup
         const int pieces = M * (K >> 3);  // 16-byte pieces of x (8 values)
@@ -291,12 +313,12 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
         for (int t = 0; t < kSW; ++t) {
             const int n = n0 + t * 16 + i16;
             const int nn = n < p.N ? n : p.N - 1;
-            sb_raw[t] = p.scale[nn];
-            const uint16_t* bp = has_bias ? p.bias : p.scale;
+            sb_raw[t] = load_raw<!kF32>(p.scale, nn);
+            const void* bp = has_bias ? p.bias : p.scale;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = 4 * g + r;
-                bias_raw[t][r] = bp[(has_bias && m < M ? (int64_t)m * p.bias_stride : 0) + nn];
+                bias_raw[t][r] = load_raw<!kF32>(bp, (has_bias && m < M ? (int64_t)m * p.bias_stride : 0) + nn);
             }
         }
         v4i acc[kSW];
@@ -343,13 +365,17 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
             }
             const int n = n0 + q * 16 + i16;
             if (n < p.N) {
-                const float sb = bf16_bits_to_f32(sbq);
+                const float sb = raw_to_f32<!kF32>(sbq);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int m = 4 * g + r;
                     if (m < M) {
-                        const float yv = descale_exact_bf16(tot[r], sa[m], sb, bf16_bits_to_f32(bq[r]), has_bias);
-                        p.y[(int64_t)m * p.N + n] = (uint16_t)f32_to_bf16_bits(yv);
+                        const float bv = raw_to_f32<!kF32>(bq[r]);
+                        if constexpr (kF32)
+                            ((float*)p.y)[(int64_t)m * p.N + n] = descale_exact_f32(tot[r], sa[m], sb, bv, has_bias);
+                        else
+                            ((uint16_t*)p.y)[(int64_t)m * p.N + n] =
+                                (uint16_t)f32_to_bf16_bits(descale_exact_bf16(tot[r], sa[m], sb, bv, has_bias));
                     }
                 }
             }
@@ -361,6 +387,13 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
 template <int kSW, int kD, int kNP>
 __global__ __launch_bounds__(kT) void gemv_w8s(W8sParams p) {
     gemv_w8s_body<kSW, kD, kNP>(p, (int)blockIdx.x, (int)gridDim.x);
+}
+// Rows that arrive quantised: float32 results, ragged K.  Bound by the kernel's bytes and a launch's fixed
+// part, as the bfloat16 form; 16 x 4096 x 4096 in float32 behind its quantizer launch 29.4 -> 10.3 us (it ran
+// on 32 of the chip's 512 tile slots before), 16 x 8192 x 8192 62.0 -> 19.4, 1 x 1600 x 6400 10.6 -> 8.5.
+template <int kSW, int kD, bool kF32, bool kTail>
+__global__ __launch_bounds__(kT) void gemv_w8s_rows(W8sParams p) {
+    gemv_w8s_body<kSW, kD, -1, false, kF32, kTail>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Up to kMaxProblems8 kernels against one x in one launch (the query / key / value projections of
@@ -446,6 +479,34 @@ W8sPlan w8s_plan(int64_t M, int64_t K, int64_t N, bool shared = false) {
     return pl;
 }
 
+// Plan for rows that arrive quantised, any K % 64 == 0 and any N: the limits of w8s_plan that come from the
+// quantizer inside the workgroup (K % 512) or from sharing a launch do not apply.  All of K still stays inside a
+// workgroup, also where the strips are fewer than the CUs: one strip of K = 14336 is 224 KiB, which a CU
+// takes in under 4 us, about what the second launch of a K split costs.
+W8sPlan w8s_rows_plan(int64_t M, int64_t K, int64_t N, bool* tail) {
+    W8sPlan pl = w8s_plan(M, K, N);
+    *tail = false;
+    if (pl.ok) return pl;
+    pl = W8sPlan{};
+    if (M < 1 || M > kMaxRows8 || K < 64 || (K % 64) != 0 || N < 1) return pl;
+    const int64_t units = K / 64, strips = (N + 15) / 16;
+    pl.d = units >= 2 * 4 * kQ ? 4 : 2;
+    pl.sw = strips >= 2 * kResident8 ? 2 : 1;
+    const int64_t blocks = (units + pl.d - 1) / pl.d;
+    *tail = (units % pl.d) != 0 || blocks < kQ;
+    pl.resident = kResident8;
+    pl.groups = (strips + pl.sw - 1) / pl.sw;
+    const int64_t turns = (pl.groups + pl.resident - 1) / pl.resident;
+    pl.blocks = (pl.groups + turns - 1) / turns;
+    pl.np = -1;
+    const int64_t pitch = blocks * pl.d * 64 + 16;
+    const size_t red_one = (size_t)kQ * pl.sw * ((M + 3) / 4) * 16 * 4 * 4;
+    // (+ 64: a fragment read may run that far past the last row)
+    pl.lds = (size_t)((M * pitch + 255) & ~255) + 2 * kMaxRows8 * 4 + (turns > 1 ? 2 : 1) * red_one + 64;
+    pl.ok = pl.lds <= 160 * 1024;
+    return pl;
+}
+
 typedef void (*W8sKernel)(W8sParams);
 typedef void (*W8sMultiKernel)(W8sMulti);
 
@@ -491,6 +552,12 @@ W8sMultiKernel pick_kernel8_multi(const W8sPlan& pl) {
     return pl.d == 4 ? pick_np8_multi<1, 4>(pl.np) : pick_np8_multi<1, 2>(pl.np);
 }
 
+template <bool kF32, bool kTail>
+W8sKernel pick_kernel8_rows(const W8sPlan& pl) {
+    if (pl.sw == 2) return pl.d == 4 ? gemv_w8s_rows<2, 4, kF32, kTail> : gemv_w8s_rows<2, 2, kF32, kTail>;
+    return pl.d == 4 ? gemv_w8s_rows<1, 4, kF32, kTail> : gemv_w8s_rows<1, 2, kF32, kTail>;
+}
+
 W8sKernel pick_kernel8(const W8sPlan& pl) {
     if (pl.sw == 2) return pl.d == 4 ? pick_np8<2, 4>(pl.np) : pick_np8<2, 2>(pl.np);
     return pl.d == 4 ? pick_np8<1, 4>(pl.np) : pick_np8<1, 2>(pl.np);
@@ -518,24 +585,30 @@ extern "C" int k3q_w8s_pack(const int8_t* w, int64_t K, int64_t N, void* shadow,
 
 extern "C" int k3q_dense_i8_w8s_supported(int64_t M, int64_t K, int64_t N) { return w8s_plan(M, K, N).ok ? 1 : 0; }
 
+extern "C" int k3q_gemm_i8_w8s_supported(int64_t M, int64_t K, int64_t N) {
+    bool tail;
+    return w8s_rows_plan(M, K, N, &tail).ok ? 1 : 0;
+}
+
 namespace {
 // checks the operands of one problem and fills its kernel parameters
 int fill_params8(W8sParams& p, const W8sPlan& pl, const void* x, const int8_t* xq, const void* xs, int64_t M,
                  int64_t K, int64_t N, const void* shadow, const void* kernel_scale, const void* bias,
-                 int64_t bias_stride, float epsilon, float range_lo, float range_hi, void* y) {
+                 int64_t bias_stride, float epsilon, float range_lo, float range_hi, void* y, bool f32 = false) {
+    const size_t el = f32 ? 4 : 2;
     if (bias_stride != 0 && bias_stride != N) return K3Q_ERR_SHAPE;
     const bool quantised = xq != nullptr;
     if (!(quantised ? (const void*)xs : x) || !shadow || !kernel_scale || !y) return K3Q_ERR_NULL;
-    if (!aligned_to(quantised ? (const void*)xq : x, 16) || !aligned_to(shadow, 16) || !aligned_to(y, 2) ||
-        !aligned_to(kernel_scale, 2) || (bias && !aligned_to(bias, 2)) || (xs && !aligned_to(xs, 2)))
+    if (!aligned_to(quantised ? (const void*)xq : x, 16) || !aligned_to(shadow, 16) || !aligned_to(y, el) ||
+        !aligned_to(kernel_scale, el) || (bias && !aligned_to(bias, el)) || (xs && !aligned_to(xs, el)))
         return K3Q_ERR_ALIGN;
     p.x = (const uint16_t*)x;
     p.xq = xq;
-    p.xs = (const uint16_t*)xs;
+    p.xs = xs;
     p.w = (const v4i*)shadow;
-    p.scale = (const uint16_t*)kernel_scale;
-    p.bias = (const uint16_t*)bias;
-    p.y = (uint16_t*)y;
+    p.scale = kernel_scale;
+    p.bias = bias;
+    p.y = y;
     p.bias_stride = bias ? bias_stride : 0;
     p.M = (int)M;
     p.K = (int)K;
@@ -563,18 +636,17 @@ int raise_lds(const void* kernel) {
     return K3Q_OK;
 }
 
-int launch_w8s(const void* x, const int8_t* xq, const void* xs, int64_t M, int64_t K, int64_t N,
-               const void* shadow, const void* kernel_scale, const void* bias, int64_t bias_stride,
-               float epsilon, float range_lo, float range_hi, void* y, hipStream_t stream) {
+int launch_w8s(const void* x, int64_t M, int64_t K, int64_t N, const void* shadow, const void* kernel_scale,
+               const void* bias, int64_t bias_stride, float epsilon, float range_lo, float range_hi, void* y,
+               hipStream_t stream) {
     if (M < 0 || K <= 0 || N <= 0) return K3Q_ERR_SHAPE;
     if (M == 0) return K3Q_OK;
     W8sPlan pl = w8s_plan(M, K, N);
     if (!pl.ok) return K3Q_ERR_SHAPE;
     W8sParams p;
-    int rc = fill_params8(p, pl, x, xq, xs, M, K, N, shadow, kernel_scale, bias, bias_stride, epsilon, range_lo,
-                          range_hi, y);
+    int rc = fill_params8(p, pl, x, nullptr, nullptr, M, K, N, shadow, kernel_scale, bias, bias_stride, epsilon,
+                          range_lo, range_hi, y);
     if (rc != K3Q_OK) return rc;
-    if (xq) pl.np = -1;
     const W8sKernel kernel = pick_kernel8(pl);
     if ((rc = raise_lds((const void*)kernel)) != K3Q_OK) return rc;
     kernel<<<(unsigned)pl.blocks, kT, pl.lds, stream>>>(p);
@@ -589,17 +661,32 @@ extern "C" int k3q_dense_i8_w8s(const void* x, int x_dtype, int64_t M, int64_t K
     if (!(range_lo >= -128.f && range_hi <= 127.f && range_lo < range_hi)) return K3Q_ERR_SHAPE;
     // (the in-kernel quantizer clips before it rounds: exact only between integer ends)
     if (range_lo != rintf(range_lo) || range_hi != rintf(range_hi)) return K3Q_ERR_RANGE;
-    return launch_w8s(x, nullptr, nullptr, M, K, N, shadow, kernel_scale, bias, bias_stride, epsilon, range_lo,
-                      range_hi, y, (hipStream_t)stream);
+    return launch_w8s(x, M, K, N, shadow, kernel_scale, bias, bias_stride, epsilon, range_lo, range_hi, y,
+                      (hipStream_t)stream);
 }
 
 extern "C" int k3q_gemm_i8_w8s(const int8_t* a, const void* a_scale, int scale_dtype, int64_t M, int64_t K,
                                int64_t N, const void* shadow, const void* kernel_scale, const void* bias,
                                int64_t bias_stride, void* y, void* stream) {
-    if (scale_dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
-    if (M > 0 && !a) return K3Q_ERR_NULL;
-    return launch_w8s(nullptr, a, a_scale, M, K, N, shadow, kernel_scale, bias, bias_stride, 0.f, -127.f, 127.f,
-                      y, (hipStream_t)stream);
+    if (scale_dtype != K3Q_BF16 && scale_dtype != K3Q_F32) return K3Q_ERR_DTYPE;
+    if (M < 0 || K <= 0 || N <= 0) return K3Q_ERR_SHAPE;
+    if (M == 0) return K3Q_OK;
+    if (!a) return K3Q_ERR_NULL;
+    const bool f32 = scale_dtype == K3Q_F32;
+    bool tail = false;
+    W8sPlan pl = w8s_rows_plan(M, K, N, &tail);
+    if (!pl.ok) return K3Q_ERR_SHAPE;
+    pl.np = -1;
+    W8sParams p;
+    int rc = fill_params8(p, pl, nullptr, a, a_scale, M, K, N, shadow, kernel_scale, bias, bias_stride, 0.f, -127.f,
+                          127.f, y, f32);
+    if (rc != K3Q_OK) return rc;
+    const W8sKernel kernel = f32 ? (tail ? pick_kernel8_rows<true, true>(pl) : pick_kernel8_rows<true, false>(pl))
+                             : tail ? pick_kernel8_rows<false, true>(pl)
+                                    : pick_kernel8(pl);
+    if ((rc = raise_lds((const void*)kernel)) != K3Q_OK) return rc;
+    kernel<<<(unsigned)pl.blocks, kT, pl.lds, (hipStream_t)stream>>>(p);
+    return launch_status();
 }
 
 namespace {

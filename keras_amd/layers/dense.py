@@ -104,13 +104,22 @@ def kmajor_rows(rows, units, input_dim=0):
     return low <= rows <= KMAJOR_MAX_ROWS
 
 
-def int8_strip_route(quantizer, x2, units):
-    """Whether an int8 call of these rows goes to `ops.int8_dense_strip`: bfloat16 rows on the
-    device, few enough, a plain abs-max quantizer (whatever its range and epsilon), a shape the
-    kernel takes."""
-    return (type(quantizer) is quantizers.AbsMaxQuantizer and quantizer.output_dtype == "int8"
-            and x2.is_cuda and x2.dtype == torch.bfloat16 and 0 < x2.shape[0] <= kops.INT8_STRIP_MAX_ROWS
-            and kops.int8_strip_supported(x2.shape[0], x2.shape[1], units))
+def int8_strip_route(quantizer, x2, units, strict=False):
+    """Whether an int8 call of these rows goes to `ops.int8_dense_strip`: rows on the device, few
+    enough, a plain abs-max quantizer (whatever its range and epsilon), a shape the kernel takes.
+    Every shape it takes is faster there than behind the two-launch routes (rows 1, 4, 8 and 16,
+    quantizer included, us, strip against stored kernel or tiles: K=N=4096 float32 8.8 / 9.6 / 9.8 / 10.3
+    against 12.2 / 13.3 / 14.0 / 29.4; K=1600, N=6400 8.5 ... 10.6 against 10.6 ... 12.2; K=8192, N=1024
+    8.6 ... 11.9 against 13.9 ... 48.7; K=N=768 6.7 ... 7.5 against 9.2 ... 13.3).
+    strict: only bfloat16 rows and the widths of `ops.int8_strip_supported`: what a launch that several
+    layers share takes, and what a tied table keeps a copy for."""
+    if not (type(quantizer) is quantizers.AbsMaxQuantizer and quantizer.output_dtype == "int8"
+            and x2.is_cuda and 0 < x2.shape[0] <= kops.INT8_STRIP_MAX_ROWS):
+        return False
+    if x2.dtype == torch.bfloat16 and kops.int8_strip_supported(x2.shape[0], x2.shape[1], units):
+        return True
+    return (not strict and x2.dtype in (torch.float32, torch.bfloat16)
+            and kops.int8_strip_rows_supported(x2.shape[0], x2.shape[1], units))
 
 
 class Dense(Layer):
@@ -528,7 +537,7 @@ class Dense(Layer):
                 or self.exact_epilogue is False):
             return None
         x2 = inputs.reshape(-1, inputs.shape[-1])
-        if not int8_strip_route(self.inputs_quantizer, x2, self.units):
+        if not int8_strip_route(self.inputs_quantizer, x2, self.units, strict=True):
             return None
         bias = self._call_bias()
         if bias is not None and bias.numel() != self.units:

@@ -858,7 +858,7 @@ class EinsumDense(Layer):
         n = 1
         for c in gv.kept:
             n *= self.full_output_shape_of(c)
-        if not int8_strip_route(self.inputs_quantizer, x2, n):
+        if not int8_strip_route(self.inputs_quantizer, x2, n, strict=True):
             return None
         bias, fused = self._fusable_bias(gv, n)
         if bias is not None and bias.numel() != n:

@@ -574,7 +574,7 @@ class ReversibleEmbedding(Embedding):
         if exact is None:
             exact = True
         if (self.tie_weights and exact and out_dtype == torch.bfloat16
-                and int8_strip_route(self.inputs_quantizer, x2, N)):
+                and int8_strip_route(self.inputs_quantizer, x2, N, strict=True)):
             # decode sizes: the table's strip-linear copy as the [dim, vocab] kernel of the projection
             # (made once, as many bytes as the table): quantizer, exact int8 matmul and de-scale in
             # one launch, the bits of the route below

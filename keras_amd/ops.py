@@ -607,14 +607,14 @@ def int8_matmul(a, kernel, a_scale=None, kernel_scale=None, bias=None, out_dtype
         if strip.numel() != lib.k3q_w8s_shadow_bytes(K, N):
             raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
         b, layout = strip, 2
-        nbytes = max(0, nbytes - (N * K + 15) // 16 * 16)  # (room for the partials of a K split only)
+        nbytes = lib.k3q_gemm_i8_split_bytes(M, N, K)  # (room for the partials of a K split only)
     elif prepacked is not None and not skinny:
         # no per-call [N,K] copy: only the part of the scratch beyond it (partial sums of a
         # K split, taken for few-tile problems) is of use; a K that is not a multiple of 128
         # keeps all of it (both operands are zero-padded into it)
         b, layout = prepacked, 1
         if K % 128 == 0:
-            nbytes = max(0, nbytes - (N * K + 15) // 16 * 16)
+            nbytes = max(lib.k3q_gemm_i8_split_bytes(M, N, K), nbytes if M <= 64 else 0)
     else:
         b = kernel if kernel.is_contiguous() else kernel.contiguous()
         layout = 0
@@ -859,6 +859,12 @@ def int8_strip_supported(M, K, N):
     return bool(_lib.load().k3q_dense_i8_w8s_supported(int(M), int(K), int(N)))
 
 
+def int8_strip_rows_supported(M, K, N):
+    """Whether `int8_dense_strip` takes M rows, float32 or bfloat16, that a quantizer launch has
+    quantised first: any K % 64 == 0 and any N while the rows fit a workgroup's LDS."""
+    return bool(_lib.load().k3q_gemm_i8_w8s_supported(int(M), int(K), int(N)))
+
+
 def int8_strip_copy(kernel):
     """The strip-linear copy of a stored int8 kernel `[K, N]` that `int8_dense_strip` reads
     (include/k3q.h, k3q_w8s_pack): uint8 bytes, made once per layer."""
@@ -893,46 +899,52 @@ def int8_strip_quantises_inside(M, K, value_range):
 
 def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, value_range=(-127, 127),
                      quantize=None):
-    """The int8 Dense forward for up to 16 bfloat16 rows: abs-max quantisation of the rows, exact
-    int8 matmul against `int8_strip_copy(kernel)`, bit-exact bfloat16 de-scale, bias (N values)
-    or addend (a row per row of x).  One launch for small x; for larger x the rows are
-    quantised by `quantize(x2)` (default: `quantizers.abs_max_quantize` with these settings)
-    first.  Same bits as `abs_max_quantize` + `int8_matmul(..., exact_epilogue=True)`.
+    """The int8 Dense forward for up to 16 rows: abs-max quantisation of the rows, exact int8 matmul
+    against `int8_strip_copy(kernel)`, bit-exact de-scale in the rows' dtype, bias (N values)
+    or addend (a row per row of x).  One launch for small bfloat16 x; for larger x, float32 x and
+    widths outside `int8_strip_supported` the rows are quantised by `quantize(x2)` (default:
+    `quantizers.abs_max_quantize` with these settings) first.  Same bits as `abs_max_quantize` +
+    `int8_matmul(..., exact_epilogue=True)`.
     Reference: keras/src/layers/core/dense.py:956-972."""
     _lib.require_device(x, shadow, kernel_scale, bias)
     lib = _lib.load()
-    if x.dtype != torch.bfloat16 or kernel_scale.dtype != torch.bfloat16:
-        raise TypeError("the strip route computes in bfloat16")
+    code = _lib.dtype_code(x.dtype)
+    if kernel_scale.dtype != x.dtype:
+        raise TypeError("kernel_scale must be read in the input's dtype")
     K, N = int(x.shape[-1]), int(units)
     lead = x.shape[:-1]
     x2 = x.reshape(-1, K)
     x2 = x2 if x2.is_contiguous() else x2.contiguous()
     M = x2.shape[0]
-    if not lib.k3q_dense_i8_w8s_supported(M, K, N):
+    inside = (code == _lib.K3Q_BF16 and int8_strip_quantises_inside(M, K, value_range)
+              and lib.k3q_dense_i8_w8s_supported(M, K, N))
+    if not inside and not lib.k3q_gemm_i8_w8s_supported(M, K, N):
         raise ValueError(f"int8_dense_strip does not take M={M}, K={K}, N={N}")
     if shadow.dtype != torch.uint8 or shadow.numel() != lib.k3q_w8s_shadow_bytes(K, N):
         raise ValueError("shadow is not int8_strip_copy(kernel) of this [K, N]")
     if kernel_scale.numel() != N:
         raise ValueError(f"kernel_scale holds {kernel_scale.numel()} values, expected {N}")
     _check_bias_size(bias, M, N)
-    if bias is not None and bias.dtype != torch.bfloat16:
-        raise TypeError("bias must be bfloat16")
+    if bias is not None and bias.dtype != x.dtype:
+        raise TypeError("bias must be read in the input's dtype")
     stride = N if (bias is not None and M > 1 and bias.numel() == M * N) else 0
     ks = kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous()
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    if not int8_strip_quantises_inside(M, K, value_range):
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    if not inside:
         if quantize is None:
             from keras_amd import quantizers
 
             q, s = quantizers.abs_max_quantize(x2, axis=-1, value_range=value_range, epsilon=epsilon)
         else:
             q, s = quantize(x2)
-        rc = lib.k3q_gemm_i8_w8s(_lib.ptr(q), _lib.ptr(s), _lib.dtype_code(s.dtype), M, K, N, _lib.ptr(shadow),
+        if s.dtype != x.dtype:
+            raise TypeError("the rows' scales must have the input's dtype")
+        rc = lib.k3q_gemm_i8_w8s(_lib.ptr(q), _lib.ptr(s), code, M, K, N, _lib.ptr(shadow),
                                  _lib.ptr(ks), _lib.ptr(bias) if bias is not None else None, stride,
                                  _lib.ptr(y), _lib.stream_ptr(x.device))
         _lib.check(rc, "k3q_gemm_i8_w8s")
         return y.reshape(*lead, N)
-    rc = lib.k3q_dense_i8_w8s(_lib.ptr(x2), _lib.dtype_code(x.dtype), M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
+    rc = lib.k3q_dense_i8_w8s(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
                               _lib.ptr(bias) if bias is not None else None, stride, float(epsilon),
                               float(value_range[0]), float(value_range[1]), _lib.ptr(y),
                               _lib.stream_ptr(x.device))

@@ -204,3 +204,31 @@ def test_dense_int8_strip_fractional_range(dev):
                               1e-7, -100.5, 90.25, _lib.ptr(y), _lib.stream_ptr(dev))
     assert rc == -7
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("K,N", [(64, 1), (448, 17), (512, 40), (960, 3200), (1600, 515), (4096, 4096), (8192, 48),
+                                 (1088, 8208)])
+def test_quantised_rows_any_width(dev, M, K, N, dtype):
+    # the form for rows that arrive quantised: one unit of K to a ragged number of them (with and
+    # without a tail, fewer blocks than waves), one column to more strips than workgroups, both dtypes
+    g = torch.Generator().manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    qk, ks = ref.dense_quantize_int8(ref.glorot_uniform(K, N, generator=g))
+    bias = (torch.randn(N, generator=g) * 0.1).to(dtype)
+    assert kops.int8_strip_rows_supported(M, K, N)
+    y = kops.int8_dense_strip(x.to(dev), kops.int8_strip_copy(qk.to(dev)), N, ks.to(dtype).to(dev), bias=bias.to(dev))
+    want = ref.dense_int8_call(x, qk, ks, bias.float(), compute_dtype=dtype)
+    assert y.dtype == dtype and torch.equal(y.cpu(), want)
+
+
+@pytest.mark.parametrize("M", [17, 64])
+def test_split_of_few_rows_on_the_strip_copy(dev, M):
+    # 17 ... 64 rows leave most of the chip idle unless K is split: same accumulators either way
+    K, N = 4096, 512
+    g = torch.Generator().manual_seed(M)
+    a = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).to(dev)
+    w = torch.randint(-127, 128, (K, N), generator=g, dtype=torch.int8).to(dev)
+    acc = kops.int8_matmul(a, w, strip=kops.int8_strip_copy(w), want_acc=True, want_y=False)
+    assert torch.equal(acc.cpu(), torch.mm(a.cpu().int(), w.cpu().int()))
