@@ -347,6 +347,20 @@ int k3q_gemv_w4s_supported(int64_t M, int64_t K, int64_t N, int64_t block_size);
 int k3q_gemv_w4s(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
                  const void* scale, const void* gparams, int64_t block_size, const void* bias,
                  int64_t bias_stride, void* y, void* stream);
+/* The general form: bfloat16 or float32 x (scales, bias and y in the same type), 1 <= M <= 16, any K % 8 == 0 from
+ * 16 on, any N.  The copy is k3q_w4s_pack's (the last unit's nibbles past K are zero); grouped parameters are
+ * k3q_w4s_rows_pack_params' (records of four scales in `dtype` and four bytes zero + 128, per strip, unit and
+ * quarter strip).  Rows whose x does not fit a workgroup's LDS go in several launches
+ * (k3q_gemv_w4s_rows_launches: how many; 0: not taken, K3Q_ERR_SHAPE). */
+int64_t k3q_w4s_rows_params_bytes(int64_t K, int64_t N, int64_t block_size, int dtype);
+int k3q_w4s_rows_pack_params(const void* scale, int dtype, const int8_t* zero, int64_t K, int64_t N,
+                             int64_t block_size, void* params, void* stream);
+int k3q_gemv_w4s_rows_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size);
+int k3q_gemv_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                      const void* scale, const void* gparams, int64_t block_size, const void* bias,
+                      int64_t bias_stride, void* y, void* stream);
+int k3q_gemv_w4s_rows_multi(const void* x, int x_dtype, int64_t M, int64_t K, int count,
+                            const k3q_gemv_w4s_problem* problems, int64_t block_size, void* stream);
 int k3q_gemv_w4s_multi(const void* x, int x_dtype, int64_t M, int64_t K, int count,
                        const k3q_gemv_w4s_problem* problems, int64_t block_size, void* stream);
 

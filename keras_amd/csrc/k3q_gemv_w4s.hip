@@ -46,19 +46,20 @@ constexpr int kRedStride = 20;   // floats per (row, strip) line of the cross-wa
 constexpr int kMaxProblems = 4;
 
 struct W4sParams {
-    const uint16_t* x;       // [M, K] bf16
+    const uint16_t* x;       // [M, K] bf16 (or float32: kernels built with kParts >= 2; so are scale, bias and y)
     const v4u* w;            // strip-linear copy
     const uint16_t* scale;   // per-channel: bf16 [N]
-    const uint8_t* gparams;  // grouped/128: [strip][unit][4][{4 bf16 scales, 4 (zero + 128)}] = 48 B
+    const uint8_t* gparams;  // grouped/128: [strip][unit][4][{4 bf16 scales, 4 (zero + 128)}] = 48 B (float32: 80)
     const uint16_t* bias;    // bf16 [N] or [M, N], or null
     uint16_t* y;             // [M, N] bf16
     int64_t bias_stride;     // 0 or N
-    int M, K, N, units;      // units = K / 128
+    int M, K, N, units;      // units = ceil(K / 128)
     int row_magic;           // ceil(2^32 / pieces per staged row): piece -> row without a division
     int slice_magic;         // (x staged in two parts) ceil(2^32 / pieces of a slice's first part); row_magic: of a row's
     int row_magic2, slice_magic2;  // the same for the second part
     int own_magic[2];        // (waves stage their own slices) ceil(2^32 / pieces per row of a slice): short, long slice
     int own;                 // 1: every wave stages its own slice of x; 0: the workgroup's threads share all of x
+    int one_red;             // (kParts) 1: room for one reduction buffer only, whatever the number of turns
     // an operation on x on its way into LDS (kernels built with kPre only):
     int pre_kind;             // 1: rms_norm(x) * pre_op (bf16 [K]); 2: silu(pre_op) * x (pre_op bf16 [M, K])
     float pre_eps;            // rms_norm's epsilon
@@ -87,30 +88,39 @@ __device__ __forceinline__ float bf_hi(u32 d) { return __uint_as_float(d & 0xfff
 // gain, as k3q_rmsnorm does, same bits) or multiplied by silu of a second input (as k3q_silu_mul).
 // Every workgroup repeats the transform on all of x -- a few hundred float operations per thread,
 // against a launch and a round trip through memory for the separate kernel.
-template <int kSW, int kD, int kNP, bool kGrouped, bool kHalves, bool kPre = false>
+// kParts: 0 for the forms above.  1, 2, 3: any K % 8 == 0 and any N.  A unit past the last one re-reads the
+// last one and meets rows of x that are zero in LDS past K; columns past N are computed and not stored.  2 and 3:
+// float32 rows.  A row travels as that many bfloat16 rows that add up to it (its top 16 bits, the top 16 bits of
+// the rest, ...: to 2^-17, or exactly), side by side in the sixteen rows the matrix instruction has anyway, and
+// the float32 results of a row's parts are added at the end.  The weights sit at 24 + w instead of 136 + w there
+// (the nibble three bits higher in the mantissa: as many operations), a fifth of the offset to cancel.
+template <int kSW, int kD, int kNP, bool kGrouped, bool kHalves, bool kPre = false, int kParts = 0>
 __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int block, const int stride) {
     extern __shared__ __attribute__((aligned(16))) char w4s_lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int q = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int units = p.units;
+    constexpr bool kRows = kParts > 0, kF32 = kParts >= 2;
+    static_assert(!(kRows && (kHalves || kPre)), "the general form stages x whole and as it is");
     const int M = p.M, K = p.K;
+    const int MX = kF32 ? kParts * M : M;  // rows in LDS: part h of row m is row h M + m
     const int j = lane & 15, g = lane >> 4;
-    const int jj = j < M ? j : M - 1;
-    const int groups = (p.N / 16 + kSW - 1) / kSW;
-    // slices of K: whole blocks of kD units, the first (blocks % kQ) waves take one more
-    const int blocks = units / kD;
+    const int jj = j < MX ? j : MX - 1;
+    const int groups = ((p.N + 15) / 16 + kSW - 1) / kSW;
+    // slices of K: whole blocks of kD units, the first (blocks % kQ) waves take one more (kRows: one at least)
+    const int blocks = !kRows ? units / kD : units > kQ * kD ? (units + kD - 1) / kD : kQ;
     const int base = blocks / kQ, extra = blocks - base * kQ;
     const int U = (base + (q < extra ? 1 : 0)) * kD;
     const int u0 = (q * base + (q < extra ? q : extra)) * kD;
-    const int R = U / kD;  // >= 2 (the launch plan sees to it)
+    const int R = U / kD;  // >= 2 (the launch plan sees to it; kRows: >= 1)
     // kHalves: LDS holds the first Rh rounds' worth of every wave's slice, then the rest (the two parts
     // are equal when the slice has an even number of rounds)
     const int Rh = kHalves ? (R + 1) / 2 : R;
     const int Uh = Rh * kD;    // units of a slice whose x is in LDS at a time (the first part)
     const int Uh2 = U - Uh;    // (kHalves) the second part
-    const int pitch = (kHalves ? kQ * Uh * 256 : K * 2) + 16;
+    const int pitch = (kHalves ? kQ * Uh * 256 : kRows ? blocks * kD * 256 : K * 2) + 16;
     // (two buffers, one per parity of the turn, when a workgroup takes several turns)
-    float* red = (float*)(w4s_lds + ((M * pitch + 255) & ~255));
+    float* red = (float*)(w4s_lds + ((MX * pitch + 255) & ~255));
 
     // ---- x into registers first (every load unconditional: pieces past the end re-read piece 0) ----
     // Whole rows (kHalves: half h of every wave's slice, row m = [slice 0 | slice 1 | ...]), spread over
@@ -119,14 +129,14 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
     // barrier stands between a wave's x (the oldest requests in its queue) and its first weights.
     // (Measured: worth 0.3 us up to 32 KiB of x, a loss beyond.)
     static_assert(!(kPre && kHalves), "no transform of x staged in halves");
-    const bool own = !kHalves && !kPre && p.own;
+    const bool own = !kHalves && !kPre && !kRows && p.own;
     const int per_row = own ? U * 16 : K >> 3;  // (kHalves: per part, below)
     const int pieces = M * per_row;
     const u32 row_magic = own ? (u32)p.own_magic[q < extra ? 1 : 0] : (u32)p.row_magic;
     const int own_col = own ? u0 * 16 : 0;  // first piece of the wave's slice within a row
     const int row_pieces = K >> 3;
     v4u xst[kNP];
-    v4u xop[kPre ? kNP : 1];
+    v4u xop[kPre || kF32 ? kNP : 1];
     auto stage_load = [&](const int h) {
         if constexpr (kHalves) {
             // part h of every wave's slice: row m of LDS = [slice 0's part | slice 1's part | ...]
@@ -150,7 +160,11 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
             pi = pi < pieces ? pi : 0;
             const int m = (int)__umulhi((unsigned)pi, row_magic);
             const int c = pi - m * per_row;
-            {
+            if constexpr (kF32) {
+                const v4u* src = (const v4u*)((const float*)p.x + ((int64_t)m * row_pieces + c) * 8);
+                xst[i] = src[0];
+                xop[i] = src[1];
+            } else {
                 xst[i] = *(const v4u*)(p.x + ((int64_t)m * row_pieces + own_col + c) * 8);
                 if constexpr (kPre)  // the gain's piece of this column, or the second input's piece
                     xop[i] = *(const v4u*)(p.pre_op + (p.pre_kind == 1 ? (int64_t)c : (int64_t)m * row_pieces + c) * 8);
@@ -177,8 +191,39 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
             if (pi < pieces) {
                 const int m = (int)__umulhi((unsigned)pi, row_magic);
                 const int c = pi - m * per_row;
-                *(v4u*)(w4s_lds + m * pitch + (own_col + c) * 16) = xst[i];
+                char* dst = w4s_lds + m * pitch + (own_col + c) * 16;
+                if constexpr (kF32) {
+                    // parts by truncation, each exact, the last one rounded: top 16 bits of what is left
+                    float rest[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) rest[e] = __uint_as_float(e < 4 ? xst[i][e & 3] : xop[i][e & 3]);
+#pragma unroll
+                    for (int h = 0; h < kParts; ++h) {
+                        v4u part;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if (h == kParts - 1) {
+                                part[e] = f32_to_bf16_bits(rest[2 * e]) | (f32_to_bf16_bits(rest[2 * e + 1]) << 16);
+                            } else {
+                                const u32 t0 = __float_as_uint(rest[2 * e]) & 0xffff0000u;
+                                const u32 t1 = __float_as_uint(rest[2 * e + 1]) & 0xffff0000u;
+                                part[e] = (t0 >> 16) | t1;
+                                rest[2 * e] -= __uint_as_float(t0);
+                                rest[2 * e + 1] -= __uint_as_float(t1);
+                            }
+                        }
+                        *(v4u*)(dst + h * M * pitch) = part;
+                    }
+                } else {
+                    *(v4u*)dst = xst[i];
+                }
             }
+        }
+        if constexpr (kRows) {  // zeros past K: whatever weights they meet there add nothing
+            const int tail = blocks * kD * 16 - per_row;
+            for (int m = q; m < MX; m += kQ)
+                for (int c = lane; c < tail; c += 64)
+                    *(v4u*)(w4s_lds + m * pitch + (per_row + c) * 16) = v4u{0u, 0u, 0u, 0u};
         }
     };
     stage_load(0);
@@ -195,13 +240,16 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
     auto place = [&](const int gi) {
         return rotate && (gi | 7) < groups ? (gi & ~7) | ((gi + (gi >> 3)) & 7) : gi;
     };
+    // (kRows: of the strip's first unit -- the unit is clamped at each request)
+    constexpr int kZ = kF32 ? 5 : 3;  // words per record: four scales, four bytes of zero points
+    const int ub = kRows ? 0 : u0;
     auto w_base = [&](const int grp, const int t) {
-        return (const char*)p.w + ((int64_t)(place(grp) * kSW + t) * units + u0) * 1024;
+        return (const char*)p.w + ((int64_t)(place(grp) * kSW + t) * units + ub) * 1024;
     };
     auto z_base = [&](const int grp, const int t) {
-        return (const char*)p.gparams + ((int64_t)(place(grp) * kSW + t) * units + u0) * 48;
+        return (const char*)p.gparams + ((int64_t)(place(grp) * kSW + t) * units + ub) * (16 * kZ);
     };
-    const unsigned lane_w = lane * 16u, lane_z = 12u * g;  // (unsigned: a scalar base + a 32-bit lane offset is one address form)
+    const unsigned lane_w = lane * 16u, lane_z = 4u * kZ * g;  // (unsigned: a scalar base + a 32-bit lane offset is one address form)
     // The weight stream of a wave: unit after unit of its slice, group after group of the workgroup.
     // The cursor (group, unit) is where the next request goes; the ring is refilled in stream order,
     // so a request needs no index, and the stream may run any number of groups ahead of the sums (a
@@ -219,21 +267,21 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
     };
     at_group();
     v4u W[kD][kSW];
-    u32 Z[kGrouped ? kD : 1][kSW][3];
+    u32 Z[kGrouped ? kD : 1][kSW][kZ];
     auto fetch = [&](const int d) {
+        const int at = !kRows ? 0 : u0 + cu < units ? u0 + cu : units - 1;
 #pragma unroll
         for (int t = 0; t < kSW; ++t) {
-            W[d][t] = __builtin_nontemporal_load((const v4u*)(cw[t] + lane_w));
-            cw[t] += 1024;
+            W[d][t] = __builtin_nontemporal_load((const v4u*)(cw[t] + (int64_t)at * 1024 + lane_w));
+            if (!kRows) cw[t] += 1024;
         }
         if constexpr (kGrouped) {
 #pragma unroll
             for (int t = 0; t < kSW; ++t) {
-                const u32* z = (const u32*)(cz[t] + lane_z);
-                Z[d][t][0] = z[0];
-                Z[d][t][1] = z[1];
-                Z[d][t][2] = z[2];
-                cz[t] += 48;
+                const u32* z = (const u32*)(cz[t] + (int64_t)at * (16 * kZ) + lane_z);
+#pragma unroll
+                for (int c = 0; c < kZ; ++c) Z[d][t][c] = z[c];
+                if (!kRows) cz[t] += 16 * kZ;
             }
         }
         if (++cu == U) {
@@ -288,12 +336,15 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
     // (three MFMAs per step with kSW = 2, two with one strip: a strip's own chain has the others between
     // its links, which is enough for the matrix pipe's latency)
     v4f acc[2][kSW], accs[2], tot[kSW];
-    u32 Zk[2][kSW][3];
+    u32 Zk[2][kSW][kZ];
     v4u av[2][kSW][4], xf[2][4];
 
     auto cvt1 = [&](const u32 w, v4u& out) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) out[e] = ((w >> (4 * e)) & 0x000F000Fu) ^ 0x43084308u;
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (kRows) out[e] = ((e ? w >> (4 * e - 3) : w << 3) & 0x00780078u) ^ 0x41C041C0u;
+            else out[e] = ((w >> (4 * e)) & 0x000F000Fu) ^ 0x43084308u;
+        }
     };
     auto read_x = [&](const int b, const int i) {
 #pragma unroll
@@ -306,9 +357,12 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 // (136 + zero) * sum(x) = (zero + 128) * sum(x) + 8 * sum(x); the byte converts in one operation
-                const float sc = (r & 1) ? bf_hi(Zk[a][t][r >> 1]) : bf_lo(Zk[a][t][r >> 1]);
-                const float zu = (float)((Zk[a][t][2] >> (8 * r)) & 0xffu);
-                const float d = __builtin_fmaf(-zu, accs[a][r], acc[a][t][r] - 8.0f * accs[a][r]);
+                const float sc = kF32 ? __uint_as_float(Zk[a][t][r])
+                                      : (r & 1) ? bf_hi(Zk[a][t][r >> 1]) : bf_lo(Zk[a][t][r >> 1]);
+                const float zu = (float)((Zk[a][t][kZ - 1] >> (8 * r)) & 0xffu);
+                // (kRows: (24 + zero) * sum(x), the factor exact)
+                const float d = kRows ? __builtin_fmaf(104.0f - zu, accs[a][r], acc[a][t][r])
+                                      : __builtin_fmaf(-zu, accs[a][r], acc[a][t][r] - 8.0f * accs[a][r]);
                 tot[t][r] = __builtin_fmaf(sc, d, tot[t][r]);
             }
     };
@@ -346,10 +400,11 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
             if (s == 1) {
                 if (kGrouped && fold_prev) fold(b ^ 1);
                 if constexpr (kGrouped && has_next) {
+                    const bool real = !kRows || u0 + (i + 1 < U ? i + 1 : 0) < units;
 #pragma unroll
                     for (int t = 0; t < kSW; ++t)
 #pragma unroll
-                        for (int c = 0; c < 3; ++c) Zk[b ^ 1][t][c] = Z[dn][t][c];
+                        for (int c = 0; c < kZ; ++c) Zk[b ^ 1][t][c] = real ? Z[dn][t][c] : 0u;
                 }
             }
         }
@@ -398,13 +453,14 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
 #pragma unroll
         for (int t = 0; t < kSW; ++t)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) Zk[0][t][c] = Z[0][t][c];
+            for (int c = 0; c < kZ; ++c) Zk[0][t][c] = !kRows || u0 < units ? Z[0][t][c] : 0u;
     }
     __builtin_amdgcn_sched_barrier(0);
     fetch(0);
     __builtin_amdgcn_sched_barrier(0);
 
-    u32 esc[kSW][2], ebi[kSW][2];
+    constexpr int kEW = kRows ? 4 : 2;  // (kRows: a value per word)
+    u32 esc[kSW][kEW], ebi[kSW][kEW];
     // a group's set-up: where the group after it lies, fresh sums, and the epilogue's operands
     // requested now rather than at the end of the group's stream
     auto begin = [&](const int grp, const int nxt_grp) {
@@ -418,6 +474,16 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
 #pragma unroll
         for (int t = 0; t < kSW; ++t) {
             int n = (place(grp) * kSW + t) * 16 + 4 * g;
+            if constexpr (kRows) {  // column by column: rows of any length, and the last columns stand in past N
+                const int64_t row = (int64_t)(j < M ? j : M - 1) * p.bias_stride;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int c = n + r < p.N ? n + r : p.N - 1;
+                    esc[t][r] = kGrouped ? 0u : load_raw<!kF32>(p.scale, c);
+                    ebi[t][r] = load_raw<!kF32>(p.bias ? p.bias : p.x, p.bias ? row + c : 0);
+                }
+                continue;
+            }
             n = n < p.N ? n : p.N - 4;  // N % 16 == 0: a valid stand-in, never stored
             esc[t][0] = esc[t][1] = 0;
             if (!kGrouped) {
@@ -445,18 +511,47 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
             for (int t = 0; t < kSW; ++t)
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr)
-                    tot[t][rr] = acc[0][t][rr] - 136.0f * accs[0][rr];
+                    tot[t][rr] = kRows ? __builtin_fmaf(-24.0f, accs[0][rr], acc[0][t][rr])
+                                       : acc[0][t][rr] - 136.0f * accs[0][rr];
         }
-        float* rbuf = red + (turn & 1) * (kQ * kSW * M * kRedStride);  // rows of x only
-        auto slot = [&](const int qq, const int t) { return rbuf + ((qq * kSW + t) * M + j) * kRedStride + 4 * g; };
-        if (j < M) {
+        const bool one_red = kRows && p.one_red;
+        float* rbuf = red + (one_red ? 0 : turn & 1) * (kQ * kSW * MX * kRedStride);  // rows of x only
+        if (one_red && turn > 0) __syncthreads();  // the turn before has been added up
+        auto slot = [&](const int qq, const int t) { return rbuf + ((qq * kSW + t) * MX + j) * kRedStride + 4 * g; };
+        if (j < MX) {
 #pragma unroll
             for (int t = 0; t < kSW; ++t)
-                if (q != t) *(v4f*)slot(q, t) = tot[t];
+                if (kF32 || q != t) *(v4f*)slot(q, t) = tot[t];  // (kF32: the parts of a row lie in several lanes)
         }
         __syncthreads();
         auto finalize = [&](auto t_c) {
             constexpr int t = decltype(t_c)::value;
+            if constexpr (kRows) {
+                v4f sum = zero4;
+#pragma unroll
+                for (int h = kF32 ? kParts - 1 : 0; h >= 0; --h) {  // the smallest parts first
+                    v4f part = zero4;
+#pragma unroll
+                    for (int qq = 0; qq < kQ; ++qq)
+                        part += !kF32 && qq == t ? tot[t] : *(const v4f*)(slot(qq, t) + h * M * kRedStride);
+                    sum += part;
+                }
+                const int n = (place(grp) * kSW + t) * 16 + 4 * g;
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) {
+                    if (n + rr >= p.N) continue;
+                    float v = kF32 ? sum[rr] : round_bf16(sum[rr]);
+                    if (!kGrouped) {
+                        v = v / raw_to_f32<!kF32>(esc[t][rr]);
+                        if (!kF32) v = round_bf16(v);
+                    }
+                    if (p.bias) v = v + raw_to_f32<!kF32>(ebi[t][rr]);
+                    const int64_t o = (int64_t)j * p.N + n + rr;
+                    if (kF32) ((float*)p.y)[o] = v;
+                    else p.y[o] = (uint16_t)f32_to_bf16_bits(v);
+                }
+                return;
+            }
             v4f sum = t == 0 ? tot[0] : *(const v4f*)slot(0, t);
 #pragma unroll
             for (int qq = 1; qq < kQ; ++qq) {
@@ -545,6 +640,26 @@ __global__ __launch_bounds__(kT) void gemv_w4s_one(W4sParams p) {
     gemv_w4s_body<kSW, kD, kNP, kGrouped, false>(p, blockIdx.x, gridDim.x);
 }
 
+// Any K % 8 == 0, any N, bfloat16 or float32 rows (kParts, above).  Bound by the copy's bytes and a launch's fixed
+// part, as the forms above; the clamped addresses and column-by-column epilogue cost 0.4 ... 1 us against them.  Graph
+// nodes, us, kernel on the stored weights -> this one: float32 8 x 4096 x 14336 grouped 16.5 -> 12.2, 8 x 4096 x 4096
+// 9.5 -> 6.6, 1 x 8192 x 8192 15.3 -> 9.5; bfloat16 16 x 4096 x 14336 19.2 -> 11.0, 1 x 768 x 768 5.8 -> 3.5,
+// 16 x 1600 x 6400 10.2 -> 6.1, 3 x 2048 x 5247 350 -> 5.6 (one output per thread before).  Error against 64 bits
+// (2-norm): float32 5.4e-6 ... 8.3e-6 -> 4.4e-6 ... 5e-6 in two parts, 2.1e-7 -> 1.0e-7 in three; bfloat16 the same.
+template <int kSW, int kD, int kNP, bool kGrouped, int kParts>
+__global__ __launch_bounds__(kT) void gemv_w4s_rows(W4sParams p) {
+    gemv_w4s_body<kSW, kD, kNP, kGrouped, false, false, kParts>(p, blockIdx.x, gridDim.x);
+}
+
+// the same for several kernels against one x (as gemv_w4s)
+template <int kSW, int kD, int kNP, bool kGrouped, int kParts>
+__global__ __launch_bounds__(kT) void gemv_w4s_rows_multi(W4sMulti mp) {
+    const int bx = blockIdx.x;
+    int i = 0;
+    while (i + 1 < mp.count && bx >= mp.first[i + 1]) ++i;
+    gemv_w4s_body<kSW, kD, kNP, kGrouped, false, false, kParts>(mp.p[i], bx - mp.first[i], mp.first[i + 1] - mp.first[i]);
+}
+
 // 9 ... 16 rows of a K too long for LDS: x in two halves (two strips per wave, ring of two, one turn)
 template <int kSW, bool kGrouped>
 __global__ __launch_bounds__(kT) void gemv_w4s_halves(W4sParams p) {
@@ -552,11 +667,12 @@ __global__ __launch_bounds__(kT) void gemv_w4s_halves(W4sParams p) {
 }
 
 // ---- the strip-linear copy ---------------------------------------------------------------
-// One thread per dword of the copy; strips past N (the copy holds an even number of strips) are zero.
+// One thread per dword of the copy; strips past N (the copy holds an even number of strips) are zero, and so are
+// the nibbles past K and N of the last unit and the last strip.
 __global__ __launch_bounds__(256) void w4s_pack(const uint8_t* __restrict__ w, u32* __restrict__ out,
                                                 int64_t K, int64_t N, int64_t strips_padded) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t units = K / 128;
+    const int64_t units = (K + 127) / 128;
     if (idx >= strips_padded * units * 256) return;
     const int s = (int)(idx & 3), lane = (int)((idx >> 2) & 63);
     const int64_t su = idx >> 8, unit = su % units, strip = su / units;
@@ -569,15 +685,16 @@ __global__ __launch_bounds__(256) void w4s_pack(const uint8_t* __restrict__ w, u
         const int64_t k0 = unit * 128 + 32 * s + 8 * g;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const u32 nib = (w[(k0 + e) * row_bytes + (n >> 1)] >> shift) & 0xFu;
+            const u32 nib = k0 + e < K ? (w[(k0 + e) * row_bytes + (n >> 1)] >> shift) & 0xFu : 0u;
             d |= nib << ((e & 1) ? 16 + 4 * (e >> 1) : 4 * (e >> 1));
         }
     }
     out[idx] = d;
 }
 
-// grouped parameters: [strip][unit][c = 4]{scale[4 c .. 4 c + 3] bf16, (zero + 128)[4 c .. 4 c + 3]}
-template <bool kBF16>
+// grouped parameters: [strip][unit][c = 4]{scale[4 c .. 4 c + 3], (zero + 128)[4 c .. 4 c + 3]}; the scales are
+// bfloat16 (kOutF32: float32); kBF16: the type they come in
+template <bool kBF16, bool kOutF32 = false>
 __global__ __launch_bounds__(256) void w4s_pack_params(const void* __restrict__ scale,
                                                        const int8_t* __restrict__ zero,
                                                        uint8_t* __restrict__ out, int64_t units, int64_t N,
@@ -586,24 +703,26 @@ __global__ __launch_bounds__(256) void w4s_pack_params(const void* __restrict__ 
     if (idx >= strips_padded * units * 4) return;
     const int c = (int)(idx & 3);
     const int64_t su = idx >> 2, unit = su % units, strip = su / units;
-    u32 rec[3] = {0, 0, 0x80808080u};
     const int64_t n = strip * 16 + 4 * c;
-    if (n < N) {  // N % 16 == 0: four columns in or out together
-        u32 h[4], z = 0;
+    u32 h[4] = {0, 0, 0, 0}, z = 0x80808080u;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int64_t o = unit * N + n + e;
-            h[e] = kBF16 ? (u32)((const uint16_t*)scale)[o] : f32_to_bf16_bits(((const float*)scale)[o]);
-            z |= ((u32)(uint8_t)(zero[o] ^ 0x80)) << (8 * e);  // zero + 128 as an unsigned byte
-        }
-        rec[0] = h[0] | (h[1] << 16);
-        rec[1] = h[2] | (h[3] << 16);
-        rec[2] = z;
+    for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) break;
+        const int64_t o = unit * N + n + e;
+        if (kOutF32) h[e] = ((const u32*)scale)[o];
+        else h[e] = kBF16 ? (u32)((const uint16_t*)scale)[o] : f32_to_bf16_bits(((const float*)scale)[o]);
+        z ^= ((u32)(uint8_t)zero[o]) << (8 * e);  // zero + 128 as an unsigned byte
     }
-    u32* dst = (u32*)(out + idx * 12);
-    dst[0] = rec[0];
-    dst[1] = rec[1];
-    dst[2] = rec[2];
+    constexpr int kWords = kOutF32 ? 5 : 3;
+    u32* dst = (u32*)out + idx * kWords;
+    if (kOutF32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[e] = h[e];
+    } else {
+        dst[0] = h[0] | (h[1] << 16);
+        dst[1] = h[2] | (h[3] << 16);
+    }
+    dst[kWords - 1] = z;
 }
 
 inline int64_t strips_padded(int64_t N) { return ((N + 15) / 16 + 1) / 2 * 2; }
@@ -686,6 +805,46 @@ W4sPlan w4s_plan(int64_t M, int64_t K, int64_t N, int64_t block_size, bool pre =
     return pl;
 }
 
+// Plan for the general form (kParts): `parts` bfloat16 rows per row of x, `rows` rows of x per launch.  All of K stays
+// in a workgroup also where the strips are fewer than the CUs (one strip of K = 8192 is 64 KiB, which a CU takes in
+// under 2 us).  x has to fit LDS and the registers it is staged in; the rows that do not go into a further launch.
+struct W4sRowsPlan : W4sPlan {
+    int64_t rows;
+    bool one_red;  // turns share one reduction buffer (a barrier more per turn): both do not fit beside x
+};
+
+// shared_groups: strip groups of the whole launch when several kernels share it (0: this kernel alone).
+W4sRowsPlan w4s_rows_plan(int parts, int64_t M, int64_t K, int64_t N, int64_t block_size, int64_t shared_groups = 0) {
+    W4sRowsPlan pl{};
+    if (M < 1 || M > kMaxRows || K < 16 || (K % 8) != 0 || N < 1 || K * N >= (int64_t(1) << 40)) return pl;
+    if (block_size > 0 && block_size != 128) return pl;
+    const bool f32 = parts > 1;
+    const int64_t units = (K + 127) / 128, strips = (N + 15) / 16;
+    pl.sw = strips >= 2 * kResident ? 2 : 1;
+    // (two strips, float32 scales and a ring of four together would spill)
+    pl.d = units >= 4 * 2 * kQ && !(f32 && block_size > 0 && pl.sw == 2) ? 4 : 2;
+    pl.groups = (strips + pl.sw - 1) / pl.sw;
+    pl.resident = kResident;
+    const int64_t turns = ((shared_groups ? shared_groups : pl.groups) + kResident - 1) / kResident;
+    pl.blocks = (pl.groups + turns - 1) / turns;
+    const int64_t blocks = units > kQ * pl.d ? (units + pl.d - 1) / pl.d : kQ;
+    const int64_t pitch = blocks * pl.d * 256 + 16, red = kQ * pl.sw * kRedStride * 4;
+    int64_t rows = kMaxRows / parts < M ? kMaxRows / parts : M;
+    const int64_t most_pieces = (f32 ? 8 : 16) * kT;
+    auto lds = [&](int64_t r) { return (parts * r * pitch + 255) / 256 * 256 + parts * r * red; };
+    while (rows > 0 && (lds(rows) > 160 * 1024 || rows * (K / 8) > most_pieces)) --rows;
+    if (rows < 1) return pl;
+    const int64_t launches = (M + rows - 1) / rows;
+    pl.rows = (M + launches - 1) / launches;
+    pl.lds = (size_t)lds(pl.rows);
+    pl.one_red = turns > 1 && lds(pl.rows) + parts * pl.rows * red > 160 * 1024;
+    if (turns > 1 && !pl.one_red) pl.lds += (size_t)(parts * pl.rows * red);
+    const int64_t pieces = pl.rows * (K / 8);
+    pl.np = pieces <= 2 * kT ? 2 : pieces <= 8 * kT ? 8 : 16;
+    pl.ok = true;
+    return pl;
+}
+
 struct W4sKernels {
     void (*multi)(W4sMulti);
     void (*one)(W4sParams);
@@ -713,6 +872,36 @@ W4sKernels pick_kernel(const W4sPlan& pl, bool grouped) {
     }
     if (pl.d == 4) return grouped ? pick_np<1, 4, true>(pl.np) : pick_np<1, 4, false>(pl.np);
     return grouped ? pick_np<1, 2, true>(pl.np) : pick_np<1, 2, false>(pl.np);
+}
+
+template <int kSW, int kD, int kParts>
+void (*pick_rows_multi_np(const W4sPlan& pl, bool grouped))(W4sMulti) {
+    if (pl.np == 2)
+        return grouped ? gemv_w4s_rows_multi<kSW, kD, 2, true, kParts> : gemv_w4s_rows_multi<kSW, kD, 2, false, kParts>;
+    return grouped ? gemv_w4s_rows_multi<kSW, kD, 8, true, kParts> : gemv_w4s_rows_multi<kSW, kD, 8, false, kParts>;
+}
+
+template <int kParts>
+void (*pick_rows_multi(const W4sPlan& pl, bool grouped))(W4sMulti) {
+    if (pl.sw == 2)
+        return pl.d == 4 ? pick_rows_multi_np<2, 4, kParts>(pl, grouped) : pick_rows_multi_np<2, 2, kParts>(pl, grouped);
+    return pl.d == 4 ? pick_rows_multi_np<1, 4, kParts>(pl, grouped) : pick_rows_multi_np<1, 2, kParts>(pl, grouped);
+}
+
+template <int kSW, int kD, int kParts>
+void (*pick_rows_np(const W4sPlan& pl, bool grouped))(W4sParams) {
+    if (pl.np == 2) return grouped ? gemv_w4s_rows<kSW, kD, 2, true, kParts> : gemv_w4s_rows<kSW, kD, 2, false, kParts>;
+    if constexpr (kParts == 1) {
+        if (pl.np == 16)
+            return grouped ? gemv_w4s_rows<kSW, kD, 16, true, 1> : gemv_w4s_rows<kSW, kD, 16, false, 1>;
+    }
+    return grouped ? gemv_w4s_rows<kSW, kD, 8, true, kParts> : gemv_w4s_rows<kSW, kD, 8, false, kParts>;
+}
+
+template <int kParts>
+void (*pick_rows(const W4sPlan& pl, bool grouped))(W4sParams) {
+    if (pl.sw == 2) return pl.d == 4 ? pick_rows_np<2, 4, kParts>(pl, grouped) : pick_rows_np<2, 2, kParts>(pl, grouped);
+    return pl.d == 4 ? pick_rows_np<1, 4, kParts>(pl, grouped) : pick_rows_np<1, 2, kParts>(pl, grouped);
 }
 
 int fill_params(W4sParams& p, const W4sPlan& pl, const void* x, int64_t M, int64_t K, int64_t N,
@@ -758,6 +947,19 @@ int fill_params(W4sParams& p, const W4sPlan& pl, const void* x, int64_t M, int64
     return K3Q_OK;
 }
 
+// more than 64 KiB of dynamic LDS has to be allowed per kernel, once
+int raise_lds(const void* kernel) {
+    static std::mutex mu;
+    static std::set<const void*> raised;
+    std::lock_guard<std::mutex> lock(mu);
+    if (!raised.count(kernel)) {
+        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+            return K3Q_ERR_LAUNCH;
+        raised.insert(kernel);
+    }
+    return K3Q_OK;
+}
+
 int launch_w4s(const W4sPlan& pl, bool grouped, const W4sMulti& mp, int total_blocks, size_t lds, hipStream_t s,
                bool pre = false) {
     W4sKernels ks = pick_kernel(pl, grouped);
@@ -768,17 +970,8 @@ int launch_w4s(const W4sPlan& pl, bool grouped, const W4sMulti& mp, int total_bl
                             : (grouped ? gemv_w4s_halves<1, true> : gemv_w4s_halves<1, false>);
     }
     const void* kernel = pre ? (const void*)ks.pre : mp.count == 1 ? (const void*)ks.one : (const void*)ks.multi;
-    // more than 64 KiB of dynamic LDS has to be allowed per kernel, once
-    {
-        static std::mutex mu;
-        static std::set<const void*> raised;
-        std::lock_guard<std::mutex> lock(mu);
-        if (!raised.count(kernel)) {
-            if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-                return K3Q_ERR_LAUNCH;
-            raised.insert(kernel);
-        }
-    }
+    const int rc = raise_lds(kernel);
+    if (rc != K3Q_OK) return rc;
     if (pre) ks.pre<<<(unsigned)total_blocks, kT, lds, s>>>(mp);
     else if (mp.count == 1) ks.one<<<(unsigned)total_blocks, kT, lds, s>>>(mp.p[0]);
     else ks.multi<<<(unsigned)total_blocks, kT, lds, s>>>(mp);
@@ -791,8 +984,8 @@ int launch_w4s(const W4sPlan& pl, bool grouped, const W4sMulti& mp, int total_bl
 using namespace k3q;
 
 extern "C" int64_t k3q_w4s_shadow_bytes(int64_t K, int64_t N) {
-    if (K <= 0 || N <= 0 || (K % 128) != 0) return 0;
-    return strips_padded(N) * (K / 128) * 1024;
+    if (K <= 0 || N <= 0 || (K % 8) != 0) return 0;
+    return strips_padded(N) * ((K + 127) / 128) * 1024;
 }
 
 extern "C" int64_t k3q_w4s_params_bytes(int64_t K, int64_t N, int64_t block_size) {
@@ -801,7 +994,7 @@ extern "C" int64_t k3q_w4s_params_bytes(int64_t K, int64_t N, int64_t block_size
 }
 
 extern "C" int k3q_w4s_pack(const int8_t* w_packed, int64_t K, int64_t N, void* shadow, void* stream) {
-    if (K <= 0 || N <= 0 || (K % 128) != 0) return K3Q_ERR_SHAPE;
+    if (K <= 0 || N <= 0 || (K % 8) != 0) return K3Q_ERR_SHAPE;
     if (!w_packed || !shadow) return K3Q_ERR_NULL;
     if (!aligned_to(shadow, 16)) return K3Q_ERR_ALIGN;
     const int64_t dwords = k3q_w4s_shadow_bytes(K, N) / 4;
@@ -825,6 +1018,165 @@ extern "C" int k3q_w4s_pack_params(const void* scale, int scale_dtype, const int
         w4s_pack_params<false><<<grid, 256, 0, (hipStream_t)stream>>>(scale, zero, (uint8_t*)params, K / 128, N,
                                                                        strips_padded(N));
     return launch_status();
+}
+
+extern "C" int64_t k3q_w4s_rows_params_bytes(int64_t K, int64_t N, int64_t block_size, int dtype) {
+    if (K <= 0 || N <= 0 || (K % 8) != 0 || block_size != 128 || (dtype != K3Q_F32 && dtype != K3Q_BF16)) return 0;
+    return strips_padded(N) * ((K + 127) / 128) * (dtype == K3Q_F32 ? 80 : 48);
+}
+
+extern "C" int k3q_w4s_rows_pack_params(const void* scale, int dtype, const int8_t* zero, int64_t K, int64_t N,
+                                        int64_t block_size, void* params, void* stream) {
+    if (dtype != K3Q_F32 && dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
+    if (K <= 0 || N <= 0 || (K % 8) != 0 || block_size != 128) return K3Q_ERR_SHAPE;
+    if (!scale || !zero || !params) return K3Q_ERR_NULL;
+    if (!aligned_to(params, 4) || !aligned_to(scale, dtype == K3Q_F32 ? 4 : 2)) return K3Q_ERR_ALIGN;
+    const int64_t units = (K + 127) / 128, padded = strips_padded(N);
+    const unsigned grid = (unsigned)((padded * units * 4 + 255) / 256);
+    if (dtype == K3Q_BF16)
+        w4s_pack_params<true><<<grid, 256, 0, (hipStream_t)stream>>>(scale, zero, (uint8_t*)params, units, N, padded);
+    else
+        w4s_pack_params<false, true><<<grid, 256, 0, (hipStream_t)stream>>>(scale, zero, (uint8_t*)params, units, N,
+                                                                            padded);
+    return launch_status();
+}
+
+namespace {
+// Parts of a float32 row: two (to 2^-17) where the kernel on the stored weights splits x in two as well, three
+// (exact) where that kernel has float32 products (N % 8, K % 16).
+int parts_of(int x_dtype, int64_t K, int64_t N) {
+    return x_dtype != K3Q_F32 ? 1 : (N % 8) == 0 && (K % 16) == 0 ? 2 : 3;
+}
+}  // namespace
+
+extern "C" int k3q_gemv_w4s_rows_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size) {
+    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return 0;
+    const W4sRowsPlan pl = w4s_rows_plan(parts_of(x_dtype, K, N), M, K, N, block_size);
+    return pl.ok ? (int)((M + pl.rows - 1) / pl.rows) : 0;
+}
+
+namespace {
+int check_rows(const void* x, const void* shadow, const void* scale, const void* gparams, bool grouped, const void* bias,
+               const void* y, size_t el) {
+    if (!x || !shadow || !y || (grouped ? !gparams : !scale)) return K3Q_ERR_NULL;
+    if (!aligned_to(x, 16) || !aligned_to(shadow, 16) || !aligned_to(y, el) || (scale && !aligned_to(scale, el)) ||
+        (gparams && !aligned_to(gparams, 4)) || (bias && !aligned_to(bias, el)))
+        return K3Q_ERR_ALIGN;
+    return K3Q_OK;
+}
+
+W4sParams rows_params(const W4sRowsPlan& pl, const void* x, int64_t M, int64_t K, int64_t N, const void* shadow,
+                      const void* scale, const void* gparams, const void* bias, int64_t bias_stride, void* y) {
+    W4sParams p{};
+    p.x = (const uint16_t*)x;
+    p.w = (const v4u*)shadow;
+    p.scale = (const uint16_t*)scale;
+    p.gparams = (const uint8_t*)gparams;
+    p.bias = (const uint16_t*)bias;
+    p.bias_stride = bias ? bias_stride : 0;
+    p.y = (uint16_t*)y;
+    p.M = (int)M;
+    p.K = (int)K;
+    p.N = (int)N;
+    p.units = (int)((K + 127) / 128);
+    p.one_red = pl.one_red ? 1 : 0;
+    const uint64_t per_row = (uint64_t)K / 8;
+    p.row_magic = (int)(uint32_t)((((uint64_t)1 << 32) + per_row - 1) / per_row);
+    return p;
+}
+}  // namespace
+
+// Kernels against one x (up to kMaxProblems per launch) in one launch where their plans agree and the rows fit one
+// launch; one after the other with the same bits where not.
+extern "C" int k3q_gemv_w4s_rows_multi(const void* x, int x_dtype, int64_t M, int64_t K, int count,
+                                       const k3q_gemv_w4s_problem* problems, int64_t block_size, void* stream) {
+    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
+    if (count < 0 || M < 0 || K <= 0) return K3Q_ERR_SHAPE;
+    if (count == 0 || M == 0) return K3Q_OK;
+    if (!problems) return K3Q_ERR_NULL;
+    const bool grouped = block_size > 0;
+    const size_t el = x_dtype == K3Q_F32 ? 4 : 2;
+    for (int i = 0; i < count; ++i) {
+        const k3q_gemv_w4s_problem& q = problems[i];
+        if (q.N <= 0 || !w4s_rows_plan(parts_of(x_dtype, K, q.N), M, K, q.N, block_size).ok) return K3Q_ERR_SHAPE;
+        const int rc = check_rows(x, q.shadow, q.scale, q.gparams, grouped, q.bias, q.y, el);
+        if (rc != K3Q_OK) return rc;
+    }
+    auto plan_of = [&](int i, int64_t shared) {
+        return w4s_rows_plan(parts_of(x_dtype, K, problems[i].N), M, K, problems[i].N, block_size, shared);
+    };
+    for (int at = 0; at < count;) {
+        const int parts = parts_of(x_dtype, K, problems[at].N);
+        const W4sRowsPlan first = plan_of(at, 0);
+        int n = 1;
+        int64_t total = first.groups;
+        if (first.rows >= M && first.np <= 8)
+            for (; at + n < count && n < kMaxProblems; ++n) {
+                const W4sRowsPlan pl = plan_of(at + n, 0);
+                if (parts_of(x_dtype, K, problems[at + n].N) != parts || pl.sw != first.sw || pl.d != first.d ||
+                    pl.np != first.np || pl.rows < M)
+                    break;
+                total += pl.groups;
+            }
+        if (n == 1) {
+            const k3q_gemv_w4s_problem& q = problems[at];
+            const int rc = k3q_gemv_w4s_rows(x, x_dtype, M, K, q.N, q.shadow, q.scale, q.gparams, block_size, q.bias, 0,
+                                             q.y, stream);
+            if (rc != K3Q_OK) return rc;
+            ++at;
+            continue;
+        }
+        W4sMulti mp{};
+        int next_block = 0;
+        W4sRowsPlan pl{};
+        for (int i = 0; i < n; ++i) {
+            const k3q_gemv_w4s_problem& q = problems[at + i];
+            pl = plan_of(at + i, total);  // (lds and one_red depend on the launch as a whole: alike for all)
+            mp.p[i] = rows_params(pl, x, M, K, q.N, q.shadow, q.scale, q.gparams, q.bias, 0, q.y);
+            mp.first[i] = next_block;
+            next_block += (int)pl.blocks;
+        }
+        mp.first[n] = next_block;
+        mp.count = n;
+        void (*kernel)(W4sMulti) = parts == 1   ? pick_rows_multi<1>(pl, grouped)
+                                   : parts == 2 ? pick_rows_multi<2>(pl, grouped)
+                                                : pick_rows_multi<3>(pl, grouped);
+        int rc = raise_lds((const void*)kernel);
+        if (rc != K3Q_OK) return rc;
+        kernel<<<(unsigned)next_block, kT, pl.lds, (hipStream_t)stream>>>(mp);
+        if ((rc = launch_status()) != K3Q_OK) return rc;
+        at += n;
+    }
+    return K3Q_OK;
+}
+
+extern "C" int k3q_gemv_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                                 const void* scale, const void* gparams, int64_t block_size, const void* bias,
+                                 int64_t bias_stride, void* y, void* stream) {
+    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
+    if (M < 0 || K <= 0 || N <= 0) return K3Q_ERR_SHAPE;
+    if (M == 0) return K3Q_OK;
+    if (bias_stride != 0 && bias_stride != N) return K3Q_ERR_SHAPE;
+    const bool grouped = block_size > 0;
+    const int parts = parts_of(x_dtype, K, N);
+    const W4sRowsPlan pl = w4s_rows_plan(parts, M, K, N, block_size);
+    if (!pl.ok) return K3Q_ERR_SHAPE;
+    const size_t el = parts > 1 ? 4 : 2;
+    int rc = check_rows(x, shadow, scale, gparams, grouped, bias, y, el);
+    if (rc != K3Q_OK) return rc;
+    void (*kernel)(W4sParams) = parts == 1   ? pick_rows<1>(pl, grouped)
+                                : parts == 2 ? pick_rows<2>(pl, grouped)
+                                             : pick_rows<3>(pl, grouped);
+    rc = raise_lds((const void*)kernel);
+    for (int64_t m0 = 0; m0 < M && rc == K3Q_OK; m0 += pl.rows) {
+        const int64_t stride = bias ? bias_stride : 0;
+        const W4sParams p = rows_params(pl, (const char*)x + m0 * K * el, M - m0 < pl.rows ? M - m0 : pl.rows, K, N, shadow,
+                                        scale, gparams, bias ? (const char*)bias + m0 * stride * el : nullptr, stride,
+                                        (char*)y + m0 * N * el);
+        kernel<<<(unsigned)pl.blocks, kT, pl.lds, (hipStream_t)stream>>>(p);
+        rc = launch_status();
+    }
+    return rc;
 }
 
 extern "C" int k3q_gemv_w4s_supported(int64_t M, int64_t K, int64_t N, int64_t block_size) {

@@ -104,6 +104,38 @@ def kmajor_rows(rows, units, input_dim=0):
     return low <= rows <= KMAJOR_MAX_ROWS
 
 
+def int4_strip_rows_route(x2, units, block_size):
+    """Whether an int4 call of these rows goes to `ops.int4_matmul_strip_rows`: what the strip kernel proper
+    (`ops.int4_strip_supported`) does not take of up to 16 rows -- float32 rows, narrow, short or ragged kernels.
+    A launch costs what one of the kernel on the stored weights costs, which takes 8 float32 or 16 bfloat16 rows
+    (us, 1 / 8 / 16 rows, stored against strip: K=4096, N=14336 float32 15.5 / 16.5 / 31.8 against 10.9 / 12.1 / 33.9
+    in three launches; K=N=4096 8.2 / 9.5 / 18.6 against 4.7 / 6.6 / 12.3; bfloat16 K=1600, N=6400 7.1 / 8.4 / 10.2
+    against 5.4 / 5.9 / 6.1; K=11008, N=4096 at 8 rows 16.1 against 16.5 in two launches).  Where N % 8 or K % 16
+    leave only the kernel of one output per thread (N = 5247: 220 ... 490 us) every shape goes here."""
+    if not (x2.is_cuda and x2.dtype in (torch.float32, torch.bfloat16) and 0 < x2.shape[0] <= kops.STRIP_MAX_ROWS):
+        return False
+    rows, input_dim = x2.shape
+    launches = kops.int4_strip_rows_launches(x2.dtype, rows, input_dim, units, block_size)
+    if units % 8 or input_dim % 16:
+        return launches > 0
+    return 0 < launches <= (-(-rows // 8) if x2.dtype == torch.float32 else 1)
+
+
+def strip_rows_params(layer, dtype, input_dim, units, block_size):
+    """The grouped parameters of `ops.int4_matmul_strip_rows` in `dtype`: made on first use, rebuilt in place
+    when a variable they come from is assigned (a captured graph holds their address)."""
+    scale, zero = layer.kernel_scale, layer.kernel_zero
+    stamp = (id(scale), scale.version, id(zero), zero.version, dtype)
+    hit = layer._cache.get("w4s_rows_params")
+    if hit is None or hit[0] != stamp:
+        value = kops.int4_strip_rows_params(as_tensor(scale).to(dtype), as_tensor(zero), input_dim, units, block_size)
+        if hit is not None and hit[2].shape == value.shape and hit[2].device == value.device:
+            hit[2].copy_(value)
+            value = hit[2]
+        hit = layer._cache["w4s_rows_params"] = (stamp, None, value)
+    return hit[2]
+
+
 def int8_strip_route(quantizer, x2, units, strict=False):
     """Whether an int8 call of these rows goes to `ops.int8_dense_strip`: rows on the device, few
     enough, a plain abs-max quantizer (whatever its range and epsilon), a shape the kernel takes.
@@ -374,6 +406,16 @@ class Dense(Layer):
             spec["kernel_scale"] = self._read_cached("kernel_scale", self.kernel_scale)
         return spec
 
+    def _strip_rows_operands(self, inputs, grouped, block_size):
+        """The operands of `ops.int4_matmul_strip_rows` for these inputs."""
+        units = self._orig_output_dim
+        spec = dict(units=units, shadow=self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)))
+        if grouped:
+            spec["gparams"] = strip_rows_params(self, inputs.dtype, inputs.shape[-1], units, block_size)
+        else:
+            spec["kernel_scale"] = self._read_cached("kernel_scale", self.kernel_scale)
+        return spec
+
     def _tile_operand(self, input_dim):
         """The derived copy of the int8 kernel that the tile GEMM reads, as a keyword of
         `ops.int8_matmul`: the decode kernel's strip-linear copy where the tile kernel can take it
@@ -481,6 +523,10 @@ class Dense(Layer):
                 inputs, strip["shadow"], self._orig_output_dim, kernel_scale=strip.get("kernel_scale"),
                 gparams=strip.get("gparams"), block_size=block_size if grouped else None,
                 bias=None if per_row else bias, addend=bias if per_row else None)
+        elif int4_strip_rows_route(inputs.reshape(rows, inputs.shape[-1]), self._orig_output_dim,
+                                   block_size if grouped else None):
+            y = kops.int4_matmul_strip_rows(inputs, block_size=block_size if grouped else None, bias=self._call_bias(),
+                                            **self._strip_rows_operands(inputs, grouped, block_size))
         elif (inputs.dtype == torch.bfloat16 and kmajor_rows(rows, self._orig_output_dim, inputs.shape[-1])
                 and kops.int4_kmajor_supported(rows, inputs.shape[-1], self._orig_output_dim,
                                                block_size if grouped else None)):
@@ -575,10 +621,13 @@ class Dense(Layer):
         x2 = inputs.reshape(-1, inputs.shape[-1])
         strip = (self._strip_operands(x2.shape[0], x2.shape[1], self._orig_output_dim, grouped, block_size)
                  if x2.dtype == torch.bfloat16 else None)
+        rows = None
         if strip is not None:
             strip["bias"] = self._call_bias()
+        elif int4_strip_rows_route(x2, self._orig_output_dim, block_size if grouped else None):
+            rows = dict(self._strip_rows_operands(x2, grouped, block_size), bias=self._call_bias())
         return dict(
-            x2=x2, block_size=block_size if grouped else None, strip=strip,
+            x2=x2, block_size=block_size if grouped else None, strip=strip, rows=rows,
             kernel=dict(kernel_packed=as_tensor(self._kernel),
                         kernel_scale=self._read_cached("kernel_scale", self.kernel_scale),
                         units=self._orig_output_dim,

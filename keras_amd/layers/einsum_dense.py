@@ -556,6 +556,19 @@ class EinsumDense(Layer):
                                                 lambda t: t.to(cd).reshape(-1).contiguous())
         return spec
 
+    def _strip_rows_operands(self, x2, grouped, block_size):
+        """As Dense._strip_rows_operands."""
+        from keras_amd.layers.dense import strip_rows_params
+
+        units = self._int4_unpacked_column_size
+        spec = dict(units=units, shadow=self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)))
+        if grouped:
+            spec["gparams"] = strip_rows_params(self, x2.dtype, x2.shape[1], units, block_size)
+        else:
+            spec["kernel_scale"] = self._cached("kernel_scale", self.kernel_scale,
+                                                lambda t: t.to(x2.dtype).reshape(-1).contiguous())
+        return spec
+
     def _input_rows(self, inputs, gv):
         x = inputs if gv.in_is_view else inputs.permute(gv.in_perm)
         k = 1
@@ -802,7 +815,7 @@ class EinsumDense(Layer):
                                           lambda t: t.to(cd).reshape(-1).contiguous()),
                 bias=bias, out_dtype=cd, exact_epilogue=True)
             return self._finish(y2, free_shape, gv, fused)
-        from keras_amd.layers.dense import kmajor_rows
+        from keras_amd.layers.dense import int4_strip_rows_route, kmajor_rows
 
         units = self._int4_unpacked_column_size
         strip = (self._strip_operands(x2.shape[0], x2.shape[1], units, grouped, block_size)
@@ -814,6 +827,10 @@ class EinsumDense(Layer):
                 x2, strip["shadow"], units, kernel_scale=strip.get("kernel_scale"),
                 gparams=strip.get("gparams"), block_size=block_size if grouped else None,
                 bias=None if per_row else bias, addend=bias if per_row else None)
+            return self._finish(y2, free_shape, gv, fused)
+        if x2.dtype == cd and int4_strip_rows_route(x2, units, block_size if grouped else None):
+            y2 = kops.int4_matmul_strip_rows(x2, block_size=block_size if grouped else None, bias=bias,
+                                             **self._strip_rows_operands(x2, grouped, block_size))
             return self._finish(y2, free_shape, gv, fused)
         if (x2.dtype == torch.bfloat16 and kmajor_rows(x2.shape[0], units, x2.shape[1])
                 and kops.int4_kmajor_supported(x2.shape[0], x2.shape[1], units,
@@ -890,10 +907,16 @@ class EinsumDense(Layer):
         bias, fused = self._fusable_bias(gv, self._int4_unpacked_column_size)
         strip = (self._strip_operands(x2.shape[0], x2.shape[1], self._int4_unpacked_column_size, grouped,
                                       block_size) if x2.dtype == torch.bfloat16 else None)
+        rows = None
         if strip is not None:
             strip["bias"] = bias
+        elif x2.dtype == cd:
+            from keras_amd.layers.dense import int4_strip_rows_route
+
+            if int4_strip_rows_route(x2, self._int4_unpacked_column_size, block_size if grouped else None):
+                rows = dict(self._strip_rows_operands(x2, grouped, block_size), bias=bias)
         return dict(
-            x2=x2, block_size=block_size if grouped else None, strip=strip,
+            x2=x2, block_size=block_size if grouped else None, strip=strip, rows=rows,
             kernel=dict(kernel_packed=as_tensor(self._kernel),
                         kernel_scale=self._cached("kernel_scale", self.kernel_scale,
                                                   lambda t: t.to(cd).contiguous()),

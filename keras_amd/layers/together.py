@@ -167,6 +167,12 @@ def _call_together(layers, inputs, input_op=None):
         # every kernel has its strip-linear copy for these rows: one launch, no scratch
         outs = kops.int4_matmul_strip_multi(x2, [s["strip"] for s in specs], block_size=specs[0]["block_size"],
                                             input_op=input_op)
+    elif all(s.get("rows") is not None and (s["rows"]["bias"] is None or s["rows"]["bias"].numel() == s["rows"]["units"])
+             for s in specs):
+        # the general form of the same kernel takes them all
+        outs = kops.int4_matmul_strip_rows_multi(x2, [s["rows"] for s in specs], block_size=specs[0]["block_size"])
+    elif any(s.get("strip") is not None or s.get("rows") is not None for s in specs):
+        return [layer(x) for layer in layers]  # (some on their strip copies: each takes its own route)
     else:
         outs = kops.int4_matmul_multi(x2, [s["kernel"] for s in specs], block_size=specs[0]["block_size"])
     return [s["finish"](y) for s, y in zip(specs, outs)]

@@ -220,7 +220,7 @@ def int4_strip_copy(kernel_packed, units):
     lib = _lib.load()
     nbytes = lib.k3q_w4s_shadow_bytes(K, N)
     if nbytes <= 0:
-        raise ValueError("the strip-linear copy needs K % 128 == 0")
+        raise ValueError("the strip-linear copy needs K % 8 == 0")
     kp = kernel_packed if kernel_packed.is_contiguous() else kernel_packed.contiguous()
     out = torch.empty(nbytes, dtype=torch.uint8, device=kp.device)
     _lib.check(lib.k3q_w4s_pack(_lib.ptr(kp), K, N, _lib.ptr(out), _lib.stream_ptr(kp.device)), "k3q_w4s_pack")
@@ -292,6 +292,113 @@ def int4_matmul_strip(x, shadow, units, kernel_scale=None, gparams=None, block_s
                           _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_gemv_w4s")
     return y.reshape(*lead, N)
+
+
+def int4_strip_rows_launches(dtype, M, K, N, block_size=None):
+    """How many launches `int4_matmul_strip_rows` needs for M rows of `dtype`; 0: it does not take them."""
+    bs = int(block_size) if block_size is not None and block_size > 0 else -1
+    return _lib.load().k3q_gemv_w4s_rows_launches(_lib.dtype_code(dtype), int(M), int(K), int(N), bs)
+
+
+def int4_strip_rows_params(kernel_scale, kernel_zero, K, units, block_size):
+    """As `int4_strip_params`, for `int4_matmul_strip_rows`: scales in their own dtype, any K % 8, any N."""
+    _lib.require_device(kernel_scale, kernel_zero)
+    lib = _lib.load()
+    K, N, code = int(K), int(units), _lib.dtype_code(kernel_scale.dtype)
+    nbytes = lib.k3q_w4s_rows_params_bytes(K, N, int(block_size), code)
+    if nbytes <= 0:
+        raise ValueError("strip parameters: groups of 128 and K % 8 == 0 only")
+    sc = kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous()
+    zp = kernel_zero if kernel_zero.is_contiguous() else kernel_zero.contiguous()
+    shape = ((K + 127) // 128, N)
+    if tuple(sc.shape) != shape or tuple(zp.shape) != shape or zp.dtype != torch.int8:
+        raise ValueError("scale / zero must be [ceil(K / 128), N], zero int8")
+    out = torch.empty(nbytes, dtype=torch.uint8, device=sc.device)
+    rc = lib.k3q_w4s_rows_pack_params(_lib.ptr(sc), code, _lib.ptr(zp), K, N, int(block_size), _lib.ptr(out),
+                                      _lib.stream_ptr(sc.device))
+    _lib.check(rc, "k3q_w4s_rows_pack_params")
+    return out
+
+
+def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, block_size=None, bias=None):
+    """`x[..., K] . W4[K, N]` for up to 16 float32 or bfloat16 rows, any K % 8 and any N, from
+    `int4_strip_copy(kernel)`.  Per-channel: `kernel_scale` [N] in x's dtype; grouped (block 128): `gparams` from
+    `int4_strip_rows_params`.  `bias` [N], or [M, N]: a row per row of x.
+    Reference: keras/src/layers/core/dense.py:988-1095."""
+    _lib.require_device(x, shadow, kernel_scale, gparams, bias)
+    lib = _lib.load()
+    code = _lib.dtype_code(x.dtype)
+    grouped = block_size is not None and block_size > 0
+    bs = int(block_size) if grouped else -1
+    K, N = x.shape[-1], int(units)
+    lead = x.shape[:-1]
+    x2 = x.reshape(-1, K)
+    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    if x2.data_ptr() % 16:  # a view into a larger buffer
+        x2 = x2.clone()
+    M = x2.shape[0]
+    if shadow.numel() != lib.k3q_w4s_shadow_bytes(K, N):
+        raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
+    _check_bias_size(bias, M, N)
+    if bias is not None and bias.dtype != x.dtype:
+        raise TypeError("bias must be read in the input's dtype")
+    stride = N if bias is not None and M > 1 and bias.numel() == M * N else 0
+    b = bias if bias is None or bias.is_contiguous() else bias.contiguous()
+    if grouped:
+        if gparams is None or gparams.numel() != lib.k3q_w4s_rows_params_bytes(K, N, bs, code):
+            raise ValueError("grouped int4 needs the strip parameters of this kernel")
+    elif kernel_scale is None or kernel_scale.dtype != x.dtype or kernel_scale.numel() != N:
+        raise ValueError("per-channel int4 needs scales [N] in the input's dtype")
+    ks = None if grouped else (kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous())
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    rc = lib.k3q_gemv_w4s_rows(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
+                               _lib.ptr(gparams) if grouped else None, bs, _lib.ptr(b), stride, _lib.ptr(y),
+                               _lib.stream_ptr(x.device))
+    _lib.check(rc, "k3q_gemv_w4s_rows")
+    return y.reshape(*lead, N)
+
+
+def int4_matmul_strip_rows_multi(x, kernels, block_size=None):
+    """`[int4_matmul_strip_rows(x, **k) for k in kernels]` (dicts of its arguments; biases [N]) in one launch where
+    the kernels' plans agree: the same bits."""
+    code = _lib.dtype_code(x.dtype)
+    grouped = block_size is not None and block_size > 0
+    bs = int(block_size) if grouped else -1
+    K = x.shape[-1]
+    lead = x.shape[:-1]
+    x2 = x.reshape(-1, K)
+    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    if x2.data_ptr() % 16:
+        x2 = x2.clone()
+    M = x2.shape[0]
+    lib = _lib.load()
+    problems = (_lib.GemvW4sProblem * len(kernels))()
+    outs, keep = [], []
+    for i, k in enumerate(kernels):
+        N, shadow, bias = int(k["units"]), k["shadow"], k.get("bias")
+        scale, gparams = k.get("kernel_scale"), k.get("gparams")
+        _lib.require_device(x, shadow, scale, gparams, bias)
+        if shadow.numel() != lib.k3q_w4s_shadow_bytes(K, N):
+            raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
+        if grouped:
+            if gparams is None or gparams.numel() != lib.k3q_w4s_rows_params_bytes(K, N, bs, code):
+                raise ValueError("grouped int4 needs the strip parameters of this kernel")
+        elif scale is None or scale.dtype != x.dtype or scale.numel() != N:
+            raise ValueError("per-channel int4 needs scales [N] in the input's dtype")
+        if bias is not None and (bias.dtype != x.dtype or bias.numel() != N):
+            raise ValueError("bias must hold N values of the input's dtype")
+        scale = scale if grouped or scale.is_contiguous() else scale.contiguous()
+        bias = bias if bias is None or bias.is_contiguous() else bias.contiguous()
+        y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        keep.append((scale, bias))
+        outs.append(y)
+        problems[i] = _lib.GemvW4sProblem(
+            N, shadow.data_ptr(), None if grouped else scale.data_ptr(), gparams.data_ptr() if grouped else None,
+            bias.data_ptr() if bias is not None else None, y.data_ptr())
+    rc = lib.k3q_gemv_w4s_rows_multi(_lib.ptr(x2), code, M, K, len(kernels), ctypes.byref(problems), bs,
+                                     _lib.stream_ptr(x.device))
+    _lib.check(rc, "k3q_gemv_w4s_rows_multi")
+    return [y.reshape(*lead, y.shape[1]) for y in outs]
 
 
 def int4_matmul_strip_multi(x, kernels, block_size=None, input_op=None, bias_rows=False):
