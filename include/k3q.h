@@ -406,6 +406,14 @@ int k3q_gemv_w4s_pre(const void* x, int x_dtype, int64_t M, int64_t K, const k3q
  * Replaces what k3q_gemv_w4 replaces (keras/src/layers/core/dense.py:988-1095).
  */
 int k3q_w4_kmajor_pack(const int8_t* w_packed, int64_t K, int64_t N, int32_t* w_kmajor, void* stream);
+/* k3q_gemm_w4_rows: the tile kernel on k3q_w4s_pack's copy for any M, any K % 8 == 0 from 16 on, any N, bfloat16 or
+ * float32 x (scales, bias and y in the same type; a float32 row travels as two or three bfloat16 rows that add
+ * up to it).  Grouped (block_size 128): scale and zero are [ceil(K / 128), Np] with Np = N rounded up to 32; per-channel
+ * (block_size <= 0): scale [N].  bias [N], or [M, N] with bias_stride N.  workspace: aligned to 256. */
+int64_t k3q_gemm_w4_rows_workspace_bytes(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size);
+int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* w_strip,
+                     const void* scale, const void* zero, int64_t block_size, const void* bias,
+                     int64_t bias_stride, void* y, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t k3q_gemm_w4_kmajor_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t block_size);
 int k3q_gemm_w4_kmajor(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N,
                        const void* w_kmajor, const void* scale, const void* zero, int64_t block_size,

@@ -106,6 +106,9 @@ SIGNATURES = {
         _int,
         [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr],
     ),
+    "k3q_gemm_w4_rows_workspace_bytes": (_i64, [_int, _i64, _i64, _i64, _i64]),
+    "k3q_gemm_w4_rows": (
+        _int, [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _ptr]),
     "k3q_w4s_rows_params_bytes": (_i64, [_i64, _i64, _i64, _int]),
     "k3q_w4s_rows_pack_params": (_int, [_ptr, _int, _ptr, _i64, _i64, _i64, _ptr, _ptr]),
     "k3q_gemv_w4s_rows_launches": (_int, [_int, _i64, _i64, _i64, _i64]),

@@ -1154,14 +1154,16 @@ bool try_gemv_w4_multi(const void* x, int x_dtype, int64_t M, int64_t K, int cou
 // kernel does: tot += scale * (acc - (136 + zero) * sum_k x).
 constexpr int kKmBM = 128, kKmBN = 256, kKmStage = 64;  // tile; values of K per stage
 constexpr int kKmThreads = 512;                        // 8 waves: 2 (M) x 4 (N), 64 x 64 each
-constexpr u32 kKmNibbles = 0x000F000Fu, kKmFlip = 0x00080008u, kKmExp = 0x43004300u;
+// bfloat16 pair (24 + w, 24 + w'): the nibbles in mantissa bits 3 ... 6 of 16.0, their sign bits flipped.  (In bits
+// 0 ... 3 of 128.0, 136 + w, they cost the same and leave an offset almost six times as large to cancel.)
+constexpr u32 kKmNibbles = 0x00780078u, kKmBase = 0x41C041C0u;
 
 __device__ __forceinline__ int km_swz(int row) { return (row & 6) | ((row ^ (row >> 3)) & 1); }
 
 struct KmParams {
     const uint16_t* x;      // [M, K] bf16
     const uint8_t* shadow;  // [N, K/2]
-    const void* scale;      // bf16 [G, N] (grouped) or unused
+    const void* scale;      // bf16 [G, N] (grouped; kernels built with kF32S: float32) or unused
     const int8_t* zero;     // [G, N] (grouped)
     const v2u* sx;          // [K / gsize, M] sums of x over each group of K, as three bfloat16 parts
     float* part;            // [KS, M, N]
@@ -1201,6 +1203,86 @@ __global__ __launch_bounds__(256) void km_group_sums(const uint16_t* __restrict_
     }
 }
 
+// The rows of x for shapes the tile kernel does not take as they lie: bfloat16 rows of Kp = ceil(K / 128) 128 values,
+// zero past K, and their sums per group of 128 as above.  kParts 2 or 3: float32 rows, each as that many bfloat16
+// rows that add up to it (top 16 bits, top 16 bits of the rest, ...; the last one rounded), part h of row m being row
+// h M + m; the tile kernel and its partials then know nothing of it, the second pass adds a row's parts.
+// One wave per (group, row), a lane two neighbouring values.
+template <int kParts>
+__global__ __launch_bounds__(256) void km_prepare_rows(const void* __restrict__ x, u32* __restrict__ xp,
+                                                       v2u* __restrict__ sx, int64_t M, int64_t K, int64_t Kp) {
+    const int lane = threadIdx.x & 63;
+    const int64_t m = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+    const int64_t g = blockIdx.x, k = g * 128 + lane * 2;  // (K is even: both values are inside or outside)
+    if (m >= M) return;
+    float v[2] = {0.f, 0.f};
+    if (k < K) {
+        if (kParts == 1) {
+            const u32 d = *(const u32*)((const uint16_t*)x + m * K + k);
+            v[0] = bf16_bits_to_f32(d & 0xffffu);
+            v[1] = bf16_bits_to_f32(d >> 16);
+        } else {
+            const v2u d = *(const v2u*)((const float*)x + m * K + k);
+            v[0] = __uint_as_float(d[0]);
+            v[1] = __uint_as_float(d[1]);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < kParts; ++h) {
+        u32 b[2];
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            b[e] = h == kParts - 1 ? f32_to_bf16_bits(v[e]) : __float_as_uint(v[e]) >> 16;
+            const float part = bf16_bits_to_f32(b[e]);
+            v[e] -= part;
+            sum += part;
+        }
+        const int64_t row = h * M + m;
+        xp[(row * Kp + k) >> 1] = b[0] | (b[1] << 16);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        if (lane == 0) {
+            const u32 hi = f32_to_bf16_bits(sum);
+            const float r1 = sum - bf16_bits_to_f32(hi);
+            const u32 lo = f32_to_bf16_bits(r1);
+            v2u o;
+            o[0] = hi | (lo << 16);
+            o[1] = f32_to_bf16_bits(r1 - bf16_bits_to_f32(lo));
+            sx[g * (kParts * M) + row] = o;
+        }
+    }
+}
+
+// Second pass of the same: y[m][n] from part[split][part of the row][m][Np], the smallest parts first, every part's
+// splits in order; then scale (per-channel) and bias.
+template <bool kBF16, bool kGrouped, int kParts>
+__global__ __launch_bounds__(256) void km_finish(const float* __restrict__ part, const void* __restrict__ scale,
+                                                 const void* __restrict__ bias, void* __restrict__ y, int64_t M,
+                                                 int64_t N, int64_t Np, int64_t bias_stride, int splits) {
+    const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4, m = blockIdx.y;
+    if (n >= N) return;
+    v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int h = kParts - 1; h >= 0; --h) {
+        v4f t = *(const v4f*)(part + (h * M + m) * Np + n);
+        for (int s = 1; s < splits; ++s) t += *(const v4f*)(part + (((int64_t)s * kParts + h) * M + m) * Np + n);
+        sum += t;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) break;
+        float v = kBF16 ? round_bf16(sum[e]) : sum[e];
+        if (!kGrouped) {
+            v = v / load_t<kBF16>(scale, n + e);
+            if (kBF16) v = round_bf16(v);
+        }
+        if (bias) v = v + load_t<kBF16>(bias, m * bias_stride + n + e);
+        if (kBF16) ((uint16_t*)y)[m * N + n + e] = (uint16_t)f32_to_bf16_bits(v);
+        else ((float*)y)[m * N + n + e] = v;
+    }
+}
+
 // Everything the loop consumes arrives by LDS-DMA (global_load_lds), nothing through
 // registers: the compiler then places no waits of its own in the loop (a register load there
 // made it wait for every outstanding operation at each use, which serialised the pipeline:
@@ -1218,9 +1300,13 @@ constexpr int kKmParScale = 0, kKmParZero = 512, kKmParSx = 768, kKmParSpare = 1
 // kNB: blocks of 32 kernel rows per wave: 2 (tiles of 128 x 256) or 1 (128 x 128, for kernels so
 // narrow that wide tiles leave CUs idle even at eight splits).
 // kWM: waves along M: 2 (tiles of 128 rows) or 1 (64 rows, eight waves side by side, kNB = 1).
-template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB>
+// kF32S: float32 scales (twice the bytes: tiles of 128 x 128 or 64 x 256 only, whose parameters still fit).
+template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB, bool kF32S = false>
 __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
     constexpr int kWaveN = 32 * kNB, kBN = kWaveN * (8 / kWM), kBM = 64 * kWM;
+    static_assert(!kF32S || (kGrouped && kBN * kBM <= 128 * 128), "parameters of a stage");
+    // where a stage's parameters lie (kF32S: scales, then zero points, then the sums of x)
+    constexpr int kParZero = kF32S ? kBN * 4 : kKmParZero, kParSx = kF32S ? kBN * 4 + 256 : kKmParSx;
     extern __shared__ char km_lds[];
     constexpr int kXOps = kWM;               // x-tile DMA instructions a wave issues per stage
     constexpr int kOpsPerStage = kXOps + 2;  // DMA instructions a wave issues per stage
@@ -1278,7 +1364,28 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
     int par_dst;
     {
         const int w = wave;
-        if (kGrouped && w < 2) {
+        constexpr int kScaleWaves = kBN / 64;  // (kF32S: a column per lane)
+        if (kF32S) {
+            if (w < kScaleWaves) {
+                par_base = (const char*)p.scale + (n0 + w * 64 + lane < p.N ? n0 + w * 64 + lane : p.N - 1) * 4;
+                par_step = p.N * 4;
+                par_dst = w * 256;
+            } else if (w == kScaleWaves) {
+                int64_t n = n0 + lane * 4;
+                if (n > p.N - 4) n = p.N - 4;
+                par_base = (const char*)p.zero + n;
+                par_step = p.N;
+                par_dst = kParZero;
+            } else {
+                const int sw = w - kScaleWaves - 1;
+                const bool sums = sw < kBM / 32;
+                int64_t m = m0 + ((sums ? sw * 64 + lane : lane) >> 1);
+                if (m >= p.M) m = p.M - 1;
+                par_base = (const char*)(p.sx + m) + (lane & 1) * 4;
+                par_step = p.M * 8;
+                par_dst = sums ? kParSx + sw * 256 : kKmParSpare;
+            }
+        } else if (kGrouped && w < 2) {
             int64_t n = n0 + w * 128 + lane * 2;
             if (n > p.N - 2) n = p.N - 2;
             par_base = (const char*)p.scale + n * 2;
@@ -1383,7 +1490,7 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
                 for (int nb = 0; nb < kNB; ++nb) {
                     const u32 d = wq[nb][s];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) wb[nb][q] = (((d >> (4 * q)) & kKmNibbles) ^ kKmFlip) | kKmExp;
+                    for (int q = 0; q < 4; ++q) wb[nb][q] = ((q ? d >> (4 * q - 3) : d << 3) & kKmNibbles) ^ kKmBase;
                 }
 #pragma unroll
                 for (int nb = 0; nb < kNB; ++nb)
@@ -1402,14 +1509,14 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
             }
             if (group_last) {
                 const char* par = cur + kKmXBytes + kKmWBytes;
-                // acc -= (136 + zero) * sum(x) as one more MFMA step: k = 0 ... 2 carry -128 on the
+                // acc -= (24 + zero) * sum(x) as one more MFMA step: k = 0 ... 2 carry -16 on the
                 // kernel side, k = 3 ... 5 carry -(8 + zero) (any int8 zero point is exact in
                 // bfloat16), both against the three bfloat16 parts of the sum of x; products of
                 // two bfloat16 are exact in float32, so the cancellation happens in the accumulator
                 v4u xs[2], wz[kNB];
 #pragma unroll
                 for (int mb = 0; mb < 2; ++mb) {
-                    v2u raw = *(const v2u*)(par + kKmParSx + a_row[mb] * 8);
+                    v2u raw = *(const v2u*)(par + kParSx + a_row[mb] * 8);
                     if (g) raw[0] = raw[1] = 0;  // lanes 32 ... 63 hold k = 8 ... 15: nothing there
                     xs[mb][0] = raw[0];                                   // hi, lo
                     xs[mb][1] = (raw[1] & 0xffffu) | (raw[0] << 16);      // lolo, hi
@@ -1419,10 +1526,10 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
 #pragma unroll
                 for (int nb = 0; nb < kNB; ++nb) {
                     int zp = 0;
-                    if (kGrouped) zp = *(const int8_t*)(par + kKmParZero + wn * kWaveN + nb * 32 + i);
+                    if (kGrouped) zp = *(const int8_t*)(par + kParZero + wn * kWaveN + nb * 32 + i);
                     const u32 cz = __float_as_uint(-(float)(8 + zp)) >> 16;
-                    wz[nb][0] = 0xC300C300u;                              // -128, -128
-                    wz[nb][1] = 0xC300u | (cz << 16);                     // -128, -(8 + zero)
+                    wz[nb][0] = 0xC180C180u;                              // -16, -16
+                    wz[nb][1] = 0xC180u | (cz << 16);                     // -16, -(8 + zero)
                     wz[nb][2] = cz | (cz << 16);
                     wz[nb][3] = 0;
                 }
@@ -1439,11 +1546,17 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
                         float sc[4] = {1.f, 1.f, 1.f, 1.f};
                         if (kGrouped) {
                             const int nl = wn * kWaveN + nb * 32 + 8 * rg + 4 * g;
-                            const v2u sraw = *(const v2u*)(par + kKmParScale + nl * 2);
+                            if (kF32S) {
+                                const v4f sraw = *(const v4f*)(par + kKmParScale + nl * 4);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const u32 w = sraw[e >> 1];
-                                sc[e] = __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
+                                for (int e = 0; e < 4; ++e) sc[e] = sraw[e];
+                            } else {
+                                const v2u sraw = *(const v2u*)(par + kKmParScale + nl * 2);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const u32 w = sraw[e >> 1];
+                                    sc[e] = __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
+                                }
                             }
                         }
 #pragma unroll
@@ -1494,10 +1607,10 @@ struct KmPlan {
     int bm;  // tile rows: 128, or 64 (with 256 columns) up to 64 rows
 };
 
-inline KmPlan kmajor_plan(int64_t M, int64_t K, int64_t N, int64_t gsize) {
+inline KmPlan kmajor_plan(int64_t M, int64_t K, int64_t N, int64_t gsize, bool f32_scales = false) {
     const int bm = M <= 64 ? 64 : kKmBM;
     const int64_t m_tiles = (M + bm - 1) / bm;
-    const int bn = (bm == kKmBM && m_tiles * ((N + kKmBN - 1) / kKmBN) * 8 < kTargetWorkgroups) ? kKmBN / 2
+    const int bn = (bm == kKmBM && f32_scales) || (bm == kKmBM && m_tiles * ((N + kKmBN - 1) / kKmBN) * 8 < kTargetWorkgroups) ? kKmBN / 2
                                                                                                : kKmBN;
     const int64_t tiles = m_tiles * ((N + bn - 1) / bn);
     // about one workgroup per CU, at most eight splits (every split writes and the reduction
@@ -1680,6 +1793,48 @@ extern "C" int64_t k3q_gemm_w4_kmajor_workspace_bytes(int64_t M, int64_t K, int6
     return ((K / gsize) * M * 8 + 255) / 256 * 256 + (int64_t)pl.ks * M * N * 4;
 }
 
+// One launch of the tile kernel over the operands of kp (any split count; the partials stay in kp.part).
+static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, bool f32_scales, hipStream_t s) {
+    dim3 grid((unsigned)((kp.N + pl.bn - 1) / pl.bn), (unsigned)((kp.M + pl.bm - 1) / pl.bm), (unsigned)pl.ks);
+    constexpr int kDepth = 4;
+    const size_t lds = (size_t)kDepth * kKmSlotBytes;
+    using KmKernel = void (*)(KmParams);
+#define K3Q_KM_ROW(G, WM, NB)                                                               \
+    {gemm_w4_kmajor<G, kDepth, 0, WM, NB>, gemm_w4_kmajor<G, kDepth, 1, WM, NB>,             \
+     gemm_w4_kmajor<G, kDepth, 2, WM, NB>, gemm_w4_kmajor<G, kDepth, 4, WM, NB>}
+    // tile shapes: 128 x 128, 128 x 256, 64 x 256
+    static const KmKernel kernels[2][3][4] = {
+        {K3Q_KM_ROW(false, 2, 1), K3Q_KM_ROW(false, 2, 2), K3Q_KM_ROW(false, 1, 1)},
+        {K3Q_KM_ROW(true, 2, 1), K3Q_KM_ROW(true, 2, 2), K3Q_KM_ROW(true, 1, 1)}};
+#undef K3Q_KM_ROW
+    static const KmKernel f32_kernels[2] = {gemm_w4_kmajor<true, kDepth, 2, 2, 1, true>,
+                                            gemm_w4_kmajor<true, kDepth, 2, 1, 1, true>};
+    static const bool raised = [] {
+        bool ok = true;
+        for (const KmKernel k : f32_kernels)
+            ok = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget) ==
+                     hipSuccess && ok;
+        for (int a = 0; a < 2; ++a)
+            for (int b = 0; b < 3; ++b)
+                for (int c = 0; c < 4; ++c)
+                    ok = hipFuncSetAttribute((const void*)kernels[a][b][c],
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             kLdsBudget) == hipSuccess && ok;
+        return ok;
+    }();
+    if (!raised) return K3Q_ERR_LAUNCH;
+    const int gs = kp.gsize / kKmStage;
+    const int variant = gs == 1 ? 1 : gs == 2 ? 2 : gs == 4 ? 3 : 0;
+    const int shape = pl.bm == 64 ? 2 : pl.bn == kKmBN ? 1 : 0;
+    if (f32_scales) {  // (groups of 128)
+        const KmKernel k = shape == 2 ? f32_kernels[1] : f32_kernels[0];
+        k<<<grid, kKmThreads, lds, s>>>(kp);
+    } else {
+        kernels[grouped ? 1 : 0][shape][variant]<<<grid, kKmThreads, lds, s>>>(kp);
+    }
+    return launch_status();
+}
+
 static int run_gemm_w4_tiles(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N,
                              const void* w_kmajor, bool strip, const void* scale, const void* zero,
                              int64_t block_size, const void* bias, void* y, void* workspace,
@@ -1721,33 +1876,8 @@ static int run_gemm_w4_tiles(const void* x, int x_dtype, int64_t M, int64_t K, i
     kp.klen = (int)pl.klen;
     kp.strip = strip ? 1 : 0;
     kp.units = (int)(K / 128);
-    dim3 grid((unsigned)((N + pl.bn - 1) / pl.bn), (unsigned)((M + pl.bm - 1) / pl.bm), (unsigned)pl.ks);
-    constexpr int kDepth = 4;
-    const size_t lds = (size_t)kDepth * kKmSlotBytes;
-    using KmKernel = void (*)(KmParams);
-#define K3Q_KM_ROW(G, WM, NB)                                                               \
-    {gemm_w4_kmajor<G, kDepth, 0, WM, NB>, gemm_w4_kmajor<G, kDepth, 1, WM, NB>,             \
-     gemm_w4_kmajor<G, kDepth, 2, WM, NB>, gemm_w4_kmajor<G, kDepth, 4, WM, NB>}
-    // tile shapes: 128 x 128, 128 x 256, 64 x 256
-    static const KmKernel kernels[2][3][4] = {
-        {K3Q_KM_ROW(false, 2, 1), K3Q_KM_ROW(false, 2, 2), K3Q_KM_ROW(false, 1, 1)},
-        {K3Q_KM_ROW(true, 2, 1), K3Q_KM_ROW(true, 2, 2), K3Q_KM_ROW(true, 1, 1)}};
-#undef K3Q_KM_ROW
-    static const bool raised = [] {
-        bool ok = true;
-        for (int a = 0; a < 2; ++a)
-            for (int b = 0; b < 3; ++b)
-                for (int c = 0; c < 4; ++c)
-                    ok = hipFuncSetAttribute((const void*)kernels[a][b][c],
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             kLdsBudget) == hipSuccess && ok;
-        return ok;
-    }();
-    (void)raised;
-    const int gs = (int)(gsize / kKmStage);
-    const int variant = gs == 1 ? 1 : gs == 2 ? 2 : gs == 4 ? 3 : 0;
-    const int shape = pl.bm == 64 ? 2 : pl.bn == kKmBN ? 1 : 0;
-    kernels[grouped ? 1 : 0][shape][variant]<<<grid, kKmThreads, lds, s>>>(kp);
+    const int lrc = launch_w4_tiles(kp, pl, grouped, false, s);
+    if (lrc != K3Q_OK) return lrc;
     // the decode kernel's second pass: sums the splits in order, applies scale and bias
     GemvParams gp{};
     gp.scale = scale;
@@ -1779,6 +1909,115 @@ extern "C" int k3q_gemm_w4_strip(const void* x, int x_dtype, int64_t M, int64_t 
                                  int64_t workspace_bytes, void* stream) {
     return run_gemm_w4_tiles(x, x_dtype, M, K, N, w_strip, true, scale, zero, block_size, bias, y, workspace,
                              workspace_bytes, stream);
+}
+
+// ---- any K % 8, any N, float32 or bfloat16 rows ------------------------------------------------------------------
+// Three launches: the rows made ready (km_prepare_rows), the tile kernel on the strip-linear copy, the second pass.  The
+// padding costs a pass over x (3 us) where it spares the kernel a copy.  Graph nodes, us, before -> now: bfloat16
+// K=1600, N=6400 300 rows 137 -> 31 and 1200 rows 570 -> 74 (passes of 32 rows); K=2048, N=5247 64 rows 484 -> 18 (one
+// output per thread); float32 K=4096, N=14336 64 rows 127 -> 37 (passes of 8 rows), 300 rows 298 -> 156 (the kernel
+// de-quantised to parts).  A float32 row doubles the matrix work, which bounds the larger sizes; up to a few dozen rows
+// it is the launches, the start of the ring and the partials.  Error against 64 bits (2-norm), before / now:
+// float32 5.3e-6 / 4.9e-6 (de-quantised kernel 1.3e-5), ragged 2.1e-7 / 1.0e-7, bfloat16 1.66e-3 / 1.66e-3.
+namespace k3q {
+namespace {
+struct KmRowsPlan {
+    int parts;      // bfloat16 rows per row of x
+    int64_t Kp, Np, rows, sx_bytes, x_bytes, part_bytes;
+    KmPlan tiles;   // of a launch of `rows` rows
+};
+
+// Rows go in launches of 1024 bfloat16 rows at most: the partials of one stay in the memory-side cache.
+constexpr int64_t kKmMostRows = 1024;
+
+bool km_rows_plan(KmRowsPlan& pl, int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size) {
+    if (M < 1 || K < 16 || (K % 8) != 0 || N < 1 || N > (int64_t(1) << 24) || (block_size > 0 && block_size != 128))
+        return false;
+    const bool f32 = x_dtype == K3Q_F32;
+    // parts of a float32 row: as in the kernels on the stored weights, which split x in two for these shapes and
+    // have float32 products for the others
+    pl.parts = !f32 ? 1 : (N % 8) == 0 && (K % 16) == 0 ? 2 : 3;
+    pl.Kp = (K + 127) / 128 * 128;
+    pl.Np = (N + 31) / 32 * 32;  // the strips of the copy
+    pl.rows = M < kKmMostRows / pl.parts ? M : kKmMostRows / pl.parts;
+    const int64_t mx = pl.rows * pl.parts;
+    pl.tiles = kmajor_plan(mx, pl.Kp, pl.Np, 128, f32 && block_size > 0);
+    pl.x_bytes = mx * pl.Kp * 2;  // (a multiple of 256)
+    pl.sx_bytes = (pl.Kp / 128 * mx * 8 + 255) / 256 * 256;
+    pl.part_bytes = (int64_t)pl.tiles.ks * mx * pl.Np * 4;
+    return true;
+}
+}  // namespace
+}  // namespace k3q
+
+extern "C" int64_t k3q_gemm_w4_rows_workspace_bytes(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size) {
+    KmRowsPlan pl;
+    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return 0;
+    return km_rows_plan(pl, x_dtype, M, K, N, block_size) ? pl.x_bytes + pl.sx_bytes + pl.part_bytes : 0;
+}
+
+extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* w_strip,
+                                const void* scale, const void* zero, int64_t block_size, const void* bias,
+                                int64_t bias_stride, void* y, void* workspace, int64_t workspace_bytes, void* stream) {
+    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
+    if (M < 0 || K <= 0 || N <= 0) return K3Q_ERR_SHAPE;
+    if (M == 0) return K3Q_OK;
+    if (bias_stride != 0 && bias_stride != N) return K3Q_ERR_SHAPE;
+    KmRowsPlan pl;
+    if (!km_rows_plan(pl, x_dtype, M, K, N, block_size)) return K3Q_ERR_SHAPE;
+    const bool f32 = x_dtype == K3Q_F32, grouped = block_size > 0;
+    const int el = f32 ? 4 : 2;
+    if (!x || !w_strip || !scale || !y || (grouped && !zero)) return K3Q_ERR_NULL;
+    if (!aligned_to(x, 2 * el) || !aligned_to(w_strip, 16) || !aligned_to(scale, grouped ? 8 : el) ||
+        (grouped && !aligned_to(zero, 4)) || !aligned_to(y, el) || (bias && !aligned_to(bias, el)))
+        return K3Q_ERR_ALIGN;
+    if (!workspace || workspace_bytes < pl.x_bytes + pl.sx_bytes + pl.part_bytes) return K3Q_ERR_WORKSPACE;
+    if (!aligned_to(workspace, 256)) return K3Q_ERR_ALIGN;
+    hipStream_t s = (hipStream_t)stream;
+    KmParams kp{};
+    kp.x = (const uint16_t*)workspace;
+    kp.sx = (const v2u*)((char*)workspace + pl.x_bytes);
+    kp.part = (float*)((char*)workspace + pl.x_bytes + pl.sx_bytes);
+    kp.shadow = (const uint8_t*)w_strip;
+    kp.scale = scale;
+    kp.zero = (const int8_t*)zero;
+    kp.N = pl.Np;
+    kp.K = pl.Kp;
+    kp.gsize = 128;
+    kp.strip = 1;
+    kp.units = (int)(pl.Kp / 128);
+    for (int64_t m0 = 0; m0 < M; m0 += pl.rows) {
+        const int64_t rows = M - m0 < pl.rows ? M - m0 : pl.rows;
+        const void* xm = (const char*)x + m0 * K * el;
+        void* ym = (char*)y + m0 * N * el;
+        const void* bm = bias ? (const char*)bias + m0 * bias_stride * el : nullptr;
+        const dim3 pgrid((unsigned)kp.units, (unsigned)((rows + 3) / 4));
+        kp.M = rows * pl.parts;
+        KmPlan tiles = kmajor_plan(kp.M, pl.Kp, pl.Np, 128, f32 && grouped);
+        if ((int64_t)tiles.ks * kp.M * pl.Np * 4 > pl.part_bytes) {  // fewer rows would split further than there is room
+            tiles.ks = pl.tiles.ks;
+            tiles.klen = pl.tiles.klen;
+        }
+        kp.klen = (int)tiles.klen;
+        u32* xp = (u32*)workspace;
+        v2u* sx = (v2u*)((char*)workspace + pl.x_bytes);
+        if (pl.parts == 1) km_prepare_rows<1><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
+        else if (pl.parts == 2) km_prepare_rows<2><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
+        else km_prepare_rows<3><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
+        const int rc = launch_w4_tiles(kp, tiles, grouped, f32 && grouped, s);
+        if (rc != K3Q_OK) return rc;
+        const dim3 fgrid((unsigned)((N + 1023) / 1024), (unsigned)rows);
+#define K3Q_KM_FINISH(B, P)                                                                                          \
+    if (grouped) km_finish<B, true, P><<<fgrid, 256, 0, s>>>(kp.part, scale, bm, ym, rows, N, pl.Np, bias_stride, tiles.ks); \
+    else km_finish<B, false, P><<<fgrid, 256, 0, s>>>(kp.part, scale, bm, ym, rows, N, pl.Np, bias_stride, tiles.ks)
+        if (pl.parts == 1) { K3Q_KM_FINISH(true, 1); }
+        else if (pl.parts == 2) { K3Q_KM_FINISH(false, 2); }
+        else { K3Q_KM_FINISH(false, 3); }
+#undef K3Q_KM_FINISH
+        const int rc2 = launch_status();
+        if (rc2 != K3Q_OK) return rc2;
+    }
+    return K3Q_OK;
 }
 
 // ---- the decode-sized call for callers that cannot allocate -----------------------------

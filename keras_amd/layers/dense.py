@@ -136,6 +136,42 @@ def strip_rows_params(layer, dtype, input_dim, units, block_size):
     return hit[2]
 
 
+# float32 rows up to which the int4 tile kernel beats the GEMM on the kernel de-quantised to bfloat16 parts (us, GEMM
+# route / tiles: K=N=4096 grouped 64 rows 50 / 27, 300 80 / 62, 600 137 / 90, 1200 188 / 166; per channel 38 / 28,
+# 59 / 46, 99 / 87, 131 / 153; K=4096, N=14336 at 300 rows 298 / 156)
+TILE_ROWS_MAX_F32 = 768
+
+
+def int4_tile_rows_route(x2, units, block_size):
+    """Whether an int4 call of more rows than the decode kernels take goes to `ops.int4_matmul_tiles_rows`: shapes
+    that neither the tile kernel proper (`ops.int4_kmajor_supported`) nor the GEMM on the de-quantised kernel takes
+    (K % 128, N % 64), which went in passes of 32 bfloat16 or 8 float32 rows over the kernel, and float32 rows up to
+    `TILE_ROWS_MAX_F32` (us, passes / tiles: K=1600, N=6400 bfloat16 48 rows 25.6 / 17.0, 300 137 / 31, 1200 570 / 74;
+    float32 17 rows 25 / 17, 300 307 / 38; one pass, up to 32 bfloat16 rows of a kernel this small, is as good: 15.7 /
+    15.7).  Where N % 8 or K % 16 leave only the kernel of one output per thread (K=2048, N=5247: 480 us at 32
+    rows, 6.1 ms at 1200, against 15 and 82) every shape goes here."""
+    rows, input_dim = x2.shape
+    if not (x2.is_cuda and x2.dtype in (torch.float32, torch.bfloat16) and rows > kops.STRIP_MAX_ROWS
+            and kops.int4_tiles_rows_supported(input_dim, units, block_size)):
+        return False
+    if units % 8 or input_dim % 16:
+        return True
+    gemm = input_dim % 128 == 0 and units % 64 == 0
+    if x2.dtype == torch.float32:
+        return not gemm or rows <= TILE_ROWS_MAX_F32
+    return not gemm and (rows >= KMAJOR_MIN_ROWS or kmajor_rows(rows, units, input_dim))
+
+
+def tile_rows_operands(layer, dtype, units, grouped):
+    """Scales and zero points of `ops.int4_matmul_tiles_rows` in `dtype`, kept while the variables do not change."""
+    if not grouped:
+        return dict(kernel_scale=layer._cached("kernel_scale", layer.kernel_scale, lambda t: t.to(dtype).contiguous()))
+    return dict(kernel_scale=layer._cached("tile_scale", layer.kernel_scale,
+                                           lambda t: kops.int4_tile_columns(t.to(dtype), units)),
+                kernel_zero=(layer._cached("tile_zero", layer.kernel_zero, lambda t: kops.int4_tile_columns(t, units))
+                             if units % 32 else as_tensor(layer.kernel_zero)))
+
+
 def int8_strip_route(quantizer, x2, units, strict=False):
     """Whether an int8 call of these rows goes to `ops.int8_dense_strip`: rows on the device, few
     enough, a plain abs-max quantizer (whatever its range and epsilon), a shape the kernel takes.
@@ -548,6 +584,13 @@ class Dense(Layer):
                     block_size=block_size if grouped else None,
                     bias=self._call_bias(),
                 )
+        elif int4_tile_rows_route(inputs.reshape(rows, inputs.shape[-1]), self._orig_output_dim,
+                                  block_size if grouped else None):
+            units = self._orig_output_dim
+            y = kops.int4_matmul_tiles_rows(
+                inputs, self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)), units,
+                block_size=block_size if grouped else None, bias=self._call_bias(),
+                **tile_rows_operands(self, inputs.dtype, units, grouped))
         else:
             y = kops.int4_matmul(
                 inputs, as_tensor(self._kernel),

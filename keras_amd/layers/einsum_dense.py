@@ -815,7 +815,8 @@ class EinsumDense(Layer):
                                           lambda t: t.to(cd).reshape(-1).contiguous()),
                 bias=bias, out_dtype=cd, exact_epilogue=True)
             return self._finish(y2, free_shape, gv, fused)
-        from keras_amd.layers.dense import int4_strip_rows_route, kmajor_rows
+        from keras_amd.layers.dense import (int4_strip_rows_route, int4_tile_rows_route, kmajor_rows,
+                                            tile_rows_operands)
 
         units = self._int4_unpacked_column_size
         strip = (self._strip_operands(x2.shape[0], x2.shape[1], units, grouped, block_size)
@@ -848,6 +849,11 @@ class EinsumDense(Layer):
                     x2, self._cached("kmajor", self._kernel, lambda t: kops.int4_kmajor_copy(t, units)),
                     scale_cd, kernel_zero=as_tensor(self.kernel_zero) if grouped else None,
                     block_size=block_size if grouped else None, bias=bias)
+            return self._finish(y2, free_shape, gv, fused)
+        if x2.dtype == cd and int4_tile_rows_route(x2, units, block_size if grouped else None):
+            y2 = kops.int4_matmul_tiles_rows(
+                x2, self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)), units,
+                block_size=block_size if grouped else None, bias=bias, **tile_rows_operands(self, cd, units, grouped))
             return self._finish(y2, free_shape, gv, fused)
         y2 = kops.int4_matmul(
             x2, as_tensor(self._kernel),

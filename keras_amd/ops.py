@@ -651,6 +651,60 @@ GEMM_EXACT_EPILOGUE = 1
 SKINNY_MAX_ROWS = 8
 
 
+def int4_tile_columns(t, units):
+    """`[G, N]` scales or zero points with the columns padded to a multiple of 32, as `int4_matmul_tiles_rows` reads
+    them (the tensor itself where nothing is missing)."""
+    pad = -int(units) % 32
+    return torch.nn.functional.pad(t, (0, pad)) if pad else t.contiguous()
+
+
+def int4_tiles_rows_supported(K, N, block_size=None):
+    """Whether `int4_matmul_tiles_rows` takes a [K, N] int4 kernel."""
+    bs = int(block_size) if block_size is not None and block_size > 0 else -1
+    return _lib.load().k3q_gemm_w4_rows_workspace_bytes(_lib.K3Q_BF16, 1, int(K), int(N), bs) > 0
+
+
+def int4_matmul_tiles_rows(x, shadow, units, kernel_scale, kernel_zero=None, block_size=None, bias=None):
+    """`x[..., K] . W4[K, N]` for any number of float32 or bfloat16 rows, any K % 8 and any N, by the int4 tile kernel
+    from `int4_strip_copy(kernel)`.  Per-channel: `kernel_scale` [N]; grouped (block 128): `kernel_scale` and
+    `kernel_zero` through `int4_tile_columns`.  `bias` [N], or [M, N]: a row per row of x.
+    Reference: keras/src/layers/core/dense.py:988-1095."""
+    _lib.require_device(x, shadow, kernel_scale, kernel_zero, bias)
+    lib = _lib.load()
+    code = _lib.dtype_code(x.dtype)
+    grouped = block_size is not None and block_size > 0
+    bs = int(block_size) if grouped else -1
+    K, N = x.shape[-1], int(units)
+    lead = x.shape[:-1]
+    x2 = x.reshape(-1, K)
+    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    if x2.data_ptr() % 16:  # a view into a larger buffer
+        x2 = x2.clone()
+    M = x2.shape[0]
+    if shadow.numel() != lib.k3q_w4s_shadow_bytes(K, N):
+        raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
+    _check_bias_size(bias, M, N)
+    if kernel_scale.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
+        raise TypeError("kernel_scale and bias must be read in the input's dtype")
+    if grouped:
+        shape = ((K + 127) // 128, -(-N // 32) * 32)
+        if (kernel_zero is None or tuple(kernel_scale.shape) != shape or tuple(kernel_zero.shape) != shape
+                or kernel_zero.dtype != torch.int8):
+            raise ValueError("scale / zero must be [ceil(K / 128), N rounded up to 32], zero int8")
+    elif kernel_scale.numel() != N:
+        raise ValueError("per-channel int4 needs scales [N]")
+    ks = kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous()
+    kz = None if not grouped else (kernel_zero if kernel_zero.is_contiguous() else kernel_zero.contiguous())
+    b = bias if bias is None or bias.is_contiguous() else bias.contiguous()
+    stride = N if bias is not None and M > 1 and bias.numel() == M * N else 0
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    ws = _workspace(x.device, lib.k3q_gemm_w4_rows_workspace_bytes(code, M, K, N, bs))
+    rc = lib.k3q_gemm_w4_rows(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks), _lib.ptr(kz), bs,
+                              _lib.ptr(b), stride, _lib.ptr(y), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(x.device))
+    _lib.check(rc, "k3q_gemm_w4_rows")
+    return y.reshape(*lead, N)
+
+
 def prepack_int8_kernel(kernel):
     """[K, N] int8 kernel -> the [N, K] shadow copy the MFMA GEMM consumes.
 

@@ -1,0 +1,51 @@
+"""GPU parity: the int4 tile kernel for any K % 8, any N, float32 or bfloat16 rows (k3q_gemm_w4_rows) against
+the float64 value of the same stored operands."""
+
+import pytest
+import torch
+
+from keras_amd import ops as kops
+from tests.helpers import c_w4_matmul_f64
+from tests.test_gpu_int4_matmul import make_layer
+from tests.test_gpu_int4_strip_rows import magnitude
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N,block_size", [
+    (1, 16, 1, None), (17, 24, 33, 128), (31, 136, 5, 128), (32, 1600, 6400, 128), (33, 960, 1003, 128),
+    (64, 128, 128, None), (65, 2048, 5247, 128), (128, 768, 2094, None), (129, 4544, 3200, 128), (300, 1600, 6400, 128),
+    (342, 1000, 777, 128), (513, 320, 1028, 128), (1025, 192, 100, None), (2050, 448, 260, 128), (64, 4096, 14336, 128),
+])
+def test_tiles_rows(dev, dtype, M, K, N, block_size):
+    qk, bias = make_layer(K, N, block_size, seed=M + K, with_bias=(M % 2 == 1))
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    scale, kernel = qk["kernel_scale"].to(dtype), qk["kernel"].to(dev)
+    zero = qk["kernel_zero"] if block_size else None
+    b = None if bias is None else bias.to(dtype)
+    per_row = M == 33
+    if per_row:
+        b = torch.randn(M, N, generator=g).to(dtype)
+    # poisoned scratch: a partial or a row that is read before it is written shows
+    kops._workspace(dev, 64 << 20).fill_(0xFF)
+    got = kops.int4_matmul_tiles_rows(
+        x.to(dev), kops.int4_strip_copy(kernel, N), N,
+        kops.int4_tile_columns(scale.to(dev), N) if block_size else scale.to(dev),
+        kernel_zero=kops.int4_tile_columns(zero.to(dev), N) if block_size else None,
+        block_size=block_size, bias=None if b is None else b.to(dev))
+    torch.cuda.synchronize()
+    assert got.dtype == dtype and tuple(got.shape) == (M, N)
+    exact = c_w4_matmul_f64(x, qk["kernel"], scale, zero, block_size, None if per_row else b, N)
+    if per_row:
+        exact = exact + b.double()
+    mag = magnitude(x, kernel, scale, zero, block_size, N)
+    err = (got.double().cpu() - exact).abs()
+    if dtype == torch.float32:  # (as in test_rows_shapes)
+        split = 2.0 ** -17 if N % 8 == 0 and K % 16 == 0 else 0.0
+        bound = mag * (split + 4 * 2.0 ** -24 * K ** 0.5) + exact.abs() * 2.0 ** -22
+    else:  # sum, quotient and biased result are each rounded to bfloat16: half an ulp is up to 2^-8 of the value
+        size = exact.abs() + (0 if b is None else 2 * b.double().abs())
+        bound = mag * 4 * 2.0 ** -24 * K ** 0.5 + size * 3.05 * 2.0 ** -8
+    assert bool((err <= bound).all()), float((err / bound).max())
