@@ -28,14 +28,14 @@ namespace k3q {
 namespace {
 
 constexpr int kBK = 128;  // bytes of K per stage: one full 128-byte line per row
-constexpr int kStages = 2;
 constexpr int kKSteps = kBK / 32;  // MFMA K steps per stage
 constexpr int kRowChunks = kBK / 16;  // 16-byte chunks per LDS row
 
 // Tile shape of a workgroup: BM rows of a / y, BN rows of the prepacked weight (= columns of
-// y), waves laid out WN (along N) x WM (along M).
-template <int BM, int BN, int WN_, int WM_>
+// y), waves laid out WN (along N) x WM (along M), LDS stages.
+template <int BM, int BN, int WN_, int WM_, int STAGES = 2>
 struct Tile {
+    static constexpr int kStages = STAGES;
     static constexpr int kBM = BM, kBN = BN, kWavesN = WN_, kWavesM = WM_;
     static constexpr int kThreads = 64 * WN_ * WM_;
     static constexpr int kWN = BN / WN_;      // columns per wave
@@ -55,6 +55,9 @@ typedef Tile<256, 256, 4, 2> TileLarge;
 // 128 x 128, 4 waves, 64 KiB of LDS: two workgroups per CU; used while the large tile would
 // leave CUs without work.
 typedef Tile<128, 128, 2, 2> TileSmall;
+
+// The small tile with four stages, 128 KiB: one workgroup per CU, for problems that have no second one for it.
+typedef Tile<128, 128, 2, 2, 4> TileDeep;
 
 constexpr int kFlagExactEpilogue = 1;
 constexpr int kFlagRoundAccBF16 = 2;   // float32 output of a bfloat16 layer: acc is cast to bfloat16 first
@@ -94,9 +97,10 @@ __device__ __forceinline__ int swz(int row) {
 
 // gfx9 s_waitcnt encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]
 __device__ __forceinline__ void wait_vmcnt0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-template <int kDmaPerWave>
-__device__ __forceinline__ void wait_vmcnt_one_stage() {
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (kDmaPerWave & 0xF) | ((kDmaPerWave >> 4) << 14));
+template <int kCount>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(kCount < 64, "six bits");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (kCount & 0xF) | ((kCount >> 4) << 14));
 }
 __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 __device__ __forceinline__ void bare_barrier() {
@@ -192,7 +196,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
     constexpr int kBM = T::kBM, kBN = T::kBN, kWavesN = T::kWavesN, kThreads = T::kThreads;
     constexpr int kWN = T::kWN, kWM = T::kWM, kNBlk = T::kNBlk, kMBlk = T::kMBlk;
     constexpr int kATileBytes = T::kATileBytes, kStageBytes = T::kStageBytes;
-    constexpr int kDmaA = T::kDmaA, kDmaPerWave = T::kDmaPerWave;
+    constexpr int kDmaA = T::kDmaA, kDmaPerWave = T::kDmaPerWave, kStages = T::kStages;
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -269,7 +273,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
         // (row base | ((g ^ swz(i)) << 4)) ^ (32 * ks) + block * 32 rows: one register per
         // operand, one XOR per K step, the blocks as immediate offsets.  The stage is a bit of
         // that register, flipped at the hand-over.
-        static_assert((kStageBytes & (kStageBytes - 1)) == 0 && kWM % 32 == 0 && kWN % 32 == 0, "addressing");
+        static_assert((kStageBytes & (kStageBytes - 1)) == 0 && (kStages & (kStages - 1)) == 0 && kWM % 32 == 0 && kWN % 32 == 0, "addressing");
         const int lane_chunk = (fg ^ swz(fi)) << 4;
         int ra = (wm * kWM + fi) * kBK + lane_chunk;
         int rb = kATileBytes + (wn * kWN + fi) * kBK + lane_chunk;
@@ -294,19 +298,27 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
                 for (int r = 0; r < 16; ++r) acc[nb][mb][r] = 0;
 
         // ---- main loop ----
-        // Two LDS stages.  The fragments of K step ks+1 are read in the middle of the MFMAs of
+        // A ring of kStages LDS stages.  The fragments of K step ks+1 are read in the middle of the MFMAs of
         // step ks; the one barrier per stage sits in the middle of the LAST step's MFMAs, so the
         // matrix core has work queued while waves meet.  At that barrier every wave holds its
-        // last fragments of stage kt in registers, so stage kt+2 may be DMA-ed over stage kt, and
+        // last fragments of stage kt in registers, so stage kt+kStages may be DMA-ed over stage kt, and
         // stage kt+1 (whose DMA every wave has waited for) may be read.
         const int kt_first = sp * p.kt_split;  // this split's stages (all of K without a split)
         const int KT = min(p.kt_split, (int)(p.row_bytes / kBK) - kt_first);
         issue_stage(0);
-        if (KT > 1) {
-            issue_stage(1);
-            wait_vmcnt_one_stage<kDmaPerWave>();
+        if constexpr (kStages == 2) {
+            if (KT > 1) {
+                issue_stage(1);
+                wait_vmcnt<kDmaPerWave>();
+            } else {
+                wait_vmcnt0();
+            }
         } else {
-            wait_vmcnt0();
+#pragma unroll
+            for (int st = 1; st < kStages; ++st)
+                if (st < KT) issue_stage(st);
+            if (KT >= kStages) wait_vmcnt<(kStages - 1) * kDmaPerWave>();
+            else wait_vmcnt0();
         }
         bare_barrier();
         read_frags(0, 0);
@@ -326,8 +338,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
                 (__attribute__((address_space(3))) void*)(dst + d * 1024), 16, 0, 0);
         };
         auto mma_half = [&](int ks, int half, int kt) {
-            // halves since the hand-over: 0 = second half of the last step (feeds stage kt+2),
-            // 1..4 = the two halves of steps 0 and 1 (feed stage kt+1, begun one stage earlier)
+            // halves since the hand-over: 0 = second half of the last step (feeds stage kt+kStages),
+            // 1..4 = the two halves of steps 0 and 1 (feed stage kt+kStages-1, begun one stage earlier)
             const int hh = (ks == kKSteps - 1 && half == 1) ? 0 : (ks <= 1 ? 1 + 2 * ks + half : -1);
 #pragma unroll
             for (int j = 0; j < kHalfMmas; ++j) {
@@ -335,7 +347,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
                 acc[nb][mb] = Mma<kKind>::run(bf[ks & 1][nb], af[ks & 1][mb], acc[nb][mb]);
                 const int pos = hh * kHalfMmas + j;
                 if (hh >= 0 && pos % kDmaStride == kDmaStride - 1 && pos / kDmaStride < kDmaPerWave) {
-                    const int target = hh == 0 ? kt + 2 : kt + 1;
+                    const int target = hh == 0 ? kt + kStages : kt + kStages - 1;
                     if ((hh == 0 || kt >= 1) && target < KT) {
                         __builtin_amdgcn_sched_barrier(0);
                         issue_one(target, pos / kDmaStride);
@@ -360,10 +372,22 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
                 if (ks + 1 < kKSteps) {
                     read_frags((ks + 1) & 1, ks + 1);
                 } else if (kt + 1 < KT) {
-                    wait_vmcnt0();  // own DMA of stage kt+1 has landed (own reads of stage kt are done)
+                    // own DMA of stage kt+1 has landed (own reads of stage kt are done): every stage up to
+                    // kt+kStages-1 has been issued whole, in order, and the ones behind kt+1 may be in flight
+                    if constexpr (kStages > 2) {
+                        if (kt + kStages <= KT) wait_vmcnt<(kStages - 2) * kDmaPerWave>();
+                        else wait_vmcnt0();
+                    } else {
+                        wait_vmcnt0();
+                    }
                     bare_barrier();
-                    ra ^= kStageBytes;
-                    rb ^= kStageBytes;
+                    if constexpr (kStages == 2) {
+                        ra ^= kStageBytes;
+                        rb ^= kStageBytes;
+                    } else {
+                        ra = (ra + kStageBytes) & (kStages * kStageBytes - 1);
+                        rb = (rb + kStageBytes) & (kStages * kStageBytes - 1);
+                    }
                     read_frags(0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -815,8 +839,7 @@ __global__ __launch_bounds__(256) void gemm_split_reduce(GemmParams p) {
 // 14336): an unsplit tile walks its stages at 0.65 us each, a split into sp saves
 // (1 - 1/sp) of that, costs 4 us for the second kernel and 0.052 us per tile and split for
 // writing and reading its 64 KiB of partials, and is taken while tiles * sp still fit on the
-// chip at once.  E.g. 32 tiles x 32 stages: 4; 64 x 64: 4; 32 x 112: 8; 128 x 64: 3;
-// 128 x 16 or 96 x 32: none.
+// chip at once.
 inline int choose_splits(int64_t tiles, int64_t stages, int resident) {
     int best = 1;
     int64_t best_gain_ns = 0;
@@ -831,13 +854,23 @@ inline int choose_splits(int64_t tiles, int64_t stages, int resident) {
     return best;
 }
 
+// Whether the small tile runs with four stages and one workgroup per CU (TileDeep): while its tiles are no more
+// than the CUs and more than half of them, so that neither a second workgroup nor a split of K has a place, and
+// the walk is long enough to be worth a deeper start.  One workgroup alone on a CU waits for the memory
+// behind two stages (us, two stages / four, bfloat16 operands and int8: 1024 x 4096 x 4096 48.8 / 42.4 and
+// 30.4 / 27.8; 300 x 3200 x 8192 38.0 / 29.8 and 23.5 / 20.6; 512 x 8192 x 8192 79.0 / 75.8 and 49.6 / 45.4).
+// With fewer tiles a split of K over two workgroups per CU stays ahead (128 x 4096 x 4096 int8 16.9 / 22.6), and
+// so do two stages on a short walk (300 x 1664 x 6400 int8, 13 stages: 14.0 / 14.7).
+inline bool deep_tile(int64_t tiles, int64_t stages, int cus) {
+    return 2 * tiles > cus && tiles <= cus && stages >= 20;
+}
 
 // Room for the partials of the largest split the launch may choose (sized for a chip of up
 // to 256 CUs; a launch that finds less room splits less).
 inline int64_t split_workspace_bytes(int64_t M, int64_t N, int64_t row_bytes) {
     if (M <= 0 || (row_bytes % kBK) != 0 || (N % 4) != 0) return 0;
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    const int splits = choose_splits(tiles, row_bytes / kBK, 512);
+    const int splits = deep_tile(tiles, row_bytes / kBK, 256) ? 1 : choose_splits(tiles, row_bytes / kBK, 512);
     return splits > 1 ? (int64_t)splits * M * N * 4 : 0;
 }
 
@@ -882,13 +915,16 @@ template <int kKind, bool kBF16, bool kExact>
 int launch_mfma(const GemmParams& p, hipStream_t s) {
     const int64_t large_tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
     const bool large = large_tiles >= kLargeTileMinTiles;
+    const bool deep = deep_tile(((p.M + 127) / 128) * ((p.N + 127) / 128), p.row_bytes / kBK, cu_count());
     if constexpr (kKind == kKindI8) {
         if (p.b_strip) {
             if (large) return launch_tile<TileLarge, kKind, kBF16, kExact, true>(p, s);
+            if (deep) return launch_tile<TileDeep, kKind, kBF16, kExact, true>(p, s);
             return launch_tile<TileSmall, kKind, kBF16, kExact, true>(p, s);
         }
     }
     if (large) return launch_tile<TileLarge, kKind, kBF16, kExact>(p, s);
+    if (deep) return launch_tile<TileDeep, kKind, kBF16, kExact>(p, s);
     return launch_tile<TileSmall, kKind, kBF16, kExact>(p, s);
 }
 
