@@ -591,6 +591,13 @@ int k3q_decode_attention(const void* q, const void* k, const void* v, int dtype,
                          const int64_t* pos, void* k_cache, void* v_cache, void* out, int* oob_flag,
                          void* stream);
 
+/* The rotation and the cache update alone, for T positions (pos: T int64 in device memory): q, k, v [B, T, H, 128];
+ * q_out [B, T, H, 128] gets the rotated queries, row pos[t] of the caches the rotated keys and the values, with the
+ * roundings of the torch sequence.  A position outside [0, max_len) writes nothing to the caches and sets *oob_flag. */
+int k3q_rope_cache(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t T, int64_t H,
+                   int64_t head_dim, int64_t max_len, const void* cos_table, const void* sin_table,
+                   const int64_t* pos, void* k_cache, void* v_cache, void* q_out, int* oob_flag, void* stream);
+
 /*
  * Two more pieces of the decoder harness's glue (no counterpart in the quantized layers; they
  * stand for `rms_norm` and `silu(gate) * up` between the Dense calls of a decoder block), bfloat16:

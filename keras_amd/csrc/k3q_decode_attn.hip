@@ -238,10 +238,110 @@ __global__ __launch_bounds__(kAT) void decode_attention(AttnParams p) {
     }
 }
 
+// ---- several positions: the prompt's rotation and cache update -------------------------------------------------
+// out = rotated q, the cache rows at pos[t] = rotated k and v, with the roundings of the torch sequence
+// (bf16(x cos) + bf16(swapped sin), rounded), which cost eight passes over q and k (cat, swap, two products, sum, two
+// index copies): 104 us per block of 8 x 128 tokens of 32 heads.  Here every value is read and written once.
+// Bound by memory: a thread takes pieces c and c + 8 (16 bytes each) of a head's 128 values of q, k and v, so that it
+// holds both halves of a rotation and eight threads read and write whole 128-byte lines.
+struct RopeParams {
+    const uint16_t *q, *k, *v;      // [B, T, H, 128]
+    const uint16_t *cos_t, *sin_t;  // [max_len, 128]
+    const int64_t* pos;             // device [T]
+    uint16_t *kc, *vc;              // [B, H, max_len, 128]
+    uint16_t* out;                  // [B, T, H, 128]
+    int* oob;                       // device flag, may be null: 1 when a position is outside the cache (not written)
+    int64_t heads;                  // B T H
+    int T, H, max_len;
+};
+
+// x cos + swapped sin for one 16-byte piece, each step rounded to bfloat16
+__device__ __forceinline__ v4u rotate_piece(const v4u& x, const v4u& swapped, const v4u& cs, const v4u& sn) {
+    v4u o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float lo = round_bf16(__uint_as_float(x[e] << 16) * __uint_as_float(cs[e] << 16)) +
+                         round_bf16(__uint_as_float(swapped[e] << 16) * __uint_as_float(sn[e] << 16));
+        const float hi = round_bf16(__uint_as_float(x[e] & 0xffff0000u) * __uint_as_float(cs[e] & 0xffff0000u)) +
+                         round_bf16(__uint_as_float(swapped[e] & 0xffff0000u) * __uint_as_float(sn[e] & 0xffff0000u));
+        o[e] = f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+    }
+    return o;
+}
+
+__global__ __launch_bounds__(256) void rope_cache_rows(RopeParams p) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t row = i >> 3;  // (b, t, h)
+    const int c = (int)(i & 7);
+    if (row >= p.heads) return;
+    const int h = (int)(row % p.H);
+    const int64_t bt = row / p.H;
+    const int t = (int)(bt % p.T);
+    const int64_t b = bt / p.T;
+    const v4u* q = (const v4u*)(p.q + row * kHd);
+    const v4u* k = (const v4u*)(p.k + row * kHd);
+    const v4u* v = (const v4u*)(p.v + row * kHd);
+    const v4u q0 = q[c], q1 = q[c + 8], k0 = k[c], k1 = k[c + 8], v0 = v[c], v1 = v[c + 8];
+    const int64_t pos = p.pos[t];
+    const bool inside = pos >= 0 && pos < p.max_len;
+    const int64_t at = inside ? pos : 0;
+    const v4u* cs = (const v4u*)(p.cos_t + at * kHd);
+    const v4u* sn = (const v4u*)(p.sin_t + at * kHd);
+    const v4u c0 = cs[c], c1 = cs[c + 8], s0 = sn[c], s1 = sn[c + 8];
+    v4u* o = (v4u*)(p.out + row * kHd);
+    o[c] = rotate_piece(q0, q1, c0, s0);
+    o[c + 8] = rotate_piece(q1, q0, c1, s1);
+    if (!inside) {
+        if (p.oob) p.oob[0] = 1;
+        return;
+    }
+    const int64_t crow = ((b * p.H + h) * p.max_len + pos) * kHd;
+    v4u* kc = (v4u*)(p.kc + crow);
+    v4u* vc = (v4u*)(p.vc + crow);
+    kc[c] = rotate_piece(k0, k1, c0, s0);
+    kc[c + 8] = rotate_piece(k1, k0, c1, s1);
+    vc[c] = v0;
+    vc[c + 8] = v1;
+}
+
 }  // namespace
 }  // namespace k3q
 
 using namespace k3q;
+
+extern "C" int k3q_rope_cache(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t T, int64_t H,
+                              int64_t head_dim, int64_t max_len, const void* cos_table, const void* sin_table,
+                              const int64_t* pos, void* k_cache, void* v_cache, void* q_out, int* oob_flag,
+                              void* stream) {
+    if (dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
+    if (B < 0 || T < 0 || H <= 0 || head_dim != kHd || max_len <= 0 || max_len >= (1 << 30) || T >= (1 << 30) ||
+        H >= (1 << 20))
+        return K3Q_ERR_SHAPE;
+    if (B == 0 || T == 0) return K3Q_OK;
+    if (B > (int64_t(1) << 33) / T / H) return K3Q_ERR_SHAPE;
+    if (!q || !k || !v || !cos_table || !sin_table || !pos || !k_cache || !v_cache || !q_out) return K3Q_ERR_NULL;
+    if (!aligned_to(q, 16) || !aligned_to(k, 16) || !aligned_to(v, 16) || !aligned_to(cos_table, 16) ||
+        !aligned_to(sin_table, 16) || !aligned_to(pos, 8) || !aligned_to(k_cache, 16) || !aligned_to(v_cache, 16) ||
+        !aligned_to(q_out, 16))
+        return K3Q_ERR_ALIGN;
+    RopeParams p;
+    p.q = (const uint16_t*)q;
+    p.k = (const uint16_t*)k;
+    p.v = (const uint16_t*)v;
+    p.cos_t = (const uint16_t*)cos_table;
+    p.sin_t = (const uint16_t*)sin_table;
+    p.pos = pos;
+    p.kc = (uint16_t*)k_cache;
+    p.vc = (uint16_t*)v_cache;
+    p.out = (uint16_t*)q_out;
+    p.oob = oob_flag;
+    p.heads = B * T * H;
+    p.T = (int)T;
+    p.H = (int)H;
+    p.max_len = (int)max_len;
+    rope_cache_rows<<<(unsigned)((p.heads * 8 + 255) / 256), 256, 0, (hipStream_t)stream>>>(p);
+    return launch_status();
+}
 
 extern "C" int k3q_decode_attention(const void* q, const void* k, const void* v, int dtype, int64_t B,
                                     int64_t H, int64_t head_dim, int64_t max_len, const void* cos_table,

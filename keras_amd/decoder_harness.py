@@ -114,13 +114,18 @@ class DecoderBlock(Layer):
             # one position: rotation, cache update and attention in one launch (5 launches per block)
             a = kops.decode_attention(q, k, v, tables[0], tables[1], pos, cache[0], cache[1], oob_flag=oob_flag)
         else:
-            # one rotation over the query and key heads together (half the elementwise launches)
             cos, sin, mask = rows()
-            qk = apply_rope(torch.cat((q, k), dim=2), cos, sin)
-            q, k = qk[:, :, : self.n_heads], qk[:, :, self.n_heads:]
             kc, vc = cache
-            kc.index_copy_(2, pos, k.transpose(1, 2))
-            vc.index_copy_(2, pos, v.transpose(1, 2))
+            if (tables is not None and pos.is_contiguous()
+                    and kops.rope_cache_supported(q, k, v, tables[0], tables[1], kc, vc)):
+                # rotation and cache update in one launch, the bits of the sequence below
+                q = kops.rope_cache(q, k, v, tables[0], tables[1], pos, kc, vc, oob_flag=oob_flag)
+            else:
+                # one rotation over the query and key heads together (half the elementwise launches)
+                qk = apply_rope(torch.cat((q, k), dim=2), cos, sin)
+                q, k = qk[:, :, : self.n_heads], qk[:, :, self.n_heads:]
+                kc.index_copy_(2, pos, k.transpose(1, 2))
+                vc.index_copy_(2, pos, v.transpose(1, 2))
             a = torch.nn.functional.scaled_dot_product_attention(
                 q.transpose(1, 2), kc, vc, attn_mask=mask[None, None]).transpose(1, 2)
         # (the residual rides in the projection's bias slot where it can, same bits as the add)

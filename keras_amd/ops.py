@@ -1230,6 +1230,43 @@ def decode_attention(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_f
     return out
 
 
+def rope_cache_supported(q, k, v, cos_table, sin_table, cache_k, cache_v):
+    """bfloat16, head width 128, caches and tables that are contiguous, all on one device."""
+    return (q.dim() == 4 and q.shape[-1] == 128 and q.shape[1] > 0 and k.shape == q.shape and v.shape == q.shape
+            and cache_k.is_contiguous() and cache_v.is_contiguous()
+            and tuple(cos_table.shape) == (cache_k.shape[2], 128) and sin_table.shape == cos_table.shape
+            and cos_table.is_contiguous() and sin_table.is_contiguous()
+            and all(t.is_cuda and t.device == q.device and t.dtype == torch.bfloat16
+                    for t in (q, k, v, cos_table, sin_table, cache_k, cache_v)))
+
+
+def rope_cache(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_flag=None):
+    """Rotate q and k `[B, T, H, 128]` at the positions `pos` `[T]` (int64, on the device), write the rotated keys and
+    the values into the caches `[B, H, max_len, 128]` at those rows, return the rotated queries: the torch sequence
+    of rotation and two `index_copy_` in one launch, the same bits.  Positions outside the cache: as
+    `decode_attention`, without its own check."""
+    _lib.require_device(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_flag)
+    B, T, H, hd = q.shape
+    max_len = cache_k.shape[2]
+    if not rope_cache_supported(q, k, v, cos_table, sin_table, cache_k, cache_v):
+        raise ValueError("rope_cache takes bfloat16 q, k, v [B, T, H, 128] and contiguous caches and tables")
+    if tuple(cache_k.shape) != (B, H, max_len, hd) or cache_v.shape != cache_k.shape:
+        raise ValueError(f"caches must be [B, H, max_len, hd], got {tuple(cache_k.shape)}")
+    if pos.dtype != torch.int64 or tuple(pos.shape) != (T,) or not pos.is_contiguous():
+        raise ValueError("pos must hold T contiguous int64 values on the device")
+    if oob_flag is not None and (oob_flag.dtype != torch.int32 or oob_flag.numel() != 1):
+        raise ValueError("oob_flag must be one int32 value on the device")
+    q, k, v = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+               for t in (q, k, v))
+    out = torch.empty_like(q)
+    rc = _lib.load().k3q_rope_cache(
+        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.dtype_code(q.dtype), B, T, H, hd, max_len, _lib.ptr(cos_table),
+        _lib.ptr(sin_table), _lib.ptr(pos), _lib.ptr(cache_k), _lib.ptr(cache_v), _lib.ptr(out), _lib.ptr(oob_flag),
+        _lib.stream_ptr(q.device))
+    _lib.check(rc, "k3q_rope_cache")
+    return out
+
+
 def _rows_view(t):
     """[rows, dim] view of a tensor whose last axis is contiguous and whose leading axes collapse
     into one stride (else a contiguous copy): (tensor, rows, dim, row stride in elements)."""
