@@ -87,6 +87,12 @@ int k3q_weight_quantize_grouped(const void* x, int x_dtype, int64_t K, int64_t N
                                 float epsilon, float range_lo, float range_hi, int8_t* q, void* scale,
                                 int8_t* zero, void* stream);
 
+/* The int4 form with its integers packed as k3q_pack_int4 packs them along N: range [-8, 7], packed [K, N / 2], the same
+ * bits as the two calls.  N % 4 == 0, block_size <= 128, epsilon > 0, x aligned to four values, packed to 4 bytes;
+ * K3Q_ERR_SHAPE otherwise. */
+int k3q_weight_quantize_grouped_int4(const void* x, int x_dtype, int64_t K, int64_t N, int64_t block_size,
+                                     float epsilon, int8_t* packed, void* scale, int8_t* zero, void* stream);
+
 /*
  * pack_int4 along the middle axis of a contiguous [outer, len, inner] int8 or
  * uint8 tensor -> [outer, ceil(len/2), inner]; byte = (lo & 15) | ((hi & 15) << 4),

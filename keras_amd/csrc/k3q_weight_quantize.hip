@@ -215,24 +215,36 @@ __global__ __launch_bounds__(kWqT) void grouped_zp(GroupedParams p) {
 // (correctly rounded) is at hand.  r = x * (1 / s) lies within 3 * 2^-24 |r| of the correctly rounded
 // quotient t, so rint(t) = rint(r) unless r is that close to a half-integer; there (and for
 // anything that is not a number) the division is done.  The margin used is 2^-20 |r|.
-__device__ __forceinline__ float rint_quotient(float x, float s, float inv_s) {
-    const float r = x * inv_s;
-    float n = rintf(r);
-    const float d = fabsf(r - n);
-    if (!(0.5f - d > fabsf(r) * 0x1p-20f)) n = rintf(x / s);
-    return n;
+// Four columns of a row share one branch (a value in 2^15 takes it; the quotient is right for all of them).
+__device__ __forceinline__ void rint_quotients(const float (&x)[4], const float (&s)[4], const float (&inv_s)[4],
+                                               float (&n)[4]) {
+    bool safe = true;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float r = x[e] * inv_s[e];
+        n[e] = rintf(r);
+        safe &= 0.5f - fabsf(r - n[e]) > fabsf(r) * 0x1p-20f;
+    }
+    if (!safe) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) n[e] = rintf(x[e] / s[e]);
+    }
 }
 
 // The same for groups of up to kHeldY * kHeldRows rows with N a multiple of 4.  A thread keeps its
 // rows in registers between the two passes, so memory sees x once (the groups resident on the chip
 // at one time are far larger than its caches, and the generic kernel's second read comes from
-// memory again); the integers come from rint_quotient.  A workgroup walks work items (column
+// memory again); the integers come from rint_quotients.  A workgroup walks work items (column
 // tile, group) at a stride of the grid and asks for the next item's rows before it works on the
 // current one: with one item per workgroup the whole chip alternates between loading and computing
 // (the registers allow one or two workgroups per CU), and neither memory nor the vector units see
 // more than half of the time.
 constexpr int kHeldY = 8, kHeldRows = 16;
-template <bool kBF16>
+// kPacked: the integers leave as int4 pairs along N (k3q_pack_int4's bytes; q is [K, N / 2], the range fits four bits):
+// half a byte written per weight instead of one byte written, read again and packed by a launch of its own.
+// 4096 x 14336 float32, call of the layer: 152 -> 130 us (the pack launch alone was 16, and its buffer went).  What bounds
+// the kernel: the read of x (235 MB) and, with eight waves on a CU, the vector work on it, which overlap only in part.
+template <bool kBF16, bool kPacked>
 __global__ __launch_bounds__(kWqX * kHeldY) void grouped_zp_held(GroupedParams p, int col_tiles, int items) {
     __shared__ float lo_s[2][kHeldY][kWqX * 4], hi_s[2][kHeldY][kWqX * 4];
     const int tx = threadIdx.x % kWqX, ty = threadIdx.x / kWqX;
@@ -301,11 +313,16 @@ __global__ __launch_bounds__(kWqX * kHeldY) void grouped_zp_held(GroupedParams p
         for (int j = 0; j < kHeldRows; ++j) {
             const int i = ty + j * kHeldY;
             if (i < p.block && r0 + i < p.K) {
+                float n[4];
                 int v[4];
+                rint_quotients(rows[j], scale, inv, n);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    v[e] = (int)__builtin_amdgcn_fmed3f(rint_quotient(rows[j][e], scale[e], inv[e]) + zero[e], p.qmin, p.qmax);
-                store_q<4>(p.q, (r0 + i) * p.N + col, v);
+                for (int e = 0; e < 4; ++e) v[e] = (int)__builtin_amdgcn_fmed3f(n[e] + zero[e], p.qmin, p.qmax);
+                if (kPacked)
+                    *(uint16_t*)(p.q + ((r0 + i) * p.N + col) / 2) =
+                        (uint16_t)((v[0] & 0xf) | ((v[1] & 0xf) << 4) | ((v[2] & 0xf) << 8) | ((v[3] & 0xf) << 12));
+                else
+                    store_q<4>(p.q, (r0 + i) * p.N + col, v);
             }
         }
     };
@@ -378,9 +395,9 @@ extern "C" int k3q_weight_absmax_quantize(const void* x, int x_dtype, int64_t ou
     return launch_status();
 }
 
-extern "C" int k3q_weight_quantize_grouped(const void* x, int x_dtype, int64_t K, int64_t N, int64_t block_size,
-                                           float epsilon, float range_lo, float range_hi, int8_t* q,
-                                           void* scale, int8_t* zero, void* stream) {
+static int run_weight_quantize_grouped(const void* x, int x_dtype, int64_t K, int64_t N, int64_t block_size,
+                                       float epsilon, float range_lo, float range_hi, int8_t* q, bool packed,
+                                       void* scale, int8_t* zero, void* stream) {
     if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
     if (K < 0 || N < 0 || block_size <= 0 || block_size > (1 << 20)) return K3Q_ERR_SHAPE;
     if (range_lo < -128.f || range_hi > 127.f || range_lo >= range_hi) return K3Q_ERR_RANGE;
@@ -411,13 +428,30 @@ extern "C" int k3q_weight_quantize_grouped(const void* x, int x_dtype, int64_t K
     const bool held = vec && block_size <= (int64_t)kHeldY * kHeldRows && epsilon > 0.f && items < (1ll << 30);
     if (held) {
         const unsigned blocks = (unsigned)(items < 256 ? items : 256);  // one resident workgroup per CU
-        if (bf) grouped_zp_held<true><<<blocks, kWqX * kHeldY, 0, s>>>(p, (int)col_tiles, (int)items);
-        else grouped_zp_held<false><<<blocks, kWqX * kHeldY, 0, s>>>(p, (int)col_tiles, (int)items);
+        void (*kernel)(GroupedParams, int, int) =
+            bf ? (packed ? grouped_zp_held<true, true> : grouped_zp_held<true, false>)
+               : (packed ? grouped_zp_held<false, true> : grouped_zp_held<false, false>);
+        kernel<<<blocks, kWqX * kHeldY, 0, s>>>(p, (int)col_tiles, (int)items);
         return launch_status();
     }
+    if (packed) return K3Q_ERR_SHAPE;
     if (bf && vec) grouped_zp<true, 4><<<grid, kWqT, 0, s>>>(p);
     else if (bf) grouped_zp<true, 1><<<grid, kWqT, 0, s>>>(p);
     else if (vec) grouped_zp<false, 4><<<grid, kWqT, 0, s>>>(p);
     else grouped_zp<false, 1><<<grid, kWqT, 0, s>>>(p);
     return launch_status();
+}
+
+extern "C" int k3q_weight_quantize_grouped(const void* x, int x_dtype, int64_t K, int64_t N, int64_t block_size,
+                                           float epsilon, float range_lo, float range_hi, int8_t* q,
+                                           void* scale, int8_t* zero, void* stream) {
+    return run_weight_quantize_grouped(x, x_dtype, K, N, block_size, epsilon, range_lo, range_hi, q, false, scale, zero,
+                                       stream);
+}
+
+extern "C" int k3q_weight_quantize_grouped_int4(const void* x, int x_dtype, int64_t K, int64_t N, int64_t block_size,
+                                                float epsilon, int8_t* packed, void* scale, int8_t* zero,
+                                                void* stream) {
+    return run_weight_quantize_grouped(x, x_dtype, K, N, block_size, epsilon, -8.f, 7.f, packed, true, scale, zero,
+                                       stream);
 }

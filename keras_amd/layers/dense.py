@@ -370,13 +370,10 @@ class Dense(Layer):
                 )
                 kernel_value_int4, kernel_scale = weight_quantizer(as_tensor(self._kernel), to_numpy=True)
                 kernel_scale = torch.squeeze(kernel_scale, dim=0)
+                packed, _, _ = quantizers.pack_int4(kernel_value_int4.to(self.device), axis=-1)
             else:
-                kernel_value_int4, kernel_scale, kernel_zero = (
-                    quantizers.abs_max_quantize_grouped_with_zero_point(
-                        as_tensor(self._kernel), block_size=block_size, to_numpy=True
-                    )
-                )
-            packed, _, _ = quantizers.pack_int4(kernel_value_int4.to(self.device), axis=-1)
+                packed, kernel_scale, kernel_zero = quantizers.quantize_and_pack_grouped(
+                    as_tensor(self._kernel), block_size, self.device)
             self._drop_float_kernel()
             self.quantized_build(kernel_shape, mode, config)
             self._kernel.assign(packed)

@@ -491,11 +491,10 @@ class EinsumDense(Layer):
                     flat, axis=0, value_range=(-8, 7), dtype="int8", to_numpy=True
                 )
                 kernel_scale = torch.squeeze(kernel_scale, dim=0)
+                kernel_value, _, _ = quantizers.pack_int4(q4.to(self.device), axis=-1)
             else:
-                q4, kernel_scale, kernel_zero = quantizers.abs_max_quantize_grouped_with_zero_point(
-                    flat, block_size=block_size, to_numpy=True
-                )
-            kernel_value, _, _ = quantizers.pack_int4(q4.to(self.device), axis=-1)
+                kernel_value, kernel_scale, kernel_zero = quantizers.quantize_and_pack_grouped(
+                    flat, block_size, self.device)
         else:
             raise self._quantization_mode_error(mode)
         self._variables = [v for v in self._variables if v is not self._kernel]

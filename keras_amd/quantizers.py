@@ -307,6 +307,27 @@ def abs_max_quantize_grouped_with_zero_point(
     return qt, st, zt
 
 
+def quantize_and_pack_grouped(inputs, block_size, device):
+    """`abs_max_quantize_grouped_with_zero_point(inputs, block_size, to_numpy=True)` and `pack_int4` of its integers
+    along the last axis: `(packed, scale, zero)`.  On the device one launch where the shape allows it (the integers
+    then never exist one per byte), else the two calls; the same bits."""
+    if (_on_device(inputs) and inputs.dim() == 2 and inputs.shape[1] % 4 == 0 and 0 < block_size <= 128
+            and inputs.numel() > 0):
+        x = inputs.contiguous()
+        if x.data_ptr() % 16 == 0:
+            K, N = x.shape
+            packed = torch.empty((K, N // 2), dtype=torch.int8, device=x.device)
+            st = torch.empty((math.ceil(K / block_size), N), dtype=x.dtype, device=x.device)
+            zt = torch.empty(st.shape, dtype=torch.int8, device=x.device)
+            rc = _lib.load().k3q_weight_quantize_grouped_int4(
+                _lib.ptr(x), _lib.dtype_code(x.dtype), K, N, int(block_size), float(EPSILON), _lib.ptr(packed),
+                _lib.ptr(st), _lib.ptr(zt), _lib.stream_ptr(x.device))
+            _lib.check(rc, "k3q_weight_quantize_grouped_int4")
+            return packed, st, zt
+    q, st, zt = abs_max_quantize_grouped_with_zero_point(inputs, block_size=block_size, to_numpy=True)
+    return pack_int4(q.to(device), axis=-1)[0], st, zt
+
+
 def _packing_dtype(dtype):
     if dtype not in ("int8", "uint8"):
         raise ValueError(
