@@ -191,7 +191,11 @@ __device__ __forceinline__ float descale_f(float acc, float sb, float bv, bool h
 // of [row][chunk]: the eight rows of a block fetch one chunk from 128 contiguous bytes of the copy.
 // The chunk position is flipped in every second block (neighbouring blocks then sit in different
 // halves of the banks for one fragment read), and a K step is still one XOR on the fragment address.
-template <class T, int kKind, bool kBF16, bool kExact, bool kBStrip = false>
+// kHalfTail (with kBStrip): K is an odd multiple of 64 (widths like 1600 or 960).  The last stage has one half: the
+// lanes that would fetch the other one fetch the first again, and its two K steps are left out.  Padding both
+// operands to 128 in scratch instead cost two launches per call (graph nodes, float32 results, us: 1000 x 1600 x 6400
+// 37.5 -> 24.6, 64 rows 32.0 -> 15.4, 4096 rows 86.6 -> 76.9; 500 x 4544 x 4544 40.6 -> 30.5).
+template <class T, int kKind, bool kBF16, bool kExact, bool kBStrip = false, bool kHalfTail = false>
 __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
     constexpr int kBM = T::kBM, kBN = T::kBN, kWavesN = T::kWavesN, kThreads = T::kThreads;
     constexpr int kWN = T::kWN, kWM = T::kWM, kNBlk = T::kNBlk, kMBlk = T::kMBlk;
@@ -253,12 +257,21 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
         // (all DMA instructions of a wave belong to the same operand: kDmaA is a multiple of kDmaPerWave)
         static_assert(kDmaA % kDmaPerWave == 0, "a wave's DMA instructions fill one operand");
         const int kstep = (kBStrip && wave * kDmaPerWave >= kDmaA) ? 2048 : kBK;
+        const int kt_first = sp * p.kt_split;  // this split's stages (all of K without a split)
+        const int kt_all = (int)((p.row_bytes + (kHalfTail ? kBK / 2 : 0)) / kBK);
+        const int KT = min(p.kt_split, kt_all - kt_first);
+        // the stage with one half, and how far back a lane of the missing half (chunks 4 ... 7) goes in it
+        const int kt_half = kHalfTail && kt_first + KT == kt_all ? KT - 1 : -1;
+        const int back = !kHalfTail ? 0
+                         : wave * kDmaPerWave >= kDmaA ? (lane >= 32 ? 1024 : 0)
+                                                       : (((lane >> 2) ^ (lane >> 5)) & 1) * 64;
         auto issue_stage = [&](int kt) {
             char* dst = lds + (kt % kStages) * kStageBytes + wave * kDmaPerWave * 1024;
+            const int64_t at = (int64_t)kt * kstep - (kHalfTail && kt == kt_half ? back : 0);
 #pragma unroll
             for (int d = 0; d < kDmaPerWave; ++d) {
                 __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void*)(src[d] + (int64_t)kt * kstep),
+                    (const __attribute__((address_space(1))) void*)(src[d] + at),
                     (__attribute__((address_space(3))) void*)(dst + d * 1024), 16, 0, 0);
             }
         };
@@ -303,8 +316,6 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
         // matrix core has work queued while waves meet.  At that barrier every wave holds its
         // last fragments of stage kt in registers, so stage kt+kStages may be DMA-ed over stage kt, and
         // stage kt+1 (whose DMA every wave has waited for) may be read.
-        const int kt_first = sp * p.kt_split;  // this split's stages (all of K without a split)
-        const int KT = min(p.kt_split, (int)(p.row_bytes / kBK) - kt_first);
         issue_stage(0);
         if constexpr (kStages == 2) {
             if (KT > 1) {
@@ -334,7 +345,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
         auto issue_one = [&](int kt, int d) {
             char* dst = lds + (kt % kStages) * kStageBytes + wave * kDmaPerWave * 1024;
             __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void*)(src[d] + (int64_t)kt * kstep),
+                (const __attribute__((address_space(1))) void*)(src[d] + (int64_t)kt * kstep -
+                                                                (kHalfTail && kt == kt_half ? back : 0)),
                 (__attribute__((address_space(3))) void*)(dst + d * 1024), 16, 0, 0);
         };
         auto mma_half = [&](int ks, int half, int kt) {
@@ -394,6 +406,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
                 mma_half(ks, 1, kt);
                 __builtin_amdgcn_s_setprio(0);
                 __builtin_amdgcn_sched_barrier(0);
+                if (kHalfTail && ks == kKSteps / 2 - 1 && kt == kt_half) break;
             }
         }
 
@@ -874,11 +887,11 @@ inline int64_t split_workspace_bytes(int64_t M, int64_t N, int64_t row_bytes) {
     return splits > 1 ? (int64_t)splits * M * N * 4 : 0;
 }
 
-template <class T, int kKind, bool kBF16, bool kExact, bool kBStrip = false>
+template <class T, int kKind, bool kBF16, bool kExact, bool kBStrip = false, bool kHalfTail = false>
 int launch_tile(GemmParams p, hipStream_t s) {
     // more than 64 KiB of dynamic LDS needs the attribute raised once per kernel
     static const bool raised =
-        hipFuncSetAttribute((const void*)gemm_mfma<T, kKind, kBF16, kExact, kBStrip>,
+        hipFuncSetAttribute((const void*)gemm_mfma<T, kKind, kBF16, kExact, kBStrip, kHalfTail>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, T::kLdsBytes) == hipSuccess;
     if (!raised) return K3Q_ERR_LAUNCH;
     p.tiles_m = (int)((p.M + T::kBM - 1) / T::kBM);
@@ -886,7 +899,7 @@ int launch_tile(GemmParams p, hipStream_t s) {
     // one resident set of workgroups (as many as fit on the chip at once, a multiple of the
     // 8 XCDs); each walks its share of the tiles
     const int resident = cu_count() * (T::kLdsBytes <= 64 * 1024 ? 2 : 1) / 8 * 8;
-    const int stages = (int)(p.row_bytes / kBK);
+    const int stages = (int)((p.row_bytes + kBK - 1) / kBK);
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
     int splits = (p.N % 4) ? 1 : choose_splits(tiles, stages, resident);
     // partials need room and 16-byte rows (no split for N % 4 != 0, above)
@@ -899,7 +912,7 @@ int launch_tile(GemmParams p, hipStream_t s) {
     const int64_t total = tiles * p.splits;
     int64_t grid = ((total + 7) / 8) * 8;
     if (resident >= 8 && grid > resident) grid = resident;
-    gemm_mfma<T, kKind, kBF16, kExact, kBStrip><<<(unsigned)grid, T::kThreads, T::kLdsBytes, s>>>(p);
+    gemm_mfma<T, kKind, kBF16, kExact, kBStrip, kHalfTail><<<(unsigned)grid, T::kThreads, T::kLdsBytes, s>>>(p);
     if (p.splits > 1) {
         const int64_t threads = p.M * (p.N / 4);
         gemm_split_reduce<kKind, kBF16, kExact><<<(unsigned)((threads + 255) / 256), 256, 0, s>>>(p);
@@ -917,6 +930,11 @@ int launch_mfma(const GemmParams& p, hipStream_t s) {
     const bool large = large_tiles >= kLargeTileMinTiles;
     const bool deep = deep_tile(((p.M + 127) / 128) * ((p.N + 127) / 128), p.row_bytes / kBK, cu_count());
     if constexpr (kKind == kKindI8) {
+        if (p.b_strip && p.row_bytes % kBK) {
+            if (large) return launch_tile<TileLarge, kKind, kBF16, kExact, true, true>(p, s);
+            if (deep) return launch_tile<TileDeep, kKind, kBF16, kExact, true, true>(p, s);
+            return launch_tile<TileSmall, kKind, kBF16, kExact, true, true>(p, s);
+        }
         if (p.b_strip) {
             if (large) return launch_tile<TileLarge, kKind, kBF16, kExact, true>(p, s);
             if (deep) return launch_tile<TileDeep, kKind, kBF16, kExact, true>(p, s);
@@ -984,7 +1002,7 @@ extern "C" int64_t k3q_gemm_i8_workspace_bytes(int64_t M, int64_t N, int64_t K) 
 }
 
 extern "C" int64_t k3q_gemm_i8_split_bytes(int64_t M, int64_t N, int64_t K) {
-    return K > 0 && N > 0 ? split_workspace_bytes(M, N, K) : 0;
+    return K > 0 && N > 0 ? split_workspace_bytes(M, N, (K + kBK - 1) / kBK * kBK) : 0;
 }
 
 extern "C" int k3q_prepack_kernel_i8(const int8_t* kernel, int64_t K, int64_t N, int8_t* prepacked,
@@ -1040,9 +1058,10 @@ extern "C" int k3q_gemm_i8(const int8_t* a, const int8_t* b, int b_layout, int64
         return gemm_i8_skinny_run(a, b, M, N, K, a_scale, b_scale, bias, bf16, flags, y, acc_out,
                                   workspace, workspace_bytes, s);
     // K % 128 != 0 (model widths like 1600 or 960): both operands are copied into scratch with
-    // their rows zero-padded to the tile's K step; zeros add nothing, the result is the same
+    // their rows zero-padded to the tile's K step; zeros add nothing, the result is the same.  (From the strip-linear
+    // copy, whose units are 64 of K, the tile kernel takes K % 64 as it lies.)
     const int64_t Kpad = (K + kBK - 1) / kBK * kBK;
-    const bool padded = Kpad != K;
+    const bool padded = b_layout == 2 ? (K % 64) != 0 : Kpad != K;
     bool fast = (padded ? (workspace && aligned_to(workspace, 16) && workspace_bytes >= (M + N) * Kpad)
                         : (aligned_to(a, 16) && aligned_to(b, 16))) &&
                 (!y || aligned_to(y, 4 * el)) && (!acc_out || aligned_to(acc_out, 16)) &&

@@ -453,7 +453,7 @@ class Dense(Layer):
         """The derived copy of the int8 kernel that the tile GEMM reads, as a keyword of
         `ops.int8_matmul`: the decode kernel's strip-linear copy where the tile kernel can take it
         (one derived copy per layer; same bits and speed as from a [N, K] copy), else the [N, K] copy."""
-        if input_dim % 128 == 0:
+        if input_dim % 64 == 0:
             return dict(strip=self._cached("w8s", self._kernel, kops.int8_strip_copy))
         return dict(prepacked=self._cached("prepacked", self._kernel, kops.prepack_int8_kernel))
 

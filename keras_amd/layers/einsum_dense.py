@@ -668,7 +668,7 @@ class EinsumDense(Layer):
             # the tile GEMM's operand: the decode kernel's strip-linear copy where it can take it
             # (one derived copy per layer), else the [N, K] copy
             **(dict(strip=self._cached("w8s", self._kernel, lambda t: kops.int8_strip_copy(kernel_matrix(t))))
-               if x2.shape[1] % 128 == 0 else
+               if x2.shape[1] % 64 == 0 else
                dict(prepacked=self._cached("prepacked", self._kernel,
                                            lambda t: kops.prepack_int8_kernel(kernel_matrix(t))))),
         )

@@ -730,7 +730,7 @@ def int8_matmul(a, kernel, a_scale=None, kernel_scale=None, bias=None, out_dtype
     Returns y (out_dtype [M, N]); with want_acc also the int32 accumulators.
     `prepacked` is the cached result of `prepack_int8_kernel(kernel)`; without it
     the [N, K] copy is rebuilt in scratch memory on every call.  `strip` is the cached
-    `int8_strip_copy(kernel)` of the decode kernel: with K % 128 == 0 the tile kernel reads
+    `int8_strip_copy(kernel)` of the decode kernel: with K % 64 == 0 the tile kernel reads
     that copy instead (the same bits), so a layer need not keep a prepacked one beside it.
     `kernel` may be None when `strip` serves the call (more than 8 rows, K % 128 == 0) and
     `kernel_shape = (K, N)` is given.
@@ -764,7 +764,9 @@ def int8_matmul(a, kernel, a_scale=None, kernel_scale=None, bias=None, out_dtype
     lib = _lib.load()
     skinny = M <= SKINNY_MAX_ROWS and N % 16 == 0 and K % 8 == 0
     nbytes = lib.k3q_gemm_i8_workspace_bytes(M, N, K)
-    if strip is not None and not skinny and K % 128 == 0:
+    if strip is not None and not skinny and K % 64 == 0:
+        # (the tile kernel reads scales and bias in 16-byte pieces)
+        sa, sb, bias = (t.clone() if t is not None and t.data_ptr() % 16 else t for t in (sa, sb, bias))
         if strip.numel() != lib.k3q_w8s_shadow_bytes(K, N):
             raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
         b, layout = strip, 2
