@@ -246,8 +246,15 @@ def require_device(*tensors):
             )
 
 
+def raw_stream(device=None):
+    """Handle of the current stream of `device`.  (`torch.cuda.current_stream` builds a Stream object around the same
+    handle: 4 us a call, where a decode-sized layer call is 12 to 30.)"""
+    index = device.index if device is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
 def stream_ptr(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(raw_stream(device))
 
 
 def ptr(t):

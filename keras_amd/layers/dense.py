@@ -104,7 +104,7 @@ def kmajor_rows(rows, units, input_dim=0):
     return low <= rows <= KMAJOR_MAX_ROWS
 
 
-def int4_strip_rows_route(x2, units, block_size):
+def int4_strip_rows_route(dtype, rows, input_dim, units, block_size):
     """Whether an int4 call of these rows goes to `ops.int4_matmul_strip_rows`: what the strip kernel proper
     (`ops.int4_strip_supported`) does not take of up to 16 rows -- float32 rows, narrow, short or ragged kernels.
     A launch costs what one of the kernel on the stored weights costs, which takes 8 float32 or 16 bfloat16 rows
@@ -112,13 +112,12 @@ def int4_strip_rows_route(x2, units, block_size):
     in three launches; K=N=4096 8.2 / 9.5 / 18.6 against 4.7 / 6.6 / 12.3; bfloat16 K=1600, N=6400 7.1 / 8.4 / 10.2
     against 5.4 / 5.9 / 6.1; K=11008, N=4096 at 8 rows 16.1 against 16.5 in two launches).  Where N % 8 or K % 16
     leave only the kernel of one output per thread (N = 5247: 220 ... 490 us) every shape goes here."""
-    if not (x2.is_cuda and x2.dtype in (torch.float32, torch.bfloat16) and 0 < x2.shape[0] <= kops.STRIP_MAX_ROWS):
+    if not (dtype in (torch.float32, torch.bfloat16) and 0 < rows <= kops.STRIP_MAX_ROWS):
         return False
-    rows, input_dim = x2.shape
-    launches = kops.int4_strip_rows_launches(x2.dtype, rows, input_dim, units, block_size)
+    launches = kops.int4_strip_rows_launches(dtype, rows, input_dim, units, block_size)
     if units % 8 or input_dim % 16:
         return launches > 0
-    return 0 < launches <= (-(-rows // 8) if x2.dtype == torch.float32 else 1)
+    return 0 < launches <= (-(-rows // 8) if dtype == torch.float32 else 1)
 
 
 def strip_rows_params(layer, dtype, input_dim, units, block_size):
@@ -142,7 +141,7 @@ def strip_rows_params(layer, dtype, input_dim, units, block_size):
 TILE_ROWS_MAX_F32 = 768
 
 
-def int4_tile_rows_route(x2, units, block_size):
+def int4_tile_rows_route(dtype, rows, input_dim, units, block_size):
     """Whether an int4 call of more rows than the decode kernels take goes to `ops.int4_matmul_tiles_rows`: shapes
     that neither the tile kernel proper (`ops.int4_kmajor_supported`) nor the GEMM on the de-quantised kernel takes
     (K % 128, N % 64), which went in passes of 32 bfloat16 or 8 float32 rows over the kernel, and float32 rows up to
@@ -150,14 +149,13 @@ def int4_tile_rows_route(x2, units, block_size):
     float32 17 rows 25 / 17, 300 307 / 38; one pass, up to 32 bfloat16 rows of a kernel this small, is as good: 15.7 /
     15.7).  Where N % 8 or K % 16 leave only the kernel of one output per thread (K=2048, N=5247: 480 us at 32
     rows, 6.1 ms at 1200, against 15 and 82) every shape goes here."""
-    rows, input_dim = x2.shape
-    if not (x2.is_cuda and x2.dtype in (torch.float32, torch.bfloat16) and rows > kops.STRIP_MAX_ROWS
+    if not (dtype in (torch.float32, torch.bfloat16) and rows > kops.STRIP_MAX_ROWS
             and kops.int4_tiles_rows_supported(input_dim, units, block_size)):
         return False
     if units % 8 or input_dim % 16:
         return True
     gemm = input_dim % 128 == 0 and units % 64 == 0
-    if x2.dtype == torch.float32:
+    if dtype == torch.float32:
         return not gemm or rows <= TILE_ROWS_MAX_F32
     return not gemm and (rows >= KMAJOR_MIN_ROWS or kmajor_rows(rows, units, input_dim))
 
@@ -474,7 +472,7 @@ class Dense(Layer):
                 y = self.activation(y)
             return y
         lead = inputs.shape[:-1]
-        x2 = inputs.reshape(-1, inputs.shape[-1])
+        x2 = inputs if inputs.dim() == 2 else inputs.reshape(-1, inputs.shape[-1])
         M, N = x2.shape[0], self.units
         exact = self.exact_epilogue
         if exact is None:
@@ -486,7 +484,7 @@ class Dense(Layer):
                 self._read_cached("kernel_scale", self.kernel_scale), bias=self._call_bias(),
                 epsilon=self.inputs_quantizer.epsilon, value_range=self.inputs_quantizer.value_range,
                 quantize=lambda rows: quantize_rows(self.inputs_quantizer, rows))
-            y = y.reshape(*lead, N)
+            y = y if len(lead) == 1 else y.reshape(*lead, N)
             if self.activation is not None:
                 y = self.activation(y)
             return y
@@ -498,7 +496,7 @@ class Dense(Layer):
             out_dtype=to_torch_dtype(self.compute_dtype),
             exact_epilogue=exact, **self._tile_operand(x2.shape[1]),
         )
-        y = y.reshape(*lead, N)
+        y = y if len(lead) == 1 else y.reshape(*lead, N)
         if self.activation is not None:
             y = self.activation(y)
         return y
@@ -556,7 +554,7 @@ class Dense(Layer):
                 inputs, strip["shadow"], self._orig_output_dim, kernel_scale=strip.get("kernel_scale"),
                 gparams=strip.get("gparams"), block_size=block_size if grouped else None,
                 bias=None if per_row else bias, addend=bias if per_row else None)
-        elif int4_strip_rows_route(inputs.reshape(rows, inputs.shape[-1]), self._orig_output_dim,
+        elif int4_strip_rows_route(inputs.dtype, rows, inputs.shape[-1], self._orig_output_dim,
                                    block_size if grouped else None):
             y = kops.int4_matmul_strip_rows(inputs, block_size=block_size if grouped else None, bias=self._call_bias(),
                                             **self._strip_rows_operands(inputs, grouped, block_size))
@@ -581,7 +579,7 @@ class Dense(Layer):
                     block_size=block_size if grouped else None,
                     bias=self._call_bias(),
                 )
-        elif int4_tile_rows_route(inputs.reshape(rows, inputs.shape[-1]), self._orig_output_dim,
+        elif int4_tile_rows_route(inputs.dtype, rows, inputs.shape[-1], self._orig_output_dim,
                                   block_size if grouped else None):
             units = self._orig_output_dim
             y = kops.int4_matmul_tiles_rows(
@@ -664,7 +662,8 @@ class Dense(Layer):
         rows = None
         if strip is not None:
             strip["bias"] = self._call_bias()
-        elif int4_strip_rows_route(x2, self._orig_output_dim, block_size if grouped else None):
+        elif int4_strip_rows_route(x2.dtype, x2.shape[0], x2.shape[1], self._orig_output_dim,
+                                   block_size if grouped else None):
             rows = dict(self._strip_rows_operands(x2, grouped, block_size), bias=self._call_bias())
         return dict(
             x2=x2, block_size=block_size if grouped else None, strip=strip, rows=rows,

@@ -828,7 +828,7 @@ class EinsumDense(Layer):
                 gparams=strip.get("gparams"), block_size=block_size if grouped else None,
                 bias=None if per_row else bias, addend=bias if per_row else None)
             return self._finish(y2, free_shape, gv, fused)
-        if x2.dtype == cd and int4_strip_rows_route(x2, units, block_size if grouped else None):
+        if x2.dtype == cd and int4_strip_rows_route(x2.dtype, x2.shape[0], x2.shape[1], units, block_size if grouped else None):
             y2 = kops.int4_matmul_strip_rows(x2, block_size=block_size if grouped else None, bias=bias,
                                              **self._strip_rows_operands(x2, grouped, block_size))
             return self._finish(y2, free_shape, gv, fused)
@@ -849,7 +849,7 @@ class EinsumDense(Layer):
                     scale_cd, kernel_zero=as_tensor(self.kernel_zero) if grouped else None,
                     block_size=block_size if grouped else None, bias=bias)
             return self._finish(y2, free_shape, gv, fused)
-        if x2.dtype == cd and int4_tile_rows_route(x2, units, block_size if grouped else None):
+        if x2.dtype == cd and int4_tile_rows_route(x2.dtype, x2.shape[0], x2.shape[1], units, block_size if grouped else None):
             y2 = kops.int4_matmul_tiles_rows(
                 x2, self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)), units,
                 block_size=block_size if grouped else None, bias=bias, **tile_rows_operands(self, cd, units, grouped))
@@ -918,7 +918,8 @@ class EinsumDense(Layer):
         elif x2.dtype == cd:
             from keras_amd.layers.dense import int4_strip_rows_route
 
-            if int4_strip_rows_route(x2, self._int4_unpacked_column_size, block_size if grouped else None):
+            if int4_strip_rows_route(x2.dtype, x2.shape[0], x2.shape[1], self._int4_unpacked_column_size,
+                                     block_size if grouped else None):
                 rows = dict(self._strip_rows_operands(x2, grouped, block_size), bias=bias)
         return dict(
             x2=x2, block_size=block_size if grouped else None, strip=strip, rows=rows,

@@ -24,8 +24,7 @@ def _workspace(device, nbytes):
     ordered, so they can share it; calls on different streams may overlap, and two threads on
     one stream may interleave the launches of a two-kernel call, so neither shares.
     """
-    stream = torch.cuda.current_stream(device)
-    key = (device.index, stream.cuda_stream, threading.get_ident())
+    key = (device.index, _lib.raw_stream(device), threading.get_ident())
     with _scratch_lock:
         ws = _workspaces.get(key)
         if ws is None or ws.numel() < nbytes:
@@ -49,8 +48,7 @@ _counters = {}
 def _arrival_counters(device, nbytes):
     """Arrival counters of the single-launch K split: zero between calls, one set per
     (device, stream, host thread), like the workspace they go with."""
-    stream = torch.cuda.current_stream(device)
-    key = (device.index, stream.cuda_stream, threading.get_ident())
+    key = (device.index, _lib.raw_stream(device), threading.get_ident())
     with _scratch_lock:
         c = _counters.get(key)
         if c is None or c.numel() < nbytes:
@@ -62,6 +60,17 @@ def _arrival_counters(device, nbytes):
 
 
 INT4_ADDEND_MAX_ROWS = 64
+
+
+def _rows_of(x, K):
+    """x as contiguous [rows, K]."""
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
+    return x2 if x2.is_contiguous() else x2.contiguous()
+
+
+def _shaped(y, lead):
+    """[rows, N] as [*lead, N]."""
+    return y if len(lead) == 1 else y.reshape(*lead, y.shape[1])
 
 
 def _check_bias_size(bias, M, N):
@@ -97,9 +106,7 @@ def int4_matmul(x, kernel_packed, kernel_scale, orig_output_dim, kernel_zero=Non
     if kernel_scale.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
         raise TypeError("kernel_scale and bias must be read in the input's dtype")
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
-    if not x2.is_contiguous():
-        x2 = x2.contiguous()
+    x2 = _rows_of(x, K)
     M = x2.shape[0]
     _check_bias_size(bias, M, N)
     kp = kernel_packed if kernel_packed.is_contiguous() else kernel_packed.contiguous()
@@ -141,7 +148,7 @@ def int4_matmul(x, kernel_packed, kernel_scale, orig_output_dim, kernel_zero=Non
         arr = (ctypes.c_int * 4)(*[int(v) for v in plan[:4]])
         rc = lib.k3qt_gemv_w4_plan(*args, arr, _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_gemv_w4")
-    return y.reshape(*lead, N)
+    return _shaped(y, lead)
 
 
 def int4_matmul_multi(x, kernels, block_size=None):
@@ -260,8 +267,7 @@ def int4_matmul_strip(x, shadow, units, kernel_scale=None, gparams=None, block_s
     N = int(units)
     K = x.shape[-1]
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
-    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    x2 = _rows_of(x, K)
     M = x2.shape[0]
     lib = _lib.load()
     if shadow.numel() != lib.k3q_w4s_shadow_bytes(K, N):
@@ -291,7 +297,7 @@ def int4_matmul_strip(x, shadow, units, kernel_scale=None, gparams=None, block_s
                           int(block_size) if grouped else -1, _lib.ptr(b), stride, _lib.ptr(y),
                           _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_gemv_w4s")
-    return y.reshape(*lead, N)
+    return _shaped(y, lead)
 
 
 def int4_strip_rows_launches(dtype, M, K, N, block_size=None):
@@ -332,8 +338,7 @@ def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, bl
     bs = int(block_size) if grouped else -1
     K, N = x.shape[-1], int(units)
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
-    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    x2 = _rows_of(x, K)
     if x2.data_ptr() % 16:  # a view into a larger buffer
         x2 = x2.clone()
     M = x2.shape[0]
@@ -355,7 +360,7 @@ def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, bl
                                _lib.ptr(gparams) if grouped else None, bs, _lib.ptr(b), stride, _lib.ptr(y),
                                _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_gemv_w4s_rows")
-    return y.reshape(*lead, N)
+    return _shaped(y, lead)
 
 
 def int4_matmul_strip_rows_multi(x, kernels, block_size=None):
@@ -624,8 +629,7 @@ def int4_matmul_tiles_strip(x, shadow, units, kernel_scale, kernel_zero=None, bl
     if shadow.numel() != lib.k3q_w4s_shadow_bytes(K, N):
         raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
-    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    x2 = _rows_of(x, K)
     M = x2.shape[0]
     if bias is not None and bias.numel() != N:
         raise ValueError(f"bias holds {bias.numel()} values, the layer has {N} units")
@@ -641,7 +645,7 @@ def int4_matmul_tiles_strip(x, shadow, units, kernel_scale, kernel_zero=None, bl
                                _lib.ptr(bias), _lib.ptr(y), _lib.ptr(ws), ws.numel(),
                                _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_gemm_w4_strip")
-    return y.reshape(*lead, N)
+    return _shaped(y, lead)
 
 
 GEMM_EXACT_EPILOGUE = 1
@@ -676,8 +680,7 @@ def int4_matmul_tiles_rows(x, shadow, units, kernel_scale, kernel_zero=None, blo
     bs = int(block_size) if grouped else -1
     K, N = x.shape[-1], int(units)
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
-    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    x2 = _rows_of(x, K)
     if x2.data_ptr() % 16:  # a view into a larger buffer
         x2 = x2.clone()
     M = x2.shape[0]
@@ -702,7 +705,7 @@ def int4_matmul_tiles_rows(x, shadow, units, kernel_scale, kernel_zero=None, blo
     rc = lib.k3q_gemm_w4_rows(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks), _lib.ptr(kz), bs,
                               _lib.ptr(b), stride, _lib.ptr(y), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_gemm_w4_rows")
-    return y.reshape(*lead, N)
+    return _shaped(y, lead)
 
 
 def prepack_int8_kernel(kernel):
@@ -1076,8 +1079,7 @@ def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, va
         raise TypeError("kernel_scale must be read in the input's dtype")
     K, N = int(x.shape[-1]), int(units)
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
-    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    x2 = _rows_of(x, K)
     M = x2.shape[0]
     inside = (code == _lib.K3Q_BF16 and int8_strip_quantises_inside(M, K, value_range)
               and lib.k3q_dense_i8_w8s_supported(M, K, N))
@@ -1106,13 +1108,13 @@ def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, va
                                  _lib.ptr(ks), _lib.ptr(bias) if bias is not None else None, stride,
                                  _lib.ptr(y), _lib.stream_ptr(x.device))
         _lib.check(rc, "k3q_gemm_i8_w8s")
-        return y.reshape(*lead, N)
+        return _shaped(y, lead)
     rc = lib.k3q_dense_i8_w8s(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
                               _lib.ptr(bias) if bias is not None else None, stride, float(epsilon),
                               float(value_range[0]), float(value_range[1]), _lib.ptr(y),
                               _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_dense_i8_w8s")
-    return y.reshape(*lead, N)
+    return _shaped(y, lead)
 
 
 def int8_dense_strip_multi(x, kernels, epsilon=1e-7, value_range=(-127, 127), quantize=None, input_op=None,

@@ -113,11 +113,12 @@ def abs_max_quantize(
     rows = x.numel() // cols if cols else 0
     if cols == 0:
         raise ValueError("Cannot compute the max of an empty tensor.")
-    x2 = xr.reshape(rows, cols)
+    plain = rank == 2 and ax == (1,)  # rows as they lie: results in the shapes they are returned in
+    x2 = xr if plain else xr.reshape(rows, cols)
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
     q2 = torch.empty((rows, cols), dtype=torch.int8, device=x.device)
-    s1 = torch.empty((rows,), dtype=x.dtype, device=x.device)
+    s1 = torch.empty((rows, 1) if plain else (rows,), dtype=x.dtype, device=x.device)
     lib = _lib.load()
     rc = lib.k3q_absmax_quantize(
         _lib.ptr(x2), code, rows, cols, x2.stride(0) if rows > 1 else cols,
@@ -125,6 +126,8 @@ def abs_max_quantize(
         _lib.ptr(q2), _lib.ptr(s1), _lib.stream_ptr(x.device),
     )
     _lib.check(rc, "k3q_absmax_quantize")
+    if plain:
+        return q2, s1
     scale_shape = [1 if i in ax else x.shape[i] for i in range(rank)]
     if trailing:
         q = q2.reshape(x.shape)
