@@ -608,6 +608,44 @@ class ReversibleEmbedding(Embedding):
             )
         return self._soft_cap(logits.reshape(*lead, N))
 
+    def _relay_tied(self, table):
+        """The strip-linear copy of the table as the `[dim, vocab]` int4 kernel of the projection."""
+        dense = quantizers.unpack_int4(table, self._orig_output_dim, axis=-1).t().contiguous()  # int8
+        return kops.int4_strip_copy(quantizers.pack_int4(dense, axis=-1)[0], self.input_dim)
+
+    def _tied_rows_operands(self, x2, scale, grouped, block_size):
+        """Operands of `ops.int4_matmul_strip_rows` for what `_tied_strip_operands` does not take of up to 16 rows,
+        or None: float32 scales (a mixed policy's: the table's variables are read as they are and the rows are
+        promoted to them, exactly), tables the decode kernel proper does not fit.  One launch only, and not for short
+        rows, of which a workgroup walks many with little in flight (us, in place / from the copy, a cast of the rows
+        included: 4096 x 32000 grouped, float32 scales, 1 and 8 bfloat16 rows 25.6 / 20.6 and 28.6 / 22.2, float32 rows
+        29.1 / 18.4 and 62.5 / 20.0; 2048 x 32000 bfloat16 rows 14.3 / 15.0, float32 rows 16.5 / 13.5; 768 x 50257
+        11.4 / 22.6)."""
+        K, N = self._orig_output_dim, self.input_dim
+        if K < (2048 if x2.dtype == scale.dtype else 4096):
+            return None
+        if not (x2.is_cuda and x2.dtype in (torch.float32, torch.bfloat16) and scale.dtype in (torch.float32, torch.bfloat16)
+                and _promote(x2.dtype, scale.dtype) == scale.dtype and (grouped or x2.dtype == scale.dtype)
+                and 0 < x2.shape[0] <= kops.STRIP_MAX_ROWS and x2.shape[1] == K
+                and kops.int4_strip_rows_launches(scale.dtype, x2.shape[0], K, N, block_size if grouped else None) == 1):
+            return None
+        spec = dict(shadow=self._cached("w4s", self._embeddings, self._relay_tied))
+        if not grouped:
+            spec["kernel_scale"] = scale if scale.is_contiguous() else scale.contiguous()
+            return spec
+        sv, zv = self.embeddings_scale, self.embeddings_zero
+        stamp = (id(sv), sv.version, id(zv), zv.version)
+        hit = self._cache.get("w4s_rows_params")
+        if hit is None or hit[0] != stamp:
+            value = kops.int4_strip_rows_params(as_tensor(sv).t().contiguous(),
+                                                as_tensor(zv).to(torch.int8).t().contiguous(), K, N, block_size)
+            if hit is not None and hit[2].shape == value.shape and hit[2].device == value.device:
+                hit[2].copy_(value)  # (a captured graph holds the address)
+                value = hit[2]
+            hit = self._cache["w4s_rows_params"] = (stamp, None, value)
+        spec["gparams"] = hit[2]
+        return spec
+
     def _tied_strip_operands(self, x2, scale, grouped, block_size):
         """Operands of `ops.int4_matmul_strip` for the tied int4 table used as the LM head, or None
         when that route does not take these rows: the table (packed along its last axis, K of the
@@ -620,11 +658,7 @@ class ReversibleEmbedding(Embedding):
                 and kops.int4_strip_supported(x2.shape[0], K, N, block_size if grouped else None)):
             return None
 
-        def relay(table):
-            dense = quantizers.unpack_int4(table, K, axis=-1).t().contiguous()  # [dim, vocab] int8
-            return kops.int4_strip_copy(quantizers.pack_int4(dense, axis=-1)[0], N)
-
-        spec = dict(shadow=self._cached("w4s", self._embeddings, relay))
+        spec = dict(shadow=self._cached("w4s", self._embeddings, self._relay_tied))
         if grouped:
             sv, zv = self.embeddings_scale, self.embeddings_zero
             stamp = (id(sv), sv.version, id(zv), zv.version)
@@ -680,6 +714,9 @@ class ReversibleEmbedding(Embedding):
                 # Dense decode kernel
                 logits = kops.int4_matmul_strip(x2, strip["shadow"], self.input_dim, block_size=block_size if grouped else None,
                                                 kernel_scale=strip.get("kernel_scale"), gparams=strip.get("gparams"))
+            elif in_scale is None and (rows := self._tied_rows_operands(x2, scale, grouped, block_size)):
+                logits = kops.int4_matmul_strip_rows(x2.to(scale.dtype), units=self.input_dim,
+                                                     block_size=block_size if grouped else None, **rows)
             else:
                 logits = kops.int4_matmul_nk(
                     x2 if in_scale is None else x2.to(cd), as_tensor(self._embeddings), scale,
