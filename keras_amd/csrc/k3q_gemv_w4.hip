@@ -1154,9 +1154,12 @@ bool try_gemv_w4_multi(const void* x, int x_dtype, int64_t M, int64_t K, int cou
 // kernel does: tot += scale * (acc - (136 + zero) * sum_k x).
 constexpr int kKmBM = 128, kKmBN = 256, kKmStage = 64;  // tile; values of K per stage
 constexpr int kKmThreads = 512;                        // 8 waves: 2 (M) x 4 (N), 64 x 64 each
-// bfloat16 pair (24 + w, 24 + w'): the nibbles in mantissa bits 3 ... 6 of 16.0, their sign bits flipped.  (In bits
-// 0 ... 3 of 128.0, 136 + w, they cost the same and leave an offset almost six times as large to cancel.)
-constexpr u32 kKmNibbles = 0x00780078u, kKmBase = 0x41C041C0u;
+constexpr u32 kKmNibbles = 0x000F000Fu, kKmFlip = 0x00080008u, kKmExp = 0x43004300u;
+// The general form (k3q_gemm_w4_rows) puts the nibbles into mantissa bits 3 ... 6 of 16.0, their sign bits flipped: the
+// bfloat16 pair (24 + w, 24 + w').  A shift more per dword and a sixth of the offset to cancel, which the float32 sums of
+// its rows need; where the sums are rounded to bfloat16 it buys nothing and the shift shows (96 rows of 4096 x 14336:
+// 27.5 -> 27.6 us in the kernel, 0.7 % of the call).
+constexpr u32 kKmNibbles24 = 0x00780078u, kKmBase24 = 0x41C041C0u;
 
 __device__ __forceinline__ int km_swz(int row) { return (row & 6) | ((row ^ (row >> 3)) & 1); }
 
@@ -1301,7 +1304,8 @@ constexpr int kKmParScale = 0, kKmParZero = 512, kKmParSx = 768, kKmParSpare = 1
 // narrow that wide tiles leave CUs idle even at eight splits).
 // kWM: waves along M: 2 (tiles of 128 rows) or 1 (64 rows, eight waves side by side, kNB = 1).
 // kF32S: float32 scales (twice the bytes: tiles of 128 x 128 or 64 x 256 only, whose parameters still fit).
-template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB, bool kF32S = false>
+// kRows: the weights at 24 + w instead of 136 + w (above).
+template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB, bool kF32S = false, bool kRows = kF32S>
 __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
     constexpr int kWaveN = 32 * kNB, kBN = kWaveN * (8 / kWM), kBM = 64 * kWM;
     static_assert(!kF32S || (kGrouped && kBN * kBM <= 128 * 128), "parameters of a stage");
@@ -1490,7 +1494,9 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
                 for (int nb = 0; nb < kNB; ++nb) {
                     const u32 d = wq[nb][s];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) wb[nb][q] = ((q ? d >> (4 * q - 3) : d << 3) & kKmNibbles) ^ kKmBase;
+                    for (int q = 0; q < 4; ++q)
+                        wb[nb][q] = kRows ? ((q ? d >> (4 * q - 3) : d << 3) & kKmNibbles24) ^ kKmBase24
+                                          : (((d >> (4 * q)) & kKmNibbles) ^ kKmFlip) | kKmExp;
                 }
 #pragma unroll
                 for (int nb = 0; nb < kNB; ++nb)
@@ -1509,8 +1515,8 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
             }
             if (group_last) {
                 const char* par = cur + kKmXBytes + kKmWBytes;
-                // acc -= (24 + zero) * sum(x) as one more MFMA step: k = 0 ... 2 carry -16 on the
-                // kernel side, k = 3 ... 5 carry -(8 + zero) (any int8 zero point is exact in
+                // acc -= (136 + zero) * sum(x) as one more MFMA step: k = 0 ... 2 carry -128 on the
+                // kernel side (kRows: -16), k = 3 ... 5 carry -(8 + zero) (any int8 zero point is exact in
                 // bfloat16), both against the three bfloat16 parts of the sum of x; products of
                 // two bfloat16 are exact in float32, so the cancellation happens in the accumulator
                 v4u xs[2], wz[kNB];
@@ -1528,8 +1534,9 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
                     int zp = 0;
                     if (kGrouped) zp = *(const int8_t*)(par + kParZero + wn * kWaveN + nb * 32 + i);
                     const u32 cz = __float_as_uint(-(float)(8 + zp)) >> 16;
-                    wz[nb][0] = 0xC180C180u;                              // -16, -16
-                    wz[nb][1] = 0xC180u | (cz << 16);                     // -16, -(8 + zero)
+                    constexpr u32 kBase = kRows ? 0xC180u : 0xC300u;      // -16, -128
+                    wz[nb][0] = kBase | (kBase << 16);
+                    wz[nb][1] = kBase | (cz << 16);                       // ..., -(8 + zero)
                     wz[nb][2] = cz | (cz << 16);
                     wz[nb][3] = 0;
                 }
@@ -1793,8 +1800,9 @@ extern "C" int64_t k3q_gemm_w4_kmajor_workspace_bytes(int64_t M, int64_t K, int6
     return ((K / gsize) * M * 8 + 255) / 256 * 256 + (int64_t)pl.ks * M * N * 4;
 }
 
-// One launch of the tile kernel over the operands of kp (any split count; the partials stay in kp.part).
-static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, bool f32_scales, hipStream_t s) {
+// One launch of the tile kernel over the operands of kp (any split count; the partials stay in kp.part).  rows: the
+// general form (groups of 128); f32_scales: its grouped kernels with float32 scales.
+static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, bool rows, bool f32_scales, hipStream_t s) {
     dim3 grid((unsigned)((kp.N + pl.bn - 1) / pl.bn), (unsigned)((kp.M + pl.bm - 1) / pl.bm), (unsigned)pl.ks);
     constexpr int kDepth = 4;
     const size_t lds = (size_t)kDepth * kKmSlotBytes;
@@ -1807,13 +1815,21 @@ static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, b
         {K3Q_KM_ROW(false, 2, 1), K3Q_KM_ROW(false, 2, 2), K3Q_KM_ROW(false, 1, 1)},
         {K3Q_KM_ROW(true, 2, 1), K3Q_KM_ROW(true, 2, 2), K3Q_KM_ROW(true, 1, 1)}};
 #undef K3Q_KM_ROW
-    static const KmKernel f32_kernels[2] = {gemm_w4_kmajor<true, kDepth, 2, 2, 1, true>,
-                                            gemm_w4_kmajor<true, kDepth, 2, 1, 1, true>};
+#define K3Q_KM_ROWS(G) \
+    {gemm_w4_kmajor<G, kDepth, 2, 2, 1, false, true>, gemm_w4_kmajor<G, kDepth, 2, 2, 2, false, true>, \
+     gemm_w4_kmajor<G, kDepth, 2, 1, 1, false, true>}
+    // (float32 scales: 128 x 128 and 64 x 256)
+    static const KmKernel row_kernels[3][3] = {
+        K3Q_KM_ROWS(false), K3Q_KM_ROWS(true),
+        {gemm_w4_kmajor<true, kDepth, 2, 2, 1, true>, nullptr, gemm_w4_kmajor<true, kDepth, 2, 1, 1, true>}};
+#undef K3Q_KM_ROWS
     static const bool raised = [] {
         bool ok = true;
-        for (const KmKernel k : f32_kernels)
-            ok = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget) ==
-                     hipSuccess && ok;
+        for (int a = 0; a < 3; ++a)
+            for (int b = 0; b < 3; ++b)
+                ok = (!row_kernels[a][b] ||
+                      hipFuncSetAttribute((const void*)row_kernels[a][b], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          kLdsBudget) == hipSuccess) && ok;
         for (int a = 0; a < 2; ++a)
             for (int b = 0; b < 3; ++b)
                 for (int c = 0; c < 4; ++c)
@@ -1826,12 +1842,9 @@ static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, b
     const int gs = kp.gsize / kKmStage;
     const int variant = gs == 1 ? 1 : gs == 2 ? 2 : gs == 4 ? 3 : 0;
     const int shape = pl.bm == 64 ? 2 : pl.bn == kKmBN ? 1 : 0;
-    if (f32_scales) {  // (groups of 128)
-        const KmKernel k = shape == 2 ? f32_kernels[1] : f32_kernels[0];
-        k<<<grid, kKmThreads, lds, s>>>(kp);
-    } else {
-        kernels[grouped ? 1 : 0][shape][variant]<<<grid, kKmThreads, lds, s>>>(kp);
-    }
+    const KmKernel k = rows ? row_kernels[f32_scales ? 2 : grouped ? 1 : 0][shape] : kernels[grouped ? 1 : 0][shape][variant];
+    if (!k) return K3Q_ERR_SHAPE;
+    k<<<grid, kKmThreads, lds, s>>>(kp);
     return launch_status();
 }
 
@@ -1876,7 +1889,7 @@ static int run_gemm_w4_tiles(const void* x, int x_dtype, int64_t M, int64_t K, i
     kp.klen = (int)pl.klen;
     kp.strip = strip ? 1 : 0;
     kp.units = (int)(K / 128);
-    const int lrc = launch_w4_tiles(kp, pl, grouped, false, s);
+    const int lrc = launch_w4_tiles(kp, pl, grouped, false, false, s);
     if (lrc != K3Q_OK) return lrc;
     // the decode kernel's second pass: sums the splits in order, applies scale and bias
     GemvParams gp{};
@@ -2004,7 +2017,7 @@ extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K
         if (pl.parts == 1) km_prepare_rows<1><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
         else if (pl.parts == 2) km_prepare_rows<2><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
         else km_prepare_rows<3><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
-        const int rc = launch_w4_tiles(kp, tiles, grouped, f32 && grouped, s);
+        const int rc = launch_w4_tiles(kp, tiles, grouped, true, f32 && grouped, s);
         if (rc != K3Q_OK) return rc;
         const dim3 fgrid((unsigned)((N + 1023) / 1024), (unsigned)rows);
 #define K3Q_KM_FINISH(B, P)                                                                                          \
