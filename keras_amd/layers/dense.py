@@ -15,7 +15,7 @@ import math
 import torch
 
 from keras_amd import dtype_policies, ops as kops, quantizers
-from keras_amd.layers.layer import Layer, as_tensor, require_default_g_idx, to_torch_dtype
+from keras_amd.layers.layer import Layer, as_tensor, cached_operand, require_default_g_idx, to_torch_dtype
 from keras_amd.layers.together import quantize_rows
 from keras_amd.quantization_config import QuantizationConfig, get_block_size_for_layer
 
@@ -396,20 +396,7 @@ class Dense(Layer):
     # ---- cached derived operands ------------------------------------------------
     def _cached(self, key, var, make):
         """Value derived from a variable, rebuilt when the variable is assigned."""
-        if var is None:
-            return None
-        hit = self._cache.get(key)
-        if hit is not None and hit[0] == var.version and hit[1] is var:
-            return hit[2]
-        value = make(as_tensor(var))
-        if (hit is not None and isinstance(hit[2], torch.Tensor) and isinstance(value, torch.Tensor)
-                and hit[2].shape == value.shape and hit[2].dtype == value.dtype and hit[2].device == value.device):
-            # a rebuilt copy keeps its address: a captured HIP graph that holds the old copy's address
-            # goes on reading live memory (the new values) instead of memory that was freed
-            hit[2].copy_(value)
-            value = hit[2]
-        self._cache[key] = (var.version, var, value)
-        return value
+        return cached_operand(self._cache, key, var, make)
 
     def _read_cached(self, key, var):
         cd = to_torch_dtype(self.compute_dtype)

@@ -21,7 +21,7 @@ import torch
 
 from keras_amd import dtype_policies, ops as kops, quantizers
 from keras_amd.layers.dense import int8_strip_route
-from keras_amd.layers.layer import Layer, as_tensor, require_default_g_idx, to_torch_dtype
+from keras_amd.layers.layer import Layer, as_tensor, cached_operand, require_default_g_idx, to_torch_dtype
 from keras_amd.quantization_config import (
     Int4QuantizationConfig,
     QuantizationConfig,
@@ -528,18 +528,7 @@ class ReversibleEmbedding(Embedding):
 
     # ---- quantized forward -----------------------------------------------------------
     def _cached(self, key, var, make):
-        hit = self._cache.get(key)
-        if hit is not None and hit[0] == var.version and hit[1] is var:
-            return hit[2]
-        value = make(as_tensor(var))
-        if (hit is not None and isinstance(hit[2], torch.Tensor) and isinstance(value, torch.Tensor)
-                and hit[2].shape == value.shape and hit[2].dtype == value.dtype and hit[2].device == value.device):
-            # a rebuilt copy keeps its address: a captured HIP graph that holds the old copy's address
-            # goes on reading live memory (the new values) instead of memory that was freed
-            hit[2].copy_(value)
-            value = hit[2]
-        self._cache[key] = (var.version, var, value)
-        return value
+        return cached_operand(self._cache, key, var, make)
 
     def _int8_call(self, inputs, reverse=False, training=None):
         """reversible_embedding.py:272-296.  Tied weights: the `[vocab, dim]` int8 table IS

@@ -92,6 +92,39 @@ def as_tensor(x):
     return x.value if isinstance(x, Variable) else x
 
 
+def cached_operand(cache, key, var, make):
+    """`make(value of var)`, kept in `cache` and rebuilt when the variable is assigned.  A rebuilt tensor keeps its
+    address: a captured HIP graph that holds the old one's goes on reading live memory (the new values) instead of
+    memory that was freed.  The rebuild writes into the tensor that is kept, so that one never shares storage with the
+    variable's (a cast to the dtype it has already, a `contiguous()` of what lies so, return the variable's own
+    tensor, and that may be the caller's): it is cloned, and follows writes into the variable's tensor, too."""
+    if var is None:
+        return None
+    t = as_tensor(var)
+    hit = cache.get(key)
+    if (hit is not None and hit[0] == var.version and hit[1] is var
+            and (hit[3] is None or hit[3] == _writes(t))):
+        return hit[2]
+    value = make(t)
+    writes = None
+    if isinstance(value, torch.Tensor):
+        if value.untyped_storage().data_ptr() == t.untyped_storage().data_ptr():
+            writes = _writes(t)
+        if (hit is not None and isinstance(hit[2], torch.Tensor) and hit[2].shape == value.shape
+                and hit[2].dtype == value.dtype and hit[2].device == value.device):
+            hit[2].copy_(value.detach())
+            value = hit[2]
+        elif writes is not None:
+            value = value.detach().clone()
+    cache[key] = (var.version, var, value, writes)
+    return value
+
+
+def _writes(t):
+    """How often a tensor was written in place (inference tensors do not count)."""
+    return 0 if t.is_inference() else t._version
+
+
 def require_default_g_idx(layer, block_size):
     """The grouped int4 kernels take the group of row k to be `k // block_size`; the reference
     looks it up in the `g_idx` variable (keras/src/quantizers/quantizers.py:1659-1668), which
