@@ -122,16 +122,17 @@ def int4_strip_rows_route(dtype, rows, input_dim, units, block_size):
 
 def strip_rows_params(layer, dtype, input_dim, units, block_size):
     """The grouped parameters of `ops.int4_matmul_strip_rows` in `dtype`: made on first use, rebuilt in place
-    when a variable they come from is assigned (a captured graph holds their address)."""
+    when a variable they come from is assigned (a captured graph holds their address).  Each dtype has its own."""
     scale, zero = layer.kernel_scale, layer.kernel_zero
-    stamp = (id(scale), scale.version, id(zero), zero.version, dtype)
-    hit = layer._cache.get("w4s_rows_params")
+    stamp = (id(scale), scale.version, id(zero), zero.version)
+    key = ("w4s_rows_params", dtype)
+    hit = layer._cache.get(key)
     if hit is None or hit[0] != stamp:
         value = kops.int4_strip_rows_params(as_tensor(scale).to(dtype), as_tensor(zero), input_dim, units, block_size)
         if hit is not None and hit[2].shape == value.shape and hit[2].device == value.device:
             hit[2].copy_(value)
             value = hit[2]
-        hit = layer._cache["w4s_rows_params"] = (stamp, None, value)
+        hit = layer._cache[key] = (stamp, None, value)
     return hit[2]
 
 
@@ -649,8 +650,9 @@ class Dense(Layer):
         rows = None
         if strip is not None:
             strip["bias"] = self._call_bias()
-        elif int4_strip_rows_route(x2.dtype, x2.shape[0], x2.shape[1], self._orig_output_dim,
-                                   block_size if grouped else None):
+        elif x2.dtype == to_torch_dtype(self.compute_dtype) and int4_strip_rows_route(
+                x2.dtype, x2.shape[0], x2.shape[1], self._orig_output_dim, block_size if grouped else None):
+            # (`call_add` asks before the cast of its inputs: what it runs has the compute dtype)
             rows = dict(self._strip_rows_operands(x2, grouped, block_size), bias=self._call_bias())
         return dict(
             x2=x2, block_size=block_size if grouped else None, strip=strip, rows=rows,

@@ -3,8 +3,9 @@
 import pytest
 import torch
 
+from keras_amd import ops as kops
 from keras_amd.layers import Dense, EinsumDense, ReversibleEmbedding
-from keras_amd.layers.dense import tile_rows_operands
+from keras_amd.layers.dense import strip_rows_params, tile_rows_operands
 
 
 def quantized(kind, policy):
@@ -62,3 +63,32 @@ def test_operand_of_the_same_type_follows_writes_into_the_variable():
     before = read()
     layer.bias.value.add_(3.0)
     assert torch.equal(read(), layer.bias.value) and read().data_ptr() == before.data_ptr()
+
+
+def test_packed_parameters_of_two_types_live_side_by_side(monkeypatch):
+    made = []
+
+    def pack(scale, zero, input_dim, units, block_size):
+        made.append(scale.dtype)
+        return torch.full((scale.numel() * scale.element_size(),), float(scale.flatten()[0]))
+
+    monkeypatch.setattr(kops, "int4_strip_rows_params", pack)
+    layer = quantized("dense", "int4/128")
+    read = lambda dtype: strip_rows_params(layer, dtype, 256, 32, 128)
+    wide, narrow = read(torch.float32), read(torch.bfloat16)
+    assert read(torch.float32) is wide and read(torch.bfloat16) is narrow and len(made) == 2
+    layer.kernel_scale.assign(torch.full(layer.kernel_scale.shape, 3.0))
+    # rebuilt where they lie
+    assert read(torch.float32) is wide and read(torch.bfloat16) is narrow
+    assert float(wide[0]) == float(narrow[0]) == 3.0
+
+
+def test_shared_launch_packs_nothing_for_rows_of_another_type(monkeypatch):
+    packed = []
+    monkeypatch.setattr(kops, "int4_strip_rows_params", lambda *a: packed.append("params") or torch.zeros(1))
+    monkeypatch.setattr(kops, "int4_strip_copy", lambda *a: packed.append("copy") or torch.zeros(1))
+    layer = Dense(24, dtype="int4/128_from_mixed_bfloat16", device="cpu", use_bias=False)
+    layer.build((None, 256))
+    spec = layer._int4_together_spec(torch.zeros(4, 256))  # float32 rows: the layer's call casts them first
+    assert spec is not None and spec["rows"] is None and packed == []
+    assert layer._int4_together_spec(torch.zeros(4, 256, dtype=torch.bfloat16))["rows"] is not None
