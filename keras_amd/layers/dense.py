@@ -15,7 +15,8 @@ import math
 import torch
 
 from keras_amd import dtype_policies, ops as kops, quantizers
-from keras_amd.layers.layer import Layer, as_tensor, cached_operand, require_default_g_idx, to_torch_dtype
+from keras_amd.layers.layer import (Layer, as_tensor, cached_operand, cached_params, require_default_g_idx,
+                                    to_torch_dtype)
 from keras_amd.layers.together import quantize_rows
 from keras_amd.quantization_config import QuantizationConfig, get_block_size_for_layer
 
@@ -124,16 +125,8 @@ def strip_rows_params(layer, dtype, input_dim, units, block_size):
     """The grouped parameters of `ops.int4_matmul_strip_rows` in `dtype`: made on first use, rebuilt in place
     when a variable they come from is assigned (a captured graph holds their address).  Each dtype has its own."""
     scale, zero = layer.kernel_scale, layer.kernel_zero
-    stamp = (id(scale), scale.version, id(zero), zero.version)
-    key = ("w4s_rows_params", dtype)
-    hit = layer._cache.get(key)
-    if hit is None or hit[0] != stamp:
-        value = kops.int4_strip_rows_params(as_tensor(scale).to(dtype), as_tensor(zero), input_dim, units, block_size)
-        if hit is not None and hit[2].shape == value.shape and hit[2].device == value.device:
-            hit[2].copy_(value)
-            value = hit[2]
-        hit = layer._cache[key] = (stamp, None, value)
-    return hit[2]
+    return cached_params(layer._cache, ("w4s_rows_params", dtype), (scale, zero), lambda: kops.int4_strip_rows_params(
+        as_tensor(scale).to(dtype), as_tensor(zero), input_dim, units, block_size))
 
 
 # float32 rows up to which the int4 tile kernel beats the GEMM on the kernel de-quantised to bfloat16 parts (us, GEMM
@@ -415,12 +408,8 @@ class Dense(Layer):
                     shadow=self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)))
         if grouped:
             scale, zero = self.kernel_scale, self.kernel_zero
-            stamp = (id(scale), scale.version, id(zero), zero.version)
-            hit = self._cache.get("w4s_params")
-            if hit is None or hit[0] != stamp:
-                value = kops.int4_strip_params(as_tensor(scale), as_tensor(zero), input_dim, units, block_size)
-                hit = self._cache["w4s_params"] = (stamp, None, value)
-            spec["gparams"] = hit[2]
+            spec["gparams"] = cached_params(self._cache, "w4s_params", (scale, zero), lambda: kops.int4_strip_params(
+                as_tensor(scale), as_tensor(zero), input_dim, units, block_size))
         else:
             spec["kernel_scale"] = self._read_cached("kernel_scale", self.kernel_scale)
         return spec

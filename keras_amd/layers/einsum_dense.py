@@ -21,7 +21,8 @@ from keras_amd import dtype_policies, ops as kops, quantizers
 from keras_amd.layers.dense import (_ACTIVATIONS, activation_name, glorot_uniform, int8_strip_route,
                                     lora_initializer,
                                     serialize_quantization_config)
-from keras_amd.layers.layer import Layer, as_tensor, cached_operand, require_default_g_idx, to_torch_dtype
+from keras_amd.layers.layer import (Layer, as_tensor, cached_operand, cached_params, require_default_g_idx,
+                                    to_torch_dtype)
 from keras_amd.layers.together import quantize_rows
 from keras_amd.quantization_config import QuantizationConfig, get_block_size_for_layer
 
@@ -531,12 +532,8 @@ class EinsumDense(Layer):
                     shadow=self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)))
         if grouped:
             scale, zero = self.kernel_scale, self.kernel_zero
-            stamp = (id(scale), scale.version, id(zero), zero.version)
-            hit = self._cache.get("w4s_params")
-            if hit is None or hit[0] != stamp:
-                value = kops.int4_strip_params(as_tensor(scale), as_tensor(zero), input_dim, units, block_size)
-                hit = self._cache["w4s_params"] = (stamp, None, value)
-            spec["gparams"] = hit[2]
+            spec["gparams"] = cached_params(self._cache, "w4s_params", (scale, zero), lambda: kops.int4_strip_params(
+                as_tensor(scale), as_tensor(zero), input_dim, units, block_size))
         else:
             spec["kernel_scale"] = self._cached("kernel_scale", self.kernel_scale,
                                                 lambda t: t.to(cd).reshape(-1).contiguous())

@@ -21,7 +21,8 @@ import torch
 
 from keras_amd import dtype_policies, ops as kops, quantizers
 from keras_amd.layers.dense import int8_strip_route
-from keras_amd.layers.layer import Layer, as_tensor, cached_operand, require_default_g_idx, to_torch_dtype
+from keras_amd.layers.layer import (Layer, as_tensor, cached_operand, cached_params, require_default_g_idx,
+                                    to_torch_dtype)
 from keras_amd.quantization_config import (
     Int4QuantizationConfig,
     QuantizationConfig,
@@ -623,16 +624,8 @@ class ReversibleEmbedding(Embedding):
             spec["kernel_scale"] = scale if scale.is_contiguous() else scale.contiguous()
             return spec
         sv, zv = self.embeddings_scale, self.embeddings_zero
-        stamp = (id(sv), sv.version, id(zv), zv.version)
-        hit = self._cache.get("w4s_rows_params")
-        if hit is None or hit[0] != stamp:
-            value = kops.int4_strip_rows_params(as_tensor(sv).t().contiguous(),
-                                                as_tensor(zv).to(torch.int8).t().contiguous(), K, N, block_size)
-            if hit is not None and hit[2].shape == value.shape and hit[2].device == value.device:
-                hit[2].copy_(value)  # (a captured graph holds the address)
-                value = hit[2]
-            hit = self._cache["w4s_rows_params"] = (stamp, None, value)
-        spec["gparams"] = hit[2]
+        spec["gparams"] = cached_params(self._cache, "w4s_rows_params", (sv, zv), lambda: kops.int4_strip_rows_params(
+            as_tensor(sv).t().contiguous(), as_tensor(zv).to(torch.int8).t().contiguous(), K, N, block_size))
         return spec
 
     def _tied_strip_operands(self, x2, scale, grouped, block_size):
@@ -650,13 +643,8 @@ class ReversibleEmbedding(Embedding):
         spec = dict(shadow=self._cached("w4s", self._embeddings, self._relay_tied))
         if grouped:
             sv, zv = self.embeddings_scale, self.embeddings_zero
-            stamp = (id(sv), sv.version, id(zv), zv.version)
-            hit = self._cache.get("w4s_params")
-            if hit is None or hit[0] != stamp:
-                value = kops.int4_strip_params(as_tensor(sv).t().contiguous(),
-                                               as_tensor(zv).to(torch.int8).t().contiguous(), K, N, block_size)
-                hit = self._cache["w4s_params"] = (stamp, None, value)
-            spec["gparams"] = hit[2]
+            spec["gparams"] = cached_params(self._cache, "w4s_params", (sv, zv), lambda: kops.int4_strip_params(
+                as_tensor(sv).t().contiguous(), as_tensor(zv).to(torch.int8).t().contiguous(), K, N, block_size))
         else:
             spec["kernel_scale"] = scale if scale.is_contiguous() else scale.contiguous()
         return spec

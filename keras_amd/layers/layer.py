@@ -120,6 +120,21 @@ def cached_operand(cache, key, var, make):
     return value
 
 
+def cached_params(cache, key, variables, make):
+    """`make()`, a tensor packed from several variables, kept in `cache` and rebuilt in place (as `cached_operand`)
+    when one of them is assigned."""
+    stamp = tuple((id(v), v.version) for v in variables)
+    hit = cache.get(key)
+    if hit is None or hit[0] != stamp:
+        value = make()
+        if (hit is not None and hit[2].shape == value.shape and hit[2].dtype == value.dtype
+                and hit[2].device == value.device):
+            hit[2].copy_(value)
+            value = hit[2]
+        hit = cache[key] = (stamp, None, value)
+    return hit[2]
+
+
 def _writes(t):
     """How often a tensor was written in place (inference tensors do not count)."""
     return 0 if t.is_inference() else t._version

@@ -8,9 +8,9 @@ from keras_amd.layers import Dense, EinsumDense, ReversibleEmbedding
 from keras_amd.layers.dense import strip_rows_params, tile_rows_operands
 
 
-def quantized(kind, policy):
+def quantized(kind, policy, source="_from_float32"):
     """A layer built in its quantized form."""
-    policy += "_from_float32"
+    policy += source
     if kind == "einsum":
         layer = EinsumDense("btd,dnh->btnh", (None, 4, 8), bias_axes="nh", dtype=policy, device="cpu")
         layer.build((None, None, 256))
@@ -92,3 +92,16 @@ def test_shared_launch_packs_nothing_for_rows_of_another_type(monkeypatch):
     spec = layer._int4_together_spec(torch.zeros(4, 256))  # float32 rows: the layer's call casts them first
     assert spec is not None and spec["rows"] is None and packed == []
     assert layer._int4_together_spec(torch.zeros(4, 256, dtype=torch.bfloat16))["rows"] is not None
+
+
+@pytest.mark.parametrize("kind", ["dense", "einsum"])
+def test_packed_parameters_of_the_decode_kernel_keep_their_address(monkeypatch, kind):
+    monkeypatch.setattr(kops, "int4_strip_supported", lambda *a: True)
+    monkeypatch.setattr(kops, "int4_strip_copy", lambda *a: torch.zeros(1))
+    monkeypatch.setattr(kops, "int4_strip_params", lambda scale, *a: scale.clone())
+    layer = quantized(kind, "int4/128", "_from_mixed_bfloat16")
+    read = lambda: layer._strip_operands(1, 256, 32, True, 128)["gparams"]
+    before = read()
+    layer.kernel_scale.assign(torch.full(layer.kernel_scale.shape, 3.0))
+    after = read()
+    assert after.data_ptr() == before.data_ptr() and bool((after == 3.0).all())
