@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "k3q_common.h"
+#include "k3q_testing.h"
 #include "k3q_gemm_bf16.h"
 #include "k3q_gemm_i8_skinny.h"
 #include "k3q_gemv_w8.h"
@@ -874,7 +875,9 @@ inline int choose_splits(int64_t tiles, int64_t stages, int resident) {
 // 30.4 / 27.8; 300 x 3200 x 8192 38.0 / 29.8 and 23.5 / 20.6; 512 x 8192 x 8192 79.0 / 75.8 and 49.6 / 45.4).
 // With fewer tiles a split of K over two workgroups per CU stays ahead (128 x 4096 x 4096 int8 16.9 / 22.6), and
 // so do two stages on a short walk (300 x 1664 x 6400 int8, 13 stages: 14.0 / 14.7).
-inline bool deep_tile(int64_t tiles, int64_t stages, int cus) {
+// (row_bytes: as the operands lie, or padded to whole stages -- the launch and the workspace ask with either.)
+inline bool deep_tile(int64_t M, int64_t N, int64_t row_bytes, int cus) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), stages = (row_bytes + kBK - 1) / kBK;
     return 2 * tiles > cus && tiles <= cus && stages >= 20;
 }
 
@@ -883,7 +886,7 @@ inline bool deep_tile(int64_t tiles, int64_t stages, int cus) {
 inline int64_t split_workspace_bytes(int64_t M, int64_t N, int64_t row_bytes) {
     if (M <= 0 || (row_bytes % kBK) != 0 || (N % 4) != 0) return 0;
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    const int splits = deep_tile(tiles, row_bytes / kBK, 256) ? 1 : choose_splits(tiles, row_bytes / kBK, 512);
+    const int splits = deep_tile(M, N, row_bytes, 256) ? 1 : choose_splits(tiles, row_bytes / kBK, 512);
     return splits > 1 ? (int64_t)splits * M * N * 4 : 0;
 }
 
@@ -928,7 +931,7 @@ template <int kKind, bool kBF16, bool kExact>
 int launch_mfma(const GemmParams& p, hipStream_t s) {
     const int64_t large_tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
     const bool large = large_tiles >= kLargeTileMinTiles;
-    const bool deep = deep_tile(((p.M + 127) / 128) * ((p.N + 127) / 128), p.row_bytes / kBK, cu_count());
+    const bool deep = deep_tile(p.M, p.N, p.row_bytes, cu_count());
     if constexpr (kKind == kKindI8) {
         if (p.b_strip && p.row_bytes % kBK) {
             if (large) return launch_tile<TileLarge, kKind, kBF16, kExact, true, true>(p, s);
@@ -1003,6 +1006,10 @@ extern "C" int64_t k3q_gemm_i8_workspace_bytes(int64_t M, int64_t N, int64_t K) 
 
 extern "C" int64_t k3q_gemm_i8_split_bytes(int64_t M, int64_t N, int64_t K) {
     return K > 0 && N > 0 ? split_workspace_bytes(M, N, (K + kBK - 1) / kBK * kBK) : 0;
+}
+
+extern "C" int k3qt_gemm_deep_tile(int64_t M, int64_t N, int64_t row_bytes, int cus) {
+    return deep_tile(M, N, row_bytes, cus) ? 1 : 0;
 }
 
 extern "C" int k3q_prepack_kernel_i8(const int8_t* kernel, int64_t K, int64_t N, int8_t* prepacked,

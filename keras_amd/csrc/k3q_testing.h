@@ -25,6 +25,10 @@ int k3qt_gemv_w4_plan(const void* x, int x_dtype, int64_t M, int64_t K, int64_t 
                      int64_t workspace_bytes, void* counters, int64_t counters_bytes,
                      const int* plan, void* stream);
 
+/* Whether the tile GEMM takes its four-stage tile for operand rows of row_bytes on a chip of `cus` compute units: the
+ * rule that both the launch and the size of the workspace follow (host only). */
+int k3qt_gemm_deep_tile(int64_t M, int64_t N, int64_t row_bytes, int cus);
+
 #ifdef __cplusplus
 }
 #endif

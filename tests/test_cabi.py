@@ -100,3 +100,17 @@ def test_error_codes_become_python_exceptions():
     with pytest.raises(RuntimeError):
         _lib.check(-6, "x")
     _lib.check(0, "x")
+
+
+@pytest.mark.parametrize("K", [2432, 2496, 2560, 2624])
+def test_four_stage_tile_is_chosen_alike_by_launch_and_workspace(K):
+    """K in half stages of 64: the launch asks with the rows as they lie, the workspace with rows of whole stages."""
+    lib = _lib.load()
+    whole = -(-K // 128) * 128
+    for M in (100, 300, 1000, 1024, 2000):
+        for N in (256, 1600, 3200, 4096):
+            deep = lib.k3qt_gemm_deep_tile(M, N, K, 256)
+            assert deep == lib.k3qt_gemm_deep_tile(M, N, whole, 256)
+            assert not (deep and lib.k3q_gemm_i8_split_bytes(M, N, K))
+            tiles = -(-M // 128) * -(-N // 128)
+            assert bool(deep) == (128 < tiles <= 256 and whole >= 20 * 128)
