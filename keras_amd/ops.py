@@ -768,8 +768,8 @@ def int8_matmul(a, kernel, a_scale=None, kernel_scale=None, bias=None, out_dtype
     skinny = M <= SKINNY_MAX_ROWS and N % 16 == 0 and K % 8 == 0
     nbytes = lib.k3q_gemm_i8_workspace_bytes(M, N, K)
     if strip is not None and not skinny and K % 64 == 0:
-        # (the tile kernel reads scales and bias in 16-byte pieces)
-        sa, sb, bias = (t.clone() if t is not None and t.data_ptr() % 16 else t for t in (sa, sb, bias))
+        # (the tile kernel reads rows, scales and bias in 16-byte pieces)
+        a, sa, sb, bias = (t.clone() if t is not None and t.data_ptr() % 16 else t for t in (a, sa, sb, bias))
         if strip.numel() != lib.k3q_w8s_shadow_bytes(K, N):
             raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
         b, layout = strip, 2

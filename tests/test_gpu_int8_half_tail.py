@@ -47,3 +47,14 @@ def test_half_tail_layer_with_unaligned_bias(dev):
     y = layer(x)
     layer.bias.assign(b[1:].clone())
     assert torch.equal(y, layer(x))
+
+
+@pytest.mark.parametrize("K", [192, 256])
+def test_rows_that_do_not_start_on_16_bytes(dev, K):
+    """Quantised rows that are a view into a larger buffer, with the strip-linear copy at hand."""
+    g = torch.Generator().manual_seed(K)
+    w = torch.randint(-128, 128, (K, 96), generator=g, dtype=torch.int8).to(dev)
+    flat = torch.randint(-128, 128, (40 * K + 3,), generator=g, dtype=torch.int8).to(dev)
+    a = flat[3:].view(40, K)
+    acc = kops.int8_matmul(a, w, strip=kops.int8_strip_copy(w), want_acc=True, want_y=False)
+    assert torch.equal(acc.cpu(), c_gemm_i8(a.cpu(), w.cpu()))
