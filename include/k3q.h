@@ -357,7 +357,9 @@ int k3q_gemv_w4s(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, co
  * 16 on, any N.  The copy is k3q_w4s_pack's (the last unit's nibbles past K are zero); grouped parameters are
  * k3q_w4s_rows_pack_params' (records of four scales in `dtype` and four bytes zero + 128, per strip, unit and
  * quarter strip).  Rows whose x does not fit a workgroup's LDS go in several launches
- * (k3q_gemv_w4s_rows_launches: how many; 0: not taken, K3Q_ERR_SHAPE). */
+ * (k3q_gemv_w4s_rows_launches: how many; 0: not taken, K3Q_ERR_SHAPE).  Where N % 8 or K % 16 the weights enter the sums
+ * as they are and float32 rows in three bfloat16 parts, exactly; elsewhere with an offset that is taken out afterwards (a
+ * row with an infinity is NaN then, as in k3q_gemv_w4 and k3q_gemv_w4s) and in two parts, to 2^-17. */
 int64_t k3q_w4s_rows_params_bytes(int64_t K, int64_t N, int64_t block_size, int dtype);
 int k3q_w4s_rows_pack_params(const void* scale, int dtype, const int8_t* zero, int64_t K, int64_t N,
                              int64_t block_size, void* params, void* stream);
@@ -414,7 +416,7 @@ int k3q_gemv_w4s_pre(const void* x, int x_dtype, int64_t M, int64_t K, const k3q
 int k3q_w4_kmajor_pack(const int8_t* w_packed, int64_t K, int64_t N, int32_t* w_kmajor, void* stream);
 /* k3q_gemm_w4_rows: the tile kernel on k3q_w4s_pack's copy for any M, any K % 8 == 0 from 16 on, any N, bfloat16 or
  * float32 x (scales, bias and y in the same type; a float32 row travels as two or three bfloat16 rows that add
- * up to it).  Grouped (block_size 128): scale and zero are [ceil(K / 128), Np] with Np = N rounded up to 32; per-channel
+ * up to it; weights and parts as in k3q_gemv_w4s_rows).  Grouped (block_size 128): scale and zero are [ceil(K / 128), Np] with Np = N rounded up to 32; per-channel
  * (block_size <= 0): scale [N].  bias [N], or [M, N] with bias_stride N.  workspace: aligned to 256. */
 int64_t k3q_gemm_w4_rows_workspace_bytes(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size);
 int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* w_strip,

@@ -1160,6 +1160,9 @@ constexpr u32 kKmNibbles = 0x000F000Fu, kKmFlip = 0x00080008u, kKmExp = 0x430043
 // its rows need; where the sums are rounded to bfloat16 it buys nothing and the shift shows (96 rows of 4096 x 14336:
 // 27.5 -> 27.6 us in the kernel, 0.7 % of the call).
 constexpr u32 kKmNibbles24 = 0x00780078u, kKmBase24 = 0x41C041C0u;
+// How a kernel converts the nibbles: the layers' own shapes, the general form, and the general form for shapes whose kernel
+// on the stored weights multiplies float32 values (N % 8, K % 16) -- no offset there, the sums are no larger than its own.
+constexpr int kKm136 = 0, kKm24 = 1, kKmPlain = 2;
 
 __device__ __forceinline__ int km_swz(int row) { return (row & 6) | ((row ^ (row >> 3)) & 1); }
 
@@ -1210,8 +1213,9 @@ __global__ __launch_bounds__(256) void km_group_sums(const uint16_t* __restrict_
 // zero past K, and their sums per group of 128 as above.  kParts 2 or 3: float32 rows, each as that many bfloat16
 // rows that add up to it (top 16 bits, top 16 bits of the rest, ...; the last one rounded), part h of row m being row
 // h M + m; the tile kernel and its partials then know nothing of it, the second pass adds a row's parts.
+// kPlain: for the kernel without an offset, which reads no sums; nothing is left of an infinity's first part.
 // One wave per (group, row), a lane two neighbouring values.
-template <int kParts>
+template <int kParts, bool kPlain>
 __global__ __launch_bounds__(256) void km_prepare_rows(const void* __restrict__ x, u32* __restrict__ xp,
                                                        v2u* __restrict__ sx, int64_t M, int64_t K, int64_t Kp) {
     const int lane = threadIdx.x & 63;
@@ -1238,11 +1242,12 @@ __global__ __launch_bounds__(256) void km_prepare_rows(const void* __restrict__ 
         for (int e = 0; e < 2; ++e) {
             b[e] = h == kParts - 1 ? f32_to_bf16_bits(v[e]) : __float_as_uint(v[e]) >> 16;
             const float part = bf16_bits_to_f32(b[e]);
-            v[e] -= part;
+            v[e] = kPlain && v[e] == part ? 0.f : v[e] - part;
             sum += part;
         }
         const int64_t row = h * M + m;
         xp[(row * Kp + k) >> 1] = b[0] | (b[1] << 16);
+        if (kPlain) continue;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
         if (lane == 0) {
@@ -1304,8 +1309,8 @@ constexpr int kKmParScale = 0, kKmParZero = 512, kKmParSx = 768, kKmParSpare = 1
 // narrow that wide tiles leave CUs idle even at eight splits).
 // kWM: waves along M: 2 (tiles of 128 rows) or 1 (64 rows, eight waves side by side, kNB = 1).
 // kF32S: float32 scales (twice the bytes: tiles of 128 x 128 or 64 x 256 only, whose parameters still fit).
-// kRows: the weights at 24 + w instead of 136 + w (above).
-template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB, bool kF32S = false, bool kRows = kF32S>
+// kForm: the conversion (above).
+template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB, int kForm = kKm136, bool kF32S = false>
 __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
     constexpr int kWaveN = 32 * kNB, kBN = kWaveN * (8 / kWM), kBM = 64 * kWM;
     static_assert(!kF32S || (kGrouped && kBN * kBM <= 128 * 128), "parameters of a stage");
@@ -1481,6 +1486,12 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
 #pragma unroll
             for (int nb = 0; nb < kNB; ++nb)
                 wq[nb] = *(const v4u*)(cur + kKmXBytes + (wn * kWaveN + nb * 32 + i) * 32 + g * 16);
+            float off[kNB];  // (kKmPlain) 8 + the zero point of this lane's column
+#pragma unroll
+            for (int nb = 0; nb < kNB; ++nb)
+                off[nb] = kForm == kKmPlain && kGrouped
+                              ? 8.f + (float)*(const int8_t*)(cur + kKmXBytes + kKmWBytes + kParZero + wn * kWaveN + nb * 32 + i)
+                              : 8.f;
             // (kDepth is a multiple of kGroupStages and a split starts on a group: u tells)
             constexpr bool kStatic = kGroupStages > 0;
             const bool group_first = kStatic && (u % (kStatic ? kGroupStages : 1)) == 0;
@@ -1493,9 +1504,14 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
 #pragma unroll
                 for (int nb = 0; nb < kNB; ++nb) {
                     const u32 d = wq[nb][s];
+                    if constexpr (kForm == kKmPlain) {
+                        wb[nb] = plain_nibbles(d, off[nb]);
+                        continue;
+                    }
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
-                        wb[nb][q] = kRows ? ((q ? d >> (4 * q - 3) : d << 3) & kKmNibbles24) ^ kKmBase24
+                        wb[nb][q] = kForm == kKm24
+                                        ? ((q ? d >> (4 * q - 3) : d << 3) & kKmNibbles24) ^ kKmBase24
                                           : (((d >> (4 * q)) & kKmNibbles) ^ kKmFlip) | kKmExp;
                 }
 #pragma unroll
@@ -1516,7 +1532,7 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
             if (group_last) {
                 const char* par = cur + kKmXBytes + kKmWBytes;
                 // acc -= (136 + zero) * sum(x) as one more MFMA step: k = 0 ... 2 carry -128 on the
-                // kernel side (kRows: -16), k = 3 ... 5 carry -(8 + zero) (any int8 zero point is exact in
+                // kernel side (kKm24: -16; kKmPlain has nothing to take out), k = 3 ... 5 carry -(8 + zero) (any int8 zero point is exact in
                 // bfloat16), both against the three bfloat16 parts of the sum of x; products of
                 // two bfloat16 are exact in float32, so the cancellation happens in the accumulator
                 v4u xs[2], wz[kNB];
@@ -1534,14 +1550,14 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
                     int zp = 0;
                     if (kGrouped) zp = *(const int8_t*)(par + kParZero + wn * kWaveN + nb * 32 + i);
                     const u32 cz = __float_as_uint(-(float)(8 + zp)) >> 16;
-                    constexpr u32 kBase = kRows ? 0xC180u : 0xC300u;      // -16, -128
+                    constexpr u32 kBase = kForm == kKm24 ? 0xC180u : 0xC300u;  // -16, -128
                     wz[nb][0] = kBase | (kBase << 16);
                     wz[nb][1] = kBase | (cz << 16);                       // ..., -(8 + zero)
                     wz[nb][2] = cz | (cz << 16);
                     wz[nb][3] = 0;
                 }
 #pragma unroll
-                for (int nb = 0; nb < kNB; ++nb)
+                for (int nb = 0; nb < kNB && kForm != kKmPlain; ++nb)
 #pragma unroll
                     for (int mb = 0; mb < 2; ++mb)
                         acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf(wz[nb]), as_bf(xs[mb]),
@@ -1800,9 +1816,9 @@ extern "C" int64_t k3q_gemm_w4_kmajor_workspace_bytes(int64_t M, int64_t K, int6
     return ((K / gsize) * M * 8 + 255) / 256 * 256 + (int64_t)pl.ks * M * N * 4;
 }
 
-// One launch of the tile kernel over the operands of kp (any split count; the partials stay in kp.part).  rows: the
-// general form (groups of 128); f32_scales: its grouped kernels with float32 scales.
-static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, bool rows, bool f32_scales, hipStream_t s) {
+// One launch of the tile kernel over the operands of kp (any split count; the partials stay in kp.part).  form: other
+// than kKm136 for groups of 128 only; f32_scales: its grouped kernels with float32 scales.
+static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, int form, bool f32_scales, hipStream_t s) {
     dim3 grid((unsigned)((kp.N + pl.bn - 1) / pl.bn), (unsigned)((kp.M + pl.bm - 1) / pl.bm), (unsigned)pl.ks);
     constexpr int kDepth = 4;
     const size_t lds = (size_t)kDepth * kKmSlotBytes;
@@ -1815,21 +1831,22 @@ static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, b
         {K3Q_KM_ROW(false, 2, 1), K3Q_KM_ROW(false, 2, 2), K3Q_KM_ROW(false, 1, 1)},
         {K3Q_KM_ROW(true, 2, 1), K3Q_KM_ROW(true, 2, 2), K3Q_KM_ROW(true, 1, 1)}};
 #undef K3Q_KM_ROW
-#define K3Q_KM_ROWS(G) \
-    {gemm_w4_kmajor<G, kDepth, 2, 2, 1, false, true>, gemm_w4_kmajor<G, kDepth, 2, 2, 2, false, true>, \
-     gemm_w4_kmajor<G, kDepth, 2, 1, 1, false, true>}
+#define K3Q_KM_ROWS(G, F) \
+    {gemm_w4_kmajor<G, kDepth, 2, 2, 1, F>, gemm_w4_kmajor<G, kDepth, 2, 2, 2, F>, gemm_w4_kmajor<G, kDepth, 2, 1, 1, F>}
     // (float32 scales: 128 x 128 and 64 x 256)
-    static const KmKernel row_kernels[3][3] = {
-        K3Q_KM_ROWS(false), K3Q_KM_ROWS(true),
-        {gemm_w4_kmajor<true, kDepth, 2, 2, 1, true>, nullptr, gemm_w4_kmajor<true, kDepth, 2, 1, 1, true>}};
+#define K3Q_KM_FORM(F) \
+    {K3Q_KM_ROWS(false, F), K3Q_KM_ROWS(true, F), \
+     {gemm_w4_kmajor<true, kDepth, 2, 2, 1, F, true>, nullptr, gemm_w4_kmajor<true, kDepth, 2, 1, 1, F, true>}}
+    static const KmKernel row_kernels[2][3][3] = {K3Q_KM_FORM(kKm24), K3Q_KM_FORM(kKmPlain)};
+#undef K3Q_KM_FORM
 #undef K3Q_KM_ROWS
     static const bool raised = [] {
         bool ok = true;
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b)
-                ok = (!row_kernels[a][b] ||
-                      hipFuncSetAttribute((const void*)row_kernels[a][b], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          kLdsBudget) == hipSuccess) && ok;
+        for (const auto& form : row_kernels)
+            for (const auto& scales : form)
+                for (const KmKernel k : scales)
+                    ok = (!k || hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    kLdsBudget) == hipSuccess) && ok;
         for (int a = 0; a < 2; ++a)
             for (int b = 0; b < 3; ++b)
                 for (int c = 0; c < 4; ++c)
@@ -1842,7 +1859,8 @@ static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, b
     const int gs = kp.gsize / kKmStage;
     const int variant = gs == 1 ? 1 : gs == 2 ? 2 : gs == 4 ? 3 : 0;
     const int shape = pl.bm == 64 ? 2 : pl.bn == kKmBN ? 1 : 0;
-    const KmKernel k = rows ? row_kernels[f32_scales ? 2 : grouped ? 1 : 0][shape] : kernels[grouped ? 1 : 0][shape][variant];
+    const KmKernel k = form != kKm136 ? row_kernels[form - kKm24][f32_scales ? 2 : grouped ? 1 : 0][shape]
+                                      : kernels[grouped ? 1 : 0][shape][variant];
     if (!k) return K3Q_ERR_SHAPE;
     k<<<grid, kKmThreads, lds, s>>>(kp);
     return launch_status();
@@ -1889,7 +1907,7 @@ static int run_gemm_w4_tiles(const void* x, int x_dtype, int64_t M, int64_t K, i
     kp.klen = (int)pl.klen;
     kp.strip = strip ? 1 : 0;
     kp.units = (int)(K / 128);
-    const int lrc = launch_w4_tiles(kp, pl, grouped, false, false, s);
+    const int lrc = launch_w4_tiles(kp, pl, grouped, kKm136, false, s);
     if (lrc != K3Q_OK) return lrc;
     // the decode kernel's second pass: sums the splits in order, applies scale and bias
     GemvParams gp{};
@@ -1928,14 +1946,16 @@ extern "C" int k3q_gemm_w4_strip(const void* x, int x_dtype, int64_t M, int64_t 
 // Three launches: the rows made ready (km_prepare_rows), the tile kernel on the strip-linear copy, the second pass.  The
 // padding costs a pass over x (3 us) where it spares the kernel a copy.  Graph nodes, us, before -> now: bfloat16
 // K=1600, N=6400 300 rows 137 -> 31 and 1200 rows 570 -> 74 (passes of 32 rows); K=2048, N=5247 64 rows 484 -> 18 (one
-// output per thread); float32 K=4096, N=14336 64 rows 127 -> 37 (passes of 8 rows), 300 rows 298 -> 156 (the kernel
+// output per thread; 48 rows 16.2, 15.6 with an offset on the weights); float32 K=4096, N=14336 64 rows 127 -> 37 (passes of 8 rows), 300 rows 298 -> 156 (the kernel
 // de-quantised to parts).  A float32 row doubles the matrix work, which bounds the larger sizes; up to a few dozen rows
 // it is the launches, the start of the ring and the partials.  Error against 64 bits (2-norm), before / now:
-// float32 5.3e-6 / 4.9e-6 (de-quantised kernel 1.3e-5), ragged 2.1e-7 / 1.0e-7, bfloat16 1.66e-3 / 1.66e-3.
+// float32 5.3e-6 / 4.9e-6 (de-quantised kernel 1.3e-5), bfloat16 1.66e-3 / 1.66e-3, without an offset 2.1e-7 / 8e-8 and
+// 1.4e-7 / 8e-8 for rows without negative values (1.3e-7 with one; K=8192: 1.9e-7 / 1.5e-7, 1.8e-7).
 namespace k3q {
 namespace {
 struct KmRowsPlan {
     int parts;      // bfloat16 rows per row of x
+    bool plain;     // the weights without an offset
     int64_t Kp, Np, rows, sx_bytes, x_bytes, part_bytes;
     KmPlan tiles;   // of a launch of `rows` rows
 };
@@ -1947,9 +1967,10 @@ bool km_rows_plan(KmRowsPlan& pl, int x_dtype, int64_t M, int64_t K, int64_t N, 
     if (M < 1 || K < 16 || (K % 8) != 0 || N < 1 || N > (int64_t(1) << 24) || (block_size > 0 && block_size != 128))
         return false;
     const bool f32 = x_dtype == K3Q_F32;
-    // parts of a float32 row: as in the kernels on the stored weights, which split x in two for these shapes and
-    // have float32 products for the others
-    pl.parts = !f32 ? 1 : (N % 8) == 0 && (K % 16) == 0 ? 2 : 3;
+    // as in the kernels on the stored weights, which split x in two and add an offset for most shapes, and have float32
+    // products for the others
+    pl.plain = (N % 8) != 0 || (K % 16) != 0;
+    pl.parts = !f32 ? 1 : pl.plain ? 3 : 2;
     pl.Kp = (K + 127) / 128 * 128;
     pl.Np = (N + 31) / 32 * 32;  // the strips of the copy
     pl.rows = M < kKmMostRows / pl.parts ? M : kKmMostRows / pl.parts;
@@ -2014,10 +2035,11 @@ extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K
         kp.klen = (int)tiles.klen;
         u32* xp = (u32*)workspace;
         v2u* sx = (v2u*)((char*)workspace + pl.x_bytes);
-        if (pl.parts == 1) km_prepare_rows<1><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
-        else if (pl.parts == 2) km_prepare_rows<2><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
-        else km_prepare_rows<3><<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
-        const int rc = launch_w4_tiles(kp, tiles, grouped, true, f32 && grouped, s);
+        (pl.parts == 3   ? km_prepare_rows<3, true>
+         : pl.parts == 2 ? km_prepare_rows<2, false>
+         : pl.plain      ? km_prepare_rows<1, true>
+                         : km_prepare_rows<1, false>)<<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
+        const int rc = launch_w4_tiles(kp, tiles, grouped, pl.plain ? kKmPlain : kKm24, f32 && grouped, s);
         if (rc != K3Q_OK) return rc;
         const dim3 fgrid((unsigned)((N + 1023) / 1024), (unsigned)rows);
 #define K3Q_KM_FINISH(B, P)                                                                                          \

@@ -93,8 +93,12 @@ __device__ __forceinline__ float bf_hi(u32 d) { return __uint_as_float(d & 0xfff
 // float32 rows.  A row travels as that many bfloat16 rows that add up to it (its top 16 bits, the top 16 bits of
 // the rest, ...: to 2^-17, or exactly), side by side in the sixteen rows the matrix instruction has anyway, and
 // the float32 results of a row's parts are added at the end.  The weights sit at 24 + w instead of 136 + w there
-// (the nibble three bits higher in the mantissa: as many operations), a fifth of the offset to cancel.
-template <int kSW, int kD, int kNP, bool kGrouped, bool kHalves, bool kPre = false, int kParts = 0>
+// (the nibble three bits higher in the mantissa), a fifth of the offset to cancel.
+// kPlain (kParts 1 or 3): the weights without an offset, w - zero, nothing to take out of the sums.  For shapes whose
+// kernel on the stored weights multiplies float32 values (N % 8, K % 16): sums no larger than its own, so that
+// rows without negative values lose nothing and a row with an infinity or with huge values gives what a float product
+// gives.  (The zero point is needed where the weights are converted, by column: a word more per unit and strip.)
+template <int kSW, int kD, int kNP, bool kGrouped, bool kHalves, bool kPre = false, int kParts = 0, bool kPlain = false>
 __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int block, const int stride) {
     extern __shared__ __attribute__((aligned(16))) char w4s_lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -102,6 +106,7 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
     const int units = p.units;
     constexpr bool kRows = kParts > 0, kF32 = kParts >= 2;
     static_assert(!(kRows && (kHalves || kPre)), "the general form stages x whole and as it is");
+    static_assert(!kPlain || kRows, "weights without an offset: a variant of the general form");
     const int M = p.M, K = p.K;
     const int MX = kF32 ? kParts * M : M;  // rows in LDS: part h of row m is row h M + m
     const int j = lane & 15, g = lane >> 4;
@@ -208,8 +213,10 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
                                 const u32 t0 = __float_as_uint(rest[2 * e]) & 0xffff0000u;
                                 const u32 t1 = __float_as_uint(rest[2 * e + 1]) & 0xffff0000u;
                                 part[e] = (t0 >> 16) | t1;
-                                rest[2 * e] -= __uint_as_float(t0);
-                                rest[2 * e + 1] -= __uint_as_float(t1);
+                                // (kPlain: nothing is left of an infinity)
+                                const float f0 = __uint_as_float(t0), f1 = __uint_as_float(t1);
+                                rest[2 * e] = kPlain && rest[2 * e] == f0 ? 0.f : rest[2 * e] - f0;
+                                rest[2 * e + 1] = kPlain && rest[2 * e + 1] == f1 ? 0.f : rest[2 * e + 1] - f1;
                             }
                         }
                         *(v4u*)(dst + h * M * pitch) = part;
@@ -268,6 +275,7 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
     at_group();
     v4u W[kD][kSW];
     u32 Z[kGrouped ? kD : 1][kSW][kZ];
+    u32 ZC[kPlain && kGrouped ? kD : 1][kSW];  // the zero points of this lane's column and its three neighbours
     auto fetch = [&](const int d) {
         const int at = !kRows ? 0 : u0 + cu < units ? u0 + cu : units - 1;
 #pragma unroll
@@ -281,6 +289,8 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
                 const u32* z = (const u32*)(cz[t] + (int64_t)at * (16 * kZ) + lane_z);
 #pragma unroll
                 for (int c = 0; c < kZ; ++c) Z[d][t][c] = z[c];
+                if constexpr (kPlain)
+                    ZC[d][t] = *(const u32*)(cz[t] + (int64_t)at * (16 * kZ) + (4u * kZ * (j >> 2) + 4u * (kZ - 1)));
                 if (!kRows) cz[t] += 16 * kZ;
             }
         }
@@ -339,7 +349,15 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
     u32 Zk[2][kSW][kZ];
     v4u av[2][kSW][4], xf[2][4];
 
-    auto cvt1 = [&](const u32 w, v4u& out) {
+    // 8 + the zero point of this lane's column in slot d (kPlain)
+    auto column_off = [&](const int d, const int t) {
+        return kPlain && kGrouped ? (float)((ZC[d][t] >> (8 * (j & 3))) & 0xffu) - 120.0f : 8.0f;
+    };
+    auto cvt1 = [&](const u32 w, const float off, v4u& out) {
+        if constexpr (kPlain) {
+            out = plain_nibbles(w, off);
+            return;
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             if constexpr (kRows) out[e] = ((e ? w >> (4 * e - 3) : w << 3) & 0x00780078u) ^ 0x41C041C0u;
@@ -360,8 +378,9 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
                 const float sc = kF32 ? __uint_as_float(Zk[a][t][r])
                                       : (r & 1) ? bf_hi(Zk[a][t][r >> 1]) : bf_lo(Zk[a][t][r >> 1]);
                 const float zu = (float)((Zk[a][t][kZ - 1] >> (8 * r)) & 0xffu);
-                // (kRows: (24 + zero) * sum(x), the factor exact)
-                const float d = kRows ? __builtin_fmaf(104.0f - zu, accs[a][r], acc[a][t][r])
+                // (kRows: (24 + zero) * sum(x), the factor exact; kPlain: nothing)
+                const float d = kPlain  ? acc[a][t][r]
+                                : kRows ? __builtin_fmaf(104.0f - zu, accs[a][r], acc[a][t][r])
                                       : __builtin_fmaf(-zu, accs[a][r], acc[a][t][r] - 8.0f * accs[a][r]);
                 tot[t][r] = __builtin_fmaf(sc, d, tot[t][r]);
             }
@@ -379,6 +398,9 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
         constexpr bool x_later = decltype(x_later_c)::value;
         constexpr int b = d & 1, dn = (d + 1) % kD;
         constexpr int ab = kGrouped ? b : 0;
+        float off[kSW];
+#pragma unroll
+        for (int t = 0; t < kSW; ++t) off[t] = has_next ? column_off(dn, t) : 0.f;
         if (has_next && !x_later) {
             int nx = i + 1 < U ? i + 1 : 0;
             if (kHalves) nx = nx >= Uh ? nx - Uh : nx;
@@ -387,15 +409,16 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const bool fresh = kGrouped && s == 0;  // (constant once unrolled)
-            accs[ab] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(ones), as_bf8(xf[b][s]),
-                                                               fresh ? zero4 : accs[ab], 0, 0, 0);
+            if constexpr (!kPlain)
+                accs[ab] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(ones), as_bf8(xf[b][s]),
+                                                                   fresh ? zero4 : accs[ab], 0, 0, 0);
 #pragma unroll
             for (int t = 0; t < kSW; ++t)
                 acc[ab][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     as_bf8(av[b][t][s]), as_bf8(xf[b][s]), fresh ? zero4 : acc[ab][t], 0, 0, 0);
             if (has_next) {
 #pragma unroll
-                for (int t = 0; t < kSW; ++t) cvt1(W[dn][t][s], av[b ^ 1][t][s]);
+                for (int t = 0; t < kSW; ++t) cvt1(W[dn][t][s], off[t], av[b ^ 1][t][s]);
             }
             if (s == 1) {
                 if (kGrouped && fold_prev) fold(b ^ 1);
@@ -408,7 +431,14 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
                 }
             }
         }
-        if (has_next) {
+        if (has_next && kPlain) {
+            // per step: kSW MFMAs against about 24 kSW conversions
+#pragma unroll
+            for (int k = 0; k < 4 * kSW; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 24, 0);
+            }
+        } else if (has_next) {
             // per step: (1 + kSW) MFMAs against 7 kSW conversions
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -448,7 +478,7 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
 #pragma unroll
     for (int t = 0; t < kSW; ++t)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) cvt1(W[0][t][s], av[0][t][s]);
+        for (int s = 0; s < 4; ++s) cvt1(W[0][t][s], column_off(0, t), av[0][t][s]);
     if constexpr (kGrouped) {
 #pragma unroll
         for (int t = 0; t < kSW; ++t)
@@ -511,7 +541,8 @@ __device__ __forceinline__ void gemv_w4s_body(const W4sParams& p, const int bloc
             for (int t = 0; t < kSW; ++t)
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr)
-                    tot[t][rr] = kRows ? __builtin_fmaf(-24.0f, accs[0][rr], acc[0][t][rr])
+                    tot[t][rr] = kPlain  ? acc[0][t][rr]
+                                 : kRows ? __builtin_fmaf(-24.0f, accs[0][rr], acc[0][t][rr])
                                        : acc[0][t][rr] - 136.0f * accs[0][rr];
         }
         const bool one_red = kRows && p.one_red;
@@ -644,20 +675,24 @@ __global__ __launch_bounds__(kT) void gemv_w4s_one(W4sParams p) {
 // part, as the forms above; the clamped addresses and column-by-column epilogue cost 0.4 ... 1 us against them.  Graph
 // nodes, us, kernel on the stored weights -> this one: float32 8 x 4096 x 14336 grouped 16.5 -> 12.2, 8 x 4096 x 4096
 // 9.5 -> 6.6, 1 x 8192 x 8192 15.3 -> 9.5; bfloat16 16 x 4096 x 14336 19.2 -> 11.0, 1 x 768 x 768 5.8 -> 3.5,
-// 16 x 1600 x 6400 10.2 -> 6.1, 3 x 2048 x 5247 350 -> 5.6 (one output per thread before).  Error against 64 bits
-// (2-norm): float32 5.4e-6 ... 8.3e-6 -> 4.4e-6 ... 5e-6 in two parts, 2.1e-7 -> 1.0e-7 in three; bfloat16 the same.
-template <int kSW, int kD, int kNP, bool kGrouped, int kParts>
+// 16 x 1600 x 6400 10.2 -> 6.1.  Error against 64 bits (2-norm): float32 in two parts 5.4e-6 ... 8.3e-6 -> 4.4e-6 ...
+// 5e-6; bfloat16 the same.
+// kPlain (one output per thread before): 5 x 2048 x 5247 bfloat16 350 -> 6.3, float32 7.9.  The conversion's 24 operations
+// per dword, twice those with an offset, show once a workgroup walks much: 6.1 and 7.2 with an offset, 4096 x 14001 at one
+// bfloat16 row 11.6 against 9.8.  Error of float32 rows of 2048 x 5247: grouped 2.1e-7 -> 7e-8, without negative values
+// 1.4e-7 -> 7e-8 (1.2e-7 with an offset); per channel 7.9e-7 -> 6e-8 and 4.6e-7 -> 5e-8 (5.8e-7 with an offset).
+template <int kSW, int kD, int kNP, bool kGrouped, int kParts, bool kPlain>
 __global__ __launch_bounds__(kT) void gemv_w4s_rows(W4sParams p) {
-    gemv_w4s_body<kSW, kD, kNP, kGrouped, false, false, kParts>(p, blockIdx.x, gridDim.x);
+    gemv_w4s_body<kSW, kD, kNP, kGrouped, false, false, kParts, kPlain>(p, blockIdx.x, gridDim.x);
 }
 
 // the same for several kernels against one x (as gemv_w4s)
-template <int kSW, int kD, int kNP, bool kGrouped, int kParts>
+template <int kSW, int kD, int kNP, bool kGrouped, int kParts, bool kPlain>
 __global__ __launch_bounds__(kT) void gemv_w4s_rows_multi(W4sMulti mp) {
     const int bx = blockIdx.x;
     int i = 0;
     while (i + 1 < mp.count && bx >= mp.first[i + 1]) ++i;
-    gemv_w4s_body<kSW, kD, kNP, kGrouped, false, false, kParts>(mp.p[i], bx - mp.first[i], mp.first[i + 1] - mp.first[i]);
+    gemv_w4s_body<kSW, kD, kNP, kGrouped, false, false, kParts, kPlain>(mp.p[i], bx - mp.first[i], mp.first[i + 1] - mp.first[i]);
 }
 
 // 9 ... 16 rows of a K too long for LDS: x in two halves (two strips per wave, ring of two, one turn)
@@ -874,34 +909,34 @@ W4sKernels pick_kernel(const W4sPlan& pl, bool grouped) {
     return grouped ? pick_np<1, 2, true>(pl.np) : pick_np<1, 2, false>(pl.np);
 }
 
-template <int kSW, int kD, int kParts>
+template <int kSW, int kD, int kParts, bool kPlain>
 void (*pick_rows_multi_np(const W4sPlan& pl, bool grouped))(W4sMulti) {
     if (pl.np == 2)
-        return grouped ? gemv_w4s_rows_multi<kSW, kD, 2, true, kParts> : gemv_w4s_rows_multi<kSW, kD, 2, false, kParts>;
-    return grouped ? gemv_w4s_rows_multi<kSW, kD, 8, true, kParts> : gemv_w4s_rows_multi<kSW, kD, 8, false, kParts>;
+        return grouped ? gemv_w4s_rows_multi<kSW, kD, 2, true, kParts, kPlain> : gemv_w4s_rows_multi<kSW, kD, 2, false, kParts, kPlain>;
+    return grouped ? gemv_w4s_rows_multi<kSW, kD, 8, true, kParts, kPlain> : gemv_w4s_rows_multi<kSW, kD, 8, false, kParts, kPlain>;
 }
 
-template <int kParts>
+template <int kParts, bool kPlain>
 void (*pick_rows_multi(const W4sPlan& pl, bool grouped))(W4sMulti) {
     if (pl.sw == 2)
-        return pl.d == 4 ? pick_rows_multi_np<2, 4, kParts>(pl, grouped) : pick_rows_multi_np<2, 2, kParts>(pl, grouped);
-    return pl.d == 4 ? pick_rows_multi_np<1, 4, kParts>(pl, grouped) : pick_rows_multi_np<1, 2, kParts>(pl, grouped);
+        return pl.d == 4 ? pick_rows_multi_np<2, 4, kParts, kPlain>(pl, grouped) : pick_rows_multi_np<2, 2, kParts, kPlain>(pl, grouped);
+    return pl.d == 4 ? pick_rows_multi_np<1, 4, kParts, kPlain>(pl, grouped) : pick_rows_multi_np<1, 2, kParts, kPlain>(pl, grouped);
 }
 
-template <int kSW, int kD, int kParts>
+template <int kSW, int kD, int kParts, bool kPlain>
 void (*pick_rows_np(const W4sPlan& pl, bool grouped))(W4sParams) {
-    if (pl.np == 2) return grouped ? gemv_w4s_rows<kSW, kD, 2, true, kParts> : gemv_w4s_rows<kSW, kD, 2, false, kParts>;
+    if (pl.np == 2) return grouped ? gemv_w4s_rows<kSW, kD, 2, true, kParts, kPlain> : gemv_w4s_rows<kSW, kD, 2, false, kParts, kPlain>;
     if constexpr (kParts == 1) {
         if (pl.np == 16)
-            return grouped ? gemv_w4s_rows<kSW, kD, 16, true, 1> : gemv_w4s_rows<kSW, kD, 16, false, 1>;
+            return grouped ? gemv_w4s_rows<kSW, kD, 16, true, 1, kPlain> : gemv_w4s_rows<kSW, kD, 16, false, 1, kPlain>;
     }
-    return grouped ? gemv_w4s_rows<kSW, kD, 8, true, kParts> : gemv_w4s_rows<kSW, kD, 8, false, kParts>;
+    return grouped ? gemv_w4s_rows<kSW, kD, 8, true, kParts, kPlain> : gemv_w4s_rows<kSW, kD, 8, false, kParts, kPlain>;
 }
 
-template <int kParts>
+template <int kParts, bool kPlain>
 void (*pick_rows(const W4sPlan& pl, bool grouped))(W4sParams) {
-    if (pl.sw == 2) return pl.d == 4 ? pick_rows_np<2, 4, kParts>(pl, grouped) : pick_rows_np<2, 2, kParts>(pl, grouped);
-    return pl.d == 4 ? pick_rows_np<1, 4, kParts>(pl, grouped) : pick_rows_np<1, 2, kParts>(pl, grouped);
+    if (pl.sw == 2) return pl.d == 4 ? pick_rows_np<2, 4, kParts, kPlain>(pl, grouped) : pick_rows_np<2, 2, kParts, kPlain>(pl, grouped);
+    return pl.d == 4 ? pick_rows_np<1, 4, kParts, kPlain>(pl, grouped) : pick_rows_np<1, 2, kParts, kPlain>(pl, grouped);
 }
 
 int fill_params(W4sParams& p, const W4sPlan& pl, const void* x, int64_t M, int64_t K, int64_t N,
@@ -1042,11 +1077,10 @@ extern "C" int k3q_w4s_rows_pack_params(const void* scale, int dtype, const int8
 }
 
 namespace {
-// Parts of a float32 row: two (to 2^-17) where the kernel on the stored weights splits x in two as well, three
-// (exact) where that kernel has float32 products (N % 8, K % 16).
-int parts_of(int x_dtype, int64_t K, int64_t N) {
-    return x_dtype != K3Q_F32 ? 1 : (N % 8) == 0 && (K % 16) == 0 ? 2 : 3;
-}
+// Where the kernel on the stored weights has float32 products (N % 8, K % 16): the weights without an offset, and
+// float32 rows in three parts (exact); two (to 2^-17) where that kernel splits x in two as well.
+bool plain_of(int64_t K, int64_t N) { return (N % 8) != 0 || (K % 16) != 0; }
+int parts_of(int x_dtype, int64_t K, int64_t N) { return x_dtype != K3Q_F32 ? 1 : plain_of(K, N) ? 3 : 2; }
 }  // namespace
 
 extern "C" int k3q_gemv_w4s_rows_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size) {
@@ -1107,13 +1141,14 @@ extern "C" int k3q_gemv_w4s_rows_multi(const void* x, int x_dtype, int64_t M, in
     };
     for (int at = 0; at < count;) {
         const int parts = parts_of(x_dtype, K, problems[at].N);
+        const bool plain = plain_of(K, problems[at].N);
         const W4sRowsPlan first = plan_of(at, 0);
         int n = 1;
         int64_t total = first.groups;
         if (first.rows >= M && first.np <= 8)
             for (; at + n < count && n < kMaxProblems; ++n) {
                 const W4sRowsPlan pl = plan_of(at + n, 0);
-                if (parts_of(x_dtype, K, problems[at + n].N) != parts || pl.sw != first.sw || pl.d != first.d ||
+                if (plain_of(K, problems[at + n].N) != plain || pl.sw != first.sw || pl.d != first.d ||
                     pl.np != first.np || pl.rows < M)
                     break;
                 total += pl.groups;
@@ -1138,9 +1173,10 @@ extern "C" int k3q_gemv_w4s_rows_multi(const void* x, int x_dtype, int64_t M, in
         }
         mp.first[n] = next_block;
         mp.count = n;
-        void (*kernel)(W4sMulti) = parts == 1   ? pick_rows_multi<1>(pl, grouped)
-                                   : parts == 2 ? pick_rows_multi<2>(pl, grouped)
-                                                : pick_rows_multi<3>(pl, grouped);
+        void (*kernel)(W4sMulti) = parts == 3   ? pick_rows_multi<3, true>(pl, grouped)
+                                   : parts == 2 ? pick_rows_multi<2, false>(pl, grouped)
+                                   : plain      ? pick_rows_multi<1, true>(pl, grouped)
+                                                : pick_rows_multi<1, false>(pl, grouped);
         int rc = raise_lds((const void*)kernel);
         if (rc != K3Q_OK) return rc;
         kernel<<<(unsigned)next_block, kT, pl.lds, (hipStream_t)stream>>>(mp);
@@ -1164,9 +1200,10 @@ extern "C" int k3q_gemv_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t 
     const size_t el = parts > 1 ? 4 : 2;
     int rc = check_rows(x, shadow, scale, gparams, grouped, bias, y, el);
     if (rc != K3Q_OK) return rc;
-    void (*kernel)(W4sParams) = parts == 1   ? pick_rows<1>(pl, grouped)
-                                : parts == 2 ? pick_rows<2>(pl, grouped)
-                                             : pick_rows<3>(pl, grouped);
+    void (*kernel)(W4sParams) = parts == 3       ? pick_rows<3, true>(pl, grouped)
+                                : parts == 2     ? pick_rows<2, false>(pl, grouped)
+                                : plain_of(K, N) ? pick_rows<1, true>(pl, grouped)
+                                                 : pick_rows<1, false>(pl, grouped);
     rc = raise_lds((const void*)kernel);
     for (int64_t m0 = 0; m0 < M && rc == K3Q_OK; m0 += pl.rows) {
         const int64_t stride = bias ? bias_stride : 0;

@@ -698,6 +698,8 @@ def int4_matmul_tiles_rows(x, shadow, units, kernel_scale, kernel_zero=None, blo
         raise ValueError("per-channel int4 needs scales [N]")
     ks = kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous()
     kz = None if not grouped else (kernel_zero if kernel_zero.is_contiguous() else kernel_zero.contiguous())
+    if grouped:  # (views into larger buffers: the kernel reads four zero points, four scales at a time)
+        ks, kz = (t.clone() if t.data_ptr() % 16 else t for t in (ks, kz))
     b = bias if bias is None or bias.is_contiguous() else bias.contiguous()
     stride = N if bias is not None and M > 1 and bias.numel() == M * N else 0
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)

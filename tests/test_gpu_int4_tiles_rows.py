@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from keras_amd import ops as kops
+from keras_amd.layers import Dense
 from tests.helpers import c_w4_matmul_f64
 from tests.test_gpu_int4_matmul import make_layer
 from tests.test_gpu_int4_strip_rows import magnitude
@@ -49,3 +50,17 @@ def test_tiles_rows(dev, dtype, M, K, N, block_size):
         size = exact.abs() + (0 if b is None else 2 * b.double().abs())
         bound = mag * 4 * 2.0 ** -24 * K ** 0.5 + size * 3.05 * 2.0 ** -8
     assert bool((err <= bound).all()), float((err / bound).max())
+
+
+def test_layer_with_parameters_that_start_anywhere(dev):
+    """Scales and zero points assigned from views into larger buffers, which the kernels on the stored weights take."""
+    layer = Dense(96, device="cuda:0")
+    layer.build((None, 256))
+    layer.quantize("int4")
+    x = torch.randn(40, 256, generator=torch.Generator().manual_seed(0)).to(dev)
+    want = layer(x)
+    for var in (layer.kernel_scale, layer.kernel_zero):
+        buffer = torch.empty(var.value.numel() + 1, dtype=var.value.dtype, device=dev)
+        buffer[1:] = var.value.flatten()
+        var.assign(buffer[1:].view(var.shape))
+    assert torch.equal(layer(x), want)
