@@ -367,6 +367,12 @@ int k3q_gemv_w4s_rows_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int
 int k3q_gemv_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
                       const void* scale, const void* gparams, int64_t block_size, const void* bias,
                       int64_t bias_stride, void* y, void* stream);
+/* The same with weights and rows as for N % 8, whatever the shape: for callers whose other kernel multiplies float32
+ * values (k3q_gemv_w4_nk where K % 128). */
+int k3q_gemv_w4s_rows_plain_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size);
+int k3q_gemv_w4s_rows_plain(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                            const void* scale, const void* gparams, int64_t block_size, const void* bias,
+                            int64_t bias_stride, void* y, void* stream);
 int k3q_gemv_w4s_rows_multi(const void* x, int x_dtype, int64_t M, int64_t K, int count,
                             const k3q_gemv_w4s_problem* problems, int64_t block_size, void* stream);
 int k3q_gemv_w4s_multi(const void* x, int x_dtype, int64_t M, int64_t K, int count,

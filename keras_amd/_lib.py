@@ -115,6 +115,9 @@ SIGNATURES = {
     "k3q_gemv_w4s_rows_launches": (_int, [_int, _i64, _i64, _i64, _i64]),
     "k3q_gemv_w4s_rows": (
         _int, [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
+    "k3q_gemv_w4s_rows_plain_launches": (_int, [_int, _i64, _i64, _i64, _i64]),
+    "k3q_gemv_w4s_rows_plain": (
+        _int, [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
     "k3q_gemv_w4s_rows_multi": (_int, [_ptr, _int, _i64, _i64, _int, _ptr, _i64, _ptr]),
     "k3q_gemv_w4s_multi": (_int, [_ptr, _int, _i64, _i64, _int, _ptr, _i64, _ptr]),
     "k3q_gemv_w4s_pre": (_int, [_ptr, _int, _i64, _i64, _ptr, _int, _ptr, _i64, _int, _ptr]),

@@ -1080,13 +1080,21 @@ namespace {
 // Where the kernel on the stored weights has float32 products (N % 8, K % 16): the weights without an offset, and
 // float32 rows in three parts (exact); two (to 2^-17) where that kernel splits x in two as well.
 bool plain_of(int64_t K, int64_t N) { return (N % 8) != 0 || (K % 16) != 0; }
-int parts_of(int x_dtype, int64_t K, int64_t N) { return x_dtype != K3Q_F32 ? 1 : plain_of(K, N) ? 3 : 2; }
+int parts_of(int x_dtype, bool plain) { return x_dtype != K3Q_F32 ? 1 : plain ? 3 : 2; }
+
+int rows_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, bool plain) {
+    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return 0;
+    const W4sRowsPlan pl = w4s_rows_plan(parts_of(x_dtype, plain), M, K, N, block_size);
+    return pl.ok ? (int)((M + pl.rows - 1) / pl.rows) : 0;
+}
 }  // namespace
 
 extern "C" int k3q_gemv_w4s_rows_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size) {
-    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return 0;
-    const W4sRowsPlan pl = w4s_rows_plan(parts_of(x_dtype, K, N), M, K, N, block_size);
-    return pl.ok ? (int)((M + pl.rows - 1) / pl.rows) : 0;
+    return rows_launches(x_dtype, M, K, N, block_size, plain_of(K, N));
+}
+
+extern "C" int k3q_gemv_w4s_rows_plain_launches(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size) {
+    return rows_launches(x_dtype, M, K, N, block_size, true);
 }
 
 namespace {
@@ -1132,16 +1140,17 @@ extern "C" int k3q_gemv_w4s_rows_multi(const void* x, int x_dtype, int64_t M, in
     const size_t el = x_dtype == K3Q_F32 ? 4 : 2;
     for (int i = 0; i < count; ++i) {
         const k3q_gemv_w4s_problem& q = problems[i];
-        if (q.N <= 0 || !w4s_rows_plan(parts_of(x_dtype, K, q.N), M, K, q.N, block_size).ok) return K3Q_ERR_SHAPE;
+        if (q.N <= 0 || !w4s_rows_plan(parts_of(x_dtype, plain_of(K, q.N)), M, K, q.N, block_size).ok) return K3Q_ERR_SHAPE;
         const int rc = check_rows(x, q.shadow, q.scale, q.gparams, grouped, q.bias, q.y, el);
         if (rc != K3Q_OK) return rc;
     }
     auto plan_of = [&](int i, int64_t shared) {
-        return w4s_rows_plan(parts_of(x_dtype, K, problems[i].N), M, K, problems[i].N, block_size, shared);
+        const int64_t N = problems[i].N;
+        return w4s_rows_plan(parts_of(x_dtype, plain_of(K, N)), M, K, N, block_size, shared);
     };
     for (int at = 0; at < count;) {
-        const int parts = parts_of(x_dtype, K, problems[at].N);
         const bool plain = plain_of(K, problems[at].N);
+        const int parts = parts_of(x_dtype, plain);
         const W4sRowsPlan first = plan_of(at, 0);
         int n = 1;
         int64_t total = first.groups;
@@ -1186,24 +1195,24 @@ extern "C" int k3q_gemv_w4s_rows_multi(const void* x, int x_dtype, int64_t M, in
     return K3Q_OK;
 }
 
-extern "C" int k3q_gemv_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
-                                 const void* scale, const void* gparams, int64_t block_size, const void* bias,
-                                 int64_t bias_stride, void* y, void* stream) {
+static int run_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                        const void* scale, const void* gparams, int64_t block_size, const void* bias,
+                        int64_t bias_stride, void* y, void* stream, bool plain) {
     if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
     if (M < 0 || K <= 0 || N <= 0) return K3Q_ERR_SHAPE;
     if (M == 0) return K3Q_OK;
     if (bias_stride != 0 && bias_stride != N) return K3Q_ERR_SHAPE;
     const bool grouped = block_size > 0;
-    const int parts = parts_of(x_dtype, K, N);
+    const int parts = parts_of(x_dtype, plain);
     const W4sRowsPlan pl = w4s_rows_plan(parts, M, K, N, block_size);
     if (!pl.ok) return K3Q_ERR_SHAPE;
     const size_t el = parts > 1 ? 4 : 2;
     int rc = check_rows(x, shadow, scale, gparams, grouped, bias, y, el);
     if (rc != K3Q_OK) return rc;
-    void (*kernel)(W4sParams) = parts == 3       ? pick_rows<3, true>(pl, grouped)
-                                : parts == 2     ? pick_rows<2, false>(pl, grouped)
-                                : plain_of(K, N) ? pick_rows<1, true>(pl, grouped)
-                                                 : pick_rows<1, false>(pl, grouped);
+    void (*kernel)(W4sParams) = parts == 3   ? pick_rows<3, true>(pl, grouped)
+                                : parts == 2 ? pick_rows<2, false>(pl, grouped)
+                                : plain      ? pick_rows<1, true>(pl, grouped)
+                                             : pick_rows<1, false>(pl, grouped);
     rc = raise_lds((const void*)kernel);
     for (int64_t m0 = 0; m0 < M && rc == K3Q_OK; m0 += pl.rows) {
         const int64_t stride = bias ? bias_stride : 0;
@@ -1214,6 +1223,19 @@ extern "C" int k3q_gemv_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t 
         rc = launch_status();
     }
     return rc;
+}
+
+extern "C" int k3q_gemv_w4s_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                                 const void* scale, const void* gparams, int64_t block_size, const void* bias,
+                                 int64_t bias_stride, void* y, void* stream) {
+    return run_w4s_rows(x, x_dtype, M, K, N, shadow, scale, gparams, block_size, bias, bias_stride, y, stream,
+                        plain_of(K, N));
+}
+
+extern "C" int k3q_gemv_w4s_rows_plain(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                                       const void* scale, const void* gparams, int64_t block_size, const void* bias,
+                                       int64_t bias_stride, void* y, void* stream) {
+    return run_w4s_rows(x, x_dtype, M, K, N, shadow, scale, gparams, block_size, bias, bias_stride, y, stream, true);
 }
 
 extern "C" int k3q_gemv_w4s_supported(int64_t M, int64_t K, int64_t N, int64_t block_size) {

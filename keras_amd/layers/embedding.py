@@ -610,16 +610,20 @@ class ReversibleEmbedding(Embedding):
         rows, of which a workgroup walks many with little in flight (us, in place / from the copy, a cast of the rows
         included: 4096 x 32000 grouped, float32 scales, 1 and 8 bfloat16 rows 25.6 / 20.6 and 28.6 / 22.2, float32 rows
         29.1 / 18.4 and 62.5 / 20.0; 2048 x 32000 bfloat16 rows 14.3 / 15.0, float32 rows 16.5 / 13.5; 768 x 50257
-        11.4 / 22.6)."""
+        11.4 / 22.6).  Where K % 128 the kernel in place multiplies float32 values, one output per thread: the rows go in
+        full there, against weights without an offset (4544 x 32000 grouped, 1 and 4 rows: float32 669 / 28 and 2405 / 30,
+        bfloat16 677 / 25 and 2411 / 26; with an offset 23 and 20, but 2.2e-7 -> 4.9e-6 from 64 bits)."""
         K, N = self._orig_output_dim, self.input_dim
+        plain = K % 128 != 0
         if K < (2048 if x2.dtype == scale.dtype else 4096):
             return None
         if not (x2.is_cuda and x2.dtype in (torch.float32, torch.bfloat16) and scale.dtype in (torch.float32, torch.bfloat16)
                 and _promote(x2.dtype, scale.dtype) == scale.dtype and (grouped or x2.dtype == scale.dtype)
                 and 0 < x2.shape[0] <= kops.STRIP_MAX_ROWS and x2.shape[1] == K
-                and kops.int4_strip_rows_launches(scale.dtype, x2.shape[0], K, N, block_size if grouped else None) == 1):
+                and kops.int4_strip_rows_launches(scale.dtype, x2.shape[0], K, N, block_size if grouped else None,
+                                                  plain=plain) == 1):
             return None
-        spec = dict(shadow=self._cached("w4s", self._embeddings, self._relay_tied))
+        spec = dict(shadow=self._cached("w4s", self._embeddings, self._relay_tied), plain=plain)
         if not grouped:
             spec["kernel_scale"] = scale if scale.is_contiguous() else scale.contiguous()
             return spec

@@ -300,10 +300,12 @@ def int4_matmul_strip(x, shadow, units, kernel_scale=None, gparams=None, block_s
     return _shaped(y, lead)
 
 
-def int4_strip_rows_launches(dtype, M, K, N, block_size=None):
+def int4_strip_rows_launches(dtype, M, K, N, block_size=None, plain=False):
     """How many launches `int4_matmul_strip_rows` needs for M rows of `dtype`; 0: it does not take them."""
     bs = int(block_size) if block_size is not None and block_size > 0 else -1
-    return _lib.load().k3q_gemv_w4s_rows_launches(_lib.dtype_code(dtype), int(M), int(K), int(N), bs)
+    lib = _lib.load()
+    launches = lib.k3q_gemv_w4s_rows_plain_launches if plain else lib.k3q_gemv_w4s_rows_launches
+    return launches(_lib.dtype_code(dtype), int(M), int(K), int(N), bs)
 
 
 def int4_strip_rows_params(kernel_scale, kernel_zero, K, units, block_size):
@@ -326,10 +328,11 @@ def int4_strip_rows_params(kernel_scale, kernel_zero, K, units, block_size):
     return out
 
 
-def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, block_size=None, bias=None):
+def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, block_size=None, bias=None, plain=False):
     """`x[..., K] . W4[K, N]` for up to 16 float32 or bfloat16 rows, any K % 8 and any N, from
     `int4_strip_copy(kernel)`.  Per-channel: `kernel_scale` [N] in x's dtype; grouped (block 128): `gparams` from
-    `int4_strip_rows_params`.  `bias` [N], or [M, N]: a row per row of x.
+    `int4_strip_rows_params`.  `bias` [N], or [M, N]: a row per row of x.  `plain`: the weights without an offset and
+    float32 rows in full, as where N % 8 or K % 16, whatever the shape.
     Reference: keras/src/layers/core/dense.py:988-1095."""
     _lib.require_device(x, shadow, kernel_scale, gparams, bias)
     lib = _lib.load()
@@ -356,9 +359,9 @@ def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, bl
         raise ValueError("per-channel int4 needs scales [N] in the input's dtype")
     ks = None if grouped else (kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous())
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    rc = lib.k3q_gemv_w4s_rows(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
-                               _lib.ptr(gparams) if grouped else None, bs, _lib.ptr(b), stride, _lib.ptr(y),
-                               _lib.stream_ptr(x.device))
+    run = lib.k3q_gemv_w4s_rows_plain if plain else lib.k3q_gemv_w4s_rows
+    rc = run(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks), _lib.ptr(gparams) if grouped else None, bs,
+             _lib.ptr(b), stride, _lib.ptr(y), _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_gemv_w4s_rows")
     return _shaped(y, lead)
 
