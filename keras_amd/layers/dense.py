@@ -118,6 +118,12 @@ def int4_strip_rows_route(dtype, rows, input_dim, units, block_size):
     launches = kops.int4_strip_rows_launches(dtype, rows, input_dim, units, block_size)
     if units % 8 or input_dim % 16:
         return launches > 0
+    # All of K stays inside a workgroup here, however few columns there are; the kernel on the stored weights splits K.  At
+    # the widths it fills the chip with, a long enough K is faster split (us, stored against strip, 1 row: 24576 x 768
+    # float32 12.1 / 13.3, 28672 x 1024 13.9 / 14.9, 32768 x 576 13.2 / 16.0; bfloat16 43008 x 512 15.4 / 17.6).  Wider or
+    # narrower it is not (24576 x 512 float32 16.5 / 13.1, 28672 x 512 25.5 / 14.6, 32768 x 256 25.7 / 15.6, 1152 16.8 / 16.4).
+    if 384 < units <= 1024 and input_dim >= (24576 if units > 640 else 32768):
+        return False
     return 0 < launches <= (-(-rows // 8) if dtype == torch.float32 else 1)
 
 
@@ -170,7 +176,9 @@ def int8_strip_route(quantizer, x2, units, strict=False):
     Every shape it takes is faster there than behind the two-launch routes (rows 1, 4, 8 and 16,
     quantizer included, us, strip against stored kernel or tiles: K=N=4096 float32 8.8 / 9.6 / 9.8 / 10.3
     against 12.2 / 13.3 / 14.0 / 29.4; K=1600, N=6400 8.5 ... 10.6 against 10.6 ... 12.2; K=8192, N=1024
-    8.6 ... 11.9 against 13.9 ... 48.7; K=N=768 6.7 ... 7.5 against 9.2 ... 13.3).
+    8.6 ... 11.9 against 13.9 ... 48.7; K=N=768 6.7 ... 7.5 against 9.2 ... 13.3).  So it is for a long K on few columns,
+    all of which stays in a workgroup (cold weights: K=28672, 1 row, N=16 / 512 / 1024 / 8192 float32 19.0 / 20.8 / 23.1 /
+    51.4 against 27.9 / 35.1 / 40.6 / 58.1; K=14336, N=128, 8 rows 16.2 against 21.5).
     strict: only bfloat16 rows and the widths of `ops.int8_strip_supported`: what a launch that several
     layers share takes, and what a tied table keeps a copy for."""
     if not (type(quantizer) is quantizers.AbsMaxQuantizer and quantizer.output_dtype == "int8"

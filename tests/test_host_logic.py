@@ -248,3 +248,14 @@ def test_resident_bytes_counts_variables_once():
     layer = Dense(8, dtype="float32", device="cpu")
     layer.build((None, 4))
     assert layer.resident_bytes() == {"stored": 4 * 8 * 4 + 8 * 4, "derived": 0}
+
+
+@pytest.mark.parametrize("input_dim,units,takes", [
+    (28672, 1024, False), (24576, 768, False), (32768, 576, False), (28672, 512, True), (24576, 640, True),
+    (28672, 1152, True), (32768, 256, True), (22528, 1024, True), (16384, 1001, True)])
+def test_long_narrow_int4_kernels_are_left_to_the_kernel_that_splits_their_input_width(input_dim, units, takes):
+    """(N % 8: only one output per thread is left there, every such shape stays.)"""
+    from keras_amd.layers.dense import int4_strip_rows_route
+
+    assert int4_strip_rows_route(torch.float32, 1, input_dim, units, 128) is takes
+    assert int4_strip_rows_route(torch.bfloat16, 1, input_dim, units, 128) is takes
