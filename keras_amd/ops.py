@@ -1240,7 +1240,9 @@ def decode_attention(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_f
 
 
 def rope_cache_supported(q, k, v, cos_table, sin_table, cache_k, cache_v):
-    """bfloat16, head width 128, caches and tables that are contiguous, all on one device."""
+    """bfloat16, head width 128, caches and tables that are contiguous, all on one device, nothing to differentiate."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v, cache_k, cache_v)):
+        return False  # (the launch is none of autograd's)
     return (q.dim() == 4 and q.shape[-1] == 128 and q.shape[1] > 0 and k.shape == q.shape and v.shape == q.shape
             and cache_k.is_contiguous() and cache_v.is_contiguous()
             and tuple(cos_table.shape) == (cache_k.shape[2], 128) and sin_table.shape == cos_table.shape
@@ -1258,7 +1260,8 @@ def rope_cache(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_flag=No
     B, T, H, hd = q.shape
     max_len = cache_k.shape[2]
     if not rope_cache_supported(q, k, v, cos_table, sin_table, cache_k, cache_v):
-        raise ValueError("rope_cache takes bfloat16 q, k, v [B, T, H, 128] and contiguous caches and tables")
+        raise ValueError("rope_cache takes bfloat16 q, k, v [B, T, H, 128] that need no gradient and contiguous caches "
+                         "and tables")
     if tuple(cache_k.shape) != (B, H, max_len, hd) or cache_v.shape != cache_k.shape:
         raise ValueError(f"caches must be [B, H, max_len, hd], got {tuple(cache_k.shape)}")
     if pos.dtype != torch.int64 or tuple(pos.shape) != (T,) or not pos.is_contiguous():

@@ -4,7 +4,8 @@ import pytest
 import torch
 
 from keras_amd import ops as kops
-from keras_amd.decoder_harness import apply_rope, rope_tables
+from keras_amd.decoder_harness import DecoderBlock, apply_rope, rope_tables
+from keras_amd.layers.layer import as_tensor
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +40,26 @@ def test_rope_cache_position_outside(dev):
     x = 2 * mk(1, 2, 2, 128)
     kops.rope_cache(x, x, x, cos_t, sin_t, torch.tensor([7, 8], device=dev), kc, vc, oob_flag=flag)
     assert int(flag) == 1 and float(vc[:, :, 7].min()) == 2.0 and float(vc[:, :, :7].max()) == 1.0
+
+
+def test_prompt_keeps_the_gradient_of_the_attention_projections(dev):
+    """The launch is none of autograd's: where a gradient is asked for, the torch sequence runs."""
+    block = DecoderBlock(256, 2, 512, dtype="bfloat16", device=dev, name="block")
+    cos_t, sin_t = rope_tables(128, 16, dev, dtype=torch.bfloat16)
+    pos = torch.arange(6, device=dev)
+    mask = torch.zeros(6, 16, dtype=torch.bfloat16, device=dev)
+    rows = lambda: (cos_t[:6], sin_t[:6], mask)
+    x = torch.randn(2, 6, 256, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16).to(dev)
+
+    def run():
+        cache = tuple(torch.zeros(2, 2, 16, 128, dtype=torch.bfloat16, device=dev) for _ in range(2))
+        return block.forward(x, rows, cache, pos, tables=(cos_t, sin_t))
+
+    assert not run().requires_grad
+    for projection in (block.query, block.key, block.value):
+        kernel = as_tensor(projection._kernel)
+        kernel.requires_grad_()
+        assert run().requires_grad
+        with torch.no_grad():
+            assert not run().requires_grad
+        kernel.requires_grad_(False)
