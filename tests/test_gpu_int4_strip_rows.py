@@ -93,3 +93,35 @@ def test_rows_layer_routes(dev):
         ein.quantize("int4")
         assert tuple(ein(torch.randn(2, 2, 192, generator=g).to(dt).to(dev)).shape) == (2, 2, 4, 64)
         assert "w4s" in ein._cache
+
+
+@pytest.mark.parametrize("dtype,M,K,widths,block_size", [
+    (torch.float32, 4, 256, (1003, 1001, 777), 128),          # three parts, weights without an offset
+    (torch.float32, 8, 1024, (96, 64, 48), 128),              # two parts
+    (torch.float32, 3, 512, (3200, 3200, 40), None),          # more strip groups than workgroups
+    (torch.float32, 8, 4096, (8192, 8208), 128),              # ... and room for one reduction buffer
+    (torch.bfloat16, 16, 1000, (1003, 9, 5247), 128),
+    (torch.bfloat16, 5, 1600, (6400, 6400, 1600, 1600, 1600), None),  # more kernels than a launch takes
+    (torch.float32, 2, 384, (1003, 96, 9000, 1000), 128),     # plans that differ
+    (torch.bfloat16, 2, 384, (1003, 96, 9000, 1000), 128),
+    (torch.float32, 16, 256, (96, 104), 128),                 # more rows than a launch takes
+])
+def test_shared_launch_has_the_bits_of_the_separate_calls(dev, dtype, M, K, widths, block_size):
+    g = torch.Generator(device=dev).manual_seed(K + M)
+    rand = lambda *s: torch.rand(*s, generator=g, device=dev)
+    kernels = []
+    for i, N in enumerate(widths):
+        packed = torch.randint(-128, 128, (K, (N + 1) // 2), generator=g, device=dev, dtype=torch.int8)
+        kernel = dict(units=N, shadow=kops.int4_strip_copy(packed, N),
+                      bias=rand(N).to(dtype) if i % 2 else None)
+        if block_size:
+            groups = -(-K // block_size)
+            zero = torch.randint(-8, 8, (groups, N), generator=g, device=dev, dtype=torch.int8)
+            kernel["gparams"] = kops.int4_strip_rows_params((rand(groups, N) + 1).to(dtype), zero, K, N, block_size)
+        else:
+            kernel["kernel_scale"] = (rand(N) + 1).to(dtype)
+        kernels.append(kernel)
+    x = torch.randn(M, K, generator=g, device=dev).to(dtype)
+    together = kops.int4_matmul_strip_rows_multi(x, kernels, block_size=block_size)
+    for y, kernel in zip(together, kernels):
+        assert torch.equal(y, kops.int4_matmul_strip_rows(x, block_size=block_size, **kernel))

@@ -5,7 +5,8 @@ import pytest
 import torch
 
 from keras_amd import ops as kops
-from keras_amd.layers import Dense
+from keras_amd.layers import Dense, EinsumDense
+from keras_amd.layers.dense import TILE_ROWS_MAX_F32
 from tests.helpers import c_w4_matmul_f64
 from tests.test_gpu_int4_matmul import make_layer
 from tests.test_gpu_int4_strip_rows import magnitude
@@ -64,3 +65,50 @@ def test_layer_with_parameters_that_start_anywhere(dev):
         buffer[1:] = var.value.flatten()
         var.assign(buffer[1:].view(var.shape))
     assert torch.equal(layer(x), want)
+
+
+def check_layer(layer, x, units):
+    """A layer's output against the float64 value of its variables, with the bounds above.  Without a strip-linear copy the
+    call went to the de-quantised kernel: its weights are two bfloat16 parts (2^-16 of each is lost) for float32 rows,
+    one for bfloat16 rows (2^-8)."""
+    scale, zero = layer.kernel_scale.value, layer.kernel_zero.value
+    y = layer(x).reshape(-1, units)
+    x2 = x.reshape(y.shape[0], -1).cpu()
+    args = (layer._kernel.value, scale.to(x.dtype), zero, 128, units)
+    exact = c_w4_matmul_f64(x2, args[0].cpu(), args[1].cpu(), zero.cpu(), 128, None, units)
+    mag = magnitude(x2, args[0], args[1].cpu(), zero.cpu(), 128, units)
+    err, K = (y.double().cpu() - exact).abs(), x2.shape[1]
+    if x.dtype == torch.float32:
+        bound = mag * (2.0 ** -16 + 4 * 2.0 ** -24 * K ** 0.5) + exact.abs() * 2.0 ** -22
+    else:
+        weights = 0.0 if "w4s" in layer._cache else 2.0 ** -8
+        bound = mag * (weights + 4 * 2.0 ** -24 * K ** 0.5) + exact.abs() * 1.02 * 2.0 ** -8
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("policy", ["float32", "mixed_bfloat16"])
+@pytest.mark.parametrize("kind,K,units,rows,copy", [
+    ("dense", 1000, 1003, 40, True), ("dense", 320, 1028, 600, True), ("dense", 192, 101, 1000, True),
+    ("dense", 256, 128, TILE_ROWS_MAX_F32, None), ("dense", 256, 128, TILE_ROWS_MAX_F32 + 1, False),
+    ("einsum", 192, 105, 40, True), ("einsum", 136, 105, 900, True), ("einsum", 256, 192, 300, None),
+])
+def test_layer_routes(dev, policy, kind, K, units, rows, copy):
+    """Ragged layers and float32 rows on both sides of the line to the de-quantised kernel; copy: whether the call reads the
+    strip-linear copy (None: float32 rows do)."""
+    dtype = torch.float32 if policy == "float32" else torch.bfloat16
+    if kind == "dense":
+        layer = Dense(units, dtype=policy, device="cuda:0", use_bias=False)
+        layer.build((None, K))
+    else:
+        layer = EinsumDense("btd,dnh->btnh", (None, 3, units // 3), dtype=policy, device="cuda:0")
+        layer.build((None, None, K))
+    layer.quantize("int4")
+    x = torch.randn(2, rows // 2, K, generator=torch.Generator().manual_seed(rows)).to(dtype).to(dev)
+    x = x if rows % 2 == 0 else torch.cat((x.flatten(0, 1), x[0, :1])).unsqueeze(0)
+    check_layer(layer, x, units)
+    expected = copy if copy is not None else dtype == torch.float32 or rows <= 512
+    assert ("w4s" in layer._cache) == expected
+    # (scales and zero points padded to whole strips are rebuilt with the variables)
+    layer.kernel_scale.assign(layer.kernel_scale.value * 2)
+    layer.kernel_zero.assign(-layer.kernel_zero.value)
+    check_layer(layer, x, units)
