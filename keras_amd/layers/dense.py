@@ -127,11 +127,17 @@ def int4_strip_rows_route(dtype, rows, input_dim, units, block_size):
     return 0 < launches <= (-(-rows // 8) if dtype == torch.float32 else 1)
 
 
+ROWS_PARAMS = {torch.float32: "w4s_rows_params", torch.bfloat16: "w4s_rows_params_bfloat16"}
+
+
 def strip_rows_params(layer, dtype, input_dim, units, block_size):
     """The grouped parameters of `ops.int4_matmul_strip_rows` in `dtype`: made on first use, rebuilt in place
     when a variable they come from is assigned (a captured graph holds their address).  Each dtype has its own."""
-    scale, zero = layer.kernel_scale, layer.kernel_zero
-    return cached_params(layer._cache, ("w4s_rows_params", dtype), (scale, zero), lambda: kops.int4_strip_rows_params(
+    scale, zero, key = layer.kernel_scale, layer.kernel_zero, ROWS_PARAMS[dtype]
+    hit = layer._cache.get(key)
+    if hit is not None and hit[0] == (id(scale), scale.version, id(zero), zero.version):
+        return hit[2]
+    return cached_params(layer._cache, key, scale, zero, lambda: kops.int4_strip_rows_params(
         as_tensor(scale).to(dtype), as_tensor(zero), input_dim, units, block_size))
 
 
@@ -398,9 +404,18 @@ class Dense(Layer):
     # ---- cached derived operands ------------------------------------------------
     def _cached(self, key, var, make):
         """Value derived from a variable, rebuilt when the variable is assigned."""
+        hit = self._cache.get(key)
+        # (the test of `cached_operand`, without a call: a decode-sized call looks up three or four operands)
+        if hit is not None and hit[1] is var and hit[0] == var.version and (
+                hit[3] is None or hit[3] == var._value._version):
+            return hit[2]
         return cached_operand(self._cache, key, var, make)
 
     def _read_cached(self, key, var):
+        hit = self._cache.get(key)
+        if hit is not None and hit[1] is var and hit[0] == var.version and (
+                hit[3] is None or hit[3] == var._value._version):
+            return hit[2]
         cd = to_torch_dtype(self.compute_dtype)
         return self._cached(key, var, lambda t: t.to(cd).contiguous())
 
@@ -416,7 +431,7 @@ class Dense(Layer):
                     shadow=self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)))
         if grouped:
             scale, zero = self.kernel_scale, self.kernel_zero
-            spec["gparams"] = cached_params(self._cache, "w4s_params", (scale, zero), lambda: kops.int4_strip_params(
+            spec["gparams"] = cached_params(self._cache, "w4s_params", scale, zero, lambda: kops.int4_strip_params(
                 as_tensor(scale), as_tensor(zero), input_dim, units, block_size))
         else:
             spec["kernel_scale"] = self._read_cached("kernel_scale", self.kernel_scale)

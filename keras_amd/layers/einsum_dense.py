@@ -515,6 +515,10 @@ class EinsumDense(Layer):
 
     # ---- helpers ---------------------------------------------------------------------------
     def _cached(self, key, var, make):
+        hit = self._cache.get(key)
+        if hit is not None and hit[1] is var and hit[0] == var.version and (
+                hit[3] is None or hit[3] == var._value._version):
+            return hit[2]  # (as Dense._cached)
         return cached_operand(self._cache, key, var, make)
 
     def _gemm_view(self):
@@ -532,7 +536,7 @@ class EinsumDense(Layer):
                     shadow=self._cached("w4s", self._kernel, lambda t: kops.int4_strip_copy(t, units)))
         if grouped:
             scale, zero = self.kernel_scale, self.kernel_zero
-            spec["gparams"] = cached_params(self._cache, "w4s_params", (scale, zero), lambda: kops.int4_strip_params(
+            spec["gparams"] = cached_params(self._cache, "w4s_params", scale, zero, lambda: kops.int4_strip_params(
                 as_tensor(scale), as_tensor(zero), input_dim, units, block_size))
         else:
             spec["kernel_scale"] = self._cached("kernel_scale", self.kernel_scale,

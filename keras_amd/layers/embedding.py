@@ -529,6 +529,10 @@ class ReversibleEmbedding(Embedding):
 
     # ---- quantized forward -----------------------------------------------------------
     def _cached(self, key, var, make):
+        hit = self._cache.get(key)
+        if hit is not None and hit[1] is var and hit[0] == var.version and (
+                hit[3] is None or hit[3] == var._value._version):
+            return hit[2]  # (as Dense._cached)
         return cached_operand(self._cache, key, var, make)
 
     def _int8_call(self, inputs, reverse=False, training=None):
@@ -628,7 +632,7 @@ class ReversibleEmbedding(Embedding):
             spec["kernel_scale"] = scale if scale.is_contiguous() else scale.contiguous()
             return spec
         sv, zv = self.embeddings_scale, self.embeddings_zero
-        spec["gparams"] = cached_params(self._cache, "w4s_rows_params", (sv, zv), lambda: kops.int4_strip_rows_params(
+        spec["gparams"] = cached_params(self._cache, "w4s_rows_params", sv, zv, lambda: kops.int4_strip_rows_params(
             as_tensor(sv).t().contiguous(), as_tensor(zv).to(torch.int8).t().contiguous(), K, N, block_size))
         return spec
 
@@ -647,7 +651,7 @@ class ReversibleEmbedding(Embedding):
         spec = dict(shadow=self._cached("w4s", self._embeddings, self._relay_tied))
         if grouped:
             sv, zv = self.embeddings_scale, self.embeddings_zero
-            spec["gparams"] = cached_params(self._cache, "w4s_params", (sv, zv), lambda: kops.int4_strip_params(
+            spec["gparams"] = cached_params(self._cache, "w4s_params", sv, zv, lambda: kops.int4_strip_params(
                 as_tensor(sv).t().contiguous(), as_tensor(zv).to(torch.int8).t().contiguous(), K, N, block_size))
         else:
             spec["kernel_scale"] = scale if scale.is_contiguous() else scale.contiguous()

@@ -100,30 +100,31 @@ def cached_operand(cache, key, var, make):
     tensor, and that may be the caller's): it is cloned, and follows writes into the variable's tensor, too."""
     if var is None:
         return None
-    t = as_tensor(var)
     hit = cache.get(key)
-    if (hit is not None and hit[0] == var.version and hit[1] is var
-            and (hit[3] is None or hit[3] == _writes(t))):
+    if (hit is not None and hit[1] is var and hit[0] == var.version
+            and (hit[3] is None or hit[3] == var._value._version)):
         return hit[2]
+    t = as_tensor(var)
     value = make(t)
-    writes = None
+    writes, shared = None, False
     if isinstance(value, torch.Tensor):
         if value.untyped_storage().data_ptr() == t.untyped_storage().data_ptr():
-            writes = _writes(t)
+            writes = None if t.is_inference() else t._version  # (inference tensors do not count)
+            shared = True
         if (hit is not None and isinstance(hit[2], torch.Tensor) and hit[2].shape == value.shape
                 and hit[2].dtype == value.dtype and hit[2].device == value.device):
             hit[2].copy_(value.detach())
             value = hit[2]
-        elif writes is not None:
+        elif shared:
             value = value.detach().clone()
     cache[key] = (var.version, var, value, writes)
     return value
 
 
-def cached_params(cache, key, variables, make):
-    """`make()`, a tensor packed from several variables, kept in `cache` and rebuilt in place (as `cached_operand`)
+def cached_params(cache, key, first, second, make):
+    """`make()`, a tensor packed from two variables, kept in `cache` and rebuilt in place (as `cached_operand`)
     when one of them is assigned."""
-    stamp = tuple((id(v), v.version) for v in variables)
+    stamp = (id(first), first.version, id(second), second.version)
     hit = cache.get(key)
     if hit is None or hit[0] != stamp:
         value = make()
@@ -133,11 +134,6 @@ def cached_params(cache, key, variables, make):
             value = hit[2]
         hit = cache[key] = (stamp, None, value)
     return hit[2]
-
-
-def _writes(t):
-    """How often a tensor was written in place (inference tensors do not count)."""
-    return 0 if t.is_inference() else t._version
 
 
 def require_default_g_idx(layer, block_size):
