@@ -46,7 +46,7 @@ HBM_PEAK_GBS = 8000.0    # MI355X HBM3E, published (8 TB/s)
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_bytes.json")
 CSRC = os.path.join(ROOT, "keras_amd", "csrc")
 TRAFFIC_SOURCES = {  # key prefix -> the kernel's source files (all of them include k3q_common.h)
-    "gemm_mfma": ["k3q_gemm_i8.hip"], "quantize_rows_vec": ["k3q_quantize.hip"], "gemv_w4s": ["k3q_gemv_w4s.hip"],
+    "gemm_mfma": ["k3q_gemm_i8.hip"], "quantize_rows_vec": ["k3q_quantize.hip"], "gemv_w4s": ["k3q_gemv_w4s.hip", "k3q_nibbles.h"],
     "gemv_w8s": ["k3q_gemv_w8s.hip"], "pack_int4": ["k3q_pack.hip"], "unpack_int4": ["k3q_pack.hip"],
     "embedding_rows": ["k3q_embedding.hip"], "absmax_reduce": ["k3q_weight_quantize.hip"],
     "grouped_zp": ["k3q_weight_quantize.hip"],

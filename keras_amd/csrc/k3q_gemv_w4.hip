@@ -41,7 +41,7 @@
 // thread waits for the acknowledgement of its own stores (s_waitcnt vmcnt(0)),
 // the workgroup's barrier collects those waits, and only then is the arrival
 // counted; the last workgroup reads the partials with L2-bypassing loads (sc1).
-#include "k3q_common.h"
+#include "k3q_nibbles.h"
 #include "k3q_gemm_bf16.h"
 
 #include <mutex>

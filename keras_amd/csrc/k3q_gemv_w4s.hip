@@ -29,7 +29,7 @@
 //    matrix pipe;
 //  * x is requested before any weight: requested after them it would arrive behind the whole first
 //    burst of weights (the memory system serves a launch's first requests roughly in order).
-#include "k3q_common.h"
+#include "k3q_nibbles.h"
 
 #include <mutex>
 #include <set>
