@@ -620,8 +620,13 @@ class EinsumDense(Layer):
             k2 = t if gv.k_is_view else t.permute(gv.k_perm)
             return k2.reshape(x2.shape[1], -1).contiguous()
 
-        k2 = self._cached("kernel2d", self._kernel, kernel_matrix)
-        n = k2.shape[1]
+        def stored_matrix():
+            # (as it lies where it can: a kept operand would be a copy of the kernel)
+            if gv.k_is_view:
+                return kernel_matrix(as_tensor(self._kernel))
+            return self._cached("kernel2d", self._kernel, kernel_matrix)
+
+        n = as_tensor(self._kernel).numel() // x2.shape[1]
         bias, fused = self._fusable_bias(gv, n)
         if not self.inputs_quantizer:
             # Weight-only (einsum_dense.py:1085-1101).  The torch backend divides every weight
@@ -629,7 +634,7 @@ class EinsumDense(Layer):
             # exact int8 values and the scale divides the result -- the same quantity without
             # the per-weight rounding.
             y2 = kops.int8_weight_only_matmul(
-                x2, k2,
+                x2, stored_matrix(),
                 self._cached("kernel_scale", self.kernel_scale,
                              lambda t: t.to(cd).reshape(-1).contiguous()),
                 bias=bias,
@@ -649,7 +654,7 @@ class EinsumDense(Layer):
             return self._finish(y2, free_shape, gv, fused)
         q, scale = quantize_rows(self.inputs_quantizer, x2)
         y2 = kops.int8_matmul(
-            q, k2, a_scale=scale,
+            q, stored_matrix(), a_scale=scale,
             kernel_scale=self._cached("kernel_scale", self.kernel_scale,
                                       lambda t: t.to(cd).reshape(-1).contiguous()),
             bias=bias, out_dtype=cd, exact_epilogue=exact,
