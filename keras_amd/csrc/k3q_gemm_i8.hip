@@ -85,6 +85,7 @@ struct GemmParams {
     // accumulators to part[sp][M][N] (int32 or float32); gemm_split_reduce sums them in
     // split order and applies the epilogue
     int splits, kt_split;
+    int kt_sum;  // (four stages, bfloat16 operands) the sums are set aside every so many stages, see launch_tile
     void* part;
     int64_t part_bytes;
 };
@@ -310,6 +311,33 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
             for (int mb = 0; mb < kMBlk; ++mb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[nb][mb][r] = 0;
+        // the sums set aside so far (p.kt_sum)
+        constexpr bool kSums = kStages > 2 && kKind != kKindI8;
+        typename Mma<kKind>::Acc aside[kSums ? kNBlk : 1][kSums ? kMBlk : 1];
+        auto set_aside = [&](const bool more) {
+            if constexpr (kSums) {
+                // (the last product is on its way to the accumulators when the loop ends; without a pause their last
+                // register was read before it came)
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int nb = 0; nb < kNBlk; ++nb)
+#pragma unroll
+                    for (int mb = 0; mb < kMBlk; ++mb)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            aside[nb][mb][r] = acc[nb][mb][r] + aside[nb][mb][r];
+                            acc[nb][mb][r] = more ? 0 : aside[nb][mb][r];
+                        }
+            }
+        };
+        if constexpr (kSums) {
+#pragma unroll
+            for (int nb = 0; nb < kNBlk; ++nb)
+#pragma unroll
+                for (int mb = 0; mb < kMBlk; ++mb) aside[nb][mb] = acc[nb][mb];
+        }
 
         // ---- main loop ----
         // A ring of kStages LDS stages.  The fragments of K step ks+1 are read in the middle of the MFMAs of
@@ -369,47 +397,55 @@ __global__ __launch_bounds__(T::kThreads) void gemm_mfma(GemmParams p) {
                 }
             }
         };
-        for (int kt = 0; kt < KT; ++kt) {
+        int kt = 0;
+        for (int end = kSums ? min(p.kt_sum, KT) : KT;;) {  // (once, but for kSums)
+            for (; kt < end; ++kt) {
 #pragma unroll
-            for (int ks = 0; ks < kKSteps; ++ks) {
-                // first half of this step's MFMAs, then the reads for the next step, then the
-                // second half: the reads get half a step of matrix-core time to come back
-                __builtin_amdgcn_sched_barrier(0);
-                // Raised wave priority from the first MFMA of a step to its last, dropped between
-                // steps: measured, 2 % on the exact bfloat16 path at M = 4096, K = N = 8192
-                // (233 against 238 us), neutral to 1 % elsewhere; raising it around each half
-                // separately, or only around the second, gained less.
-                __builtin_amdgcn_s_setprio(1);
-                mma_half(ks, 0, kt);
-                __builtin_amdgcn_sched_barrier(0);
-                if (ks + 1 < kKSteps) {
-                    read_frags((ks + 1) & 1, ks + 1);
-                } else if (kt + 1 < KT) {
-                    // own DMA of stage kt+1 has landed (own reads of stage kt are done): every stage up to
-                    // kt+kStages-1 has been issued whole, in order, and the ones behind kt+1 may be in flight
-                    if constexpr (kStages > 2) {
-                        if (kt + kStages <= KT) wait_vmcnt<(kStages - 2) * kDmaPerWave>();
-                        else wait_vmcnt0();
-                    } else {
-                        wait_vmcnt0();
+                for (int ks = 0; ks < kKSteps; ++ks) {
+                    // first half of this step's MFMAs, then the reads for the next step, then the
+                    // second half: the reads get half a step of matrix-core time to come back
+                    __builtin_amdgcn_sched_barrier(0);
+                    // Raised wave priority from the first MFMA of a step to its last, dropped between
+                    // steps: measured, 2 % on the exact bfloat16 path at M = 4096, K = N = 8192
+                    // (233 against 238 us), neutral to 1 % elsewhere; raising it around each half
+                    // separately, or only around the second, gained less.
+                    __builtin_amdgcn_s_setprio(1);
+                    mma_half(ks, 0, kt);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (ks + 1 < kKSteps) {
+                        read_frags((ks + 1) & 1, ks + 1);
+                    } else if (kt + 1 < KT) {
+                        // own DMA of stage kt+1 has landed (own reads of stage kt are done): every stage up to
+                        // kt+kStages-1 has been issued whole, in order, and the ones behind kt+1 may be in flight
+                        if constexpr (kStages > 2) {
+                            if (kt + kStages <= KT) wait_vmcnt<(kStages - 2) * kDmaPerWave>();
+                            else wait_vmcnt0();
+                        } else {
+                            wait_vmcnt0();
+                        }
+                        bare_barrier();
+                        if constexpr (kStages == 2) {
+                            ra ^= kStageBytes;
+                            rb ^= kStageBytes;
+                        } else {
+                            ra = (ra + kStageBytes) & (kStages * kStageBytes - 1);
+                            rb = (rb + kStageBytes) & (kStages * kStageBytes - 1);
+                        }
+                        read_frags(0, 0);
                     }
-                    bare_barrier();
-                    if constexpr (kStages == 2) {
-                        ra ^= kStageBytes;
-                        rb ^= kStageBytes;
-                    } else {
-                        ra = (ra + kStageBytes) & (kStages * kStageBytes - 1);
-                        rb = (rb + kStageBytes) & (kStages * kStageBytes - 1);
-                    }
-                    read_frags(0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma_half(ks, 1, kt);
+                    __builtin_amdgcn_s_setprio(0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (kHalfTail && ks == kKSteps / 2 - 1 && kt == kt_half) break;
                 }
-                __builtin_amdgcn_sched_barrier(0);
-                mma_half(ks, 1, kt);
-                __builtin_amdgcn_s_setprio(0);
-                __builtin_amdgcn_sched_barrier(0);
-                if (kHalfTail && ks == kKSteps / 2 - 1 && kt == kt_half) break;
             }
+            if constexpr (!kSums) break;
+            if (end >= KT) break;
+            set_aside(true);
+            end = min(end + p.kt_sum, KT);
         }
+        if (kSums && p.kt_sum < KT) set_aside(false);
 
         if (p.splits > 1) {
             // raw accumulators of this split, as they lie (16 bytes per lane and column group)
@@ -909,6 +945,12 @@ int launch_tile(GemmParams p, hipStream_t s) {
     if (splits > 1 && (!p.part || p.part_bytes < (int64_t)splits * p.M * p.N * 4)) {
         const int64_t fit = p.part ? p.part_bytes / (p.M * p.N * 4) : 0;
         splits = fit >= 2 ? (int)fit : 1;
+    }
+    if (T::kStages > 2) {
+        // One workgroup walks all of K where two, or more, each took a part of it and a second kernel added their sums.
+        // It adds the same parts: a float32 sum of many terms keeps its order, and stays a sum of shorter ones.
+        const int parts = (p.N % 4) ? 1 : choose_splits(tiles, stages, 2 * resident);
+        p.kt_sum = (stages + parts - 1) / parts;
     }
     p.kt_split = (stages + splits - 1) / splits;
     p.splits = (stages + p.kt_split - 1) / p.kt_split;  // no empty split
