@@ -19,6 +19,7 @@ SOURCES = [
     "k3q_quantize.hip",
     "k3q_weight_quantize.hip",
     "k3q_gemv_w4.hip",
+    "k3q_gemm_w4_tiles.hip",
     "k3q_gemv_w4s.hip",
     "k3q_gemv_w4_nk.hip",
     "k3q_gemv_w8.hip",

@@ -41,6 +41,7 @@
 // thread waits for the acknowledgement of its own stores (s_waitcnt vmcnt(0)),
 // the workgroup's barrier collects those waits, and only then is the arrival
 // counted; the last workgroup reads the partials with L2-bypassing loads (sc1).
+#include "k3q_gemm_w4_tiles.h"
 #include "k3q_nibbles.h"
 #include "k3q_gemm_bf16.h"
 
@@ -1155,21 +1156,12 @@ bool try_gemv_w4_multi(const void* x, int x_dtype, int64_t M, int64_t K, int cou
 constexpr int kKmBM = 128, kKmBN = 256, kKmStage = 64;  // tile; values of K per stage
 constexpr int kKmThreads = 512;                        // 8 waves: 2 (M) x 4 (N), 64 x 64 each
 constexpr u32 kKmNibbles = 0x000F000Fu, kKmFlip = 0x00080008u, kKmExp = 0x43004300u;
-// The general form (k3q_gemm_w4_rows) puts the nibbles into mantissa bits 3 ... 6 of 16.0, their sign bits flipped: the
-// bfloat16 pair (24 + w, 24 + w').  A shift more per dword and a sixth of the offset to cancel, which the float32 sums of
-// its rows need; where the sums are rounded to bfloat16 it buys nothing and the shift shows (96 rows of 4096 x 14336:
-// 27.5 -> 27.6 us in the kernel, 0.7 % of the call).
-constexpr u32 kKmNibbles24 = 0x00780078u, kKmBase24 = 0x41C041C0u;
-// How a kernel converts the nibbles: the layers' own shapes, the general form, and the general form for shapes whose kernel
-// on the stored weights multiplies float32 values (N % 8, K % 16) -- no offset there, the sums are no larger than its own.
-constexpr int kKm136 = 0, kKm24 = 1, kKmPlain = 2;
-
 __device__ __forceinline__ int km_swz(int row) { return (row & 6) | ((row ^ (row >> 3)) & 1); }
 
 struct KmParams {
     const uint16_t* x;      // [M, K] bf16
     const uint8_t* shadow;  // [N, K/2]
-    const void* scale;      // bf16 [G, N] (grouped; kernels built with kF32S: float32) or unused
+    const void* scale;      // bf16 [G, N] (grouped) or unused
     const int8_t* zero;     // [G, N] (grouped)
     const v2u* sx;          // [K / gsize, M] sums of x over each group of K, as three bfloat16 parts
     float* part;            // [KS, M, N]
@@ -1308,14 +1300,9 @@ constexpr int kKmParScale = 0, kKmParZero = 512, kKmParSx = 768, kKmParSpare = 1
 // kNB: blocks of 32 kernel rows per wave: 2 (tiles of 128 x 256) or 1 (128 x 128, for kernels so
 // narrow that wide tiles leave CUs idle even at eight splits).
 // kWM: waves along M: 2 (tiles of 128 rows) or 1 (64 rows, eight waves side by side, kNB = 1).
-// kF32S: float32 scales (twice the bytes: tiles of 128 x 128 or 64 x 256 only, whose parameters still fit).
-// kForm: the conversion (above).
-template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB, int kForm = kKm136, bool kF32S = false>
+template <bool kGrouped, int kDepth, int kGroupStages, int kWM, int kNB>
 __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
     constexpr int kWaveN = 32 * kNB, kBN = kWaveN * (8 / kWM), kBM = 64 * kWM;
-    static_assert(!kF32S || (kGrouped && kBN * kBM <= 128 * 128), "parameters of a stage");
-    // where a stage's parameters lie (kF32S: scales, then zero points, then the sums of x)
-    constexpr int kParZero = kF32S ? kBN * 4 : kKmParZero, kParSx = kF32S ? kBN * 4 + 256 : kKmParSx;
     extern __shared__ char km_lds[];
     constexpr int kXOps = kWM;               // x-tile DMA instructions a wave issues per stage
     constexpr int kOpsPerStage = kXOps + 2;  // DMA instructions a wave issues per stage
@@ -1373,28 +1360,7 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
     int par_dst;
     {
         const int w = wave;
-        constexpr int kScaleWaves = kBN / 64;  // (kF32S: a column per lane)
-        if (kF32S) {
-            if (w < kScaleWaves) {
-                par_base = (const char*)p.scale + (n0 + w * 64 + lane < p.N ? n0 + w * 64 + lane : p.N - 1) * 4;
-                par_step = p.N * 4;
-                par_dst = w * 256;
-            } else if (w == kScaleWaves) {
-                int64_t n = n0 + lane * 4;
-                if (n > p.N - 4) n = p.N - 4;
-                par_base = (const char*)p.zero + n;
-                par_step = p.N;
-                par_dst = kParZero;
-            } else {
-                const int sw = w - kScaleWaves - 1;
-                const bool sums = sw < kBM / 32;
-                int64_t m = m0 + ((sums ? sw * 64 + lane : lane) >> 1);
-                if (m >= p.M) m = p.M - 1;
-                par_base = (const char*)(p.sx + m) + (lane & 1) * 4;
-                par_step = p.M * 8;
-                par_dst = sums ? kParSx + sw * 256 : kKmParSpare;
-            }
-        } else if (kGrouped && w < 2) {
+        if (kGrouped && w < 2) {
             int64_t n = n0 + w * 128 + lane * 2;
             if (n > p.N - 2) n = p.N - 2;
             par_base = (const char*)p.scale + n * 2;
@@ -1486,12 +1452,6 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
 #pragma unroll
             for (int nb = 0; nb < kNB; ++nb)
                 wq[nb] = *(const v4u*)(cur + kKmXBytes + (wn * kWaveN + nb * 32 + i) * 32 + g * 16);
-            float off[kNB];  // (kKmPlain) 8 + the zero point of this lane's column
-#pragma unroll
-            for (int nb = 0; nb < kNB; ++nb)
-                off[nb] = kForm == kKmPlain && kGrouped
-                              ? 8.f + (float)*(const int8_t*)(cur + kKmXBytes + kKmWBytes + kParZero + wn * kWaveN + nb * 32 + i)
-                              : 8.f;
             // (kDepth is a multiple of kGroupStages and a split starts on a group: u tells)
             constexpr bool kStatic = kGroupStages > 0;
             const bool group_first = kStatic && (u % (kStatic ? kGroupStages : 1)) == 0;
@@ -1504,15 +1464,9 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
 #pragma unroll
                 for (int nb = 0; nb < kNB; ++nb) {
                     const u32 d = wq[nb][s];
-                    if constexpr (kForm == kKmPlain) {
-                        wb[nb] = plain_nibbles(d, off[nb]);
-                        continue;
-                    }
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
-                        wb[nb][q] = kForm == kKm24
-                                        ? ((q ? d >> (4 * q - 3) : d << 3) & kKmNibbles24) ^ kKmBase24
-                                          : (((d >> (4 * q)) & kKmNibbles) ^ kKmFlip) | kKmExp;
+                        wb[nb][q] = (((d >> (4 * q)) & kKmNibbles) ^ kKmFlip) | kKmExp;
                 }
 #pragma unroll
                 for (int nb = 0; nb < kNB; ++nb)
@@ -1532,13 +1486,13 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
             if (group_last) {
                 const char* par = cur + kKmXBytes + kKmWBytes;
                 // acc -= (136 + zero) * sum(x) as one more MFMA step: k = 0 ... 2 carry -128 on the
-                // kernel side (kKm24: -16; kKmPlain has nothing to take out), k = 3 ... 5 carry -(8 + zero) (any int8 zero point is exact in
+                // kernel side, k = 3 ... 5 carry -(8 + zero) (any int8 zero point is exact in
                 // bfloat16), both against the three bfloat16 parts of the sum of x; products of
                 // two bfloat16 are exact in float32, so the cancellation happens in the accumulator
                 v4u xs[2], wz[kNB];
 #pragma unroll
                 for (int mb = 0; mb < 2; ++mb) {
-                    v2u raw = *(const v2u*)(par + kParSx + a_row[mb] * 8);
+                    v2u raw = *(const v2u*)(par + kKmParSx + a_row[mb] * 8);
                     if (g) raw[0] = raw[1] = 0;  // lanes 32 ... 63 hold k = 8 ... 15: nothing there
                     xs[mb][0] = raw[0];                                   // hi, lo
                     xs[mb][1] = (raw[1] & 0xffffu) | (raw[0] << 16);      // lolo, hi
@@ -1548,16 +1502,15 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
 #pragma unroll
                 for (int nb = 0; nb < kNB; ++nb) {
                     int zp = 0;
-                    if (kGrouped) zp = *(const int8_t*)(par + kParZero + wn * kWaveN + nb * 32 + i);
+                    if (kGrouped) zp = *(const int8_t*)(par + kKmParZero + wn * kWaveN + nb * 32 + i);
                     const u32 cz = __float_as_uint(-(float)(8 + zp)) >> 16;
-                    constexpr u32 kBase = kForm == kKm24 ? 0xC180u : 0xC300u;  // -16, -128
-                    wz[nb][0] = kBase | (kBase << 16);
-                    wz[nb][1] = kBase | (cz << 16);                       // ..., -(8 + zero)
+                    wz[nb][0] = 0xC300C300u;                              // -128, -128
+                    wz[nb][1] = 0xC300u | (cz << 16);                      // ..., -(8 + zero)
                     wz[nb][2] = cz | (cz << 16);
                     wz[nb][3] = 0;
                 }
 #pragma unroll
-                for (int nb = 0; nb < kNB && kForm != kKmPlain; ++nb)
+                for (int nb = 0; nb < kNB; ++nb)
 #pragma unroll
                     for (int mb = 0; mb < 2; ++mb)
                         acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf(wz[nb]), as_bf(xs[mb]),
@@ -1569,11 +1522,7 @@ __global__ __launch_bounds__(kKmThreads) void gemm_w4_kmajor(KmParams p) {
                         float sc[4] = {1.f, 1.f, 1.f, 1.f};
                         if (kGrouped) {
                             const int nl = wn * kWaveN + nb * 32 + 8 * rg + 4 * g;
-                            if (kF32S) {
-                                const v4f sraw = *(const v4f*)(par + kKmParScale + nl * 4);
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) sc[e] = sraw[e];
-                            } else {
+                            {
                                 const v2u sraw = *(const v2u*)(par + kKmParScale + nl * 2);
 #pragma unroll
                                 for (int e = 0; e < 4; ++e) {
@@ -1630,11 +1579,10 @@ struct KmPlan {
     int bm;  // tile rows: 128, or 64 (with 256 columns) up to 64 rows
 };
 
-inline KmPlan kmajor_plan(int64_t M, int64_t K, int64_t N, int64_t gsize, bool f32_scales = false) {
+inline KmPlan kmajor_plan(int64_t M, int64_t K, int64_t N, int64_t gsize) {
     const int bm = M <= 64 ? 64 : kKmBM;
     const int64_t m_tiles = (M + bm - 1) / bm;
-    const int bn = (bm == kKmBM && f32_scales) || (bm == kKmBM && m_tiles * ((N + kKmBN - 1) / kKmBN) * 8 < kTargetWorkgroups) ? kKmBN / 2
-                                                                                               : kKmBN;
+    const int bn = bm == kKmBM && m_tiles * ((N + kKmBN - 1) / kKmBN) * 8 < kTargetWorkgroups ? kKmBN / 2 : kKmBN;
     const int64_t tiles = m_tiles * ((N + bn - 1) / bn);
     // about one workgroup per CU, at most eight splits (every split writes and the reduction
     // reads M x N floats: at 128 rows one split of a 4096 x 14336 kernel is a quarter of the
@@ -1720,6 +1668,16 @@ extern "C" int k3q_gemv_w4_addend(const void* x, int x_dtype, int64_t M, int64_t
     if (M > 0 && !addend) return K3Q_ERR_NULL;
     return run_gemv_w4(x, x_dtype, M, K, N, w_packed, scale, zero, block_size, addend, y, workspace,
                        workspace_bytes, nullptr, counters, counters_bytes, (hipStream_t)stream, true);
+}
+
+extern "C" int k3qt_w4_tile_plan(int64_t rows, int parts, int64_t K, int64_t N, int* plan) {
+    if (rows <= 0 || parts < 1 || parts > 3 || K <= 0 || K % 128 || N <= 0 || N % 32 || !plan) return K3Q_ERR_SHAPE;
+    const W4TilePlan pl = w4_tile_plan(rows, parts, K, N);
+    plan[0] = pl.mb;
+    plan[1] = pl.bn;
+    plan[2] = pl.ks;
+    plan[3] = pl.steps;
+    return K3Q_OK;
 }
 
 extern "C" int k3qt_gemv_w4_plan(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N,
@@ -1813,12 +1771,13 @@ extern "C" int64_t k3q_gemm_w4_kmajor_workspace_bytes(int64_t M, int64_t K, int6
     if (!kmajor_ok(M, K, N, block_size)) return 0;
     const int64_t gsize = block_size > 0 ? block_size : 128;
     const KmPlan pl = kmajor_plan(M, K, N, gsize);
-    return ((K / gsize) * M * 8 + 255) / 256 * 256 + (int64_t)pl.ks * M * N * 4;
+    const W4TilePlan tp = w4_tile_plan(M, 1, K, N);
+    const int64_t ks = gsize == 128 && tp.ks > pl.ks ? tp.ks : pl.ks;
+    return ((K / gsize) * M * 8 + 255) / 256 * 256 + ks * M * N * 4;
 }
 
-// One launch of the tile kernel over the operands of kp (any split count; the partials stay in kp.part).  form: other
-// than kKm136 for groups of 128 only; f32_scales: its grouped kernels with float32 scales.
-static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, int form, bool f32_scales, hipStream_t s) {
+// One launch of the tile kernel over the operands of kp (any split count; the partials stay in kp.part).
+static int launch_w4_kmajor(const KmParams& kp, const KmPlan& pl, bool grouped, hipStream_t s) {
     dim3 grid((unsigned)((kp.N + pl.bn - 1) / pl.bn), (unsigned)((kp.M + pl.bm - 1) / pl.bm), (unsigned)pl.ks);
     constexpr int kDepth = 4;
     const size_t lds = (size_t)kDepth * kKmSlotBytes;
@@ -1831,22 +1790,8 @@ static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, i
         {K3Q_KM_ROW(false, 2, 1), K3Q_KM_ROW(false, 2, 2), K3Q_KM_ROW(false, 1, 1)},
         {K3Q_KM_ROW(true, 2, 1), K3Q_KM_ROW(true, 2, 2), K3Q_KM_ROW(true, 1, 1)}};
 #undef K3Q_KM_ROW
-#define K3Q_KM_ROWS(G, F) \
-    {gemm_w4_kmajor<G, kDepth, 2, 2, 1, F>, gemm_w4_kmajor<G, kDepth, 2, 2, 2, F>, gemm_w4_kmajor<G, kDepth, 2, 1, 1, F>}
-    // (float32 scales: 128 x 128 and 64 x 256)
-#define K3Q_KM_FORM(F) \
-    {K3Q_KM_ROWS(false, F), K3Q_KM_ROWS(true, F), \
-     {gemm_w4_kmajor<true, kDepth, 2, 2, 1, F, true>, nullptr, gemm_w4_kmajor<true, kDepth, 2, 1, 1, F, true>}}
-    static const KmKernel row_kernels[2][3][3] = {K3Q_KM_FORM(kKm24), K3Q_KM_FORM(kKmPlain)};
-#undef K3Q_KM_FORM
-#undef K3Q_KM_ROWS
     static const bool raised = [] {
         bool ok = true;
-        for (const auto& form : row_kernels)
-            for (const auto& scales : form)
-                for (const KmKernel k : scales)
-                    ok = (!k || hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                    kLdsBudget) == hipSuccess) && ok;
         for (int a = 0; a < 2; ++a)
             for (int b = 0; b < 3; ++b)
                 for (int c = 0; c < 4; ++c)
@@ -1859,10 +1804,7 @@ static int launch_w4_tiles(const KmParams& kp, const KmPlan& pl, bool grouped, i
     const int gs = kp.gsize / kKmStage;
     const int variant = gs == 1 ? 1 : gs == 2 ? 2 : gs == 4 ? 3 : 0;
     const int shape = pl.bm == 64 ? 2 : pl.bn == kKmBN ? 1 : 0;
-    const KmKernel k = form != kKm136 ? row_kernels[form - kKm24][f32_scales ? 2 : grouped ? 1 : 0][shape]
-                                      : kernels[grouped ? 1 : 0][shape][variant];
-    if (!k) return K3Q_ERR_SHAPE;
-    k<<<grid, kKmThreads, lds, s>>>(kp);
+    kernels[grouped ? 1 : 0][shape][variant]<<<grid, kKmThreads, lds, s>>>(kp);
     return launch_status();
 }
 
@@ -1886,6 +1828,32 @@ static int run_gemm_w4_tiles(const void* x, int x_dtype, int64_t M, int64_t K, i
     if (!aligned_to(workspace, 16)) return K3Q_ERR_ALIGN;
     hipStream_t s = (hipStream_t)stream;
     int64_t gsize = grouped ? block_size : 128;
+    if (strip && gsize == 128 && w4_tile_fits(M, 1, K, N)) {
+        const W4TilePlan tp = w4_tile_plan(M, 1, K, N);
+        v2u* sums = (v2u*)workspace;
+        km_group_sums<<<dim3((unsigned)(K / 128), (unsigned)((M + 3) / 4)), 256, 0, s>>>((const uint16_t*)x, sums, M, K, 128);
+        W4TileCall c{};
+        c.x = (const uint16_t*)x;
+        c.rows = M;
+        c.K = K;
+        c.N = c.n_out = N;
+        c.parts = 1;
+        c.w = w_kmajor;
+        c.form = kW4Form136;
+        c.grouped = grouped;
+        c.scale = scale;
+        c.zero = (const int8_t*)zero;
+        c.sx = sums;
+        c.bias = bias;
+        c.y = y;
+        c.part = (float*)((char*)workspace + ((K / 128) * M * 8 + 255) / 256 * 256);
+        const int trc = w4_tile_launch(c, tp, s);
+        if (trc != K3Q_OK || w4_tile_direct(tp, 1)) return trc;
+        const dim3 fgrid((unsigned)((N + 1023) / 1024), (unsigned)M);
+        if (grouped) km_finish<true, true, 1><<<fgrid, 256, 0, s>>>(c.part, scale, bias, y, M, N, N, 0, tp.ks);
+        else km_finish<true, false, 1><<<fgrid, 256, 0, s>>>(c.part, scale, bias, y, M, N, N, 0, tp.ks);
+        return launch_status();
+    }
     const KmPlan pl = kmajor_plan(M, K, N, gsize);
     // per-channel kernels need the offset taken out only once per split
     if (!grouped && (K % pl.klen) == 0) gsize = pl.klen;
@@ -1907,7 +1875,7 @@ static int run_gemm_w4_tiles(const void* x, int x_dtype, int64_t M, int64_t K, i
     kp.klen = (int)pl.klen;
     kp.strip = strip ? 1 : 0;
     kp.units = (int)(K / 128);
-    const int lrc = launch_w4_tiles(kp, pl, grouped, kKm136, false, s);
+    const int lrc = launch_w4_kmajor(kp, pl, grouped, s);
     if (lrc != K3Q_OK) return lrc;
     // the decode kernel's second pass: sums the splits in order, applies scale and bias
     GemvParams gp{};
@@ -1943,21 +1911,20 @@ extern "C" int k3q_gemm_w4_strip(const void* x, int x_dtype, int64_t M, int64_t 
 }
 
 // ---- any K % 8, any N, float32 or bfloat16 rows ------------------------------------------------------------------
-// Three launches: the rows made ready (km_prepare_rows), the tile kernel on the strip-linear copy, the second pass.  The
-// padding costs a pass over x (3 us) where it spares the kernel a copy.  Graph nodes, us, before -> now: bfloat16
-// K=1600, N=6400 300 rows 137 -> 31 and 1200 rows 570 -> 74 (passes of 32 rows); K=2048, N=5247 64 rows 484 -> 18 (one
-// output per thread; 48 rows 16.2, 15.6 with an offset on the weights); float32 K=4096, N=14336 64 rows 127 -> 37 (passes of 8 rows), 300 rows 298 -> 156 (the kernel
-// de-quantised to parts).  A float32 row doubles the matrix work, which bounds the larger sizes; up to a few dozen rows
-// it is the launches, the start of the ring and the partials.  Error against 64 bits (2-norm), before / now:
-// float32 5.3e-6 / 4.9e-6 (de-quantised kernel 1.3e-5), bfloat16 1.66e-3 / 1.66e-3, without an offset 2.1e-7 / 8e-8 and
-// 1.4e-7 / 8e-8 for rows without negative values (1.3e-7 with one; K=8192: 1.9e-7 / 1.5e-7, 1.8e-7).
+// The rows made ready (km_prepare_rows; whole units of bfloat16 rows stay where they are, and only their sums are made), the
+// tile kernel (k3q_gemm_w4_tiles.hip) on the strip-linear copy and, where it splits K or a row has three parts, a second
+// pass.  The padding costs a pass over x (3 us) where it spares the kernel a copy.  Graph nodes, us, the kernel on the stored
+// weights -> the tile kernel with a second pass always -> now: bfloat16 K=1600, N=6400 300 rows 137 -> 29.9 -> 18.6, 900
+// rows (1200: 570) -> 48.7 -> 39.4; float32 K=N=4096 64 rows -> 26.7 -> 21.3, 300 rows -> 59.5 -> 43.8, 700 -> 102.7 -> 79.
+// A float32 row doubles the matrix work, which bounds the larger sizes.  Error against 64 bits (2-norm) of the
+// forms: float32 4.9e-6 (de-quantised kernel 1.3e-5), bfloat16 1.66e-3, without an offset 8e-8.
 namespace k3q {
 namespace {
 struct KmRowsPlan {
     int parts;      // bfloat16 rows per row of x
     bool plain;     // the weights without an offset
     int64_t Kp, Np, rows, sx_bytes, x_bytes, part_bytes;
-    KmPlan tiles;   // of a launch of `rows` rows
+    W4TilePlan tiles;   // of a launch of `rows` rows
 };
 
 // Rows go in launches of 1024 bfloat16 rows at most: the partials of one stay in the memory-side cache.
@@ -1974,11 +1941,12 @@ bool km_rows_plan(KmRowsPlan& pl, int x_dtype, int64_t M, int64_t K, int64_t N, 
     pl.Kp = (K + 127) / 128 * 128;
     pl.Np = (N + 31) / 32 * 32;  // the strips of the copy
     pl.rows = M < kKmMostRows / pl.parts ? M : kKmMostRows / pl.parts;
+    while (pl.rows > 1 && !w4_tile_fits(pl.rows, pl.parts, pl.Kp, pl.Np)) pl.rows /= 2;
     const int64_t mx = pl.rows * pl.parts;
-    pl.tiles = kmajor_plan(mx, pl.Kp, pl.Np, 128, f32 && block_size > 0);
+    pl.tiles = w4_tile_plan(pl.rows, pl.parts, pl.Kp, pl.Np);
     pl.x_bytes = mx * pl.Kp * 2;  // (a multiple of 256)
     pl.sx_bytes = (pl.Kp / 128 * mx * 8 + 255) / 256 * 256;
-    pl.part_bytes = (int64_t)pl.tiles.ks * mx * pl.Np * 4;
+    pl.part_bytes = w4_tile_direct(pl.tiles, pl.parts) ? 0 : (int64_t)pl.tiles.ks * mx * pl.Np * 4;
     return true;
 }
 }  // namespace
@@ -2008,43 +1976,52 @@ extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K
     if (!workspace || workspace_bytes < pl.x_bytes + pl.sx_bytes + pl.part_bytes) return K3Q_ERR_WORKSPACE;
     if (!aligned_to(workspace, 256)) return K3Q_ERR_ALIGN;
     hipStream_t s = (hipStream_t)stream;
-    KmParams kp{};
-    kp.x = (const uint16_t*)workspace;
-    kp.sx = (const v2u*)((char*)workspace + pl.x_bytes);
-    kp.part = (float*)((char*)workspace + pl.x_bytes + pl.sx_bytes);
-    kp.shadow = (const uint8_t*)w_strip;
-    kp.scale = scale;
-    kp.zero = (const int8_t*)zero;
-    kp.N = pl.Np;
-    kp.K = pl.Kp;
-    kp.gsize = 128;
-    kp.strip = 1;
-    kp.units = (int)(pl.Kp / 128);
+    W4TileCall c{};
+    c.x = (const uint16_t*)workspace;
+    c.sx = (const v2u*)((char*)workspace + pl.x_bytes);
+    c.part = (float*)((char*)workspace + pl.x_bytes + pl.sx_bytes);
+    c.w = w_strip;
+    c.scale = scale;
+    c.zero = (const int8_t*)zero;
+    c.N = pl.Np;
+    c.n_out = N;
+    c.K = pl.Kp;
+    c.parts = pl.parts;
+    c.form = pl.plain ? kW4FormPlain : kW4Form24;
+    c.grouped = grouped;
+    c.f32 = f32;
+    c.bias_stride = bias_stride;
+    // whole units of bfloat16 rows that start on 16 bytes are read where they lie: only their sums are made first
+    const bool as_is = !f32 && !pl.plain && K == pl.Kp && aligned_to(x, 16);
     for (int64_t m0 = 0; m0 < M; m0 += pl.rows) {
         const int64_t rows = M - m0 < pl.rows ? M - m0 : pl.rows;
         const void* xm = (const char*)x + m0 * K * el;
-        void* ym = (char*)y + m0 * N * el;
-        const void* bm = bias ? (const char*)bias + m0 * bias_stride * el : nullptr;
-        const dim3 pgrid((unsigned)kp.units, (unsigned)((rows + 3) / 4));
-        kp.M = rows * pl.parts;
-        KmPlan tiles = kmajor_plan(kp.M, pl.Kp, pl.Np, 128, f32 && grouped);
-        if ((int64_t)tiles.ks * kp.M * pl.Np * 4 > pl.part_bytes) {  // fewer rows would split further than there is room
+        const dim3 pgrid((unsigned)(pl.Kp / 128), (unsigned)((rows + 3) / 4));
+        c.rows = rows;
+        c.y = (char*)y + m0 * N * el;
+        c.bias = bias ? (const char*)bias + m0 * bias_stride * el : nullptr;
+        W4TilePlan tiles = rows == pl.rows ? pl.tiles : w4_tile_plan(rows, pl.parts, pl.Kp, pl.Np);
+        if (!w4_tile_direct(tiles, pl.parts) && (int64_t)tiles.ks * rows * pl.parts * pl.Np * 4 > pl.part_bytes) {
+            // fewer rows would split further than there is room
             tiles.ks = pl.tiles.ks;
-            tiles.klen = pl.tiles.klen;
+            tiles.steps = pl.tiles.steps;
         }
-        kp.klen = (int)tiles.klen;
-        u32* xp = (u32*)workspace;
         v2u* sx = (v2u*)((char*)workspace + pl.x_bytes);
-        (pl.parts == 3   ? km_prepare_rows<3, true>
-         : pl.parts == 2 ? km_prepare_rows<2, false>
-         : pl.plain      ? km_prepare_rows<1, true>
-                         : km_prepare_rows<1, false>)<<<pgrid, 256, 0, s>>>(xm, xp, sx, rows, K, pl.Kp);
-        const int rc = launch_w4_tiles(kp, tiles, grouped, pl.plain ? kKmPlain : kKm24, f32 && grouped, s);
+        if (as_is) {
+            c.x = (const uint16_t*)xm;
+            km_group_sums<<<pgrid, 256, 0, s>>>(c.x, sx, rows, K, 128);
+        } else
+            (pl.parts == 3   ? km_prepare_rows<3, true>
+             : pl.parts == 2 ? km_prepare_rows<2, false>
+             : pl.plain      ? km_prepare_rows<1, true>
+                             : km_prepare_rows<1, false>)<<<pgrid, 256, 0, s>>>(xm, (u32*)workspace, sx, rows, K, pl.Kp);
+        const int rc = w4_tile_launch(c, tiles, s);
         if (rc != K3Q_OK) return rc;
+        if (w4_tile_direct(tiles, pl.parts)) continue;
         const dim3 fgrid((unsigned)((N + 1023) / 1024), (unsigned)rows);
 #define K3Q_KM_FINISH(B, P)                                                                                          \
-    if (grouped) km_finish<B, true, P><<<fgrid, 256, 0, s>>>(kp.part, scale, bm, ym, rows, N, pl.Np, bias_stride, tiles.ks); \
-    else km_finish<B, false, P><<<fgrid, 256, 0, s>>>(kp.part, scale, bm, ym, rows, N, pl.Np, bias_stride, tiles.ks)
+    if (grouped) km_finish<B, true, P><<<fgrid, 256, 0, s>>>(c.part, scale, c.bias, c.y, rows, N, pl.Np, bias_stride, tiles.ks); \
+    else km_finish<B, false, P><<<fgrid, 256, 0, s>>>(c.part, scale, c.bias, c.y, rows, N, pl.Np, bias_stride, tiles.ks)
         if (pl.parts == 1) { K3Q_KM_FINISH(true, 1); }
         else if (pl.parts == 2) { K3Q_KM_FINISH(false, 2); }
         else { K3Q_KM_FINISH(false, 3); }

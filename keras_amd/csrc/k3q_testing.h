@@ -29,6 +29,10 @@ int k3qt_gemv_w4_plan(const void* x, int x_dtype, int64_t M, int64_t K, int64_t 
  * rule that both the launch and the size of the workspace follow (host only). */
 int k3qt_gemm_deep_tile(int64_t M, int64_t N, int64_t row_bytes, int cus);
 
+/* The launch plan of the int4 tile kernel for `rows` rows of `parts` bfloat16 parts (host only): plan = {blocks of 32 rows
+ * per tile, columns per tile, workgroups that share K, steps of K per split}. */
+int k3qt_w4_tile_plan(int64_t rows, int parts, int64_t K, int64_t N, int* plan);
+
 #ifdef __cplusplus
 }
 #endif

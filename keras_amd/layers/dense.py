@@ -84,12 +84,10 @@ def lora_initializer(spec):
     return LORA_INITIALIZERS[spec]
 
 
-# rows for which the int4 forward reads the K-contiguous copy of the kernel (measured against
-# the 32-row passes below it and the de-quantise + GEMM route above it, groups of 128, us:
-# K=4096, N=14336: 17 rows 22 against 27, 32 rows 23 against 31, 64 rows 26 against 60, 128 rows
-# 38 against 65, 256 rows 58 against 81, 512 rows 98 against 98; K=N=4096: 17 rows 14.5 against
-# 13.4, 32 rows 16 against 17, 64 rows 19 against 32, 128 rows 24 against 30, 512 rows 40
-# against 45; K=14336, N=4096: 17 rows 29 against 27, 512 rows 96 against 102)
+# rows for which the int4 forward reads the kernel as int4 tiles, from the strip-linear copy or (groups of 64) a
+# K-contiguous one, measured against the 32-row passes below it (17 rows 13.4 us at K=N=4096, where the tiles take 14.5)
+# and the de-quantise + GEMM route above it (512 rows: K=4096, N=14336 98 against 73; K=N=4096 45 against 30.5; K=14336,
+# N=4096 102 against 84).  What larger calls of the strip-linear copy keep on tiles: int4_tile_rows_route.
 KMAJOR_MIN_ROWS, KMAJOR_MAX_ROWS = 33, 512
 # from 17 rows on kernels at least this wide or this large (17 rows, groups of 128, us:
 # K=5120, N=13824: 26 against 36; K=13824, N=5120: 29 against 37; K=11008, N=4096: 25 against
@@ -141,29 +139,38 @@ def strip_rows_params(layer, dtype, input_dim, units, block_size):
         as_tensor(scale).to(dtype), as_tensor(zero), input_dim, units, block_size))
 
 
-# float32 rows up to which the int4 tile kernel beats the GEMM on the kernel de-quantised to bfloat16 parts (us, GEMM
-# route / tiles: K=N=4096 grouped 64 rows 50 / 27, 300 80 / 62, 600 137 / 90, 1200 188 / 166; per channel 38 / 28,
-# 59 / 46, 99 / 87, 131 / 153; K=4096, N=14336 at 300 rows 298 / 156)
-TILE_ROWS_MAX_F32 = 768
+# Rows up to which the int4 tile kernel beats the GEMM on the de-quantised kernel (us, GEMM route / tiles).  Float32: grouped
+# K=N=4096 768 rows 107 / 82, 1024 147 / 100, 2048 241 / 199; K=4096, N=11008 2048 rows 701 / 488; 1024 rows of K=N=2048 53 /
+# 45, K=4096, N=1024 60.2 / 59.9; K=N=2048 4000 rows 132 / 180: small kernels up to 1024.  Per channel (two parts a weight fewer
+# for the GEMM) 700 rows 97 / 79, 1024 104 / 101, K=2048, N=8192 96 / 98.  Bfloat16: while the tiles are one turn of the chip,
+# and enough for it: 1024 rows K=N=4096 58 / 48, K=14336, N=4096 168 / 148, K=N=2048 37 / 20, 640 rows K=N=4096 52 / 42, 700
+# rows K=4096, N=1024 28 / 25; K=4096, N=14336 138 / 143.
+TILE_ROWS_MAX_F32, TILE_ROWS_MAX_F32_LARGE, TILE_ROWS_MAX_F32_CHANNEL, TILE_LARGE_WEIGHTS = 1024, 2048, 768, 16 << 20
+TILE_ROWS_MAX_BF16, TILE_COUNTS_BF16 = 1024, (32, 256)
 
 
 def int4_tile_rows_route(dtype, rows, input_dim, units, block_size):
     """Whether an int4 call of more rows than the decode kernels take goes to `ops.int4_matmul_tiles_rows`: shapes
-    that neither the tile kernel proper (`ops.int4_kmajor_supported`) nor the GEMM on the de-quantised kernel takes
-    (K % 128, N % 64), which went in passes of 32 bfloat16 or 8 float32 rows over the kernel, and float32 rows up to
-    `TILE_ROWS_MAX_F32` (us, passes / tiles: K=1600, N=6400 bfloat16 48 rows 25.6 / 17.0, 300 137 / 31, 1200 570 / 74;
-    float32 17 rows 25 / 17, 300 307 / 38; one pass, up to 32 bfloat16 rows of a kernel this small, is as good: 15.7 /
-    15.7).  Where N % 8 or K % 16 leave only the kernel of one output per thread (K=2048, N=5247: 480 us at 32
-    rows, 6.1 ms at 1200, against 15 and 82) every shape goes here."""
+    that neither the tile kernel's aligned entry (`ops.int4_kmajor_supported`) nor the GEMM on the de-quantised kernel takes
+    (K % 128, N % 64), which went in passes of 32 bfloat16 or 8 float32 rows over the kernel (us, passes / tiles: K=1600,
+    N=6400 bfloat16 48 rows 25.6 / 15, 300 137 / 19; float32 17 rows 25 / 15, 300 307 / 30; one pass, up to 32 bfloat16 rows of a
+    kernel this small, is as good), and rows of aligned shapes up to the limits above.  Where N % 8 or K % 16 leave only the
+    kernel of one output per thread (K=2048, N=5247: 480 us at 32 rows, 6.1 ms at 1200, against 15 and 82) every shape
+    goes here."""
     if not (dtype in (torch.float32, torch.bfloat16) and rows > kops.STRIP_MAX_ROWS
             and kops.int4_tiles_rows_supported(input_dim, units, block_size)):
         return False
     if units % 8 or input_dim % 16:
         return True
     gemm = input_dim % 128 == 0 and units % 64 == 0
+    if not gemm:
+        return dtype == torch.float32 or rows >= KMAJOR_MIN_ROWS or kmajor_rows(rows, units, input_dim)
     if dtype == torch.float32:
-        return not gemm or rows <= TILE_ROWS_MAX_F32
-    return not gemm and (rows >= KMAJOR_MIN_ROWS or kmajor_rows(rows, units, input_dim))
+        if not block_size:
+            return rows <= TILE_ROWS_MAX_F32_CHANNEL
+        return rows <= (TILE_ROWS_MAX_F32_LARGE if input_dim * units >= TILE_LARGE_WEIGHTS else TILE_ROWS_MAX_F32)
+    low, high = TILE_COUNTS_BF16
+    return KMAJOR_MAX_ROWS < rows <= TILE_ROWS_MAX_BF16 and low <= -(-rows // 128) * -(-units // 128) <= high
 
 
 def tile_rows_operands(layer, dtype, units, grouped):
