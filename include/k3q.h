@@ -552,6 +552,18 @@ int k3q_gemm_i8_w8s(const int8_t* a, const void* a_scale, int scale_dtype, int64
                     const void* shadow, const void* kernel_scale, const void* bias, int64_t bias_stride,
                     void* y, void* stream);
 /*
+ * The whole int8 Dense forward of a layer that keeps the strip-linear copy (K % 64 == 0), any number of rows x [M, K] of
+ * x_dtype, dense: abs-max quantisation of the rows (k3q_absmax_quantize), the int32 product, the bit-exact de-scale, bias [N],
+ * or up to 16 rows [M, N] (bias_stride N).  The bits of the calls one by one (k3q_gemm_i8_w8s up to 16 rows it takes,
+ * k3q_gemm_i8 with b_layout 2 and the exact epilogue beyond; the alignments are theirs), in one launch where float32 rows
+ * are few enough to be quantised by the product's own workgroups, otherwise in two or three with the quantised rows in the
+ * workspace (aligned to 256 bytes).
+ */
+int64_t k3q_dense_i8_workspace_bytes(int x_dtype, int64_t M, int64_t K, int64_t N);
+int k3q_dense_i8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                 const void* kernel_scale, const void* bias, int64_t bias_stride, float epsilon, float range_lo,
+                 float range_hi, void* y, void* workspace, int64_t workspace_bytes, void* stream);
+/*
  * Several int8 layers against ONE x in one launch (the query / key / value projections of an
  * attention block, gate / up of an MLP): each result is what k3q_dense_i8_w8s (a == NULL: the rows
  * are quantised in the kernel) or k3q_gemm_i8_w8s (a, a_scale: rows already quantised) gives for

@@ -130,6 +130,12 @@ SIGNATURES = {
         [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _f32, _f32, _f32, _ptr, _ptr],
     ),
     "k3q_gemm_i8_w8s_supported": (_int, [_i64, _i64, _i64]),
+    "k3q_dense_i8_workspace_bytes": (_i64, [_int, _i64, _i64, _i64]),
+    "k3q_dense_i8": (
+        _int,
+        [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, ctypes.c_float, ctypes.c_float, ctypes.c_float, _ptr, _ptr,
+         _i64, _ptr],
+    ),
     "k3q_gemm_i8_w8s": (_int, [_ptr, _ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _ptr]),
     "k3q_dense_i8_w8s_multi": (
         _int, [_ptr, _int, _ptr, _ptr, _i64, _i64, _int, _ptr, _f32, _f32, _f32, _ptr]),

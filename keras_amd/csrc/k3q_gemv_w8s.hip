@@ -28,7 +28,7 @@ constexpr int kMaxRows8 = 16;
 constexpr int kResident8 = 256;  // workgroups the chip holds at once (one per CU)
 
 struct W8sParams {
-    const uint16_t* x;      // [M, K] bfloat16 (quantised in the kernel), or
+    const void* x;          // [M, K] bfloat16, or float32 (kernels built with kF32), quantised in the kernel, or
     const int8_t* xq;       // [M, K] int8 with
     const void* xs;         // T [M] scales (already quantised rows)
     const v4i* w;           // strip-linear copy
@@ -39,8 +39,8 @@ struct W8sParams {
     int M, K, N;
     int units;              // K / 64
     int groups;             // strip groups (kSW strips each)
-    int row_magic;          // ceil(2^32 / (K / 8)): piece -> row
-    float eps, qlo, qhi;    // quantizer settings (eps already rounded to bfloat16)
+    int row_magic;          // ceil(2^32 / (K / 8)), float32 rows K / 4: piece -> row
+    float eps, qlo, qhi;    // quantizer settings (bfloat16 rows: eps already rounded to bfloat16)
     // an operation on x before it is quantised (kernels built with kPre only):
     int pre_kind;            // 1: rms_norm(x) * pre_op (bf16 [K]); 2: silu(pre_op) * x (pre_op bf16 [M, K])
     float pre_eps;           // rms_norm's epsilon
@@ -69,7 +69,7 @@ __device__ __forceinline__ float descale_exact_f32(int acc, float sa, float sb, 
 // quantisation (0: it reads them twice); -1: the rows arrive quantised (p.xq, p.xs).
 // kPre (kNP > 0 only): the rows are transformed before they are quantised (p.pre_kind): rms_norm with
 // a gain, the bits of k3q_rmsnorm, or multiplied by silu of a second input, the bits of k3q_silu_mul.
-// kF32 (kNP < 0 only): scales, bias and result are float32.
+// kF32: scales, bias and result are float32, and the rows, where the kernel quantises them (kNP > 0).
 // kTail (kNP < 0 only): the units are no whole number of blocks of kD, or fewer blocks than waves (K = 1600
 // is 25 units): the rows of x in LDS are zero past K, and a unit past the last one reads the last one.
 template <int kSW, int kD, int kNP, bool kPre = false, bool kF32 = false, bool kTail = false>
@@ -78,7 +78,9 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
     const int tid = threadIdx.x, lane = tid & 63;
     const int q = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = p.M, K = p.K;
-    static_assert(kNP < 0 || !(kF32 || kTail), "float32 results and ragged K: rows that arrive quantised");
+    static_assert(kNP < 0 || !kTail, "ragged K: rows that arrive quantised");
+    static_assert(!kF32 || (kNP != 0 && !kPre), "float32 rows stay in registers between their maximum and their quantisation");
+    constexpr int kPieceShift = kF32 ? 2 : 3;  // values per 16-byte piece of x, as a power of two
     const int blocks = kTail ? (p.units + kD - 1) / kD : p.units / kD;
     const int pitch = (kTail ? blocks * kD * 64 : K) + 16;
     // LDS: x rows as int8 | row maxima (uint bits) | row scales | reduction buffers
@@ -187,7 +189,7 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
         if (tid < M) sa[tid] = raw_to_f32<!kF32>(load_raw<!kF32>(p.xs, tid));
     } else {
         // row maxima, scales, int8 rows: abs_max_quantize of the rows inside the workgroup
-        const int pieces = M * (K >> 3);  // 16-byte pieces of x (8 values)
+        const int pieces = M * (K >> kPieceShift);  // 16-byte pieces of x
         if (tid < kMaxRows8) rowmax[tid] = 0u;
         static_assert(!kPre || kNP > 0, "the transform works on the pieces kept in registers");
         v4u xr[kNP > 0 ? kNP : 1];
@@ -248,12 +250,16 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
             float a = 0.f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                if constexpr (kF32) {
+                    a = fmaxf(a, fabsf(__uint_as_float(c[e])));
+                    continue;
+                }
                 a = fmaxf(a, fabsf(__uint_as_float(c[e] << 16)));
                 a = fmaxf(a, fabsf(__uint_as_float(c[e] & 0xffff0000u)));
             }
             return a;
         };
-        // a wave's 64 consecutive pieces lie in one row (K % 512 == 0): one LDS atomic per wave and turn
+        // a wave's 64 consecutive pieces lie in one row (K % 512 == 0; float32 K % 256): one LDS atomic per wave and turn
         auto fold_amax = [&](int pi, float a) {
             a = wave_max(a);
             const int row = (int)__umulhi((u32)(pi < pieces ? pi : pieces - 1), (u32)p.row_magic);
@@ -273,14 +279,29 @@ __device__ __forceinline__ void gemv_w8s_body(const W8sParams& p, const int bloc
             }
         }
         __syncthreads();
-        if (tid < M) sa[tid] = scale_from_amax_bf16(__uint_as_float(rowmax[tid]), p.eps, p.qhi);
+        if (tid < M) {
+            const float amax = __uint_as_float(rowmax[tid]);
+            sa[tid] = kF32 ? p.qhi / (amax + p.eps) : scale_from_amax_bf16(amax, p.eps, p.qhi);
+        }
         __syncthreads();
         // (quantize_piece_bf16: the clip before the rounding, exact between the integer ends of the range
         // that the entry point insists on)
         auto quantize_piece = [&](int pi, const v4u& c) {
             const int row = (int)__umulhi((u32)pi, (u32)p.row_magic);
-            const int col = (pi - row * (K >> 3)) << 3;
-            *(v2u*)(xs + row * pitch + col) = quantize_piece_bf16(c, sa[row], p.qlo, p.qhi);
+            const int col = (pi - row * (K >> kPieceShift)) << kPieceShift;
+            if constexpr (kF32) {
+                // product, clip, and the rounding as the addition of 1.5 2^23, whose low byte is the result's: the clip
+                // before the rounding, as above
+                u32 t[4];
+                const float s = sa[row];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    t[e] = __float_as_uint(fminf(fmaxf(__uint_as_float(c[e]) * s, p.qlo), p.qhi) + 12582912.0f);
+                const u32 lo = byte_perm(t[1], t[0], 0x0c0c0400u), hi = byte_perm(t[3], t[2], 0x0c0c0400u);
+                *(u32*)(xs + row * pitch + col) = lo | (hi << 16);
+            } else {
+                *(v2u*)(xs + row * pitch + col) = quantize_piece_bf16(c, sa[row], p.qlo, p.qhi);
+            }
         };
         if (kNP > 0) {
 #pragma unroll
@@ -394,6 +415,12 @@ __global__ __launch_bounds__(kT) void gemv_w8s(W8sParams p) {
 template <int kSW, int kD, bool kF32, bool kTail>
 __global__ __launch_bounds__(kT) void gemv_w8s_rows(W8sParams p) {
     gemv_w8s_body<kSW, kD, -1, false, kF32, kTail>(p, (int)blockIdx.x, (int)gridDim.x);
+}
+
+// float32 rows that are quantised here.
+template <int kSW, int kD, int kNP>
+__global__ __launch_bounds__(kT) void gemv_w8s_f32(W8sParams p) {
+    gemv_w8s_body<kSW, kD, kNP, false, true>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Up to kMaxProblems8 kernels against one x in one launch (the query / key / value projections of
@@ -558,6 +585,18 @@ W8sKernel pick_kernel8_rows(const W8sPlan& pl) {
     return pl.d == 4 ? gemv_w8s_rows<1, 4, kF32, kTail> : gemv_w8s_rows<1, 2, kF32, kTail>;
 }
 
+template <int kSW, int kD>
+W8sKernel pick_np8_f32(int64_t pieces) {
+    return pieces <= kT       ? gemv_w8s_f32<kSW, kD, 1>
+           : pieces <= 4 * kT ? gemv_w8s_f32<kSW, kD, 4>
+                              : gemv_w8s_f32<kSW, kD, 8>;
+}
+
+W8sKernel pick_kernel8_f32(const W8sPlan& pl, int64_t pieces) {
+    if (pl.sw == 2) return pl.d == 4 ? pick_np8_f32<2, 4>(pieces) : pick_np8_f32<2, 2>(pieces);
+    return pl.d == 4 ? pick_np8_f32<1, 4>(pieces) : pick_np8_f32<1, 2>(pieces);
+}
+
 W8sKernel pick_kernel8(const W8sPlan& pl) {
     if (pl.sw == 2) return pl.d == 4 ? pick_np8<2, 4>(pl.np) : pick_np8<2, 2>(pl.np);
     return pl.d == 4 ? pick_np8<1, 4>(pl.np) : pick_np8<1, 2>(pl.np);
@@ -602,7 +641,7 @@ int fill_params8(W8sParams& p, const W8sPlan& pl, const void* x, const int8_t* x
     if (!aligned_to(quantised ? (const void*)xq : x, 16) || !aligned_to(shadow, 16) || !aligned_to(y, el) ||
         !aligned_to(kernel_scale, el) || (bias && !aligned_to(bias, el)) || (xs && !aligned_to(xs, el)))
         return K3Q_ERR_ALIGN;
-    p.x = (const uint16_t*)x;
+    p.x = x;
     p.xq = xq;
     p.xs = xs;
     p.w = (const v4i*)shadow;
@@ -615,9 +654,9 @@ int fill_params8(W8sParams& p, const W8sPlan& pl, const void* x, const int8_t* x
     p.N = (int)N;
     p.units = (int)(K / 64);
     p.groups = (int)pl.groups;
-    const uint64_t per_row = (uint64_t)K / (quantised ? 16 : 8);
+    const uint64_t per_row = (uint64_t)K / (quantised ? 16 : f32 ? 4 : 8);
     p.row_magic = (int)(uint32_t)((((uint64_t)1 << 32) + per_row - 1) / per_row);
-    p.eps = host_round_bf16(epsilon);  // torch rounds the epsilon operand to the tensor dtype before the add
+    p.eps = f32 ? epsilon : host_round_bf16(epsilon);  // torch rounds the epsilon operand to the tensor dtype before the add
     p.qlo = range_lo;
     p.qhi = range_hi;
     return K3Q_OK;
@@ -687,6 +726,70 @@ extern "C" int k3q_gemm_i8_w8s(const int8_t* a, const void* a_scale, int scale_d
     if ((rc = raise_lds((const void*)kernel)) != K3Q_OK) return rc;
     kernel<<<(unsigned)pl.blocks, kT, pl.lds, (hipStream_t)stream>>>(p);
     return launch_status();
+}
+
+namespace {
+// Float32 values of x up to which the kernel's workgroups quantise the rows themselves: every one of them reads and converts all
+// of x, which costs what the quantizer's launch does at about 16 K values (graph nodes, us, two launches / one, with more
+// values beside: K=N=4096 1 row 8.5 / 6.0, 4 9.2 / 8.9, 6 9.2 / 9.6, 16 10.1 / 15.4; K=N=8192 1 row 15.9 / 12.9, 2 15.6 / 14.9,
+// 4 16.5 / 16.7; K=2048, N=5632 6 rows 10.4 / 10.1, 12 10.6 / 11.3; K=1024, N=14336 16 rows 9.4 / 9.2, N=3072 7.2 / 7.6).
+constexpr int64_t kFusedF32Values = 8 * 4 * kT;
+
+int64_t dense_i8_scratch(int64_t M, int64_t K, int64_t el, int64_t* scales_at) {
+    *scales_at = (M * K + 255) / 256 * 256;
+    return *scales_at + (M * el + 255) / 256 * 256;
+}
+}  // namespace
+
+extern "C" int64_t k3q_dense_i8_workspace_bytes(int x_dtype, int64_t M, int64_t K, int64_t N) {
+    if ((x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) || M <= 0 || K <= 0 || N <= 0 || (K % 64) != 0) return 0;
+    int64_t at;
+    return dense_i8_scratch(M, K, x_dtype == K3Q_F32 ? 4 : 2, &at) + (M > kMaxRows8 ? k3q_gemm_i8_split_bytes(M, N, K) : 0);
+}
+
+extern "C" int k3q_dense_i8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t N, const void* shadow,
+                            const void* kernel_scale, const void* bias, int64_t bias_stride, float epsilon,
+                            float range_lo, float range_hi, void* y, void* workspace, int64_t workspace_bytes,
+                            void* stream) {
+    if (x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
+    if (M < 0 || K <= 0 || N <= 0 || (K % 64) != 0) return K3Q_ERR_SHAPE;
+    if (bias_stride != 0 && (bias_stride != N || M > kMaxRows8)) return K3Q_ERR_SHAPE;
+    if (!(range_lo >= -128.f && range_hi <= 127.f && range_lo <= range_hi)) return K3Q_ERR_RANGE;
+    if (M == 0) return K3Q_OK;
+    if (!x || !shadow || !kernel_scale || !y) return K3Q_ERR_NULL;
+    const bool f32 = x_dtype == K3Q_F32;
+    const int64_t el = f32 ? 4 : 2;
+    bool tail = false;
+    // (the quantizer inside the kernel clips before it rounds: exact only between integer ends)
+    if (f32 && M <= kMaxRows8 && M * K <= kFusedF32Values && range_lo < range_hi && range_lo == rintf(range_lo) &&
+        range_hi == rintf(range_hi) && aligned_to(x, 16)) {
+        const W8sPlan pl = w8s_plan(M, K, N);
+        if (pl.ok) {
+            W8sParams p;
+            int rc = fill_params8(p, pl, x, nullptr, nullptr, M, K, N, shadow, kernel_scale, bias, bias_stride, epsilon,
+                                  range_lo, range_hi, y, true);
+            if (rc != K3Q_OK) return rc;
+            const W8sKernel kernel = pick_kernel8_f32(pl, M * K / 4);
+            if ((rc = raise_lds((const void*)kernel)) != K3Q_OK) return rc;
+            kernel<<<(unsigned)pl.blocks, kT, pl.lds, (hipStream_t)stream>>>(p);
+            return launch_status();
+        }
+    }
+    int64_t scales_at;
+    const int64_t head = dense_i8_scratch(M, K, el, &scales_at);
+    if (!workspace || workspace_bytes < head) return K3Q_ERR_WORKSPACE;
+    if (!aligned_to(workspace, 256)) return K3Q_ERR_ALIGN;
+    int8_t* q = (int8_t*)workspace;
+    void* scales = (char*)workspace + scales_at;
+    const bool rows = M <= kMaxRows8 && w8s_rows_plan(M, K, N, &tail).ok;
+    if (!rows && bias_stride != 0) return K3Q_ERR_SHAPE;
+    int rc = k3q_absmax_quantize(x, x_dtype, M, K, K, epsilon, range_lo, range_hi, q, scales, stream);
+    if (rc != K3Q_OK) return rc;
+    if (rows)
+        return k3q_gemm_i8_w8s(q, scales, x_dtype, M, K, N, shadow, kernel_scale, bias, bias_stride, y, stream);
+    const int64_t rest = workspace_bytes - head;
+    return k3q_gemm_i8(q, (const int8_t*)shadow, 2, M, N, K, scales, kernel_scale, bias, x_dtype, 1 /* exact */, y, nullptr,
+                       rest > 0 ? (char*)workspace + head : nullptr, rest > 0 ? rest : 0, stream);
 }
 
 namespace {

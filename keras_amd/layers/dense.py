@@ -17,7 +17,7 @@ import torch
 from keras_amd import dtype_policies, ops as kops, quantizers
 from keras_amd.layers.layer import (Layer, as_tensor, cached_operand, cached_params, require_default_g_idx,
                                     to_torch_dtype)
-from keras_amd.layers.together import quantize_rows
+from keras_amd.layers.together import quantize_rows, quantizes_alone
 from keras_amd.quantization_config import QuantizationConfig, get_block_size_for_layer
 
 _ACTIVATIONS = {
@@ -201,6 +201,14 @@ def int8_strip_route(quantizer, x2, units, strict=False):
         return True
     return (not strict and x2.dtype in (torch.float32, torch.bfloat16)
             and kops.int8_strip_rows_supported(x2.shape[0], x2.shape[1], units))
+
+
+def int8_rows_route(x2, dtype, units, bias):
+    """Whether an int8 call of more rows than the decode kernels take goes to `ops.int8_dense_rows`: everything the tile
+    GEMM reads from the strip-linear copy, with a bias for all rows.  (The same launches as quantizer and product called one by
+    one; eager, us, one by one / in one call: 64 rows of 4096 x 4096 float32 32.0 / 20.2, 100 of 1600 x 6400 bfloat16 27.5 / 18.7.)"""
+    return (x2.is_cuda and x2.dtype == dtype and dtype in (torch.float32, torch.bfloat16) and x2.shape[1] % 64 == 0
+            and x2.shape[0] > kops.INT8_STRIP_MAX_ROWS and (bias is None or bias.numel() == units))
 
 
 class Dense(Layer):
@@ -484,25 +492,34 @@ class Dense(Layer):
         exact = self.exact_epilogue
         if exact is None:
             exact = True
+        alone = exact and quantizes_alone(self.inputs_quantizer)
         if exact and int8_strip_route(self.inputs_quantizer, x2, N):
             # decode sizes: quantizer, matmul and de-scale in one launch, from the strip-linear copy
             y = kops.int8_dense_strip(
                 x2, self._cached("w8s", self._kernel, kops.int8_strip_copy), N,
                 self._read_cached("kernel_scale", self.kernel_scale), bias=self._call_bias(),
                 epsilon=self.inputs_quantizer.epsilon, value_range=self.inputs_quantizer.value_range,
-                quantize=lambda rows: quantize_rows(self.inputs_quantizer, rows))
+                quantize=None if alone else lambda rows: quantize_rows(self.inputs_quantizer, rows))
             y = y if len(lead) == 1 else y.reshape(*lead, N)
             if self.activation is not None:
                 y = self.activation(y)
             return y
-        q, scale = quantize_rows(self.inputs_quantizer, x2)
-        y = kops.int8_matmul(
-            q, as_tensor(self._kernel), a_scale=scale,
-            kernel_scale=self._read_cached("kernel_scale", self.kernel_scale),
-            bias=self._call_bias(),
-            out_dtype=to_torch_dtype(self.compute_dtype),
-            exact_epilogue=exact, **self._tile_operand(x2.shape[1]),
-        )
+        bias = self._call_bias()
+        if alone and int8_rows_route(x2, to_torch_dtype(self.compute_dtype), N, bias):
+            # more rows: quantizer and tile GEMM in one call
+            y = kops.int8_dense_rows(
+                x2, self._cached("w8s", self._kernel, kops.int8_strip_copy), N,
+                self._read_cached("kernel_scale", self.kernel_scale), bias=bias, epsilon=self.inputs_quantizer.epsilon,
+                value_range=self.inputs_quantizer.value_range)
+        else:
+            q, scale = quantize_rows(self.inputs_quantizer, x2)
+            y = kops.int8_matmul(
+                q, as_tensor(self._kernel), a_scale=scale,
+                kernel_scale=self._read_cached("kernel_scale", self.kernel_scale),
+                bias=bias,
+                out_dtype=to_torch_dtype(self.compute_dtype),
+                exact_epilogue=exact, **self._tile_operand(x2.shape[1]),
+            )
         y = y if len(lead) == 1 else y.reshape(*lead, N)
         if self.activation is not None:
             y = self.activation(y)

@@ -18,12 +18,12 @@ import string
 import torch
 
 from keras_amd import dtype_policies, ops as kops, quantizers
-from keras_amd.layers.dense import (_ACTIVATIONS, activation_name, glorot_uniform, int8_strip_route,
+from keras_amd.layers.dense import (_ACTIVATIONS, activation_name, glorot_uniform, int8_rows_route, int8_strip_route,
                                     lora_initializer,
                                     serialize_quantization_config)
 from keras_amd.layers.layer import (Layer, as_tensor, cached_operand, cached_params, require_default_g_idx,
                                     to_torch_dtype)
-from keras_amd.layers.together import quantize_rows
+from keras_amd.layers.together import quantize_rows, quantizes_alone
 from keras_amd.quantization_config import QuantizationConfig, get_block_size_for_layer
 
 
@@ -643,6 +643,7 @@ class EinsumDense(Layer):
         exact = self.exact_epilogue
         if exact is None:
             exact = True
+        alone = exact and quantizes_alone(self.inputs_quantizer)
         if exact and int8_strip_route(self.inputs_quantizer, x2, n):
             # decode sizes, as Dense: one launch from the strip-linear copy of the [K, N] matrix
             y2 = kops.int8_dense_strip(
@@ -650,7 +651,13 @@ class EinsumDense(Layer):
                 self._cached("kernel_scale", self.kernel_scale, lambda t: t.to(cd).reshape(-1).contiguous()),
                 bias=bias, epsilon=self.inputs_quantizer.epsilon,
                 value_range=self.inputs_quantizer.value_range,
-                quantize=lambda rows: quantize_rows(self.inputs_quantizer, rows))
+                quantize=None if alone else lambda rows: quantize_rows(self.inputs_quantizer, rows))
+            return self._finish(y2, free_shape, gv, fused)
+        if alone and int8_rows_route(x2, cd, n, bias):
+            y2 = kops.int8_dense_rows(
+                x2, self._cached("w8s", self._kernel, lambda t: kops.int8_strip_copy(kernel_matrix(t))), n,
+                self._cached("kernel_scale", self.kernel_scale, lambda t: t.to(cd).reshape(-1).contiguous()),
+                bias=bias, epsilon=self.inputs_quantizer.epsilon, value_range=self.inputs_quantizer.value_range)
             return self._finish(y2, free_shape, gv, fused)
         q, scale = quantize_rows(self.inputs_quantizer, x2)
         y2 = kops.int8_matmul(

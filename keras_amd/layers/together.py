@@ -13,10 +13,11 @@ import threading
 import numpy as np
 import torch
 
-from keras_amd import ops as kops
+from keras_amd import ops as kops, quantizers
 from keras_amd.layers.layer import to_torch_dtype
 
 _state = threading.local()
+_abs_max_quantize = quantizers.abs_max_quantize
 
 # rows up to which a weight-only int4 layer runs the decode kernel proper (above, other routes)
 ADDEND_MAX_ROWS = 16
@@ -50,6 +51,13 @@ def quantize_rows(quantizer, x2):
     return hit[0]
 
 
+def quantizes_alone(quantizer):
+    """Whether a layer's quantizer is the plain abs-max one, nobody shares its rows and nobody has put a function of their own
+    in the place of `quantizers.abs_max_quantize`: its forward may then quantise the rows in the call that multiplies them."""
+    return (type(quantizer) is quantizers.AbsMaxQuantizer and quantizer.output_dtype == "int8"
+            and getattr(_state, "memo", None) is None and quantizers.abs_max_quantize is _abs_max_quantize)
+
+
 def _quantizer_key(quantizer, x2):
     return (type(quantizer), repr(sorted(quantizer.get_config().items())), x2.data_ptr(), tuple(x2.shape),
             tuple(x2.stride()), x2.dtype, x2._version)
@@ -60,8 +68,6 @@ def apply_input_op_for(layers, input_op, x):
     their input with the same plain abs-max quantizer, the operation and that quantizer run as ONE
     launch and the quantised rows are left in the enclosing `shared_input_rows()` for the layers to
     pick up (same bits as the two launches); otherwise the operation's own launch."""
-    from keras_amd import quantizers
-
     memo = getattr(_state, "memo", None)
     if memo is not None and isinstance(x, torch.Tensor) and x.dim() >= 2:
         qs = [getattr(l, "inputs_quantizer", None) for l in layers]

@@ -1072,10 +1072,9 @@ def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, va
                      quantize=None):
     """The int8 Dense forward for up to 16 rows: abs-max quantisation of the rows, exact int8 matmul
     against `int8_strip_copy(kernel)`, bit-exact de-scale in the rows' dtype, bias (N values)
-    or addend (a row per row of x).  One launch for small bfloat16 x; for larger x, float32 x and
-    widths outside `int8_strip_supported` the rows are quantised by `quantize(x2)` (default:
-    `quantizers.abs_max_quantize` with these settings) first.  Same bits as `abs_max_quantize` +
-    `int8_matmul(..., exact_epilogue=True)`.
+    or addend (a row per row of x).  One launch for small x; for larger x and widths outside
+    `int8_strip_supported` the rows are quantised first, in the same call, or by `quantize(x2)` where one is given.
+    Same bits as `abs_max_quantize` + `int8_matmul(..., exact_epilogue=True)`.
     Reference: keras/src/layers/core/dense.py:956-972."""
     _lib.require_device(x, shadow, kernel_scale, bias)
     lib = _lib.load()
@@ -1100,13 +1099,16 @@ def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, va
     stride = N if (bias is not None and M > 1 and bias.numel() == M * N) else 0
     ks = kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous()
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    if not inside and quantize is None:
+        ws = _workspace(x.device, lib.k3q_dense_i8_workspace_bytes(code, M, K, N)) if M else None
+        rc = lib.k3q_dense_i8(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
+                              _lib.ptr(bias) if bias is not None else None, stride, float(epsilon), float(value_range[0]),
+                              float(value_range[1]), _lib.ptr(y), _lib.ptr(ws), ws.numel() if ws is not None else 0,
+                              _lib.stream_ptr(x.device))
+        _lib.check(rc, "k3q_dense_i8")
+        return _shaped(y, lead)
     if not inside:
-        if quantize is None:
-            from keras_amd import quantizers
-
-            q, s = quantizers.abs_max_quantize(x2, axis=-1, value_range=value_range, epsilon=epsilon)
-        else:
-            q, s = quantize(x2)
+        q, s = quantize(x2)
         if s.dtype != x.dtype:
             raise TypeError("the rows' scales must have the input's dtype")
         rc = lib.k3q_gemm_i8_w8s(_lib.ptr(q), _lib.ptr(s), code, M, K, N, _lib.ptr(shadow),
@@ -1119,6 +1121,35 @@ def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, va
                               float(value_range[0]), float(value_range[1]), _lib.ptr(y),
                               _lib.stream_ptr(x.device))
     _lib.check(rc, "k3q_dense_i8_w8s")
+    return _shaped(y, lead)
+
+
+def int8_dense_rows(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, value_range=(-127, 127)):
+    """`int8_dense_strip` for more rows: quantizer and tile GEMM in one call, x[..., K] float32 or bfloat16 with
+    K % 64 == 0, bias of N values.  The bits of `abs_max_quantize` + `int8_matmul(..., strip=shadow, exact_epilogue=True)`.
+    Reference: keras/src/layers/core/dense.py:956-972."""
+    _lib.require_device(x, shadow, kernel_scale, bias)
+    lib = _lib.load()
+    code = _lib.dtype_code(x.dtype)
+    K, N = int(x.shape[-1]), int(units)
+    lead = x.shape[:-1]
+    x2 = _rows_of(x, K)
+    M = x2.shape[0]
+    if shadow.dtype != torch.uint8 or K % 64 or shadow.numel() != lib.k3q_w8s_shadow_bytes(K, N):
+        raise ValueError("shadow is not int8_strip_copy(kernel) of this [K, N]")
+    if kernel_scale.numel() != N or (bias is not None and bias.numel() != N):
+        raise ValueError(f"kernel_scale and bias hold {N} values each")
+    if kernel_scale.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
+        raise TypeError("kernel_scale and bias must be read in the input's dtype")
+    # (the tile kernel reads scales and bias in 16-byte pieces)
+    ks, b = (t if t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) else t.clone(memory_format=torch.contiguous_format)
+             for t in (kernel_scale, bias))
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    ws = _workspace(x.device, lib.k3q_dense_i8_workspace_bytes(code, M, K, N)) if M else None
+    rc = lib.k3q_dense_i8(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks), _lib.ptr(b), 0, float(epsilon),
+                          float(value_range[0]), float(value_range[1]), _lib.ptr(y), _lib.ptr(ws),
+                          ws.numel() if ws is not None else 0, _lib.stream_ptr(x.device))
+    _lib.check(rc, "k3q_dense_i8")
     return _shaped(y, lead)
 
 
