@@ -625,6 +625,17 @@ int k3q_rope_cache(const void* q, const void* k, const void* v, int dtype, int64
                    const int64_t* pos, void* k_cache, void* v_cache, void* q_out, int* oob_flag, void* stream);
 
 /*
+ * Attention of T positions q [B, T, H, 128] (rotated, bfloat16) over the caches [B, H, max_len, 128]:
+ * out [B, T, H, 128] = softmax(q k^T / sqrt(128) + mask) v with an additive bfloat16 mask [T, max_len], as
+ * scaled_dot_product_attention computes it; max_len % 4 == 0.  Scores, probabilities and sums are float32 (a probability
+ * enters its product as two bfloat16 parts).  Blocks of 64 cache rows that the mask closes (-inf) for 64 positions are not read.
+ * The decoder harness's prompt; no counterpart in the reference's quantized layers.
+ */
+int k3q_prompt_attention(const void* q, int dtype, int64_t B, int64_t T, int64_t H, int64_t head_dim,
+                         int64_t max_len, const void* k_cache, const void* v_cache, const void* mask, void* out,
+                         void* stream);
+
+/*
  * Two more pieces of the decoder harness's glue (no counterpart in the quantized layers; they
  * stand for `rms_norm` and `silu(gate) * up` between the Dense calls of a decoder block), bfloat16:
  * k3q_rmsnorm: y[r, :] = bf16(x[r, :] * rsqrt(mean(x[r, :]^2) + epsilon) * weight[:]), float32

@@ -145,6 +145,7 @@ SIGNATURES = {
         _int, [_ptr, _int, _i64, _i64, _ptr, _f32, _f32, _f32, _ptr, _ptr, _ptr, _ptr]),
     "k3q_rmsnorm": (_int, [_ptr, _ptr, _int, _i64, _i64, _i64, _f32, _ptr, _i64, _ptr]),
     "k3q_silu_mul": (_int, [_ptr, _ptr, _int, _i64, _i64, _i64, _i64, _ptr, _i64, _ptr]),
+    "k3q_prompt_attention": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "k3q_rope_cache": (
         _int, [_ptr, _ptr, _ptr, _int, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "k3q_decode_attention": (

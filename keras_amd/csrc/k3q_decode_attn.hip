@@ -304,10 +304,188 @@ __global__ __launch_bounds__(256) void rope_cache_rows(RopeParams p) {
     vc[c + 8] = v1;
 }
 
+// ---- several positions: a prompt's attention over the cache -------------------------------------------------------
+// out[b, t, h] = softmax(q k^T / sqrt(128) + mask[t]) v over the cache rows, the mask added as it is.  A workgroup takes 64
+// positions of a (sequence, head), a wave 16 of them, and walks the cache in blocks of 64 rows, running maximum and sum per
+// position; blocks that the mask closes for all 64 positions (an additive -inf) are not read.  Products on the matrix cores, keys
+// as the rows: a lane then holds scores of ONE position (its column), four keys of each 16, and these are, as they lie, the
+// operand of the product with the values -- whose other operand takes its keys in the same order, from a transposed tile in
+// LDS.  Scores and sums are float32; a probability goes into its product as two bfloat16 parts (2^-17), not one.
+// 8 x 128 positions of 32 heads, cache of 256: bound by its 32 MB and the chain of a block (mask, keys, scores, values); 49 us
+// in the library's kernel behind a transposed view, 10 here.
+constexpr int kPKeys = 64, kPRows = 64;             // cache rows per block, positions per workgroup
+constexpr int kPKPitch = kHd * 2 + 16;              // LDS bytes per key row
+constexpr int kPVPitch = kPKeys * 2 + 24;           // and per value column (of the transposed tile)
+struct PromptParams {
+    const uint16_t* q;      // [B, T, H, 128]
+    const uint16_t *kc, *vc;  // [B, H, max_len, 128]
+    const uint16_t* mask;   // [T, max_len] bfloat16
+    uint16_t* out;          // [B, T, H, 128]
+    int T, H, max_len;
+    float scale;
+};
+
+__global__ __launch_bounds__(256) void prompt_attention(PromptParams p) {
+    __shared__ __attribute__((aligned(16))) char ks[kPKeys * kPKPitch];
+    __shared__ __attribute__((aligned(16))) char vs[kHd * kPVPitch];
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t bh = blockIdx.x;
+    const int64_t b = bh / p.H;
+    const int h = (int)(bh - b * p.H);
+    const int t0 = (int)blockIdx.y * kPRows + wave * 16;
+    const int t = t0 + i < p.T ? t0 + i : p.T - 1;  // this lane's position (past the end: a copy of the last, not stored)
+    const int64_t qrow = ((b * p.T + t) * p.H + h) * kHd;
+    v4u qf[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) qf[s] = *(const v4u*)(p.q + qrow + 32 * s + 8 * g);
+    const uint16_t* mrow = p.mask + (int64_t)t * p.max_len;
+    const uint16_t* kb = p.kc + bh * p.max_len * kHd;
+    const uint16_t* vb = p.vc + bh * p.max_len * kHd;
+    v4f o[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[d] = v4f{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    const int blocks = (p.max_len + kPKeys - 1) / kPKeys;
+    // the mask of keys 16 kt + 4 g ... + 3 of a block (max_len % 4 == 0: four keys are inside or outside together)
+    auto load_mask = [&](v2u (&mk)[4], const int blk) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            const int j = blk * kPKeys + kt * 16 + 4 * g;
+            mk[kt] = j < p.max_len ? *(const v2u*)(mrow + j) : v2u{0xFF80FF80u, 0xFF80FF80u};  // -inf
+        }
+    };
+    v2u mk[4], mk_next[4];
+    load_mask(mk_next, 0);
+    for (int blk = 0; blk < blocks; ++blk) {
+        u32 open = 0;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            mk[kt] = mk_next[kt];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) open |= (mk[kt][e] ^ 0xFF80FF80u);
+        }
+        if (blk + 1 < blocks) load_mask(mk_next, blk + 1);
+        // (the barrier also ends the reads of the block before)
+        if (!__syncthreads_or(open != 0)) continue;
+        // ---- keys as they lie, values transposed, into LDS; rows past the cache repeat its last ----
+        {
+            const int c = tid & 15, a = tid >> 4;
+            v4u kk[4], vv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t j = blk * kPKeys + 4 * a + r;
+                const int64_t at = (j < p.max_len ? j : p.max_len - 1) * kHd + 8 * c;
+                kk[r] = *(const v4u*)(kb + at);
+                vv[r] = *(const v4u*)(vb + at);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) *(v4u*)(ks + (4 * a + r) * kPKPitch + 16 * c) = kk[r];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const u32 sel = e & 1 ? 0x07060302u : 0x05040100u;
+                const v2u w = {byte_perm(vv[1][e >> 1], vv[0][e >> 1], sel), byte_perm(vv[3][e >> 1], vv[2][e >> 1], sel)};
+                *(v2u*)(vs + (8 * c + e) * kPVPitch + 8 * a) = w;
+            }
+        }
+        __syncthreads();
+        // ---- scores ----
+        float x[4][4];
+        float top = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const v4u kf = *(const v4u*)(ks + (kt * 16 + i) * kPKPitch + 64 * s + 16 * g);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, kf), __builtin_bit_cast(v8bf, qf[s]), acc,
+                                                              0, 0, 0);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const u32 w = mk[kt][e >> 1];
+                x[kt][e] = acc[e] * p.scale + __uint_as_float(e & 1 ? w & 0xffff0000u : w << 16);
+                top = fmaxf(top, x[kt][e]);
+            }
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, kWave));
+        top = fmaxf(top, __shfl_xor(top, 32, kWave));
+        const float m_new = fmaxf(m, top);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;  // (nothing open yet: every term below is zero)
+        const float shrink = __builtin_amdgcn_exp2f((m - m_use) * 1.44269504f);
+        m = m_new;
+        float sum = 0.f;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                x[kt][e] = __builtin_amdgcn_exp2f((x[kt][e] - m_use) * 1.44269504f);
+                sum += x[kt][e];
+            }
+        l = l * shrink + sum;  // (this lane's keys; the four lanes of a position meet at the end)
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[d][e] *= shrink;
+        // ---- values: 32 keys per product, slot 8 g + e of it key 16 (2 pr) + 4 g + e, slots e >= 4 the next 16's ----
+#pragma unroll
+        for (int pr = 0; pr < 2; ++pr) {
+            v4u hi, lo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v0 = x[2 * pr + (e >> 1)][2 * (e & 1)], v1 = x[2 * pr + (e >> 1)][2 * (e & 1) + 1];
+                hi[e] = pack_bf16x2(v0, v1);
+                lo[e] = pack_bf16x2(v0 - __uint_as_float(hi[e] << 16), v1 - __uint_as_float(hi[e] & 0xffff0000u));
+            }
+#pragma unroll
+            for (int d = 0; d < 8; ++d) {
+                const char* at = vs + (16 * d + i) * kPVPitch + (32 * pr + 4 * g) * 2;
+                const v2u v0 = *(const v2u*)at, v1 = *(const v2u*)(at + 32);
+                const v8bf vf = __builtin_bit_cast(v8bf, (v4u{v0[0], v0[1], v1[0], v1[1]}));
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(v8bf, lo), o[d], 0, 0, 0);
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(v8bf, hi), o[d], 0, 0, 0);
+            }
+        }
+    }
+    l += __shfl_xor(l, 16, kWave);
+    l += __shfl_xor(l, 32, kWave);
+    if (t0 + i >= p.T) return;
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+        *(v2u*)(p.out + qrow + 16 * d + 4 * g) = v2u{pack_bf16x2(o[d][0] / l, o[d][1] / l), pack_bf16x2(o[d][2] / l, o[d][3] / l)};
+}
+
 }  // namespace
 }  // namespace k3q
 
 using namespace k3q;
+
+extern "C" int k3q_prompt_attention(const void* q, int dtype, int64_t B, int64_t T, int64_t H, int64_t head_dim,
+                                    int64_t max_len, const void* k_cache, const void* v_cache, const void* mask,
+                                    void* out, void* stream) {
+    if (dtype != K3Q_BF16) return K3Q_ERR_DTYPE;
+    if (B < 0 || T < 0 || H <= 0 || head_dim != kHd || max_len <= 0 || (max_len % 4) != 0 || max_len >= (1 << 30) ||
+        T > 65535 * kPRows || H >= (1 << 20))
+        return K3Q_ERR_SHAPE;
+    if (B == 0 || T == 0) return K3Q_OK;
+    if (B >= (int64_t(1) << 31) / H) return K3Q_ERR_SHAPE;
+    if (!q || !k_cache || !v_cache || !mask || !out) return K3Q_ERR_NULL;
+    if (!aligned_to(q, 16) || !aligned_to(k_cache, 16) || !aligned_to(v_cache, 16) || !aligned_to(mask, 8) ||
+        !aligned_to(out, 8))
+        return K3Q_ERR_ALIGN;
+    PromptParams p;
+    p.q = (const uint16_t*)q;
+    p.kc = (const uint16_t*)k_cache;
+    p.vc = (const uint16_t*)v_cache;
+    p.mask = (const uint16_t*)mask;
+    p.out = (uint16_t*)out;
+    p.T = (int)T;
+    p.H = (int)H;
+    p.max_len = (int)max_len;
+    p.scale = 0.08838834764831845f;  // 1 / sqrt(128)
+    prompt_attention<<<dim3((unsigned)(B * H), (unsigned)((T + kPRows - 1) / kPRows)), 256, 0, (hipStream_t)stream>>>(p);
+    return launch_status();
+}
 
 extern "C" int k3q_rope_cache(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t T, int64_t H,
                               int64_t head_dim, int64_t max_len, const void* cos_table, const void* sin_table,

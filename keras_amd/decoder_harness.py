@@ -126,8 +126,11 @@ class DecoderBlock(Layer):
                 q, k = qk[:, :, : self.n_heads], qk[:, :, self.n_heads:]
                 kc.index_copy_(2, pos, k.transpose(1, 2))
                 vc.index_copy_(2, pos, v.transpose(1, 2))
-            a = torch.nn.functional.scaled_dot_product_attention(
-                q.transpose(1, 2), kc, vc, attn_mask=mask[None, None]).transpose(1, 2)
+            if kops.prompt_attention_supported(q, kc, vc, mask):
+                a = kops.prompt_attention(q, kc, vc, mask)
+            else:
+                a = torch.nn.functional.scaled_dot_product_attention(
+                    q.transpose(1, 2), kc, vc, attn_mask=mask[None, None]).transpose(1, 2)
         # (the residual rides in the projection's bias slot where it can, same bits as the add)
         x = call_add(self.attn_out, a, x)
         if fused:

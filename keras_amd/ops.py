@@ -1310,6 +1310,41 @@ def rope_cache(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_flag=No
     return out
 
 
+def prompt_attention_supported(q, cache_k, cache_v, mask):
+    """bfloat16, head width 128, contiguous caches of a multiple of four rows, a mask [T, max_len] for all heads, nothing to
+    differentiate."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in (q, cache_k, cache_v, mask)):
+        return False
+    return (q.dim() == 4 and q.shape[-1] == 128 and q.shape[1] > 0 and cache_k.shape == cache_v.shape
+            and cache_k.dim() == 4 and cache_k.shape[:2] == (q.shape[0], q.shape[2]) and cache_k.shape[3] == 128
+            and cache_k.shape[2] % 4 == 0 and tuple(mask.shape) == (q.shape[1], cache_k.shape[2])
+            and cache_k.is_contiguous() and cache_v.is_contiguous()
+            and all(t.is_cuda and t.device == q.device and t.dtype == torch.bfloat16 for t in (q, cache_k, cache_v, mask)))
+
+
+def prompt_attention(q, cache_k, cache_v, mask):
+    """`scaled_dot_product_attention(q.transpose(1, 2), cache_k, cache_v, attn_mask=mask[None, None]).transpose(1, 2)` for
+    q `[B, T, H, 128]` and caches `[B, H, max_len, 128]` that `prompt_attention_supported`."""
+    _lib.require_device(q, cache_k, cache_v, mask)
+    lib = _lib.load()
+    B, T, H, hd = q.shape
+    max_len = cache_k.shape[2]
+    if (tuple(cache_k.shape) != (B, H, max_len, hd) or cache_v.shape != cache_k.shape or tuple(mask.shape) != (T, max_len)):
+        raise ValueError("prompt_attention takes caches [B, H, max_len, hd] and a mask [T, max_len], got "
+                         f"{tuple(cache_k.shape)}, {tuple(cache_v.shape)}, {tuple(mask.shape)} for q {tuple(q.shape)}")
+    for t in (q, cache_k, cache_v, mask):
+        if t.dtype != torch.bfloat16:
+            raise TypeError("prompt_attention computes in bfloat16")
+    q, cache_k, cache_v, mask = (
+        t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+        for t in (q, cache_k, cache_v, mask))
+    out = torch.empty((B, T, H, hd), dtype=torch.bfloat16, device=q.device)
+    rc = lib.k3q_prompt_attention(_lib.ptr(q), _lib.dtype_code(q.dtype), B, T, H, hd, max_len, _lib.ptr(cache_k),
+                                  _lib.ptr(cache_v), _lib.ptr(mask), _lib.ptr(out), _lib.stream_ptr(q.device))
+    _lib.check(rc, "k3q_prompt_attention")
+    return out
+
+
 def _rows_view(t):
     """[rows, dim] view of a tensor whose last axis is contiguous and whose leading axes collapse
     into one stride (else a contiguous copy): (tensor, rows, dim, row stride in elements)."""
