@@ -311,8 +311,8 @@ __global__ __launch_bounds__(256) void rope_cache_rows(RopeParams p) {
 // as the rows: a lane then holds scores of ONE position (its column), four keys of each 16, and these are, as they lie, the
 // operand of the product with the values -- whose other operand takes its keys in the same order, from a transposed tile in
 // LDS.  Scores and sums are float32; a probability goes into its product as two bfloat16 parts (2^-17), not one.
-// 8 x 128 positions of 32 heads, cache of 256: bound by its 32 MB and the chain of a block (mask, keys, scores, values); 49 us
-// in the library's kernel behind a transposed view, 10 here.
+// 8 x 128 positions of 32 heads, cache of 256: bound by the chain of a block (mask, keys, scores, values) beside its 32 MB; 49
+// us in the library's kernel behind transposed views, 16 here (dispatches in a kernel trace).
 constexpr int kPKeys = 64, kPRows = 64;             // cache rows per block, positions per workgroup
 constexpr int kPKPitch = kHd * 2 + 16;              // LDS bytes per key row
 constexpr int kPVPitch = kPKeys * 2 + 24;           // and per value column (of the transposed tile)

@@ -1201,6 +1201,52 @@ __global__ __launch_bounds__(256) void km_group_sums(const uint16_t* __restrict_
     }
 }
 
+// The same for groups of 128 with the whole of x in 16-byte pieces: a thread sums the eight values of a piece, sixteen of them a
+// group by lane exchange, so that a wave instruction reads 1 KiB (a wave per group, four bytes a lane, took 6.0 us at 1024 x
+// 4096 and 16.7 at 1024 x 14336, dispatches in a trace; the call there 147 -> 134).
+// kUnitPieces: per thread, all in flight.
+template <int kUnitPieces>
+__global__ __launch_bounds__(256) void km_unit_sums(const v4u* __restrict__ x, v2u* __restrict__ sx, int64_t pieces,
+                                                    int64_t M, int units) {
+    const int64_t first = (int64_t)blockIdx.x * (256 * kUnitPieces) + threadIdx.x;
+    v4u c[kUnitPieces];
+#pragma unroll
+    for (int j = 0; j < kUnitPieces; ++j) c[j] = x[first + j * 256 < pieces ? first + j * 256 : pieces - 1];
+#pragma unroll
+    for (int j = 0; j < kUnitPieces; ++j) {
+        float s[2] = {0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s[0] += bf16_bits_to_f32(c[j][e] & 0xffffu);
+            s[1] += bf16_bits_to_f32(c[j][e] >> 16);
+        }
+        float sum = s[0] + s[1];
+        sum += dpp_move<0xB1, 0xf>(sum);   // quad_perm [1,0,3,2]
+        sum += dpp_move<0x4E, 0xf>(sum);   // quad_perm [2,3,0,1]
+        sum += dpp_move<0x141, 0xf>(sum);  // row_half_mirror
+        sum += dpp_move<0x140, 0xf>(sum);  // row_mirror
+        const int64_t at = first + j * 256;
+        if (at < pieces && (threadIdx.x & 15) == 0) {
+            const int64_t unit = at >> 4, m = unit / units;
+            const u32 hi = f32_to_bf16_bits(sum);
+            const float r1 = sum - bf16_bits_to_f32(hi);
+            const u32 lo = f32_to_bf16_bits(r1);
+            sx[(unit - m * units) * M + m] = v2u{hi | (lo << 16), f32_to_bf16_bits(r1 - bf16_bits_to_f32(lo))};
+        }
+    }
+}
+
+// (x aligned to 16 bytes, K % 128 == 0: the pieces of a group are sixteen neighbouring threads'.)  Four pieces a thread once
+// that still gives every CU a workgroup: 96 rows of 4096 are 48 of them, 1 us slower than 192 with one piece a thread.
+void unit_sums_launch(const uint16_t* x, v2u* sx, int64_t M, int64_t K, hipStream_t s) {
+    const int64_t pieces = M * K / 8, blocks = (pieces + 255) / 256;
+    const int units = (int)(K / 128);
+    if (blocks >= 4 * kTargetWorkgroups)
+        km_unit_sums<4><<<(unsigned)((blocks + 3) / 4), 256, 0, s>>>((const v4u*)x, sx, pieces, M, units);
+    else
+        km_unit_sums<1><<<(unsigned)blocks, 256, 0, s>>>((const v4u*)x, sx, pieces, M, units);
+}
+
 // The rows of x for shapes the tile kernel does not take as they lie: bfloat16 rows of Kp = ceil(K / 128) 128 values,
 // zero past K, and their sums per group of 128 as above.  kParts 2 or 3: float32 rows, each as that many bfloat16
 // rows that add up to it (top 16 bits, top 16 bits of the rest, ...; the last one rounded), part h of row m being row
@@ -1831,7 +1877,7 @@ static int run_gemm_w4_tiles(const void* x, int x_dtype, int64_t M, int64_t K, i
     if (strip && gsize == 128 && w4_tile_fits(M, 1, K, N)) {
         const W4TilePlan tp = w4_tile_plan(M, 1, K, N);
         v2u* sums = (v2u*)workspace;
-        km_group_sums<<<dim3((unsigned)(K / 128), (unsigned)((M + 3) / 4)), 256, 0, s>>>((const uint16_t*)x, sums, M, K, 128);
+        unit_sums_launch((const uint16_t*)x, sums, M, K, s);
         W4TileCall c{};
         c.x = (const uint16_t*)x;
         c.rows = M;
@@ -2009,7 +2055,7 @@ extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K
         v2u* sx = (v2u*)((char*)workspace + pl.x_bytes);
         if (as_is) {
             c.x = (const uint16_t*)xm;
-            km_group_sums<<<pgrid, 256, 0, s>>>(c.x, sx, rows, K, 128);
+            unit_sums_launch(c.x, sx, rows, K, s);
         } else
             (pl.parts == 3   ? km_prepare_rows<3, true>
              : pl.parts == 2 ? km_prepare_rows<2, false>
