@@ -232,6 +232,31 @@ def load():
     return lib
 
 
+class _Calls:
+    """The library's entry points as the package's own calls make them: built-in functions that take addresses as integers
+    (k3q_calls.cpp), ctypes functions where an argument points to a structure."""
+
+    def __init__(self, lib):
+        try:
+            from keras_amd import _k3q_calls as native
+        except ImportError as e:
+            raise RuntimeError(f"{os.path.join(_HERE, '_k3q_calls.so')} is missing or does not load ({e}): build it with "
+                               "`python -m keras_amd.csrc.build`") from e
+        for name in list(SIGNATURES) + list(TEST_SIGNATURES):
+            setattr(self, name, getattr(native, name, None) or getattr(lib, name))
+
+
+_calls = None
+
+
+def calls():
+    """`load()` for hot calls: the same functions without what ctypes costs per argument."""
+    global _calls
+    if _calls is None:
+        _calls = _Calls(load())
+    return _calls
+
+
 def check(code, what):
     if code == 0:
         return
@@ -267,6 +292,11 @@ def raw_stream(device=None):
 
 def stream_ptr(device=None):
     return ctypes.c_void_p(raw_stream(device))
+
+
+def addr(t):
+    """A tensor's address for `calls()`; None: a null pointer."""
+    return t.data_ptr() if t is not None else None
 
 
 def ptr(t):

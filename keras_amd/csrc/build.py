@@ -1,4 +1,4 @@
-"""Compile the k3q HIP sources into keras_amd/libk3q.so for gfx950.
+"""Compile the k3q HIP sources into keras_amd/libk3q.so for gfx950, and the Python module over its entry points.
 
 Run as `python -m keras_amd.csrc.build` or through `__graft_entry__.build()`.
 hipcc cross-compiles, so no GPU is needed to build.
@@ -8,10 +8,12 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "libk3q.so")
+CALLS = os.path.join(PKG, "_k3q_calls.so")
 
 SOURCES = [
     "k3q_api.hip",
@@ -71,7 +73,17 @@ def build(verbose=True, jobs=8):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    build_calls(verbose)
     return LIB
+
+
+def build_calls(verbose=True):
+    """The Python module over the library's entry points (k3q_calls.cpp), next to the library it is linked to."""
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-I", sysconfig.get_paths()["include"],
+           os.path.join(HERE, "k3q_calls.cpp"), "-o", CALLS, "-L", PKG, "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
 
 
 def _drain(procs):

@@ -117,19 +117,19 @@ def int4_matmul(x, kernel_packed, kernel_scale, orig_output_dim, kernel_zero=Non
             raise ValueError("grouped int4 needs kernel_zero")
         kz = kernel_zero if kernel_zero.is_contiguous() else kernel_zero.contiguous()
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    lib = _lib.load()
+    lib = _lib.calls()
     nbytes = lib.k3q_gemv_w4_workspace_bytes(M, K, N)
     if plan is not None:
         # an overridden plan may split K into many more workgroups than the built-in one
         nbytes = max(nbytes, (K // 16 + 1) * min(M, 16) * N * 4)
     ws = _workspace(x.device, nbytes)
     args = [
-        _lib.ptr(x2), code, M, K, N, _lib.ptr(kp), _lib.ptr(ks), _lib.ptr(kz),
-        int(block_size) if grouped else -1, _lib.ptr(bias), _lib.ptr(y),
-        _lib.ptr(ws), ws.numel(),
+        _lib.addr(x2), code, M, K, N, _lib.addr(kp), _lib.addr(ks), _lib.addr(kz),
+        int(block_size) if grouped else -1, _lib.addr(bias), _lib.addr(y),
+        _lib.addr(ws), ws.numel(),
     ]
     cnt = _arrival_counters(x.device, lib.k3q_gemv_w4_counters_bytes(N)) if single_launch else None
-    args += [_lib.ptr(cnt), cnt.numel() if single_launch else 0]
+    args += [_lib.addr(cnt), cnt.numel() if single_launch else 0]
     if addend is None and bias is not None and M > 1 and bias.numel() == M * N:
         addend, bias = bias, None  # a bias with a row per row of x is an addend
     if addend is not None:
@@ -140,13 +140,13 @@ def int4_matmul(x, kernel_packed, kernel_scale, orig_output_dim, kernel_zero=Non
         if addend.dtype != x.dtype or addend.numel() != M * N:
             raise ValueError("addend must hold M x N values of the input's dtype")
         ad = addend.reshape(M, N)
-        args[9] = _lib.ptr(ad if ad.is_contiguous() else ad.contiguous())
-        rc = lib.k3q_gemv_w4_addend(*args, _lib.stream_ptr(x.device))
+        args[9] = _lib.addr(ad if ad.is_contiguous() else ad.contiguous())
+        rc = lib.k3q_gemv_w4_addend(*args, _lib.raw_stream(x.device))
     elif plan is None:
-        rc = lib.k3q_gemv_w4_fused(*args, _lib.stream_ptr(x.device))
+        rc = lib.k3q_gemv_w4_fused(*args, _lib.raw_stream(x.device))
     else:
         arr = (ctypes.c_int * 4)(*[int(v) for v in plan[:4]])
-        rc = lib.k3qt_gemv_w4_plan(*args, arr, _lib.stream_ptr(x.device))
+        rc = lib.k3qt_gemv_w4_plan(*args, arr, _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemv_w4")
     return _shaped(y, lead)
 
@@ -169,7 +169,7 @@ def int4_matmul_multi(x, kernels, block_size=None):
     if not x2.is_contiguous():
         x2 = x2.contiguous()
     M = x2.shape[0]
-    lib = _lib.load()
+    lib = _lib.calls()
     problems = (_lib.GemvW4Problem * len(kernels))()
     outs, keep = [], []
     ws_bytes = cnt_bytes = 0
@@ -200,9 +200,9 @@ def int4_matmul_multi(x, kernels, block_size=None):
         cnt_bytes += lib.k3q_gemv_w4_counters_bytes(N)
     ws = _workspace(x.device, ws_bytes)
     cnt = _arrival_counters(x.device, cnt_bytes)
-    rc = lib.k3q_gemv_w4_multi(_lib.ptr(x2), code, M, K, len(kernels), ctypes.byref(problems),
-                               int(block_size) if grouped else -1, _lib.ptr(ws), ws.numel(),
-                               _lib.ptr(cnt), cnt.numel(), _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemv_w4_multi(_lib.addr(x2), code, M, K, len(kernels), ctypes.byref(problems),
+                               int(block_size) if grouped else -1, _lib.addr(ws), ws.numel(),
+                               _lib.addr(cnt), cnt.numel(), _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemv_w4_multi")
     return [y.reshape(*lead, y.shape[1]) for y in outs]
 
@@ -213,7 +213,7 @@ STRIP_MAX_ROWS = 16
 def int4_strip_supported(M, K, N, block_size=None):
     """Whether `int4_matmul_strip` takes M bfloat16 rows against a [K, N] int4 kernel."""
     bs = int(block_size) if block_size is not None and block_size > 0 else -1
-    return bool(_lib.load().k3q_gemv_w4s_supported(int(M), int(K), int(N), bs))
+    return bool(_lib.calls().k3q_gemv_w4s_supported(int(M), int(K), int(N), bs))
 
 
 def int4_strip_copy(kernel_packed, units):
@@ -224,13 +224,13 @@ def int4_strip_copy(kernel_packed, units):
     K, N = kernel_packed.shape[0], int(units)
     if kernel_packed.dtype != torch.int8 or kernel_packed.shape[1] != (N + 1) // 2:
         raise ValueError("kernel must be int8 of shape [input_dim, ceil(units / 2)]")
-    lib = _lib.load()
+    lib = _lib.calls()
     nbytes = lib.k3q_w4s_shadow_bytes(K, N)
     if nbytes <= 0:
         raise ValueError("the strip-linear copy needs K % 8 == 0")
     kp = kernel_packed if kernel_packed.is_contiguous() else kernel_packed.contiguous()
     out = torch.empty(nbytes, dtype=torch.uint8, device=kp.device)
-    _lib.check(lib.k3q_w4s_pack(_lib.ptr(kp), K, N, _lib.ptr(out), _lib.stream_ptr(kp.device)), "k3q_w4s_pack")
+    _lib.check(lib.k3q_w4s_pack(_lib.addr(kp), K, N, _lib.addr(out), _lib.raw_stream(kp.device)), "k3q_w4s_pack")
     return out
 
 
@@ -238,7 +238,7 @@ def int4_strip_params(kernel_scale, kernel_zero, K, units, block_size):
     """Scales and zero points of a grouped (block 128) int4 kernel in the order the strip kernel
     reads them: per (strip, group) four records of four bfloat16 scales and four `zero + 128` bytes."""
     _lib.require_device(kernel_scale, kernel_zero)
-    lib = _lib.load()
+    lib = _lib.calls()
     N = int(units)
     nbytes = lib.k3q_w4s_params_bytes(int(K), N, int(block_size))
     if nbytes <= 0:
@@ -248,8 +248,8 @@ def int4_strip_params(kernel_scale, kernel_zero, K, units, block_size):
     if tuple(sc.shape) != (K // 128, N) or tuple(zp.shape) != (K // 128, N) or zp.dtype != torch.int8:
         raise ValueError("scale / zero must be [K / 128, N], zero int8")
     out = torch.empty(nbytes, dtype=torch.uint8, device=sc.device)
-    rc = lib.k3q_w4s_pack_params(_lib.ptr(sc), _lib.dtype_code(sc.dtype), _lib.ptr(zp), int(K), N,
-                                 int(block_size), _lib.ptr(out), _lib.stream_ptr(sc.device))
+    rc = lib.k3q_w4s_pack_params(_lib.addr(sc), _lib.dtype_code(sc.dtype), _lib.addr(zp), int(K), N,
+                                 int(block_size), _lib.addr(out), _lib.raw_stream(sc.device))
     _lib.check(rc, "k3q_w4s_pack_params")
     return out
 
@@ -269,7 +269,7 @@ def int4_matmul_strip(x, shadow, units, kernel_scale=None, gparams=None, block_s
     lead = x.shape[:-1]
     x2 = _rows_of(x, K)
     M = x2.shape[0]
-    lib = _lib.load()
+    lib = _lib.calls()
     if shadow.numel() != lib.k3q_w4s_shadow_bytes(K, N):
         raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
     stride = 0
@@ -292,10 +292,10 @@ def int4_matmul_strip(x, shadow, units, kernel_scale=None, gparams=None, block_s
     elif kernel_scale is None or kernel_scale.dtype != torch.bfloat16 or kernel_scale.numel() != N:
         raise ValueError("per-channel int4 needs bfloat16 scales [N]")
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    rc = lib.k3q_gemv_w4s(_lib.ptr(x2), _lib.K3Q_BF16, M, K, N, _lib.ptr(shadow),
-                          None if grouped else _lib.ptr(kernel_scale), _lib.ptr(gparams) if grouped else None,
-                          int(block_size) if grouped else -1, _lib.ptr(b), stride, _lib.ptr(y),
-                          _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemv_w4s(_lib.addr(x2), _lib.K3Q_BF16, M, K, N, _lib.addr(shadow),
+                          None if grouped else _lib.addr(kernel_scale), _lib.addr(gparams) if grouped else None,
+                          int(block_size) if grouped else -1, _lib.addr(b), stride, _lib.addr(y),
+                          _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemv_w4s")
     return _shaped(y, lead)
 
@@ -303,7 +303,7 @@ def int4_matmul_strip(x, shadow, units, kernel_scale=None, gparams=None, block_s
 def int4_strip_rows_launches(dtype, M, K, N, block_size=None, plain=False):
     """How many launches `int4_matmul_strip_rows` needs for M rows of `dtype`; 0: it does not take them."""
     bs = int(block_size) if block_size is not None and block_size > 0 else -1
-    lib = _lib.load()
+    lib = _lib.calls()
     launches = lib.k3q_gemv_w4s_rows_plain_launches if plain else lib.k3q_gemv_w4s_rows_launches
     return launches(_lib.dtype_code(dtype), int(M), int(K), int(N), bs)
 
@@ -311,7 +311,7 @@ def int4_strip_rows_launches(dtype, M, K, N, block_size=None, plain=False):
 def int4_strip_rows_params(kernel_scale, kernel_zero, K, units, block_size):
     """As `int4_strip_params`, for `int4_matmul_strip_rows`: scales in their own dtype, any K % 8, any N."""
     _lib.require_device(kernel_scale, kernel_zero)
-    lib = _lib.load()
+    lib = _lib.calls()
     K, N, code = int(K), int(units), _lib.dtype_code(kernel_scale.dtype)
     nbytes = lib.k3q_w4s_rows_params_bytes(K, N, int(block_size), code)
     if nbytes <= 0:
@@ -322,8 +322,8 @@ def int4_strip_rows_params(kernel_scale, kernel_zero, K, units, block_size):
     if tuple(sc.shape) != shape or tuple(zp.shape) != shape or zp.dtype != torch.int8:
         raise ValueError("scale / zero must be [ceil(K / 128), N], zero int8")
     out = torch.empty(nbytes, dtype=torch.uint8, device=sc.device)
-    rc = lib.k3q_w4s_rows_pack_params(_lib.ptr(sc), code, _lib.ptr(zp), K, N, int(block_size), _lib.ptr(out),
-                                      _lib.stream_ptr(sc.device))
+    rc = lib.k3q_w4s_rows_pack_params(_lib.addr(sc), code, _lib.addr(zp), K, N, int(block_size), _lib.addr(out),
+                                      _lib.raw_stream(sc.device))
     _lib.check(rc, "k3q_w4s_rows_pack_params")
     return out
 
@@ -335,7 +335,7 @@ def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, bl
     float32 rows in full, as where N % 8 or K % 16, whatever the shape.
     Reference: keras/src/layers/core/dense.py:988-1095."""
     _lib.require_device(x, shadow, kernel_scale, gparams, bias)
-    lib = _lib.load()
+    lib = _lib.calls()
     code = _lib.dtype_code(x.dtype)
     grouped = block_size is not None and block_size > 0
     bs = int(block_size) if grouped else -1
@@ -360,8 +360,8 @@ def int4_matmul_strip_rows(x, shadow, units, kernel_scale=None, gparams=None, bl
     ks = None if grouped else (kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous())
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     run = lib.k3q_gemv_w4s_rows_plain if plain else lib.k3q_gemv_w4s_rows
-    rc = run(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks), _lib.ptr(gparams) if grouped else None, bs,
-             _lib.ptr(b), stride, _lib.ptr(y), _lib.stream_ptr(x.device))
+    rc = run(_lib.addr(x2), code, M, K, N, _lib.addr(shadow), _lib.addr(ks), _lib.addr(gparams) if grouped else None, bs,
+             _lib.addr(b), stride, _lib.addr(y), _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemv_w4s_rows")
     return _shaped(y, lead)
 
@@ -379,7 +379,7 @@ def int4_matmul_strip_rows_multi(x, kernels, block_size=None):
     if x2.data_ptr() % 16:
         x2 = x2.clone()
     M = x2.shape[0]
-    lib = _lib.load()
+    lib = _lib.calls()
     problems = (_lib.GemvW4sProblem * len(kernels))()
     outs, keep = [], []
     for i, k in enumerate(kernels):
@@ -403,8 +403,8 @@ def int4_matmul_strip_rows_multi(x, kernels, block_size=None):
         problems[i] = _lib.GemvW4sProblem(
             N, shadow.data_ptr(), None if grouped else scale.data_ptr(), gparams.data_ptr() if grouped else None,
             bias.data_ptr() if bias is not None else None, y.data_ptr())
-    rc = lib.k3q_gemv_w4s_rows_multi(_lib.ptr(x2), code, M, K, len(kernels), ctypes.byref(problems), bs,
-                                     _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemv_w4s_rows_multi(_lib.addr(x2), code, M, K, len(kernels), ctypes.byref(problems), bs,
+                                     _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemv_w4s_rows_multi")
     return [y.reshape(*lead, y.shape[1]) for y in outs]
 
@@ -421,7 +421,7 @@ def int4_matmul_strip_multi(x, kernels, block_size=None, input_op=None, bias_row
     x2 = x.reshape(-1, K)
     x2 = x2 if x2.is_contiguous() else x2.contiguous()
     M = x2.shape[0]
-    lib = _lib.load()
+    lib = _lib.calls()
     problems = (_lib.GemvW4sProblem * len(kernels))()
     outs = []
     for i, k in enumerate(kernels):
@@ -440,14 +440,14 @@ def int4_matmul_strip_multi(x, kernels, block_size=None, input_op=None, bias_row
             k["gparams"].data_ptr() if grouped else None,
             bias.data_ptr() if bias is not None else None, y.data_ptr())
     if input_op is None and not bias_rows:
-        rc = lib.k3q_gemv_w4s_multi(_lib.ptr(x2), _lib.K3Q_BF16, M, K, len(kernels), ctypes.byref(problems),
-                                    int(block_size) if grouped else -1, _lib.stream_ptr(x.device))
+        rc = lib.k3q_gemv_w4s_multi(_lib.addr(x2), _lib.K3Q_BF16, M, K, len(kernels), ctypes.byref(problems),
+                                    int(block_size) if grouped else -1, _lib.raw_stream(x.device))
         _lib.check(rc, "k3q_gemv_w4s_multi")
     else:
         pre, keep = _input_op_struct(input_op, M, K, x.device)
-        rc = lib.k3q_gemv_w4s_pre(_lib.ptr(x2), _lib.K3Q_BF16, M, K, ctypes.byref(pre) if pre is not None else None,
+        rc = lib.k3q_gemv_w4s_pre(_lib.addr(x2), _lib.K3Q_BF16, M, K, ctypes.byref(pre) if pre is not None else None,
                                   len(kernels), ctypes.byref(problems), int(block_size) if grouped else -1,
-                                  1 if bias_rows else 0, _lib.stream_ptr(x.device))
+                                  1 if bias_rows else 0, _lib.raw_stream(x.device))
         _lib.check(rc, "k3q_gemv_w4s_pre")
         del keep
     return [y.reshape(*lead, y.shape[1]) for y in outs]
@@ -524,9 +524,9 @@ def input_op_quantize(input_op, x2, epsilon=1e-7, value_range=(-127, 127)):
     h = torch.empty_like(x2)
     q = torch.empty((M, K), dtype=torch.int8, device=x2.device)
     s = torch.empty((M,), dtype=torch.bfloat16, device=x2.device)
-    rc = _lib.load().k3q_input_op_quantize(_lib.ptr(x2), _lib.K3Q_BF16, M, K, ctypes.byref(pre), float(epsilon),
-                                           float(value_range[0]), float(value_range[1]), _lib.ptr(h), _lib.ptr(q),
-                                           _lib.ptr(s), _lib.stream_ptr(x2.device))
+    rc = _lib.calls().k3q_input_op_quantize(_lib.addr(x2), _lib.K3Q_BF16, M, K, ctypes.byref(pre), float(epsilon),
+                                           float(value_range[0]), float(value_range[1]), _lib.addr(h), _lib.addr(q),
+                                           _lib.addr(s), _lib.raw_stream(x2.device))
     _lib.check(rc, "k3q_input_op_quantize")
     del keep
     return h, q, s.reshape(M, 1)
@@ -544,13 +544,13 @@ def int4_strip_input_op_supported(input_op, M, K, N, block_size=None):
     for the gate."""
     bs = int(block_size) if block_size is not None and block_size > 0 else -1
     return (_input_op_rows_ok(input_op, M, K) and M * K <= 65536
-            and bool(_lib.load().k3q_gemv_w4s_supported(M, K, N, bs)))
+            and bool(_lib.calls().k3q_gemv_w4s_supported(M, K, N, bs)))
 
 
 def int8_strip_input_op_supported(input_op, M, K, N, value_range=(-127, 127)):
     """The same for `int8_dense_strip_multi`: sizes at which the kernel quantises the rows itself."""
     return (_input_op_rows_ok(input_op, M, K) and int8_strip_quantises_inside(M, K, value_range)
-            and bool(_lib.load().k3q_dense_i8_w8s_supported(M, K, N)))
+            and bool(_lib.calls().k3q_dense_i8_w8s_supported(M, K, N)))
 
 
 def int4_kmajor_copy(kernel_packed, units):
@@ -559,7 +559,7 @@ def int4_kmajor_copy(kernel_packed, units):
     (include/k3q.h, k3q_gemm_w4_kmajor).  Made once per layer from the stored
     `[K, ceil(N/2)]` kernel; K % 8 == 0."""
     _lib.require_device(kernel_packed)
-    lib = _lib.load()
+    lib = _lib.calls()
     K, N = int(kernel_packed.shape[0]), int(units)
     if kernel_packed.dtype != torch.int8 or kernel_packed.dim() != 2 or kernel_packed.shape[1] != (N + 1) // 2:
         raise ValueError(f"expected the stored int8 kernel [K, ceil({N}/2)], got {tuple(kernel_packed.shape)}")
@@ -567,13 +567,13 @@ def int4_kmajor_copy(kernel_packed, units):
         raise ValueError("the K-contiguous copy needs K % 8 == 0")
     src = kernel_packed if kernel_packed.is_contiguous() else kernel_packed.contiguous()
     out = torch.empty((N, K // 8), dtype=torch.int32, device=src.device)
-    _lib.check(lib.k3q_w4_kmajor_pack(_lib.ptr(src), K, N, _lib.ptr(out), _lib.stream_ptr(src.device)),
+    _lib.check(lib.k3q_w4_kmajor_pack(_lib.addr(src), K, N, _lib.addr(out), _lib.raw_stream(src.device)),
                "k3q_w4_kmajor_pack")
     return out
 
 
 def int4_kmajor_supported(M, K, N, block_size=None):
-    lib = _lib.load()
+    lib = _lib.calls()
     bs = int(block_size) if block_size is not None and block_size > 0 else -1
     return lib.k3q_gemm_w4_kmajor_workspace_bytes(M, K, N, bs) > 0
 
@@ -596,17 +596,17 @@ def int4_matmul_kmajor(x, kernel_kmajor, kernel_scale, kernel_zero=None, block_s
     if bias is not None and bias.numel() != N:
         raise ValueError(f"bias holds {bias.numel()} values, the layer has {N} units")
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    lib = _lib.load()
+    lib = _lib.calls()
     bs = int(block_size) if grouped else -1
     nbytes = lib.k3q_gemm_w4_kmajor_workspace_bytes(M, K, N, bs)
     if nbytes <= 0:
         raise ValueError(f"the K-contiguous route does not take M={M}, K={K}, N={N}, block_size={block_size}")
     ws = _workspace(x.device, nbytes)
     ks = kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous()
-    rc = lib.k3q_gemm_w4_kmajor(_lib.ptr(x2), _lib.dtype_code(x.dtype), M, K, N, _lib.ptr(kernel_kmajor),
-                                _lib.ptr(ks), _lib.ptr(kernel_zero) if grouped else None, bs,
-                                _lib.ptr(bias), _lib.ptr(y), _lib.ptr(ws), ws.numel(),
-                                _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemm_w4_kmajor(_lib.addr(x2), _lib.dtype_code(x.dtype), M, K, N, _lib.addr(kernel_kmajor),
+                                _lib.addr(ks), _lib.addr(kernel_zero) if grouped else None, bs,
+                                _lib.addr(bias), _lib.addr(y), _lib.addr(ws), ws.numel(),
+                                _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemm_w4_kmajor")
     return y.reshape(*lead, N)
 
@@ -615,7 +615,7 @@ def int4_tiles_strip_supported(M, K, N, block_size=None):
     """Whether `int4_matmul_tiles_strip` takes M bfloat16 rows against a [K, N] kernel's strip copy."""
     grouped = block_size is not None and block_size > 0
     return (int4_kmajor_supported(M, K, N, block_size) and (not grouped or block_size % 128 == 0)
-            and _lib.load().k3q_w4s_shadow_bytes(int(K), int(N)) > 0)
+            and _lib.calls().k3q_w4s_shadow_bytes(int(K), int(N)) > 0)
 
 
 def int4_matmul_tiles_strip(x, shadow, units, kernel_scale, kernel_zero=None, block_size=None, bias=None):
@@ -628,7 +628,7 @@ def int4_matmul_tiles_strip(x, shadow, units, kernel_scale, kernel_zero=None, bl
         raise TypeError("the int4 tile route computes in bfloat16")
     grouped = block_size is not None and block_size > 0
     N, K = int(units), x.shape[-1]
-    lib = _lib.load()
+    lib = _lib.calls()
     if shadow.numel() != lib.k3q_w4s_shadow_bytes(K, N):
         raise ValueError("the strip-linear copy does not belong to a [%d, %d] kernel" % (K, N))
     lead = x.shape[:-1]
@@ -643,10 +643,10 @@ def int4_matmul_tiles_strip(x, shadow, units, kernel_scale, kernel_zero=None, bl
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     ws = _workspace(x.device, nbytes)
     ks = kernel_scale if kernel_scale.is_contiguous() else kernel_scale.contiguous()
-    rc = lib.k3q_gemm_w4_strip(_lib.ptr(x2), _lib.dtype_code(x.dtype), M, K, N, _lib.ptr(shadow),
-                               _lib.ptr(ks), _lib.ptr(kernel_zero) if grouped else None, bs,
-                               _lib.ptr(bias), _lib.ptr(y), _lib.ptr(ws), ws.numel(),
-                               _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemm_w4_strip(_lib.addr(x2), _lib.dtype_code(x.dtype), M, K, N, _lib.addr(shadow),
+                               _lib.addr(ks), _lib.addr(kernel_zero) if grouped else None, bs,
+                               _lib.addr(bias), _lib.addr(y), _lib.addr(ws), ws.numel(),
+                               _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemm_w4_strip")
     return _shaped(y, lead)
 
@@ -668,7 +668,7 @@ def int4_tile_columns(t, units):
 def int4_tiles_rows_supported(K, N, block_size=None):
     """Whether `int4_matmul_tiles_rows` takes a [K, N] int4 kernel."""
     bs = int(block_size) if block_size is not None and block_size > 0 else -1
-    return _lib.load().k3q_gemm_w4_rows_workspace_bytes(_lib.K3Q_BF16, 1, int(K), int(N), bs) > 0
+    return _lib.calls().k3q_gemm_w4_rows_workspace_bytes(_lib.K3Q_BF16, 1, int(K), int(N), bs) > 0
 
 
 def int4_matmul_tiles_rows(x, shadow, units, kernel_scale, kernel_zero=None, block_size=None, bias=None):
@@ -677,7 +677,7 @@ def int4_matmul_tiles_rows(x, shadow, units, kernel_scale, kernel_zero=None, blo
     `kernel_zero` through `int4_tile_columns`.  `bias` [N], or [M, N]: a row per row of x.
     Reference: keras/src/layers/core/dense.py:988-1095."""
     _lib.require_device(x, shadow, kernel_scale, kernel_zero, bias)
-    lib = _lib.load()
+    lib = _lib.calls()
     code = _lib.dtype_code(x.dtype)
     grouped = block_size is not None and block_size > 0
     bs = int(block_size) if grouped else -1
@@ -707,8 +707,8 @@ def int4_matmul_tiles_rows(x, shadow, units, kernel_scale, kernel_zero=None, blo
     stride = N if bias is not None and M > 1 and bias.numel() == M * N else 0
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     ws = _workspace(x.device, lib.k3q_gemm_w4_rows_workspace_bytes(code, M, K, N, bs))
-    rc = lib.k3q_gemm_w4_rows(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks), _lib.ptr(kz), bs,
-                              _lib.ptr(b), stride, _lib.ptr(y), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemm_w4_rows(_lib.addr(x2), code, M, K, N, _lib.addr(shadow), _lib.addr(ks), _lib.addr(kz), bs,
+                              _lib.addr(b), stride, _lib.addr(y), _lib.addr(ws), ws.numel(), _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemm_w4_rows")
     return _shaped(y, lead)
 
@@ -724,8 +724,8 @@ def prepack_int8_kernel(kernel):
     k = kernel if kernel.is_contiguous() else kernel.contiguous()
     K, N = k.shape
     out = torch.empty((N, K), dtype=torch.int8, device=k.device)
-    rc = _lib.load().k3q_prepack_kernel_i8(_lib.ptr(k), K, N, _lib.ptr(out),
-                                           _lib.stream_ptr(k.device))
+    rc = _lib.calls().k3q_prepack_kernel_i8(_lib.addr(k), K, N, _lib.addr(out),
+                                           _lib.raw_stream(k.device))
     _lib.check(rc, "k3q_prepack_kernel_i8")
     return out
 
@@ -769,7 +769,7 @@ def int8_matmul(a, kernel, a_scale=None, kernel_scale=None, bias=None, out_dtype
     _check_bias_size(bias, M, N)
     y = torch.empty((M, N), dtype=out_dtype, device=a.device) if want_y else None
     acc = torch.empty((M, N), dtype=torch.int32, device=a.device) if want_acc else None
-    lib = _lib.load()
+    lib = _lib.calls()
     skinny = M <= SKINNY_MAX_ROWS and N % 16 == 0 and K % 8 == 0
     nbytes = lib.k3q_gemm_i8_workspace_bytes(M, N, K)
     if strip is not None and not skinny and K % 64 == 0:
@@ -798,16 +798,16 @@ def int8_matmul(a, kernel, a_scale=None, kernel_scale=None, bias=None, out_dtype
                              "and returns y only" % SKINNY_MAX_ROWS)
         ad = bias.reshape(M, N)
         rc = lib.k3q_gemm_i8_addend(
-            _lib.ptr(a), _lib.ptr(b), M, N, K, _lib.ptr(sa), _lib.ptr(sb),
-            _lib.ptr(ad if ad.is_contiguous() else ad.contiguous()), code,
-            GEMM_EXACT_EPILOGUE if exact_epilogue else 0, _lib.ptr(y), _lib.ptr(ws), ws_bytes,
-            _lib.stream_ptr(a.device))
+            _lib.addr(a), _lib.addr(b), M, N, K, _lib.addr(sa), _lib.addr(sb),
+            _lib.addr(ad if ad.is_contiguous() else ad.contiguous()), code,
+            GEMM_EXACT_EPILOGUE if exact_epilogue else 0, _lib.addr(y), _lib.addr(ws), ws_bytes,
+            _lib.raw_stream(a.device))
         _lib.check(rc, "k3q_gemm_i8_addend")
         return y
     rc = lib.k3q_gemm_i8(
-        _lib.ptr(a), _lib.ptr(b), layout, M, N, K, _lib.ptr(sa), _lib.ptr(sb), _lib.ptr(bias),
-        code, GEMM_EXACT_EPILOGUE if exact_epilogue else 0, _lib.ptr(y), _lib.ptr(acc),
-        _lib.ptr(ws), ws_bytes, _lib.stream_ptr(a.device),
+        _lib.addr(a), _lib.addr(b), layout, M, N, K, _lib.addr(sa), _lib.addr(sb), _lib.addr(bias),
+        code, GEMM_EXACT_EPILOGUE if exact_epilogue else 0, _lib.addr(y), _lib.addr(acc),
+        _lib.addr(ws), ws_bytes, _lib.raw_stream(a.device),
     )
     _lib.check(rc, "k3q_gemm_i8")
     if want_acc and want_y:
@@ -846,7 +846,7 @@ def int8_matmul_nk(a, kernel_nk, a_scale=None, kernel_scale=None, out_dtype=None
     sb = kernel_scale.reshape(-1).contiguous() if kernel_scale is not None else None
     y = torch.empty((M, N), dtype=out_dtype, device=a.device)
     acc = torch.empty((M, N), dtype=torch.int32, device=a.device) if want_acc else None
-    lib = _lib.load()
+    lib = _lib.calls()
     ws, ws_bytes = None, 0
     if M <= 64 or K % 128 != 0:
         # the decode kernels may split K and then need room for int32 partials; a K that is not
@@ -854,10 +854,10 @@ def int8_matmul_nk(a, kernel_nk, a_scale=None, kernel_scale=None, out_dtype=None
         ws = _workspace(a.device, lib.k3q_gemm_i8_workspace_bytes(M, N, K))
         ws_bytes = ws.numel()
     rc = lib.k3q_gemm_i8(
-        _lib.ptr(a), _lib.ptr(b), 1, M, N, K, _lib.ptr(sa), _lib.ptr(sb), None, code,
+        _lib.addr(a), _lib.addr(b), 1, M, N, K, _lib.addr(sa), _lib.addr(sb), None, code,
         (GEMM_EXACT_EPILOGUE if exact_epilogue else 0)
         | (GEMM_ROUND_ACC_BF16 if round_acc_bf16 else 0),
-        _lib.ptr(y), _lib.ptr(acc), _lib.ptr(ws), ws_bytes, _lib.stream_ptr(a.device),
+        _lib.addr(y), _lib.addr(acc), _lib.addr(ws), ws_bytes, _lib.raw_stream(a.device),
     )
     _lib.check(rc, "k3q_gemm_i8")
     return (y, acc) if want_acc else y
@@ -899,11 +899,11 @@ def embedding_lookup(ids, table, scale, dim, bits=8, zero=None, block_size=None,
     count = ids.numel()
     out = torch.empty((count, dim), dtype=out_dtype, device=table.device)
     flag = torch.zeros(1, dtype=torch.int32, device=table.device) if check_ids else None
-    rc = _lib.load().k3q_embedding_lookup(
-        _lib.ptr(ids), _lib.K3Q_I64 if ids.dtype == torch.int64 else _lib.K3Q_I32, count,
-        _lib.ptr(table), vocab, int(dim), int(bits), _lib.ptr(scale), _lib.dtype_code(scale.dtype),
-        _lib.ptr(zero) if grouped else None, int(block_size) if grouped else -1,
-        _lib.dtype_code(out_dtype), _lib.ptr(out), _lib.ptr(flag), _lib.stream_ptr(table.device),
+    rc = _lib.calls().k3q_embedding_lookup(
+        _lib.addr(ids), _lib.K3Q_I64 if ids.dtype == torch.int64 else _lib.K3Q_I32, count,
+        _lib.addr(table), vocab, int(dim), int(bits), _lib.addr(scale), _lib.dtype_code(scale.dtype),
+        _lib.addr(zero) if grouped else None, int(block_size) if grouped else -1,
+        _lib.dtype_code(out_dtype), _lib.addr(out), _lib.addr(flag), _lib.raw_stream(table.device),
     )
     _lib.check(rc, "k3q_embedding_lookup")
     if check_ids and int(flag.item()) != 0:
@@ -938,9 +938,9 @@ def int4_matmul_nk(x, table_packed, scale, zero=None, block_size=None):
         zp = zero if zero.is_contiguous() else zero.contiguous()
     out_dtype = torch.bfloat16 if (x.dtype == torch.bfloat16 and scale.dtype == torch.bfloat16) else torch.float32
     y = torch.empty((x2.shape[0], N), dtype=out_dtype, device=x.device)
-    rc = _lib.load().k3q_gemv_w4_nk(
-        _lib.ptr(x2), xcode, x2.shape[0], K, N, _lib.ptr(tp), _lib.ptr(sc), scode, _lib.ptr(zp),
-        int(block_size) if grouped else -1, _lib.ptr(y), _lib.stream_ptr(x.device),
+    rc = _lib.calls().k3q_gemv_w4_nk(
+        _lib.addr(x2), xcode, x2.shape[0], K, N, _lib.addr(tp), _lib.addr(sc), scode, _lib.addr(zp),
+        int(block_size) if grouped else -1, _lib.addr(y), _lib.raw_stream(x.device),
     )
     _lib.check(rc, "k3q_gemv_w4_nk")
     return y.reshape(*lead, N)
@@ -970,12 +970,12 @@ def int8_weight_only_matmul(x, kernel, kernel_scale, bias=None, prepacked=None):
         b, layout = prepacked, 1
     else:
         b, layout = (kernel if kernel.is_contiguous() else kernel.contiguous()), 0
-    lib = _lib.load()
+    lib = _lib.calls()
     ws = _workspace(x.device, lib.k3q_gemm_w8_workspace_bytes(M, N, K))
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    rc = lib.k3q_gemm_w8(_lib.ptr(x2), code, _lib.ptr(b), layout, M, N, K,
-                         _lib.ptr(kernel_scale.reshape(-1).contiguous()), _lib.ptr(bias), _lib.ptr(y),
-                         _lib.ptr(ws), ws.numel(), _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemm_w8(_lib.addr(x2), code, _lib.addr(b), layout, M, N, K,
+                         _lib.addr(kernel_scale.reshape(-1).contiguous()), _lib.addr(bias), _lib.addr(y),
+                         _lib.addr(ws), ws.numel(), _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemm_w8")
     return y.reshape(*lead, N)
 
@@ -1012,11 +1012,11 @@ def float_matmul_nk(x, wt, parts=1, bias=None):
     N = wt.shape[0]
     x = x if x.is_contiguous() else x.contiguous()
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    lib = _lib.load()
+    lib = _lib.calls()
     ws = _workspace(x.device, lib.k3q_gemm_wbf16_workspace_bytes(M, N, K, parts))
-    rc = lib.k3q_gemm_wbf16(_lib.ptr(x), _lib.dtype_code(x.dtype), _lib.ptr(wt), parts, M, N, K,
-                            _lib.ptr(bias), _lib.ptr(y), _lib.ptr(ws), ws.numel(),
-                            _lib.stream_ptr(x.device))
+    rc = lib.k3q_gemm_wbf16(_lib.addr(x), _lib.dtype_code(x.dtype), _lib.addr(wt), parts, M, N, K,
+                            _lib.addr(bias), _lib.addr(y), _lib.addr(ws), ws.numel(),
+                            _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_gemm_wbf16")
     return y
 
@@ -1027,13 +1027,13 @@ INT8_STRIP_MAX_ROWS = 16
 
 def int8_strip_supported(M, K, N):
     """Whether `int8_dense_strip` takes M rows against a [K, N] int8 kernel."""
-    return bool(_lib.load().k3q_dense_i8_w8s_supported(int(M), int(K), int(N)))
+    return bool(_lib.calls().k3q_dense_i8_w8s_supported(int(M), int(K), int(N)))
 
 
 def int8_strip_rows_supported(M, K, N):
     """Whether `int8_dense_strip` takes M rows, float32 or bfloat16, that a quantizer launch has
     quantised first: any K % 64 == 0 and any N while the rows fit a workgroup's LDS."""
-    return bool(_lib.load().k3q_gemm_i8_w8s_supported(int(M), int(K), int(N)))
+    return bool(_lib.calls().k3q_gemm_i8_w8s_supported(int(M), int(K), int(N)))
 
 
 def int8_strip_copy(kernel):
@@ -1042,14 +1042,14 @@ def int8_strip_copy(kernel):
     _lib.require_device(kernel)
     if kernel.dtype != torch.int8 or kernel.dim() != 2:
         raise ValueError(f"expected the stored int8 kernel [K, N], got {kernel.dtype} {tuple(kernel.shape)}")
-    lib = _lib.load()
+    lib = _lib.calls()
     K, N = (int(d) for d in kernel.shape)
     nbytes = lib.k3q_w8s_shadow_bytes(K, N)
     if nbytes <= 0:
         raise ValueError(f"no strip-linear copy for a [{K}, {N}] kernel (K % 64 != 0)")
     src = kernel if kernel.is_contiguous() else kernel.contiguous()
     out = torch.empty(nbytes, dtype=torch.uint8, device=src.device)
-    _lib.check(lib.k3q_w8s_pack(_lib.ptr(src), K, N, _lib.ptr(out), _lib.stream_ptr(src.device)), "k3q_w8s_pack")
+    _lib.check(lib.k3q_w8s_pack(_lib.addr(src), K, N, _lib.addr(out), _lib.raw_stream(src.device)), "k3q_w8s_pack")
     return out
 
 
@@ -1077,7 +1077,7 @@ def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, va
     Same bits as `abs_max_quantize` + `int8_matmul(..., exact_epilogue=True)`.
     Reference: keras/src/layers/core/dense.py:956-972."""
     _lib.require_device(x, shadow, kernel_scale, bias)
-    lib = _lib.load()
+    lib = _lib.calls()
     code = _lib.dtype_code(x.dtype)
     if kernel_scale.dtype != x.dtype:
         raise TypeError("kernel_scale must be read in the input's dtype")
@@ -1101,25 +1101,25 @@ def int8_dense_strip(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, va
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     if not inside and quantize is None:
         ws = _workspace(x.device, lib.k3q_dense_i8_workspace_bytes(code, M, K, N)) if M else None
-        rc = lib.k3q_dense_i8(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
-                              _lib.ptr(bias) if bias is not None else None, stride, float(epsilon), float(value_range[0]),
-                              float(value_range[1]), _lib.ptr(y), _lib.ptr(ws), ws.numel() if ws is not None else 0,
-                              _lib.stream_ptr(x.device))
+        rc = lib.k3q_dense_i8(_lib.addr(x2), code, M, K, N, _lib.addr(shadow), _lib.addr(ks),
+                              _lib.addr(bias) if bias is not None else None, stride, float(epsilon), float(value_range[0]),
+                              float(value_range[1]), _lib.addr(y), _lib.addr(ws), ws.numel() if ws is not None else 0,
+                              _lib.raw_stream(x.device))
         _lib.check(rc, "k3q_dense_i8")
         return _shaped(y, lead)
     if not inside:
         q, s = quantize(x2)
         if s.dtype != x.dtype:
             raise TypeError("the rows' scales must have the input's dtype")
-        rc = lib.k3q_gemm_i8_w8s(_lib.ptr(q), _lib.ptr(s), code, M, K, N, _lib.ptr(shadow),
-                                 _lib.ptr(ks), _lib.ptr(bias) if bias is not None else None, stride,
-                                 _lib.ptr(y), _lib.stream_ptr(x.device))
+        rc = lib.k3q_gemm_i8_w8s(_lib.addr(q), _lib.addr(s), code, M, K, N, _lib.addr(shadow),
+                                 _lib.addr(ks), _lib.addr(bias) if bias is not None else None, stride,
+                                 _lib.addr(y), _lib.raw_stream(x.device))
         _lib.check(rc, "k3q_gemm_i8_w8s")
         return _shaped(y, lead)
-    rc = lib.k3q_dense_i8_w8s(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks),
-                              _lib.ptr(bias) if bias is not None else None, stride, float(epsilon),
-                              float(value_range[0]), float(value_range[1]), _lib.ptr(y),
-                              _lib.stream_ptr(x.device))
+    rc = lib.k3q_dense_i8_w8s(_lib.addr(x2), code, M, K, N, _lib.addr(shadow), _lib.addr(ks),
+                              _lib.addr(bias) if bias is not None else None, stride, float(epsilon),
+                              float(value_range[0]), float(value_range[1]), _lib.addr(y),
+                              _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_dense_i8_w8s")
     return _shaped(y, lead)
 
@@ -1129,7 +1129,7 @@ def int8_dense_rows(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, val
     K % 64 == 0, bias of N values.  The bits of `abs_max_quantize` + `int8_matmul(..., strip=shadow, exact_epilogue=True)`.
     Reference: keras/src/layers/core/dense.py:956-972."""
     _lib.require_device(x, shadow, kernel_scale, bias)
-    lib = _lib.load()
+    lib = _lib.calls()
     code = _lib.dtype_code(x.dtype)
     K, N = int(x.shape[-1]), int(units)
     lead = x.shape[:-1]
@@ -1146,9 +1146,9 @@ def int8_dense_rows(x, shadow, units, kernel_scale, bias=None, epsilon=1e-7, val
              for t in (kernel_scale, bias))
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     ws = _workspace(x.device, lib.k3q_dense_i8_workspace_bytes(code, M, K, N)) if M else None
-    rc = lib.k3q_dense_i8(_lib.ptr(x2), code, M, K, N, _lib.ptr(shadow), _lib.ptr(ks), _lib.ptr(b), 0, float(epsilon),
-                          float(value_range[0]), float(value_range[1]), _lib.ptr(y), _lib.ptr(ws),
-                          ws.numel() if ws is not None else 0, _lib.stream_ptr(x.device))
+    rc = lib.k3q_dense_i8(_lib.addr(x2), code, M, K, N, _lib.addr(shadow), _lib.addr(ks), _lib.addr(b), 0, float(epsilon),
+                          float(value_range[0]), float(value_range[1]), _lib.addr(y), _lib.addr(ws),
+                          ws.numel() if ws is not None else 0, _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_dense_i8")
     return _shaped(y, lead)
 
@@ -1160,7 +1160,7 @@ def int8_dense_strip_multi(x, kernels, epsilon=1e-7, value_range=(-127, 127), qu
     bits as the separate calls.  kernels: dicts with `shadow`, `units`, `kernel_scale` and
     optionally `bias` [N] (bias_rows: [M, N]).  input_op: as in `int4_matmul_strip_multi`
     (`int8_strip_input_op_supported`)."""
-    lib = _lib.load()
+    lib = _lib.calls()
     K = int(x.shape[-1])
     lead = x.shape[:-1]
     x2 = x.reshape(-1, K)
@@ -1193,9 +1193,9 @@ def int8_dense_strip_multi(x, kernels, epsilon=1e-7, value_range=(-127, 127), qu
         if not int8_strip_quantises_inside(M, K, value_range):
             raise ValueError("input operations and per-row addends need rows the kernel quantises itself")
         pre, keep_op = _input_op_struct(input_op, M, K, x.device)
-        rc = lib.k3q_dense_i8_w8s_pre(_lib.ptr(x2), _lib.K3Q_BF16, M, K, ctypes.byref(pre) if pre is not None else None,
+        rc = lib.k3q_dense_i8_w8s_pre(_lib.addr(x2), _lib.K3Q_BF16, M, K, ctypes.byref(pre) if pre is not None else None,
                                       len(kernels), ctypes.byref(problems), float(epsilon), float(value_range[0]),
-                                      float(value_range[1]), 1 if bias_rows else 0, _lib.stream_ptr(x.device))
+                                      float(value_range[1]), 1 if bias_rows else 0, _lib.raw_stream(x.device))
         _lib.check(rc, "k3q_dense_i8_w8s_pre")
         del keep_op
         return [y.reshape(*lead, y.shape[1]) for y in outs]
@@ -1209,9 +1209,9 @@ def int8_dense_strip_multi(x, kernels, epsilon=1e-7, value_range=(-127, 127), qu
             q, s = quantize(x2)
         if s.dtype != torch.bfloat16:
             raise TypeError("the rows' scales must be bfloat16")
-    rc = lib.k3q_dense_i8_w8s_multi(_lib.ptr(x2), _lib.K3Q_BF16, _lib.ptr(q), _lib.ptr(s), M, K, len(kernels),
+    rc = lib.k3q_dense_i8_w8s_multi(_lib.addr(x2), _lib.K3Q_BF16, _lib.addr(q), _lib.addr(s), M, K, len(kernels),
                                     ctypes.byref(problems), float(epsilon), float(value_range[0]),
-                                    float(value_range[1]), _lib.stream_ptr(x.device))
+                                    float(value_range[1]), _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_dense_i8_w8s_multi")
     return [y.reshape(*lead, y.shape[1]) for y in outs]
 
@@ -1233,7 +1233,7 @@ def decode_attention(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_f
     that the caller reads when it synchronises anyway; without one the call checks a flag of its
     own, which costs a synchronisation)."""
     _lib.require_device(q, k, v, cos_table, sin_table, pos, cache_k, cache_v)
-    lib = _lib.load()
+    lib = _lib.calls()
     B, T, H, hd = q.shape
     if T != 1 or k.shape != q.shape or v.shape != q.shape:
         raise ValueError(f"decode_attention takes one position: q, k, v [B, 1, H, hd], got {tuple(q.shape)}")
@@ -1260,10 +1260,10 @@ def decode_attention(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_f
         _lib.require_device(oob_flag)
         if oob_flag.dtype != torch.int32 or oob_flag.numel() != 1:
             raise ValueError("oob_flag must be one int32 value on the device")
-    rc = lib.k3q_decode_attention(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.dtype_code(q.dtype), B, H, hd,
-                                  max_len, _lib.ptr(cos_table), _lib.ptr(sin_table), _lib.ptr(pos),
-                                  _lib.ptr(cache_k), _lib.ptr(cache_v), _lib.ptr(out), _lib.ptr(oob_flag),
-                                  _lib.stream_ptr(q.device))
+    rc = lib.k3q_decode_attention(_lib.addr(q), _lib.addr(k), _lib.addr(v), _lib.dtype_code(q.dtype), B, H, hd,
+                                  max_len, _lib.addr(cos_table), _lib.addr(sin_table), _lib.addr(pos),
+                                  _lib.addr(cache_k), _lib.addr(cache_v), _lib.addr(out), _lib.addr(oob_flag),
+                                  _lib.raw_stream(q.device))
     _lib.check(rc, "k3q_decode_attention")
     if own_flag and int(oob_flag.item()):
         raise IndexError(f"decode_attention: position {int(pos.item())} is outside the cache of {max_len} rows")
@@ -1302,10 +1302,10 @@ def rope_cache(q, k, v, cos_table, sin_table, pos, cache_k, cache_v, oob_flag=No
     q, k, v = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
                for t in (q, k, v))
     out = torch.empty_like(q)
-    rc = _lib.load().k3q_rope_cache(
-        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.dtype_code(q.dtype), B, T, H, hd, max_len, _lib.ptr(cos_table),
-        _lib.ptr(sin_table), _lib.ptr(pos), _lib.ptr(cache_k), _lib.ptr(cache_v), _lib.ptr(out), _lib.ptr(oob_flag),
-        _lib.stream_ptr(q.device))
+    rc = _lib.calls().k3q_rope_cache(
+        _lib.addr(q), _lib.addr(k), _lib.addr(v), _lib.dtype_code(q.dtype), B, T, H, hd, max_len, _lib.addr(cos_table),
+        _lib.addr(sin_table), _lib.addr(pos), _lib.addr(cache_k), _lib.addr(cache_v), _lib.addr(out), _lib.addr(oob_flag),
+        _lib.raw_stream(q.device))
     _lib.check(rc, "k3q_rope_cache")
     return out
 
@@ -1326,7 +1326,7 @@ def prompt_attention(q, cache_k, cache_v, mask):
     """`scaled_dot_product_attention(q.transpose(1, 2), cache_k, cache_v, attn_mask=mask[None, None]).transpose(1, 2)` for
     q `[B, T, H, 128]` and caches `[B, H, max_len, 128]` that `prompt_attention_supported`."""
     _lib.require_device(q, cache_k, cache_v, mask)
-    lib = _lib.load()
+    lib = _lib.calls()
     B, T, H, hd = q.shape
     max_len = cache_k.shape[2]
     if (tuple(cache_k.shape) != (B, H, max_len, hd) or cache_v.shape != cache_k.shape or tuple(mask.shape) != (T, max_len)):
@@ -1339,8 +1339,8 @@ def prompt_attention(q, cache_k, cache_v, mask):
         t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
         for t in (q, cache_k, cache_v, mask))
     out = torch.empty((B, T, H, hd), dtype=torch.bfloat16, device=q.device)
-    rc = lib.k3q_prompt_attention(_lib.ptr(q), _lib.dtype_code(q.dtype), B, T, H, hd, max_len, _lib.ptr(cache_k),
-                                  _lib.ptr(cache_v), _lib.ptr(mask), _lib.ptr(out), _lib.stream_ptr(q.device))
+    rc = lib.k3q_prompt_attention(_lib.addr(q), _lib.dtype_code(q.dtype), B, T, H, hd, max_len, _lib.addr(cache_k),
+                                  _lib.addr(cache_v), _lib.addr(mask), _lib.addr(out), _lib.raw_stream(q.device))
     _lib.check(rc, "k3q_prompt_attention")
     return out
 
@@ -1364,12 +1364,12 @@ def rmsnorm(x, weight, epsilon):
     """`rms_norm(x, weight, epsilon)` over the last axis, bfloat16, one short launch (the decoder
     harness's normalisation between the quantized layers)."""
     _lib.require_device(x, weight)
-    lib = _lib.load()
+    lib = _lib.calls()
     x2, rows, dim, xs = _rows_view(x)
     w = weight if weight.is_contiguous() else weight.contiguous()
     y = torch.empty((rows, dim), dtype=x.dtype, device=x.device)
-    rc = lib.k3q_rmsnorm(_lib.ptr(x2), _lib.ptr(w), _lib.dtype_code(x.dtype), rows, dim, xs, float(epsilon),
-                         _lib.ptr(y), dim, _lib.stream_ptr(x.device))
+    rc = lib.k3q_rmsnorm(_lib.addr(x2), _lib.addr(w), _lib.dtype_code(x.dtype), rows, dim, xs, float(epsilon),
+                         _lib.addr(y), dim, _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_rmsnorm")
     return y.reshape(x.shape)
 
@@ -1383,11 +1383,11 @@ def silu_mul(gate, up):
     """`silu(gate) * up`, bfloat16, one launch; the operands may be column slices of a wider
     tensor (rows given by a stride)."""
     _lib.require_device(gate, up)
-    lib = _lib.load()
+    lib = _lib.calls()
     g2, rows, dim, gs = _rows_view(gate)
     u2, _, _, us = _rows_view(up)
     y = torch.empty((rows, dim), dtype=gate.dtype, device=gate.device)
-    rc = lib.k3q_silu_mul(_lib.ptr(g2), _lib.ptr(u2), _lib.dtype_code(gate.dtype), rows, dim, gs, us,
-                          _lib.ptr(y), dim, _lib.stream_ptr(gate.device))
+    rc = lib.k3q_silu_mul(_lib.addr(g2), _lib.addr(u2), _lib.dtype_code(gate.dtype), rows, dim, gs, us,
+                          _lib.addr(y), dim, _lib.raw_stream(gate.device))
     _lib.check(rc, "k3q_silu_mul")
     return y.reshape(gate.shape)

@@ -119,11 +119,11 @@ def abs_max_quantize(
         x2 = x2.contiguous()
     q2 = torch.empty((rows, cols), dtype=torch.int8, device=x.device)
     s1 = torch.empty((rows, 1) if plain else (rows,), dtype=x.dtype, device=x.device)
-    lib = _lib.load()
+    lib = _lib.calls()
     rc = lib.k3q_absmax_quantize(
-        _lib.ptr(x2), code, rows, cols, x2.stride(0) if rows > 1 else cols,
+        _lib.addr(x2), code, rows, cols, x2.stride(0) if rows > 1 else cols,
         float(epsilon), float(value_range[0]), float(value_range[1]),
-        _lib.ptr(q2), _lib.ptr(s1), _lib.stream_ptr(x.device),
+        _lib.addr(q2), _lib.addr(s1), _lib.raw_stream(x.device),
     )
     _lib.check(rc, "k3q_absmax_quantize")
     if plain:
@@ -173,10 +173,10 @@ def _abs_max_quantize_numpy_bits(x, axis, value_range, epsilon):
     q = torch.empty(shape, dtype=torch.int8, device=x.device)
     s = torch.empty((outer * inner,), dtype=x.dtype, device=x.device)
     ws = torch.empty((outer * inner,), dtype=torch.int32, device=x.device)
-    rc = _lib.load().k3q_weight_absmax_quantize(
-        _lib.ptr(src), _lib.dtype_code(x.dtype), outer, R, inner, float(epsilon),
-        float(value_range[0]), float(value_range[1]), _lib.ptr(q), _lib.ptr(s), _lib.ptr(ws),
-        _lib.stream_ptr(x.device))
+    rc = _lib.calls().k3q_weight_absmax_quantize(
+        _lib.addr(src), _lib.dtype_code(x.dtype), outer, R, inner, float(epsilon),
+        float(value_range[0]), float(value_range[1]), _lib.addr(q), _lib.addr(s), _lib.addr(ws),
+        _lib.raw_stream(x.device))
     _lib.check(rc, "k3q_weight_absmax_quantize")
     if perm is not None:
         inv = [perm.index(i) for i in range(rank)]
@@ -275,10 +275,10 @@ def abs_max_quantize_grouped_with_zero_point(
         q = torch.empty((K, N), dtype=torch.int8, device=x.device)
         st = torch.empty((G, N), dtype=x.dtype, device=x.device)
         zt = torch.empty((G, N), dtype=torch.int8, device=x.device)
-        rc = _lib.load().k3q_weight_quantize_grouped(
-            _lib.ptr(x), _lib.dtype_code(x.dtype), K, N, int(block_size), float(epsilon),
-            float(value_range[0]), float(value_range[1]), _lib.ptr(q), _lib.ptr(st), _lib.ptr(zt),
-            _lib.stream_ptr(x.device))
+        rc = _lib.calls().k3q_weight_quantize_grouped(
+            _lib.addr(x), _lib.dtype_code(x.dtype), K, N, int(block_size), float(epsilon),
+            float(value_range[0]), float(value_range[1]), _lib.addr(q), _lib.addr(st), _lib.addr(zt),
+            _lib.raw_stream(x.device))
         _lib.check(rc, "k3q_weight_quantize_grouped")
         return q, st, zt
     device = inputs.device if isinstance(inputs, torch.Tensor) else None
@@ -322,9 +322,9 @@ def quantize_and_pack_grouped(inputs, block_size, device):
             packed = torch.empty((K, N // 2), dtype=torch.int8, device=x.device)
             st = torch.empty((math.ceil(K / block_size), N), dtype=x.dtype, device=x.device)
             zt = torch.empty(st.shape, dtype=torch.int8, device=x.device)
-            rc = _lib.load().k3q_weight_quantize_grouped_int4(
-                _lib.ptr(x), _lib.dtype_code(x.dtype), K, N, int(block_size), float(EPSILON), _lib.ptr(packed),
-                _lib.ptr(st), _lib.ptr(zt), _lib.stream_ptr(x.device))
+            rc = _lib.calls().k3q_weight_quantize_grouped_int4(
+                _lib.addr(x), _lib.dtype_code(x.dtype), K, N, int(block_size), float(EPSILON), _lib.addr(packed),
+                _lib.addr(st), _lib.addr(zt), _lib.raw_stream(x.device))
             _lib.check(rc, "k3q_weight_quantize_grouped_int4")
             return packed, st, zt
     q, st, zt = abs_max_quantize_grouped_with_zero_point(inputs, block_size=block_size, to_numpy=True)
@@ -375,8 +375,8 @@ def pack_int4(arr, axis=0, dtype="int8"):
     packed_shape = list(src.shape)
     packed_shape[axis] = (n + 1) // 2
     out = torch.empty(packed_shape, dtype=tdt, device=arr.device)
-    rc = _lib.load().k3q_pack_int4(
-        _lib.ptr(src), outer, n, inner, _lib.ptr(out), _lib.stream_ptr(arr.device)
+    rc = _lib.calls().k3q_pack_int4(
+        _lib.addr(src), outer, n, inner, _lib.addr(out), _lib.raw_stream(arr.device)
     )
     _lib.check(rc, "k3q_pack_int4")
     return out, tuple(packed_shape), n
@@ -405,9 +405,9 @@ def unpack_int4(packed, orig_len, axis=0, dtype="int8"):
     out_shape = list(src.shape)
     out_shape[axis] = orig_len
     out = torch.empty(out_shape, dtype=tdt, device=packed.device)
-    rc = _lib.load().k3q_unpack_int4(
-        _lib.ptr(src), outer, plen, inner, orig_len, 1 if dtype == "int8" else 0,
-        _lib.ptr(out), _lib.stream_ptr(packed.device),
+    rc = _lib.calls().k3q_unpack_int4(
+        _lib.addr(src), outer, plen, inner, orig_len, 1 if dtype == "int8" else 0,
+        _lib.addr(out), _lib.raw_stream(packed.device),
     )
     _lib.check(rc, "k3q_unpack_int4")
     return out
