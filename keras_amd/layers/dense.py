@@ -356,11 +356,12 @@ class Dense(Layer):
         self.kernel_scale = self.add_weight(name="kernel_scale", shape=scale_shape, initializer="ones")
         if block_size is not None and block_size > 0:
             self.kernel_zero = self.add_weight(name="kernel_zero", shape=scale_shape, dtype="int8")
-            # float32 on purpose, as in the reference (dense.py:868-889)
+            # float32 on purpose, as in the reference (dense.py:868-889); made where it stays: a copy from the host would
+            # wait for the quantizer that is running
             self.g_idx = self.add_weight(
                 name="g_idx", shape=(input_dim,), dtype="float32",
                 initializer=lambda shape, dtype: torch.floor_divide(
-                    torch.arange(input_dim, dtype=dtype), block_size),
+                    torch.arange(input_dim, dtype=dtype, device=self.device), block_size),
             )
         self._orig_input_dim = input_dim
         self._orig_output_dim = output_dim
@@ -378,7 +379,7 @@ class Dense(Layer):
             kernel_value, kernel_scale = weight_quantizer(as_tensor(self._kernel), to_numpy=True)
             kernel_scale = torch.squeeze(kernel_scale, dim=0)
             self._drop_float_kernel()
-            self.quantized_build(kernel_shape, mode, config)
+            self._quantized_build_with(kernel_shape, mode, config, kernel=kernel_value, kernel_scale=kernel_scale)
             self._kernel.assign(kernel_value)
             self.kernel_scale.assign(kernel_scale)
         elif mode == "int4":
@@ -396,7 +397,8 @@ class Dense(Layer):
                 packed, kernel_scale, kernel_zero = quantizers.quantize_and_pack_grouped(
                     as_tensor(self._kernel), block_size, self.device)
             self._drop_float_kernel()
-            self.quantized_build(kernel_shape, mode, config)
+            self._quantized_build_with(kernel_shape, mode, config, kernel=packed, kernel_scale=kernel_scale,
+                                       kernel_zero=kernel_zero)
             self._kernel.assign(packed)
             self.kernel_scale.assign(kernel_scale)
             if kernel_zero is not None:

@@ -465,7 +465,7 @@ class EinsumDense(Layer):
             self.g_idx = self.add_weight(
                 name="g_idx", shape=(rows,), dtype="float32",
                 initializer=lambda shape, dtype: torch.floor_divide(
-                    torch.arange(rows, dtype=dtype), block_size),
+                    torch.arange(rows, dtype=dtype, device=self.device), block_size),
             )
 
     # ---- quantize ---------------------------------------------------------------------
@@ -500,7 +500,8 @@ class EinsumDense(Layer):
             raise self._quantization_mode_error(mode)
         self._variables = [v for v in self._variables if v is not self._kernel]
         del self._kernel
-        self.quantized_build(kernel_shape, mode, config)
+        self._quantized_build_with(kernel_shape, mode, config, kernel=kernel_value, kernel_scale=kernel_scale,
+                                   kernel_zero=kernel_zero)
         self._kernel.assign(kernel_value)
         self.kernel_scale.assign(kernel_scale)
         if kernel_zero is not None:
