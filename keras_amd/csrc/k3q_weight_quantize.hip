@@ -15,6 +15,8 @@
 // first integer, and the kernel is larger than the chip's caches).  Groups of up to 128 rows keep
 // their rows in registers between the min / max and the integers (grouped_zp_held: one read); larger
 // groups take the generic two-pass kernel.
+#include <type_traits>
+
 #include "k3q_common.h"
 
 namespace k3q {
@@ -231,42 +233,47 @@ __device__ __forceinline__ void rint_quotients(const float (&x)[4], const float 
     }
 }
 
-// The same for groups of up to kHeldY * kHeldRows rows with N a multiple of 4.  A thread keeps its
-// rows in registers between the two passes, so memory sees x once (the groups resident on the chip
-// at one time are far larger than its caches, and the generic kernel's second read comes from
-// memory again); the integers come from rint_quotients.  A workgroup walks work items (column
-// tile, group) at a stride of the grid and asks for the next item's rows before it works on the
-// current one: with one item per workgroup the whole chip alternates between loading and computing
-// (the registers allow one or two workgroups per CU), and neither memory nor the vector units see
-// more than half of the time.
+// The same for groups of up to kHeldY * kHeldRows rows with N a multiple of 4.  A thread keeps its rows of a work item (column
+// tile, group) in registers between the two passes, so memory sees x once; the integers come from rint_quotients.  A
+// workgroup walks the items at a stride of the grid, and a row's registers take the next item's row as soon as the row's
+// integers are out: loads run through the whole of the vector work, and a workgroup holds the registers of one item only.
+// Every load of an item is unconditional, at a row and a column held inside x (what a repeated row holds is not used): with a
+// condition on each, the compiler waited for every load before the next.  4096 x 14336 float32 to int4, groups of 128:
+// 73.3 -> 51.8 us, where reading x and writing the result takes 52 at the rate of a large copy (8192 x 8192: 79.0 -> 57.9,
+// 1600 x 6400, whose last group is short: 22.1 -> 18.7).
+// kFull: every group has kHeldY * kHeldRows rows, all of them in x; no condition is left between the loads and stores, and 96
+// registers let two workgroups share a CU.  kPacked: the integers leave as int4 pairs along N (k3q_pack_int4's bytes; q is
+// [K, N / 2], the range fits four bits): half a byte written per weight instead of one byte written, read again and packed.
 constexpr int kHeldY = 8, kHeldRows = 16;
-// kPacked: the integers leave as int4 pairs along N (k3q_pack_int4's bytes; q is [K, N / 2], the range fits four bits):
-// half a byte written per weight instead of one byte written, read again and packed by a launch of its own.
-// 4096 x 14336 float32, call of the layer: 152 -> 130 us (the pack launch alone was 16, and its buffer went).  What bounds
-// the kernel: the read of x (235 MB) and, with eight waves on a CU, the vector work on it, which overlap only in part.
-template <bool kBF16, bool kPacked>
-__global__ __launch_bounds__(kWqX * kHeldY) void grouped_zp_held(GroupedParams p, int col_tiles, int items) {
+template <bool kFull, bool kBF16, bool kPacked>
+__global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(GroupedParams p, int col_tiles, int items) {
+    typedef typename std::conditional<kBF16, v2u, v4u>::type Raw;  // four values of a row as they lie in memory
     __shared__ float lo_s[2][kHeldY][kWqX * 4], hi_s[2][kHeldY][kWqX * 4];
-    const int tx = threadIdx.x % kWqX, ty = threadIdx.x / kWqX;
-    auto load_item = [&](const int item, float (&rows)[kHeldRows][4]) {
-        const int64_t g = item / col_tiles;
-        const int64_t col = ((int64_t)(item - g * col_tiles) * kWqX + tx) * 4;
-        const int64_t r0 = g * p.block;
+    const int tx = threadIdx.x % kWqX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / kWqX);
+    Raw rows[kHeldRows];
+    auto fetch = [&](const int item, const int j) {
+        const int g = item / col_tiles;
+        const int64_t col = ((int64_t)(item - g * col_tiles) * kWqX + tx) * 4, r0 = (int64_t)g * p.block;
+        const int i = ty + j * kHeldY;
+        int64_t r = r0 + (i < p.block ? i : p.block - 1);
+        r = r < p.K ? r : p.K - 1;
+        rows[j] = *(const Raw*)((const char*)p.x + (r * p.N + (col < p.N ? col : p.N - 4)) * (kBF16 ? 2 : 4));
+    };
+    auto values = [&](const int j, float (&f)[4]) {
+        if constexpr (kBF16) {
+            f[0] = __uint_as_float(rows[j][0] << 16);
+            f[1] = __uint_as_float(rows[j][0] & 0xffff0000u);
+            f[2] = __uint_as_float(rows[j][1] << 16);
+            f[3] = __uint_as_float(rows[j][1] & 0xffff0000u);
+        } else {
 #pragma unroll
-        for (int j = 0; j < kHeldRows; ++j) {
-            const int i = ty + j * kHeldY;
-            if (item < items && col < p.N && i < p.block && r0 + i < p.K) {
-                load_vals<kBF16, 4>(p.x, (r0 + i) * p.N + col, rows[j]);
-            } else {  // rows past K count as zeros; rows past the group do not count (skipped below)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) rows[j][e] = 0.f;
-            }
+            for (int e = 0; e < 4; ++e) f[e] = __uint_as_float(rows[j][e]);
         }
     };
-    auto work = [&](const int item, const int par, const float (&rows)[kHeldRows][4]) {
-        const int64_t g = item / col_tiles;
-        const int64_t col = ((int64_t)(item - g * col_tiles) * kWqX + tx) * 4;
-        const int64_t r0 = g * p.block;
+    auto work = [&](auto more, const int item, const int next, const int par) {
+        constexpr bool kMore = decltype(more)::value;  // (there is a next item)
+        const int g = item / col_tiles;
+        const int64_t col = ((int64_t)(item - g * col_tiles) * kWqX + tx) * 4, r0 = (int64_t)g * p.block;
         float lo[4], hi[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -274,21 +281,24 @@ __global__ __launch_bounds__(kWqX * kHeldY) void grouped_zp_held(GroupedParams p
             hi[e] = -INFINITY;
         }
 #pragma unroll
-        for (int j = 0; j < kHeldRows; ++j)
-            if (ty + j * kHeldY < p.block) {
+        for (int j = 0; j < kHeldRows; ++j) {
+            const int i = ty + j * kHeldY;
+            if (!kFull && i >= p.block) break;
+            float f[4];
+            values(j, f);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    lo[e] = fminf(lo[e], rows[j][e]);
-                    hi[e] = fmaxf(hi[e], rows[j][e]);
-                }
+            for (int e = 0; e < 4; ++e) {
+                const float v = kFull || r0 + i < p.K ? f[e] : 0.f;  // (rows past K count as zeros)
+                lo[e] = fminf(lo[e], v);
+                hi[e] = fmaxf(hi[e], v);
             }
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             lo_s[par][ty][tx * 4 + e] = lo[e];
             hi_s[par][ty][tx * 4 + e] = hi[e];
         }
         __syncthreads();  // (the buffers alternate, so the item after the next may overwrite this one's)
-        if (col >= p.N) return;
         float scale[4], inv[4], zero[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -302,7 +312,8 @@ __global__ __launch_bounds__(kWqX * kHeldY) void grouped_zp_held(GroupedParams p
             inv[e] = 1.0f / scale[e];
             zero[e] = fminf(fmaxf(rintf(-l / scale[e]) + p.qmin, p.qmin), p.qmax);
         }
-        if (ty == 0) {
+        const bool live = col < p.N;
+        if (ty == 0 && live) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 store_scale<kBF16>(p.scale, g * p.N + col + e, scale[e]);
@@ -312,33 +323,39 @@ __global__ __launch_bounds__(kWqX * kHeldY) void grouped_zp_held(GroupedParams p
 #pragma unroll
         for (int j = 0; j < kHeldRows; ++j) {
             const int i = ty + j * kHeldY;
-            if (i < p.block && r0 + i < p.K) {
-                float n[4];
+            if (kFull || (i < p.block && r0 + i < p.K)) {
+                float f[4], n[4];
                 int v[4];
-                rint_quotients(rows[j], scale, inv, n);
+                values(j, f);
+                rint_quotients(f, scale, inv, n);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = (int)__builtin_amdgcn_fmed3f(n[e] + zero[e], p.qmin, p.qmax);
-                if (kPacked)
-                    *(uint16_t*)(p.q + ((r0 + i) * p.N + col) / 2) =
-                        (uint16_t)((v[0] & 0xf) | ((v[1] & 0xf) << 4) | ((v[2] & 0xf) << 8) | ((v[3] & 0xf) << 12));
-                else
-                    store_q<4>(p.q, (r0 + i) * p.N + col, v);
+                if (live) {
+                    if (kPacked)
+                        *(uint16_t*)(p.q + ((r0 + i) * p.N + col) / 2) = (uint16_t)(
+                            (v[0] & 0xf) | ((v[1] & 0xf) << 4) | ((v[2] & 0xf) << 8) | ((v[3] & 0xf) << 12));
+                    else
+                        store_q<4>(p.q, (r0 + i) * p.N + col, v);
+                }
             }
+            if (kMore) fetch(next, j);
         }
     };
-    float a[kHeldRows][4], b[kHeldRows][4];
     const int step = gridDim.x;
     int item = blockIdx.x;
-    load_item(item, a);
-    while (item < items) {  // (uniform over the workgroup: every thread meets every barrier)
-        load_item(item + step, b);
-        work(item, 0, a);
-        item += step;
-        if (item >= items) break;
-        load_item(item + step, a);
-        work(item, 1, b);
-        item += step;
-    }
+#pragma unroll
+    for (int j = 0; j < kHeldRows; ++j) fetch(item, j);
+    int par = 0;
+#pragma clang loop unroll(disable)
+    for (; item + step < items; item += step, par ^= 1)  // (uniform over the workgroup: every thread meets every barrier)
+        work(std::true_type{}, item, item + step, par);
+    work(std::false_type{}, item, item, par);
+}
+
+template <bool kFull>
+void (*held_kernel(const bool bf, const bool packed))(GroupedParams, int, int) {
+    return bf ? (packed ? grouped_zp_held<kFull, true, true> : grouped_zp_held<kFull, true, false>)
+              : (packed ? grouped_zp_held<kFull, false, true> : grouped_zp_held<kFull, false, false>);
 }
 
 __global__ void clear_u32(u32* p, int64_t n) {
@@ -427,10 +444,12 @@ static int run_weight_quantize_grouped(const void* x, int x_dtype, int64_t K, in
     const int64_t col_tiles = grid.x, items = col_tiles * groups;
     const bool held = vec && block_size <= (int64_t)kHeldY * kHeldRows && epsilon > 0.f && items < (1ll << 30);
     if (held) {
-        const unsigned blocks = (unsigned)(items < 256 ? items : 256);  // one resident workgroup per CU
+        // two workgroups per CU where the registers allow it; 256, 768 and 1024 of them, and one per item, take 54.6, 56.6,
+        // 52.9 and 52.9 us where this takes 51.8 (4096 x 14336)
+        const unsigned blocks = (unsigned)(items < 512 ? items : 512);
+        const bool full = block_size == kHeldY * kHeldRows && K % block_size == 0;
         void (*kernel)(GroupedParams, int, int) =
-            bf ? (packed ? grouped_zp_held<true, true> : grouped_zp_held<true, false>)
-               : (packed ? grouped_zp_held<false, true> : grouped_zp_held<false, false>);
+            full ? held_kernel<true>(bf, packed) : held_kernel<false>(bf, packed);
         kernel<<<blocks, kWqX * kHeldY, 0, s>>>(p, (int)col_tiles, (int)items);
         return launch_status();
     }
