@@ -11,8 +11,15 @@
 // What makes the bits equal: every step is one IEEE float32 operation in numpy and here (compiled
 // with -ffp-contract=off, `/` is the correctly rounded division, rintf rounds half to even as
 // np.round does); bfloat16 inputs are widened first, as the reference's conversion to numpy does.
-// The abs-max form reads x from memory twice (a column's maximum needs all of the column before the
-// first integer, and the kernel is larger than the chip's caches).  Groups of up to 128 rows keep
+// The abs-max form reads x twice (a column's maximum needs all of the column before the first integer).
+// It is bound by memory where there are workgroups enough: a thread has kWqDeep rows in flight, and a
+// kernel that would make fewer than 1024 workgroups is cut into shorter chunks of rows -- down to 64, and
+// to 32 below 512 workgroups, since every chunk costs an atomic a column (6400 x 1600: 24 us in chunks of
+// 64, 30 of 32).  One row at a time in chunks of 256 -> now, float32 / bfloat16, us: 768 x 768 27 / 28 -> 8 / 8,
+// 1600 x 6400 46 / 45 -> 19 / 15, 4096 x 4096 45 / 52 -> 29 / 24, 4096 x 14336 111 / 84 -> 87 / 53, 8192 x 8192
+// 116 / 95 -> 113 / 59.  Pass 2 goes from the end of x to its start and stores past the caches (with ordinary stores
+// 4096 x 14336 takes 97).
+//  Groups of up to 128 rows keep
 // their rows in registers between the min / max and the integers (grouped_zp_held: one read); larger
 // groups take the generic two-pass kernel.
 #include <type_traits>
@@ -25,32 +32,47 @@ namespace {
 constexpr int kWqX = 64;   // threads along the columns
 constexpr int kWqY = 4;    // threads along the reduced rows
 constexpr int kWqT = kWqX * kWqY;
-constexpr int kWqChunk = 256;  // rows of R per workgroup in the abs-max passes
+constexpr int kWqDeep = 8;     // rows that a thread of the abs-max passes has in flight
+
+// kV values as they lie in memory, and as floats
+template <bool kBF16, int kV>
+struct RawVals {
+    typedef typename std::conditional<kBF16, v2u, v4u>::type Four;
+    typename std::conditional<kV == 4, Four, u32>::type raw;
+    __device__ __forceinline__ void load(const void* x, int64_t idx) {
+        if constexpr (kV == 4) raw = *(const Four*)((const char*)x + idx * (kBF16 ? 2 : 4));
+        else raw = load_raw<kBF16>(x, idx);
+    }
+    __device__ __forceinline__ void values(float* f) const {
+        if constexpr (kV != 4) {
+            f[0] = raw_to_f32<kBF16>(raw);
+        } else if constexpr (kBF16) {
+            f[0] = __uint_as_float(raw[0] << 16);
+            f[1] = __uint_as_float(raw[0] & 0xffff0000u);
+            f[2] = __uint_as_float(raw[1] << 16);
+            f[3] = __uint_as_float(raw[1] & 0xffff0000u);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[e] = __uint_as_float(raw[e]);
+        }
+    }
+};
 
 template <bool kBF16, int kV>
 __device__ __forceinline__ void load_vals(const void* x, int64_t idx, float* f) {
-    if (kV == 4) {
-        if (kBF16) {
-            const v2u c = *(const v2u*)((const uint16_t*)x + idx);
-            f[0] = __uint_as_float(c[0] << 16);
-            f[1] = __uint_as_float(c[0] & 0xffff0000u);
-            f[2] = __uint_as_float(c[1] << 16);
-            f[3] = __uint_as_float(c[1] & 0xffff0000u);
-        } else {
-            const v4u c = *(const v4u*)((const u32*)x + idx);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f[e] = __uint_as_float(c[e]);
-        }
-    } else {
-        f[0] = raw_to_f32<kBF16>(load_raw<kBF16>(x, idx));
-    }
+    RawVals<kBF16, kV> v;
+    v.load(x, idx);
+    v.values(f);
 }
 
-template <int kV>
+// kStream: past the caches, which keep more of the input then
+template <int kV, bool kStream = false>
 __device__ __forceinline__ void store_q(int8_t* q, int64_t idx, const int* v) {
     if (kV == 4) {
-        *(u32*)(q + idx) = (u32)(v[0] & 0xff) | ((u32)(v[1] & 0xff) << 8) | ((u32)(v[2] & 0xff) << 16) |
-                           ((u32)(v[3] & 0xff) << 24);
+        const u32 w = (u32)(v[0] & 0xff) | ((u32)(v[1] & 0xff) << 8) | ((u32)(v[2] & 0xff) << 16) |
+                      ((u32)(v[3] & 0xff) << 24);
+        if (kStream) __builtin_nontemporal_store(w, (u32*)(q + idx));
+        else *(u32*)(q + idx) = w;
     } else {
         q[idx] = (int8_t)v[0];
     }
@@ -68,6 +90,7 @@ struct ReduceParams {
     void* scale;
     u32* amax;  // [outer * inner] bit patterns of the running max of |x| (zeroed by the entry point)
     int64_t R, inner;
+    int chunk;  // rows of R per workgroup
     float eps, qlo, qhi;
 };
 
@@ -79,17 +102,24 @@ __global__ __launch_bounds__(kWqT) void absmax_reduce_max(ReduceParams p) {
     const int tx = threadIdx.x % kWqX, ty = threadIdx.x / kWqX;
     const int64_t col = ((int64_t)blockIdx.x * kWqX + tx) * kV;
     const int64_t o = blockIdx.z;
-    const int64_t r0 = (int64_t)blockIdx.y * kWqChunk;
-    const int64_t r1 = r0 + kWqChunk < p.R ? r0 + kWqChunk : p.R;
+    const int64_t r0 = (int64_t)blockIdx.y * p.chunk;
+    const int64_t r1 = r0 + p.chunk < p.R ? r0 + p.chunk : p.R;
     float m[kV];
 #pragma unroll
     for (int e = 0; e < kV; ++e) m[e] = 0.f;
     if (col < p.inner) {
-        for (int64_t r = r0 + ty; r < r1; r += kWqY) {
-            float f[kV];
-            load_vals<kBF16, kV>(p.x, (o * p.R + r) * p.inner + col, f);
+        for (int64_t r = r0 + ty; r < r1; r += kWqY * kWqDeep) {
+            RawVals<kBF16, kV> raw[kWqDeep];  // (a row past the chunk's last counts as that one again)
 #pragma unroll
-            for (int e = 0; e < kV; ++e) m[e] = fmaxf(m[e], fabsf(f[e]));
+            for (int j = 0; j < kWqDeep; ++j)
+                raw[j].load(p.x, (o * p.R + (r + j * kWqY < r1 ? r + j * kWqY : r1 - 1)) * p.inner + col);
+#pragma unroll
+            for (int j = 0; j < kWqDeep; ++j) {
+                float f[kV];
+                raw[j].values(f);
+#pragma unroll
+                for (int e = 0; e < kV; ++e) m[e] = fmaxf(m[e], fabsf(f[e]));
+            }
         }
     }
 #pragma unroll
@@ -106,15 +136,16 @@ __global__ __launch_bounds__(kWqT) void absmax_reduce_max(ReduceParams p) {
     }
 }
 
-// pass 2: scale = hi / (amax + eps), q = clip(rint(x * scale))
+// pass 2: scale = hi / (amax + eps), q = clip(rint(x * scale)); from the end of x to its start, so that what pass 1 read last
+// comes out of the caches
 template <bool kBF16, int kV>
 __global__ __launch_bounds__(kWqT) void absmax_reduce_quantize(ReduceParams p) {
     const int tx = threadIdx.x % kWqX, ty = threadIdx.x / kWqX;
-    const int64_t col = ((int64_t)blockIdx.x * kWqX + tx) * kV;
+    const int64_t col = ((int64_t)(gridDim.x - 1 - blockIdx.x) * kWqX + tx) * kV;
     if (col >= p.inner) return;
-    const int64_t o = blockIdx.z;
-    const int64_t r0 = (int64_t)blockIdx.y * kWqChunk;
-    const int64_t r1 = r0 + kWqChunk < p.R ? r0 + kWqChunk : p.R;
+    const int64_t o = gridDim.z - 1 - blockIdx.z;
+    const int64_t r0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * p.chunk;
+    const int64_t r1 = r0 + p.chunk < p.R ? r0 + p.chunk : p.R;
     float s[kV];
 #pragma unroll
     for (int e = 0; e < kV; ++e) s[e] = p.qhi / (__uint_as_float(p.amax[o * p.inner + col + e]) + p.eps);
@@ -122,14 +153,21 @@ __global__ __launch_bounds__(kWqT) void absmax_reduce_quantize(ReduceParams p) {
 #pragma unroll
         for (int e = 0; e < kV; ++e) store_scale<kBF16>(p.scale, o * p.inner + col + e, s[e]);
     }
-    for (int64_t r = r0 + ty; r < r1; r += kWqY) {
-        const int64_t idx = (o * p.R + r) * p.inner + col;
-        float f[kV];
-        load_vals<kBF16, kV>(p.x, idx, f);
-        int v[kV];
+    for (int64_t r = r0 + ty; r < r1; r += kWqY * kWqDeep) {
+        RawVals<kBF16, kV> raw[kWqDeep];
 #pragma unroll
-        for (int e = 0; e < kV; ++e) v[e] = (int)fminf(fmaxf(rintf(f[e] * s[e]), p.qlo), p.qhi);
-        store_q<kV>(p.q, idx, v);
+        for (int j = 0; j < kWqDeep; ++j)
+            raw[j].load(p.x, (o * p.R + (r + j * kWqY < r1 ? r + j * kWqY : r1 - 1)) * p.inner + col);
+#pragma unroll
+        for (int j = 0; j < kWqDeep; ++j) {
+            if (r + j * kWqY >= r1) break;
+            float f[kV];
+            int v[kV];
+            raw[j].values(f);
+#pragma unroll
+            for (int e = 0; e < kV; ++e) v[e] = (int)fminf(fmaxf(rintf(f[e] * s[e]), p.qlo), p.qhi);
+            store_q<kV, true>(p.q, (o * p.R + r + j * kWqY) * p.inner + col, v);
+        }
     }
 }
 
@@ -247,28 +285,16 @@ __device__ __forceinline__ void rint_quotients(const float (&x)[4], const float 
 constexpr int kHeldY = 8, kHeldRows = 16;
 template <bool kFull, bool kBF16, bool kPacked>
 __global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(GroupedParams p, int col_tiles, int items) {
-    typedef typename std::conditional<kBF16, v2u, v4u>::type Raw;  // four values of a row as they lie in memory
     __shared__ float lo_s[2][kHeldY][kWqX * 4], hi_s[2][kHeldY][kWqX * 4];
     const int tx = threadIdx.x % kWqX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / kWqX);
-    Raw rows[kHeldRows];
+    RawVals<kBF16, 4> rows[kHeldRows];
     auto fetch = [&](const int item, const int j) {
         const int g = item / col_tiles;
         const int64_t col = ((int64_t)(item - g * col_tiles) * kWqX + tx) * 4, r0 = (int64_t)g * p.block;
         const int i = ty + j * kHeldY;
         int64_t r = r0 + (i < p.block ? i : p.block - 1);
         r = r < p.K ? r : p.K - 1;
-        rows[j] = *(const Raw*)((const char*)p.x + (r * p.N + (col < p.N ? col : p.N - 4)) * (kBF16 ? 2 : 4));
-    };
-    auto values = [&](const int j, float (&f)[4]) {
-        if constexpr (kBF16) {
-            f[0] = __uint_as_float(rows[j][0] << 16);
-            f[1] = __uint_as_float(rows[j][0] & 0xffff0000u);
-            f[2] = __uint_as_float(rows[j][1] << 16);
-            f[3] = __uint_as_float(rows[j][1] & 0xffff0000u);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f[e] = __uint_as_float(rows[j][e]);
-        }
+        rows[j].load(p.x, r * p.N + (col < p.N ? col : p.N - 4));
     };
     auto work = [&](auto more, const int item, const int next, const int par) {
         constexpr bool kMore = decltype(more)::value;  // (there is a next item)
@@ -285,7 +311,7 @@ __global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(
             const int i = ty + j * kHeldY;
             if (!kFull && i >= p.block) break;
             float f[4];
-            values(j, f);
+            rows[j].values(f);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float v = kFull || r0 + i < p.K ? f[e] : 0.f;  // (rows past K count as zeros)
@@ -326,7 +352,7 @@ __global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(
             if (kFull || (i < p.block && r0 + i < p.K)) {
                 float f[4], n[4];
                 int v[4];
-                values(j, f);
+                rows[j].values(f);
                 rint_quotients(f, scale, inv, n);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = (int)__builtin_amdgcn_fmed3f(n[e] + zero[e], p.qmin, p.qmax);
@@ -377,8 +403,7 @@ extern "C" int k3q_weight_absmax_quantize(const void* x, int x_dtype, int64_t ou
     if (outer == 0 || inner == 0) return K3Q_OK;
     if (R == 0) return K3Q_ERR_SHAPE;  // the maximum of nothing
     if (!x || !q || !scale || !amax_workspace) return K3Q_ERR_NULL;
-    const int64_t chunks = (R + kWqChunk - 1) / kWqChunk;
-    if (chunks > 65535) return K3Q_ERR_SHAPE;
+    if ((R + 255) / 256 > 65535) return K3Q_ERR_SHAPE;
     hipStream_t s = (hipStream_t)stream;
     ReduceParams p;
     p.x = x;
@@ -395,7 +420,11 @@ extern "C" int k3q_weight_absmax_quantize(const void* x, int x_dtype, int64_t ou
     const bool bf = x_dtype == K3Q_BF16;
     const bool vec = (inner % 4) == 0 && aligned_to(x, bf ? 8 : 16) && aligned_to(q, 4);
     const int v = vec ? 4 : 1;
-    dim3 grid((unsigned)((inner + (int64_t)kWqX * v - 1) / ((int64_t)kWqX * v)), (unsigned)chunks, (unsigned)outer);
+    const int64_t col_tiles = (inner + (int64_t)kWqX * v - 1) / ((int64_t)kWqX * v);
+    p.chunk = 256;  // (the reasons stand at the top)
+    const int64_t across = col_tiles * outer;
+    while (p.chunk > 32 && across * ((R + p.chunk - 1) / p.chunk) < (p.chunk > 64 ? 1024 : 512)) p.chunk /= 2;
+    dim3 grid((unsigned)col_tiles, (unsigned)((R + p.chunk - 1) / p.chunk), (unsigned)outer);
     if (bf && vec) {
         absmax_reduce_max<true, 4><<<grid, kWqT, 0, s>>>(p);
         absmax_reduce_quantize<true, 4><<<grid, kWqT, 0, s>>>(p);
