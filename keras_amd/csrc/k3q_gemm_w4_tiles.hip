@@ -16,7 +16,7 @@
 // What bounds it: at 512 rows and more the matrix cores (128 x 256 tiles: 1.23 PFLOP/s in the loop, the library's large
 // products on this card 1.26), below that the starts of ring and launch and the rate of the requests (64 x 128: 39 bytes a ns
 // and CU).  Graph nodes, groups of 128, us, before -> now: 32 rows of 4096 x 14336 22.4 -> 19.0, 96 34.9 -> 29.0, 512 89.3 ->
-// 72.7; 128 rows of 4096 x 4096 24.3 -> 18.5, 512 40.6 -> 30.5; 128 of 14336 x 4096 37.9 -> 32.5; 256 of 8192 x 8192 58.9 ->
+// 72.7; 128 rows of 4096 x 4096 24.3 -> 18.5, 512 40.6 -> 28.9; 128 of 14336 x 4096 37.9 -> 32.5; 256 of 8192 x 8192 58.9 ->
 // 51.7.  Tried and slower: the sums of x in this kernel, from the rows in LDS (saves 2.8 us of launch, costs 0.1 us a round: 512
 // rows of 4096 x 14336 76.9); a block's four products in turn instead of a step's four blocks (80.9, the sums depend on each
 // other); an explicit wait for a step's operands ahead of the next reads (no gain).
