@@ -69,6 +69,15 @@ def apply_rope(x, cos, sin):
     return x * cos[None, :, None, :] + swapped * sin[None, :, None, :]
 
 
+def quantises_rows(layer):
+    """Whether a layer quantises the rows it multiplies (a grouped int4 `Dense` or `EinsumDense` ignores its activation
+    quantizer)."""
+    if not getattr(layer, "inputs_quantizer", None):
+        return False
+    grouped = (getattr(layer, "_int4_block_size", None) or -1) > 0
+    return not (isinstance(layer, (Dense, EinsumDense)) and layer.quantization_mode == "int4" and grouped)
+
+
 class DecoderBlock(Layer):
     def __init__(self, d_model, n_heads, ffn_dim, dtype=None, layer_dtype=None, name=None,
                  device=None, init=None):
@@ -95,12 +104,16 @@ class DecoderBlock(Layer):
         self.down.build((None, ffn_dim))
         self.built = True
 
-    def forward(self, x, rows, cache, pos, tables=None, oob_flag=None):
+    def forward(self, x, rows, cache, pos, tables=None, oob_flag=None, prompt_kernel=None):
         """x [B, T, D].  cache: (k, v) each [B, H, maxT, hd], written at positions `pos`
         (an int64 device tensor [T]); rows(): (cos, sin, mask) of these positions -- the table
         rows and mask [T, maxT], 0 where a key may be attended to, -inf elsewhere -- asked for
         only by the torch path; tables: the whole (cos, sin) tables, for the one-position kernel;
-        oob_flag: the int32 device flag that kernel raises for a position outside the cache."""
+        oob_flag: the int32 device flag that kernel raises for a position outside the cache;
+        prompt_kernel: whether the prompt's attention may run on `ops.prompt_attention` (None: where no layer of the
+        block quantises its rows).  Its results are bfloat16 ulps from the library's, and an ulp moves quantised rows by a
+        step: the logits of two correct int8 decoders lie 4 ... 5 % apart (2-norm), those of int4 ones 1 %.  Layers that
+        quantise keep the library's attention, and with it their results."""
         # The normalisations and the gate are handed to the projections that consume them as their
         # `input_op`: at one position they ride inside the projections' launches, in front of int8
         # layers they share a launch with the activation quantizer, otherwise they run as their own
@@ -126,7 +139,10 @@ class DecoderBlock(Layer):
                 q, k = qk[:, :, : self.n_heads], qk[:, :, self.n_heads:]
                 kc.index_copy_(2, pos, k.transpose(1, 2))
                 vc.index_copy_(2, pos, v.transpose(1, 2))
-            if kops.prompt_attention_supported(q, kc, vc, mask):
+            if prompt_kernel is None:
+                prompt_kernel = not any(quantises_rows(layer) for layer in (
+                    self.query, self.key, self.value, self.attn_out, self.gate, self.up, self.down))
+            if prompt_kernel and kops.prompt_attention_supported(q, kc, vc, mask):
                 a = kops.prompt_attention(q, kc, vc, mask)
             else:
                 a = torch.nn.functional.scaled_dot_product_attention(
@@ -253,8 +269,11 @@ class LlamaStyleDecoder(Model):
                 made.append((cos, sin, mask))
             return made[0]
 
+        # (one layer that quantises its rows, and every block before it keeps the library's attention)
+        prompt_kernel = ids.shape[1] > 1 and not any(quantises_rows(layer) for layer in self._flatten_layers())
         for block, kv in zip(self.blocks, cache):
-            x = block.forward(x, rows, kv, pos, tables=(self.cos, self.sin), oob_flag=self._pos_oob)
+            x = block.forward(x, rows, kv, pos, tables=(self.cos, self.sin), oob_flag=self._pos_oob,
+                              prompt_kernel=prompt_kernel)
         if last_only:
             x = x[:, -1:, :]
         return self.token_embedding(self.final_norm(x), reverse=True)

@@ -1,0 +1,64 @@
+"""GPU: which attention a decoder's prompt takes.  Layers that quantise their rows keep the library's, bit for bit."""
+
+import warnings
+
+import pytest
+import torch
+
+from keras_amd import ops as kops
+from keras_amd.decoder_harness import LlamaStyleDecoder
+
+pytestmark = pytest.mark.gpu
+
+CFG = dict(vocab=300, d_model=256, n_heads=2, ffn_dim=384, n_layers=2, max_len=64, init_on_device=True)
+
+
+def forward(model, ids):
+    cache = model.new_cache(ids.shape[0])
+    T = ids.shape[1]
+    prompt = model.forward(ids, torch.arange(T, device="cuda"), cache)
+    return prompt, model.forward(ids[:, :1], torch.full((1,), T, dtype=torch.int64, device="cuda"), cache)
+
+
+@pytest.mark.parametrize("first,rest,kernel", [
+    ("int8", "int8", False), ("int4", "int4", True), (None, None, True), ("int4", "int8", False), (None, "int8", False),
+])
+def test_prompt_attention_route(dev, monkeypatch, first, rest, kernel):
+    """first: what the first block's layers are quantized to, rest: all others."""
+    model = LlamaStyleDecoder(dtype="bfloat16", device="cuda:0", seed=5, **CFG)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        if first:
+            model.quantize(first, filters=lambda layer: layer.name.startswith("block0"))
+        if rest:
+            model.quantize(rest, filters=lambda layer: not layer.name.startswith("block0"))
+    ids = torch.randint(0, CFG["vocab"], (2, 21), generator=torch.Generator().manual_seed(2)).to(dev)
+    calls, real = [], kops.prompt_attention
+    monkeypatch.setattr(kops, "prompt_attention", lambda *a: (calls.append(1), real(*a))[1])
+    with torch.no_grad():
+        got = forward(model, ids)
+        assert len(calls) == (CFG["n_layers"] if kernel else 0)
+        monkeypatch.setattr(kops, "prompt_attention_supported", lambda *a: False)
+        library = forward(model, ids)
+    if not kernel:
+        assert all(torch.equal(a, b) for a, b in zip(got, library))
+    else:
+        assert all(float((a - b).float().norm() / b.float().norm()) < 3e-2 for a, b in zip(got, library))
+
+
+def test_block_alone(dev, monkeypatch):
+    """A block that a program calls by itself decides by its own layers."""
+    calls, real = [], kops.prompt_attention
+    monkeypatch.setattr(kops, "prompt_attention", lambda *a: (calls.append(1), real(*a))[1])
+    for mode, count in (("int4", 1), ("int8", 0)):
+        model = LlamaStyleDecoder(dtype="bfloat16", device="cuda:0", seed=5, **CFG)
+        with warnings.catch_warnings():
+            warnings.simplefilter("ignore")
+            model.quantize(mode, filters=lambda layer: layer.name.startswith("block0"))
+        mask = torch.zeros(9, 64, dtype=torch.bfloat16, device=dev).masked_fill_(
+            torch.arange(64, device=dev)[None] > torch.arange(9, device=dev)[:, None], float("-inf"))
+        del calls[:]
+        with torch.no_grad():
+            model.blocks[0].forward(torch.randn(1, 9, 256, device=dev).to(torch.bfloat16), lambda: (model.cos[:9], model.sin[:9], mask),
+                                    model.new_cache(1)[0], torch.arange(9, device=dev), tables=(model.cos, model.sin))
+        assert len(calls) == count
