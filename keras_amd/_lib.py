@@ -171,6 +171,7 @@ SIGNATURES = {
 TEST_SIGNATURES = {
     "k3qt_gemm_deep_tile": (_int, [_i64, _i64, _i64, _int]),
     "k3qt_w4_tile_plan": (_int, [_i64, _int, _i64, _i64, _ptr]),
+    "k3qt_w4_rows_launch": (_int, [_int, _i64, _i64, _i64, _i64, _i64, _ptr]),
     "k3qt_gemv_w4_plan": (
         _int,
         [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64,

@@ -13,7 +13,8 @@ struct W4TilePlan {
     int mb;      // blocks of 32 rows per tile: 1, 2 or 4
     int bn;      // columns per tile: 128 (K in two slices), or 256 with mb = 4
     int ks;      // workgroups that share K
-    int steps;   // 256 / bn units of K at a time: steps per split
+    int steps;   // of a workgroup, each kq() units of K: ks and steps cover K with this plan's own bn only
+    int kq() const { return 256 / bn; }
 };
 
 struct W4TileCall {

@@ -494,7 +494,7 @@ W4TilePlan w4_tile_plan(int64_t rows, int parts, int64_t K, int64_t N) {
     for (const Shape& sh : shapes) {
         if (parts == 2 && sh.mb == 1) continue;  // (both parts of a row in one tile)
         const int64_t tiles = ((xrows + 32 * sh.mb - 1) / (32 * sh.mb)) * ((N + sh.bn - 1) / sh.bn);
-        const int kq = 256 / sh.bn;
+        const int kq = W4TilePlan{sh.mb, sh.bn, 1, 1}.kq();
         const int64_t all = (units + kq - 1) / kq;
         for (int64_t want = 1; want <= 8; ++want) {
             const int64_t steps = (all + want - 1) / want;
@@ -541,7 +541,9 @@ int w4_tile_launch(const W4TileCall& c, const W4TilePlan& pl, hipStream_t s) {
     p.direct = w4_tile_direct(pl, c.parts) ? 1 : 0;
     p.wide = c.n_out % 4 == 0 && aligned_to(c.y, c.f32 ? 16 : 8) ? 1 : 0;
     const int64_t total = (int64_t)p.m_tiles * p.n_tiles * p.splits;
-    if (total > (1 << 28) || !w4_tile_fits(c.rows, c.parts, c.K, c.N)) return K3Q_ERR_SHAPE;
+    // (a plan that leaves a part of K out is not launched)
+    if (total > (1 << 28) || !w4_tile_fits(c.rows, c.parts, c.K, c.N) || (int64_t)pl.ks * pl.steps * pl.kq() < p.units)
+        return K3Q_ERR_SHAPE;
     int lds = 0;
     const TileKernel k = c.grouped ? (c.f32 ? pick_form<true, true>(c.form, pl, &lds) : pick_form<true, false>(c.form, pl, &lds))
                                    : (c.f32 ? pick_form<false, true>(c.form, pl, &lds) : pick_form<false, false>(c.form, pl, &lds));

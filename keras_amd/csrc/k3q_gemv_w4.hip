@@ -1971,6 +1971,13 @@ struct KmRowsPlan {
     bool plain;     // the weights without an offset
     int64_t Kp, Np, rows, sx_bytes, x_bytes, part_bytes;
     W4TilePlan tiles;   // of a launch of `rows` rows
+    W4TilePlan rest;    // of the launch of the remaining M % rows rows, if there are any
+    const W4TilePlan& tiles_of(int64_t launch_rows) const { return launch_rows == rows ? tiles : rest; }
+    // partial sums of a launch
+    int64_t partials(int64_t launch_rows) const {
+        const W4TilePlan& t = tiles_of(launch_rows);
+        return w4_tile_direct(t, parts) ? 0 : (int64_t)t.ks * launch_rows * parts * Np * 4;
+    }
 };
 
 // Rows go in launches of 1024 bfloat16 rows at most: the partials of one stay in the memory-side cache.
@@ -1992,11 +1999,28 @@ bool km_rows_plan(KmRowsPlan& pl, int x_dtype, int64_t M, int64_t K, int64_t N, 
     pl.tiles = w4_tile_plan(pl.rows, pl.parts, pl.Kp, pl.Np);
     pl.x_bytes = mx * pl.Kp * 2;  // (a multiple of 256)
     pl.sx_bytes = (pl.Kp / 128 * mx * 8 + 255) / 256 * 256;
-    pl.part_bytes = w4_tile_direct(pl.tiles, pl.parts) ? 0 : (int64_t)pl.tiles.ks * mx * pl.Np * 4;
+    pl.part_bytes = pl.partials(pl.rows);
+    // (fewer rows may want another tile and more splits: room for both)
+    if (const int64_t rest = M % pl.rows) {
+        pl.rest = w4_tile_plan(rest, pl.parts, pl.Kp, pl.Np);
+        if (pl.partials(rest) > pl.part_bytes) pl.part_bytes = pl.partials(rest);
+    }
     return true;
 }
 }  // namespace
 }  // namespace k3q
+
+extern "C" int k3qt_w4_rows_launch(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int64_t m0,
+                                   int64_t* launch) {
+    KmRowsPlan pl;
+    if ((x_dtype != K3Q_F32 && x_dtype != K3Q_BF16) || !launch) return K3Q_ERR_DTYPE;
+    if (!km_rows_plan(pl, x_dtype, M, K, N, block_size) || m0 < 0 || m0 >= M || m0 % pl.rows) return K3Q_ERR_SHAPE;
+    const int64_t rows = M - m0 < pl.rows ? M - m0 : pl.rows;
+    const W4TilePlan& t = pl.tiles_of(rows);
+    const int64_t values[7] = {rows, t.mb, t.bn, t.ks, t.steps, pl.partials(rows), pl.part_bytes};
+    for (int i = 0; i < 7; ++i) launch[i] = values[i];
+    return K3Q_OK;
+}
 
 extern "C" int64_t k3q_gemm_w4_rows_workspace_bytes(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size) {
     KmRowsPlan pl;
@@ -2046,12 +2070,7 @@ extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K
         c.rows = rows;
         c.y = (char*)y + m0 * N * el;
         c.bias = bias ? (const char*)bias + m0 * bias_stride * el : nullptr;
-        W4TilePlan tiles = rows == pl.rows ? pl.tiles : w4_tile_plan(rows, pl.parts, pl.Kp, pl.Np);
-        if (!w4_tile_direct(tiles, pl.parts) && (int64_t)tiles.ks * rows * pl.parts * pl.Np * 4 > pl.part_bytes) {
-            // fewer rows would split further than there is room
-            tiles.ks = pl.tiles.ks;
-            tiles.steps = pl.tiles.steps;
-        }
+        const W4TilePlan& tiles = pl.tiles_of(rows);
         v2u* sx = (v2u*)((char*)workspace + pl.x_bytes);
         if (as_is) {
             c.x = (const uint16_t*)xm;

@@ -33,6 +33,10 @@ int k3qt_gemm_deep_tile(int64_t M, int64_t N, int64_t row_bytes, int cus);
  * per tile, columns per tile, workgroups that share K, steps of K per split}. */
 int k3qt_w4_tile_plan(int64_t rows, int parts, int64_t K, int64_t N, int* plan);
 
+/* The launch of k3q_gemm_w4_rows that starts at row m0 (host only): launch = {rows, blocks of 32 rows per tile, columns per
+ * tile, workgroups that share K, steps of K per split, bytes of its partial sums, bytes of room for them}. */
+int k3qt_w4_rows_launch(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int64_t m0, int64_t* launch);
+
 #ifdef __cplusplus
 }
 #endif
