@@ -629,6 +629,7 @@ int k3q_rope_cache(const void* q, const void* k, const void* v, int dtype, int64
  * out [B, T, H, 128] = softmax(q k^T / sqrt(128) + mask) v with an additive bfloat16 mask [T, max_len], as
  * scaled_dot_product_attention computes it; max_len % 4 == 0.  Scores, probabilities and sums are float32 (a probability
  * enters its product as two bfloat16 parts).  Blocks of 64 cache rows that the mask closes (-inf) for 64 positions are not read.
+ * A position that sees no row gets zeros; infinite values and NaN in rows that are read go the way of float arithmetic.
  * The decoder harness's prompt; no counterpart in the reference's quantized layers.
  */
 int k3q_prompt_attention(const void* q, int dtype, int64_t B, int64_t T, int64_t H, int64_t head_dim,

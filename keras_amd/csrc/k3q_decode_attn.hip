@@ -325,27 +325,17 @@ struct PromptParams {
     float scale;
 };
 
-__global__ __launch_bounds__(256) void prompt_attention(PromptParams p) {
-    __shared__ __attribute__((aligned(16))) char ks[kPKeys * kPKPitch];
-    __shared__ __attribute__((aligned(16))) char vs[kHd * kPVPitch];
-    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t bh = blockIdx.x;
-    const int64_t b = bh / p.H;
-    const int h = (int)(bh - b * p.H);
-    const int t0 = (int)blockIdx.y * kPRows + wave * 16;
-    const int t = t0 + i < p.T ? t0 + i : p.T - 1;  // this lane's position (past the end: a copy of the last, not stored)
-    const int64_t qrow = ((b * p.T + t) * p.H + h) * kHd;
-    v4u qf[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) qf[s] = *(const v4u*)(p.q + qrow + 32 * s + 8 * g);
-    const uint16_t* mrow = p.mask + (int64_t)t * p.max_len;
-    const uint16_t* kb = p.kc + bh * p.max_len * kHd;
-    const uint16_t* vb = p.vc + bh * p.max_len * kHd;
-    v4f o[8];
+// The walk over the cache: this lane's sums o (columns 16 d + 4 g + e of its position) and its keys' share l of the
+// probabilities.  kTwo: a probability as two parts; one: where a value is no number.
+template <bool kTwo>
+__device__ __forceinline__ void prompt_walk(const PromptParams& p, char* ks, char* vs, const int tid, const v4u (&qf)[4],
+                                            const uint16_t* mrow, const uint16_t* kb, const uint16_t* vb, v4f (&o)[8],
+                                            float& l) {
+    const int lane = tid & 63, i = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int d = 0; d < 8; ++d) o[d] = v4f{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
+    float m = -INFINITY;
+    l = 0.f;
     const int blocks = (p.max_len + kPKeys - 1) / kPKeys;
     // the mask of keys 16 kt + 4 g ... + 3 of a block (max_len % 4 == 0: four keys are inside or outside together)
     auto load_mask = [&](v2u (&mk)[4], const int blk) {
@@ -378,6 +368,7 @@ __global__ __launch_bounds__(256) void prompt_attention(PromptParams p) {
                 const int64_t at = (j < p.max_len ? j : p.max_len - 1) * kHd + 8 * c;
                 kk[r] = *(const v4u*)(kb + at);
                 vv[r] = *(const v4u*)(vb + at);
+                if (!kTwo && j >= p.max_len) vv[r] = v4u{0u, 0u, 0u, 0u};  // (nothing, not 0 times what the last row holds)
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) *(v4u*)(ks + (4 * a + r) * kPKPitch + 16 * c) = kk[r];
@@ -442,18 +433,61 @@ __global__ __launch_bounds__(256) void prompt_attention(PromptParams p) {
                 const char* at = vs + (16 * d + i) * kPVPitch + (32 * pr + 4 * g) * 2;
                 const v2u v0 = *(const v2u*)at, v1 = *(const v2u*)(at + 32);
                 const v8bf vf = __builtin_bit_cast(v8bf, (v4u{v0[0], v0[1], v1[0], v1[1]}));
-                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(v8bf, lo), o[d], 0, 0, 0);
+                if (kTwo) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(v8bf, lo), o[d], 0, 0, 0);
                 o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(v8bf, hi), o[d], 0, 0, 0);
             }
         }
     }
     l += __shfl_xor(l, 16, kWave);
     l += __shfl_xor(l, 32, kWave);
-    if (t0 + i >= p.T) return;
+}
+
+// (the bound keeps three waves a SIMD, as one walk alone has; two cost 0.3 % of a prompt of 8 x 128 positions)
+__global__ __launch_bounds__(256, 3) void prompt_attention(PromptParams p) {
+    __shared__ __attribute__((aligned(16))) char ks[kPKeys * kPKPitch];
+    __shared__ __attribute__((aligned(16))) char vs[kHd * kPVPitch];
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t bh = blockIdx.x;
+    const int64_t b = bh / p.H;
+    const int h = (int)(bh - b * p.H);
+    const int t0 = (int)blockIdx.y * kPRows + wave * 16;
+    const int t = t0 + i < p.T ? t0 + i : p.T - 1;  // this lane's position (past the end: a copy of the last, not stored)
+    const int64_t qrow = ((b * p.T + t) * p.H + h) * kHd;
+    v4u qf[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) qf[s] = *(const v4u*)(p.q + qrow + 32 * s + 8 * g);
+    const uint16_t* mrow = p.mask + (int64_t)t * p.max_len;
+    const uint16_t* kb = p.kc + bh * p.max_len * kHd;
+    const uint16_t* vb = p.vc + bh * p.max_len * kHd;
+    v4f o[8];
+    float l;
+    prompt_walk<true>(p, ks, vs, tid, qf, mrow, kb, vb, o, l);
+    const bool live = t0 + i < p.T;
+    // (a position with no open row has no probabilities: zeros, as the library gives)
+    auto value = [&](const int d, const int e) { return l == 0.f ? 0.f : o[d][e] / l; };
+    u32 odd = 0;  // this lane's results that are no numbers
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            y[e] = value(d, e);
+            if (!(fabsf(y[e]) < INFINITY)) odd |= 1u << (4 * d + e);
+        }
+        if (live) *(v2u*)(p.out + qrow + 16 * d + 4 * g) = v2u{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+    }
+    // The low part of a probability may be zero or negative, so that an infinite value makes a NaN of an infinity: such
+    // results are worked out again with one part.
+    if (!__syncthreads_or(live && odd)) return;
+    prompt_walk<false>(p, ks, vs, tid, qf, mrow, kb, vb, o, l);
 #pragma unroll
     for (int d = 0; d < 8; ++d)
-        *(v2u*)(p.out + qrow + 16 * d + 4 * g) = v2u{pack_bf16x2(o[d][0] / l, o[d][1] / l), pack_bf16x2(o[d][2] / l, o[d][3] / l)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (live && ((odd >> (4 * d + e)) & 1)) p.out[qrow + 16 * d + 4 * g + e] = (uint16_t)f32_to_bf16_bits(value(d, e));
 }
+
 
 }  // namespace
 }  // namespace k3q
