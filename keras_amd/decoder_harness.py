@@ -142,7 +142,9 @@ class DecoderBlock(Layer):
             if prompt_kernel is None:
                 prompt_kernel = not any(quantises_rows(layer) for layer in (
                     self.query, self.key, self.value, self.attn_out, self.gate, self.up, self.down))
-            if prompt_kernel and kops.prompt_attention_supported(q, kc, vc, mask):
+            B, T, H, _ = q.shape
+            if (prompt_kernel and kops.prompt_attention_pays(B, T, H, kc.shape[2])
+                    and kops.prompt_attention_supported(q, kc, vc, mask)):
                 a = kops.prompt_attention(q, kc, vc, mask)
             else:
                 a = torch.nn.functional.scaled_dot_product_attention(

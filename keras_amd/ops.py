@@ -1322,6 +1322,16 @@ def prompt_attention_supported(q, cache_k, cache_v, mask):
             and all(t.is_cuda and t.device == q.device and t.dtype == torch.bfloat16 for t in (q, cache_k, cache_v, mask)))
 
 
+def prompt_attention_pays(B, T, H, max_len):
+    """Whether the prompt's kernel is the faster one wherever in the cache the T positions lie: a workgroup walks the cache
+    by itself, which a piece near the end of a long one makes long (us, library / kernel, the first and the last
+    positions: 8 x 32 heads T=128 max_len 256 46 / 15, 46 / 23, 512 75 / 18, 75 / 37; T=33 512 33 / 11, 34 / 31; T=16 256 18 / 8,
+    18 / 17, 512 31 / 11, 31 / 31, 1024 55 / 14, 55 / 59; T=512 512 139 / 98, 140 / 98, 4096 741 / 265, 741 / 929; 16 x 32 heads
+    T=16 256 22 / 10, 22 / 23, T=65 128 23 / 22, 24 / 24)."""
+    few = B * H <= 256
+    return max_len <= 512 and T >= (128 if not few else 33 if max_len > 256 else 1)
+
+
 def prompt_attention(q, cache_k, cache_v, mask):
     """`scaled_dot_product_attention(q.transpose(1, 2), cache_k, cache_v, attn_mask=mask[None, None]).transpose(1, 2)` for
     q `[B, T, H, 128]` and caches `[B, H, max_len, 128]` that `prompt_attention_supported`."""

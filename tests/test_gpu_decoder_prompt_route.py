@@ -62,3 +62,14 @@ def test_block_alone(dev, monkeypatch):
             model.blocks[0].forward(torch.randn(1, 9, 256, device=dev).to(torch.bfloat16), lambda: (model.cos[:9], model.sin[:9], mask),
                                     model.new_cache(1)[0], torch.arange(9, device=dev), tables=(model.cos, model.sin))
         assert len(calls) == count
+
+
+@pytest.mark.parametrize("max_len,T,kernel", [(256, 20, True), (512, 32, False), (512, 33, True), (516, 64, False)])
+def test_long_caches_keep_the_library(dev, monkeypatch, max_len, T, kernel):
+    model = LlamaStyleDecoder(dtype="bfloat16", device="cuda:0", seed=5, **dict(CFG, max_len=max_len, n_layers=1))
+    calls, real = [], kops.prompt_attention
+    monkeypatch.setattr(kops, "prompt_attention", lambda *a: (calls.append(1), real(*a))[1])
+    ids = torch.randint(0, CFG["vocab"], (2, T), generator=torch.Generator().manual_seed(2)).to(dev)
+    with torch.no_grad():
+        model.forward(ids, torch.arange(T, device="cuda"), model.new_cache(2))
+    assert len(calls) == kernel
