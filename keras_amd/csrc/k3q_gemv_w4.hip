@@ -1988,8 +1988,10 @@ bool km_rows_plan(KmRowsPlan& pl, int x_dtype, int64_t M, int64_t K, int64_t N, 
         return false;
     const bool f32 = x_dtype == K3Q_F32;
     // as in the kernels on the stored weights, which split x in two and add an offset for most shapes, and have float32
-    // products for the others
-    pl.plain = (N % 8) != 0 || (K % 16) != 0;
+    // products for the others; and as in the GEMM on the de-quantised kernel, whose bfloat16 shapes have no offset either (an
+    // infinity in a row stays one in the columns it reaches, and is not a NaN in all of them; eager, us, with the offset and the sums
+    // of x it needs -> without: 1024 rows of 4096 x 4096 44.0 -> 41.1, of 14336 x 4096 132 -> 128, 640 of 8192 x 3072 51.6 -> 53.8)
+    pl.plain = (N % 8) != 0 || (K % 16) != 0 || (!f32 && (K % 128) == 0 && (N % 64) == 0);
     pl.parts = !f32 ? 1 : pl.plain ? 3 : 2;
     pl.Kp = (K + 127) / 128 * 128;
     pl.Np = (N + 31) / 32 * 32;  // the strips of the copy
@@ -2061,8 +2063,9 @@ extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K
     c.grouped = grouped;
     c.f32 = f32;
     c.bias_stride = bias_stride;
-    // whole units of bfloat16 rows that start on 16 bytes are read where they lie: only their sums are made first
-    const bool as_is = !f32 && !pl.plain && K == pl.Kp && aligned_to(x, 16);
+    // whole units of bfloat16 rows that start on 16 bytes are read where they lie: only their sums are made first, and weights
+    // without an offset need none
+    const bool as_is = !f32 && K == pl.Kp && aligned_to(x, 16);
     for (int64_t m0 = 0; m0 < M; m0 += pl.rows) {
         const int64_t rows = M - m0 < pl.rows ? M - m0 : pl.rows;
         const void* xm = (const char*)x + m0 * K * el;
@@ -2074,7 +2077,7 @@ extern "C" int k3q_gemm_w4_rows(const void* x, int x_dtype, int64_t M, int64_t K
         v2u* sx = (v2u*)((char*)workspace + pl.x_bytes);
         if (as_is) {
             c.x = (const uint16_t*)xm;
-            unit_sums_launch(c.x, sx, rows, K, s);
+            if (!pl.plain) unit_sums_launch(c.x, sx, rows, K, s);
         } else
             (pl.parts == 3   ? km_prepare_rows<3, true>
              : pl.parts == 2 ? km_prepare_rows<2, false>

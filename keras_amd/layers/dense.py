@@ -143,8 +143,8 @@ def strip_rows_params(layer, dtype, input_dim, units, block_size):
 # K=N=4096 768 rows 107 / 82, 1024 147 / 100, 2048 241 / 199; K=4096, N=11008 2048 rows 701 / 488; 1024 rows of K=N=2048 53 /
 # 45, K=4096, N=1024 60.2 / 59.9; K=N=2048 4000 rows 132 / 180: small kernels up to 1024.  Per channel (two parts a weight fewer
 # for the GEMM) 700 rows 97 / 79, 1024 104 / 101, K=2048, N=8192 96 / 98.  Bfloat16: while the tiles are one turn of the chip,
-# and enough for it: 1024 rows K=N=4096 58 / 46, K=14336, N=4096 168 / 134, K=N=2048 37 / 20, 640 rows K=N=4096 52 / 42, 700
-# rows K=4096, N=1024 28 / 25; K=4096, N=14336 138 / 143.
+# and enough for it (weights without an offset, as the GEMM's): 1024 rows K=N=4096 55 / 41, K=14336, N=4096 153 / 128, K=N=2048
+# 36 / 19, 640 rows K=N=4096 51 / 38, K=4096, N=1024 28 / 24; with an offset K=4096, N=14336 138 / 143.
 TILE_ROWS_MAX_F32, TILE_ROWS_MAX_F32_LARGE, TILE_ROWS_MAX_F32_CHANNEL, TILE_LARGE_WEIGHTS = 1024, 2048, 768, 16 << 20
 TILE_ROWS_MAX_BF16, TILE_COUNTS_BF16 = 1024, (32, 256)
 
