@@ -283,11 +283,15 @@ __device__ __forceinline__ void rint_quotients(const float (&x)[4], const float 
 // registers let two workgroups share a CU.  kPacked: the integers leave as int4 pairs along N (k3q_pack_int4's bytes; q is
 // [K, N / 2], the range fits four bits): half a byte written per weight instead of one byte written, read again and packed.
 constexpr int kHeldY = 8, kHeldRows = 16;
-template <bool kFull, bool kBF16, bool kPacked>
-__global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(GroupedParams p, int col_tiles, int items) {
+// kRows: rows of a group that a thread holds, the smallest of 2, 4, 8 and 16 that takes the group.  With 16 for all of them a
+// thread loaded its last row again up to fourteen times: 4096 x 14336 float32, groups of 8, 16, 32 and 64, conditional loads /
+// 16 rows / now: 262 / 295 / 150, 155 / 168 / 97, 104 / 101 / 64, 77 / 70 / 51 us.
+template <int kRows, bool kFull, bool kBF16, bool kPacked>
+__global__ __launch_bounds__(kWqX * kHeldY, kFull || kRows < kHeldRows ? 4 : 2) void grouped_zp_held(GroupedParams p, int col_tiles,
+                                                                                                     int items) {
     __shared__ float lo_s[2][kHeldY][kWqX * 4], hi_s[2][kHeldY][kWqX * 4];
     const int tx = threadIdx.x % kWqX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / kWqX);
-    RawVals<kBF16, 4> rows[kHeldRows];
+    RawVals<kBF16, 4> rows[kRows];
     auto fetch = [&](const int item, const int j) {
         const int g = item / col_tiles;
         const int64_t col = ((int64_t)(item - g * col_tiles) * kWqX + tx) * 4, r0 = (int64_t)g * p.block;
@@ -307,7 +311,7 @@ __global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(
             hi[e] = -INFINITY;
         }
 #pragma unroll
-        for (int j = 0; j < kHeldRows; ++j) {
+        for (int j = 0; j < kRows; ++j) {
             const int i = ty + j * kHeldY;
             if (!kFull && i >= p.block) break;
             float f[4];
@@ -347,7 +351,7 @@ __global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(
             }
         }
 #pragma unroll
-        for (int j = 0; j < kHeldRows; ++j) {
+        for (int j = 0; j < kRows; ++j) {
             const int i = ty + j * kHeldY;
             if (kFull || (i < p.block && r0 + i < p.K)) {
                 float f[4], n[4];
@@ -370,7 +374,7 @@ __global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(
     const int step = gridDim.x;
     int item = blockIdx.x;
 #pragma unroll
-    for (int j = 0; j < kHeldRows; ++j) fetch(item, j);
+    for (int j = 0; j < kRows; ++j) fetch(item, j);
     int par = 0;
 #pragma clang loop unroll(disable)
     for (; item + step < items; item += step, par ^= 1)  // (uniform over the workgroup: every thread meets every barrier)
@@ -378,10 +382,10 @@ __global__ __launch_bounds__(kWqX * kHeldY, kFull ? 4 : 2) void grouped_zp_held(
     work(std::false_type{}, item, item, par);
 }
 
-template <bool kFull>
+template <int kRows, bool kFull>
 void (*held_kernel(const bool bf, const bool packed))(GroupedParams, int, int) {
-    return bf ? (packed ? grouped_zp_held<kFull, true, true> : grouped_zp_held<kFull, true, false>)
-              : (packed ? grouped_zp_held<kFull, false, true> : grouped_zp_held<kFull, false, false>);
+    return bf ? (packed ? grouped_zp_held<kRows, kFull, true, true> : grouped_zp_held<kRows, kFull, true, false>)
+              : (packed ? grouped_zp_held<kRows, kFull, false, true> : grouped_zp_held<kRows, kFull, false, false>);
 }
 
 __global__ void clear_u32(u32* p, int64_t n) {
@@ -478,7 +482,11 @@ static int run_weight_quantize_grouped(const void* x, int x_dtype, int64_t K, in
         const unsigned blocks = (unsigned)(items < 512 ? items : 512);
         const bool full = block_size == kHeldY * kHeldRows && K % block_size == 0;
         void (*kernel)(GroupedParams, int, int) =
-            full ? held_kernel<true>(bf, packed) : held_kernel<false>(bf, packed);
+            full                         ? held_kernel<kHeldRows, true>(bf, packed)
+            : block_size <= 2 * kHeldY ? held_kernel<2, false>(bf, packed)
+            : block_size <= 4 * kHeldY ? held_kernel<4, false>(bf, packed)
+            : block_size <= 8 * kHeldY ? held_kernel<8, false>(bf, packed)
+                                         : held_kernel<kHeldRows, false>(bf, packed);
         kernel<<<blocks, kWqX * kHeldY, 0, s>>>(p, (int)col_tiles, (int)items);
         return launch_status();
     }
