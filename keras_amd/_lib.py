@@ -172,6 +172,7 @@ TEST_SIGNATURES = {
     "k3qt_gemm_deep_tile": (_int, [_i64, _i64, _i64, _int]),
     "k3qt_w4_tile_plan": (_int, [_i64, _int, _i64, _i64, _ptr]),
     "k3qt_w4_rows_launch": (_int, [_int, _i64, _i64, _i64, _i64, _i64, _ptr]),
+    "k3qt_header_digest": (ctypes.c_char_p, []),
     "k3qt_gemv_w4_plan": (
         _int,
         [_ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64,
@@ -233,9 +234,16 @@ def load():
     return lib
 
 
+# what stays with ctypes: arguments that point to structures, a text as result (and the test hooks)
+BY_CTYPES = frozenset((
+    "k3q_error_string", "k3q_gemv_w4_multi", "k3q_gemv_w4s_multi", "k3q_gemv_w4s_pre", "k3q_gemv_w4s_rows_multi",
+    "k3q_dense_i8_w8s_multi", "k3q_dense_i8_w8s_pre", "k3q_input_op_quantize",
+))
+
+
 class _Calls:
     """The library's entry points as the package's own calls make them: built-in functions that take addresses as integers
-    (k3q_calls.cpp), ctypes functions where an argument points to a structure."""
+    (k3q_calls.cpp), ctypes functions for `BY_CTYPES`."""
 
     def __init__(self, lib):
         try:
@@ -243,8 +251,12 @@ class _Calls:
         except ImportError as e:
             raise RuntimeError(f"{os.path.join(_HERE, '_k3q_calls.so')} is missing or does not load ({e}): build it with "
                                "`python -m keras_amd.csrc.build`") from e
+        # (a module of an earlier header would hand over arguments in the order of that one)
+        if getattr(native, "header_digest", None) != lib.k3qt_header_digest().decode():
+            raise RuntimeError(f"{os.path.join(_HERE, '_k3q_calls.so')} and {LIB_PATH} are not built from the same header: "
+                               "build both with `python -m keras_amd.csrc.build`")
         for name in list(SIGNATURES) + list(TEST_SIGNATURES):
-            setattr(self, name, getattr(native, name, None) or getattr(lib, name))
+            setattr(self, name, getattr(lib if name in BY_CTYPES or name in TEST_SIGNATURES else native, name))
 
 
 _calls = None

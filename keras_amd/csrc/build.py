@@ -4,6 +4,7 @@ Run as `python -m keras_amd.csrc.build` or through `__graft_entry__.build()`.
 hipcc cross-compiles, so no GPU is needed to build.
 """
 
+import hashlib
 import os
 import shutil
 import subprocess
@@ -14,6 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "libk3q.so")
 CALLS = os.path.join(PKG, "_k3q_calls.so")
+HEADER = os.path.join(os.path.dirname(PKG), "include", "k3q.h")
 
 SOURCES = [
     "k3q_api.hip",
@@ -53,6 +55,13 @@ def hipcc():
     return exe
 
 
+def header_flag():
+    """The header that library and Python module are built from, as a macro of both: keras_amd/_lib.py puts them together
+    only if it is the same one."""
+    with open(HEADER, "rb") as f:
+        return '-DK3Q_HEADER_DIGEST="%s"' % hashlib.sha256(f.read()).hexdigest()[:16]
+
+
 def build(verbose=True, jobs=8):
     srcs = [os.path.join(HERE, s) for s in SOURCES if os.path.exists(os.path.join(HERE, s))]
     objdir = os.path.join(HERE, "build")
@@ -62,7 +71,7 @@ def build(verbose=True, jobs=8):
     for src in srcs:
         obj = os.path.join(objdir, os.path.basename(src) + ".o")
         objs.append(obj)
-        cmd = [hipcc(), *FLAGS, "-c", src, "-o", obj]
+        cmd = [hipcc(), *FLAGS, header_flag(), "-c", src, "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
@@ -79,7 +88,7 @@ def build(verbose=True, jobs=8):
 
 def build_calls(verbose=True):
     """The Python module over the library's entry points (k3q_calls.cpp), next to the library it is linked to."""
-    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-I", sysconfig.get_paths()["include"],
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", header_flag(), "-I", sysconfig.get_paths()["include"],
            os.path.join(HERE, "k3q_calls.cpp"), "-o", CALLS, "-L", PKG, "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN"]
     if verbose:
         print(" ".join(cmd), flush=True)

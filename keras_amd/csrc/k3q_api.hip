@@ -1,5 +1,8 @@
 // Entry points that carry no kernel: version and error text.
 #include "k3q_common.h"
+#include "k3q_testing.h"
+
+extern "C" const char* k3qt_header_digest(void) { return K3Q_HEADER_DIGEST; }
 
 extern "C" int k3q_version(void) { return 100; }
 

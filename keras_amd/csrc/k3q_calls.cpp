@@ -140,4 +140,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_k3q_calls", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__k3q_calls(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__k3q_calls(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "header_digest", K3Q_HEADER_DIGEST) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

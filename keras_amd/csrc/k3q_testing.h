@@ -37,6 +37,9 @@ int k3qt_w4_tile_plan(int64_t rows, int parts, int64_t K, int64_t N, int* plan);
  * tile, workgroups that share K, steps of K per split, bytes of its partial sums, bytes of room for them}. */
 int k3qt_w4_rows_launch(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int64_t m0, int64_t* launch);
 
+/* Digest of the include/k3q.h that the library was built from (host only); k3q_calls.cpp's module holds its own. */
+const char* k3qt_header_digest(void);
+
 #ifdef __cplusplus
 }
 #endif
