@@ -1995,6 +1995,7 @@ bool km_rows_plan(KmRowsPlan& pl, int x_dtype, int64_t M, int64_t K, int64_t N, 
     pl.parts = !f32 ? 1 : pl.plain ? 3 : 2;
     pl.Kp = (K + 127) / 128 * 128;
     pl.Np = (N + 31) / 32 * 32;  // the strips of the copy
+    if (!w4_tile_fits(1, 2, pl.Kp, pl.Np)) return false;  // (not a row of either type: the kernels on the stored weights do)
     pl.rows = M < kKmMostRows / pl.parts ? M : kKmMostRows / pl.parts;
     while (pl.rows > 1 && !w4_tile_fits(pl.rows, pl.parts, pl.Kp, pl.Np)) pl.rows /= 2;
     const int64_t mx = pl.rows * pl.parts;

@@ -46,6 +46,17 @@ def test_every_launch_covers_k_and_has_room():
     assert changes > 300
 
 
+def test_kernels_beyond_the_tiles_offsets_are_not_promised():
+    """K and N that 32-bit lane offsets do not reach are not taken (they go to the kernels on the stored weights) instead of
+    failing at the launch."""
+    assert kops.int4_tiles_rows_supported(1 << 20, 1 << 16, 128)
+    for K, N in ((1 << 24, 64), (1 << 21, 1 << 16), (1 << 21, (1 << 16) - 8)):
+        for bs in (128, None):
+            assert not kops.int4_tiles_rows_supported(K, N, bs)
+        for dtype in (_lib.K3Q_F32, _lib.K3Q_BF16):
+            assert _lib.load().k3q_gemm_w4_rows_workspace_bytes(dtype, 100, K, N, 128) == 0
+
+
 # the plans of the first and of the last launch: (blocks of rows, columns, splits)
 CASES = [
     (900, 6400, 2560, True, (4, 128, 1), (4, 256, 3)),
