@@ -104,6 +104,11 @@ class DecoderBlock(Layer):
         self.down.build((None, ffn_dim))
         self.built = True
 
+    def quantises_rows(self):
+        """Whether one of the block's layers quantises the rows it multiplies."""
+        return any(quantises_rows(layer) for layer in (
+            self.query, self.key, self.value, self.attn_out, self.gate, self.up, self.down))
+
     def forward(self, x, rows, cache, pos, tables=None, oob_flag=None, prompt_kernel=None):
         """x [B, T, D].  cache: (k, v) each [B, H, maxT, hd], written at positions `pos`
         (an int64 device tensor [T]); rows(): (cos, sin, mask) of these positions -- the table
@@ -140,8 +145,7 @@ class DecoderBlock(Layer):
                 kc.index_copy_(2, pos, k.transpose(1, 2))
                 vc.index_copy_(2, pos, v.transpose(1, 2))
             if prompt_kernel is None:
-                prompt_kernel = not any(quantises_rows(layer) for layer in (
-                    self.query, self.key, self.value, self.attn_out, self.gate, self.up, self.down))
+                prompt_kernel = not self.quantises_rows()
             B, T, H, _ = q.shape
             if (prompt_kernel and kops.prompt_attention_pays(B, T, H, kc.shape[2])
                     and kops.prompt_attention_supported(q, kc, vc, mask)):
@@ -272,7 +276,8 @@ class LlamaStyleDecoder(Model):
             return made[0]
 
         # (one layer that quantises its rows, and every block before it keeps the library's attention)
-        prompt_kernel = ids.shape[1] > 1 and not any(quantises_rows(layer) for layer in self._flatten_layers())
+        prompt_kernel = ids.shape[1] > 1 and not (quantises_rows(self.token_embedding)
+                                                  or any(block.quantises_rows() for block in self.blocks))
         for block, kv in zip(self.blocks, cache):
             x = block.forward(x, rows, kv, pos, tables=(self.cos, self.sin), oob_flag=self._pos_oob,
                               prompt_kernel=prompt_kernel)
