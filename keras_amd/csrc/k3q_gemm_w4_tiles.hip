@@ -479,15 +479,17 @@ bool w4_tile_fits(int64_t rows, int parts, int64_t K, int64_t N) {
     return ((parts == 2 ? rows : 0) + 128) * K * 2 < most && units * 4 * N < most && units * 8 * rows * parts < most;
 }
 
-// Tile shape and split of K from a model of the time (ns) fitted to a sweep of every shape and split (17 ... 900 rows, K = 768
-// ... 14336, N = 3072 ... 14336; what it chooses is within 4 % of the best measured everywhere there): a launch and the sums
-// of x 6 us; a workgroup its rounds at the shape's rate, which the start of its ring and its sums' way through LDS come on top
-// of, 256 of them at a time; partial sums a launch and their bytes out and in at 4.5 TB/s.
+// Tile shape and split of K from a model of the time (ns) fitted to a sweep of every shape and split (1469 calls of 17 ... 1024
+// rows, K = 768 ... 14336, N = 768 ... 14336; what it chooses takes 0.4 % more than the best measured one in the mean, 5.4 % in 99
+// of 100): a workgroup its rounds at the shape's rate, 7.5 % slower with all CUs at it than with one, which the start of its ring
+// and its sums' way through LDS come on top of, 256 of them at a time; partial sums a launch, something per split, and their
+// bytes out and in at 7.2 TB/s.  (A first fit, on fewer shapes and with splits dearer, left 1.0 % and 12 %, and more than the old
+// kernel took in places: 65 rows of 5120 x 11008 32.9 us, old kernel 29.5, now 29.5.)
 W4TilePlan w4_tile_plan(int64_t rows, int parts, int64_t K, int64_t N) {
     struct Shape {
         int mb, bn, round_ns, start_ns;
     };
-    static const Shape shapes[] = {{1, 128, 450, 3000}, {2, 128, 620, 4000}, {4, 128, 920, 6000}, {4, 256, 950, 6000}};
+    static const Shape shapes[] = {{1, 128, 460, 2220}, {2, 128, 600, 3370}, {4, 128, 880, 5410}, {4, 256, 820, 6560}};
     const int64_t xrows = rows * parts, units = K / 128;
     W4TilePlan best{};
     int64_t best_ns = -1;
@@ -501,9 +503,9 @@ W4TilePlan w4_tile_plan(int64_t rows, int parts, int64_t K, int64_t N) {
             const int64_t ks = (all + steps - 1) / steps;
             if (want > 1 && (steps < 4 || tiles * want > 256)) break;
             if (ks != want) continue;
-            const int64_t turns = (tiles * ks + 255) / 256;
-            int64_t ns = 6000 + turns * (2 * steps * sh.round_ns + sh.start_ns);
-            if (ks > 1 || parts == 3) ns += 2500 + ks * xrows * N * 8 / 4500;
+            const int64_t turns = (tiles * ks + 255) / 256, rounds = 2 * steps * sh.round_ns;
+            int64_t ns = turns * (rounds + sh.start_ns) + rounds * 75 * tiles * ks / 256000;
+            if (ks > 1 || parts == 3) ns += 1010 + 252 * ks + ks * xrows * N * 8 / 7170;
             if (best_ns < 0 || ns < best_ns) {
                 best_ns = ns;
                 best.mb = sh.mb;

@@ -59,12 +59,12 @@ def test_kernels_beyond_the_tiles_offsets_are_not_promised():
 
 # the plans of the first and of the last launch: (blocks of rows, columns, splits)
 CASES = [
-    (900, 6400, 2560, True, (4, 128, 1), (4, 256, 3)),
+    (612, 6400, 2560, True, (4, 256, 3), (2, 128, 3)),
     (800, 8192, 4096, True, (4, 128, 1), (4, 256, 3)),
     (648, 11008, 4096, True, (4, 128, 1), (4, 256, 5)),
     (860, 14336, 2048, True, (4, 128, 2), (4, 256, 5)),
-    (621, 4096, 2337, True, (4, 128, 1), (4, 256, 3)),     # three parts a row
-    (1985, 6400, 2049, False, (4, 128, 1), (4, 256, 3)),
+    (409, 4096, 2337, True, (4, 256, 3), (2, 128, 3)),     # three parts a row
+    (1505, 6400, 2049, False, (4, 256, 3), (4, 128, 3)),
     (1700, 11008, 3333, False, (4, 128, 1), (4, 256, 3)),
 ]
 
@@ -99,3 +99,14 @@ def test_last_launch(dev, M, K, N, f32, first, last, block_size):
     else:
         bound = mag * 4 * 2.0 ** -24 * K ** 0.5 + (exact.abs() + 2 * b.double().abs()) * 3.05 * 2.0 ** -8
     assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("rows,parts,K,N,plan", [
+    (65, 1, 5120, 11008, (4, 256, 5)), (64, 1, 5120, 11008, (2, 128, 2)), (329, 2, 8192, 2048, (4, 256, 5)),
+    (338, 1, 5120, 2048, (4, 128, 5)), (920, 1, 8192, 2048, (4, 128, 2)),
+    (96, 1, 4096, 14336, (2, 128, 1)), (102, 2, 3200, 4544, (2, 128, 1)),
+])
+def test_splits_where_they_pay(rows, parts, K, N, plan):
+    """Measured: the best plan of each, 6 to 33 % ahead of fewer splits (the last two: of more)."""
+    out = (ctypes.c_int * 4)()
+    assert _lib.load().k3qt_w4_tile_plan(rows, parts, K, N, out) == 0 and tuple(out)[:3] == plan
