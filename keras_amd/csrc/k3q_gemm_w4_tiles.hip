@@ -2,7 +2,7 @@
 // (k3q_w4s_pack), nothing de-quantised in memory; the result is written here unless K is split over workgroups.
 //
 // Eight waves, each 32 columns x 32 kMB rows: kNS of them side by side along N, kKQ slices of K (every kKQ-th unit of 128), whose
-// sums meet in LDS at the end.  The tile kernel before this one (k3q_gemv_w4.hip, which keeps the other group lengths) filled
+// sums meet in LDS at the end -- 4 x 2 in tiles of 128 columns, 8 x 1 in tiles of 256.  The tile kernel before this one (k3q_gemv_w4.hip, which keeps the other group lengths) filled
 // the chip by splitting K over workgroups: at 96 rows of 4096 x 14336 four splits wrote and read 44 MB of partial sums
 // beside 29 MB of kernel, 13 of its 34 us.  Slices inside a workgroup need none of that, and narrow tiles of few rows (64 x
 // 128) fill the chip at 96 rows without a split.  A lane's products are one column of the kernel, so that a unit's scale is one
@@ -15,9 +15,9 @@
 //
 // What bounds it: at 512 rows and more the matrix cores (128 x 256 tiles: 1.23 PFLOP/s in the loop, the library's large
 // products on this card 1.26), below that the starts of ring and launch and the rate of the requests (64 x 128: 39 bytes a ns
-// and CU).  Graph nodes, groups of 128, us, before -> now: 32 rows of 4096 x 14336 22.4 -> 19.0, 96 34.9 -> 29.0, 512 89.3 ->
-// 72.7; 128 rows of 4096 x 4096 24.3 -> 18.5, 512 40.6 -> 28.9; 128 of 14336 x 4096 37.9 -> 32.5; 256 of 8192 x 8192 58.9 ->
-// 51.7.  Tried and slower: the sums of x in this kernel, from the rows in LDS (saves 2.8 us of launch, costs 0.1 us a round: 512
+// and CU).  Graph nodes, groups of 128, us, before -> now: 32 rows of 4096 x 14336 21.7 -> 17.2, 96 32.0 -> 27.3, 512 86.2 ->
+// 68.9; 128 rows of 4096 x 4096 23.6 -> 17.3, 512 37.8 -> 28.7; 128 of 14336 x 4096 34.3 -> 29.0; 256 of 8192 x 8192 54.8 ->
+// 47.8.  Tried and slower: the sums of x in this kernel, from the rows in LDS (saves 2.8 us of launch, costs 0.1 us a round: 512
 // rows of 4096 x 14336 76.9); a block's four products in turn instead of a step's four blocks (80.9, the sums depend on each
 // other); an explicit wait for a step's operands ahead of the next reads (no gain).
 #include "k3q_gemm_w4_tiles.h"
@@ -26,7 +26,7 @@
 namespace k3q {
 namespace {
 
-constexpr int kTThreads = 512;  // 8 waves: 4 along N (32 columns each) x 2 along K
+constexpr int kTThreads = 512;  // 8 waves: kNS along N (32 columns each) x kKQ along K
 
 struct TileParams {
     const char* x;
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(kTThreads) void gemm_w4_tiles(TileParams p) {
         for (int mb = 0; mb < kMB; ++mb) fold(mb);
     }
 
-    // ---- the two slices' sums, through LDS, and the result ----
+    // ---- the slices' sums, through LDS, and the result ----
     __syncthreads();
     constexpr int kRows = 32 * kMB;
 #pragma unroll

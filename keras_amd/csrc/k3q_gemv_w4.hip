@@ -1960,8 +1960,8 @@ extern "C" int k3q_gemm_w4_strip(const void* x, int x_dtype, int64_t M, int64_t 
 // The rows made ready (km_prepare_rows; whole units of bfloat16 rows stay where they are, and only their sums are made), the
 // tile kernel (k3q_gemm_w4_tiles.hip) on the strip-linear copy and, where it splits K or a row has three parts, a second
 // pass.  The padding costs a pass over x (3 us) where it spares the kernel a copy.  Graph nodes, us, the kernel on the stored
-// weights -> the tile kernel with a second pass always -> now: bfloat16 K=1600, N=6400 300 rows 137 -> 29.9 -> 18.6, 900
-// rows (1200: 570) -> 48.7 -> 39.4; float32 K=N=4096 64 rows -> 26.7 -> 21.3, 300 rows -> 59.5 -> 43.8, 700 -> 102.7 -> 79.
+// weights -> the tile kernel with a second pass always -> now: bfloat16 K=1600, N=6400 300 rows 137 -> 28.9 -> 17.3, 900
+// rows -> 46.4 -> 38.4, 1200 570 -> 70.4 -> 55.1; float32 K=N=4096 64 rows -> 25.7 -> 20.5, 300 -> 57.5 -> 42.2, 700 -> 97.4 -> 75.0.
 // A float32 row doubles the matrix work, which bounds the larger sizes.  Error against 64 bits (2-norm) of the
 // forms: float32 4.9e-6 (de-quantised kernel 1.3e-5), bfloat16 1.66e-3, without an offset 8e-8.
 namespace k3q {

@@ -86,8 +86,8 @@ def lora_initializer(spec):
 
 # rows for which the int4 forward reads the kernel as int4 tiles, from the strip-linear copy or (groups of 64) a
 # K-contiguous one, measured against the 32-row passes below it (17 rows 13.4 us at K=N=4096, where the tiles take 14.5)
-# and the de-quantise + GEMM route above it (512 rows: K=4096, N=14336 98 against 73; K=N=4096 45 against 30.5; K=14336,
-# N=4096 102 against 84).  What larger calls of the strip-linear copy keep on tiles: int4_tile_rows_route.
+# and the de-quantise + GEMM route above it (512 rows: K=4096, N=14336 98 against 69; K=N=4096 45 against 29; K=14336,
+# N=4096 102 against 74).  What larger calls of the strip-linear copy keep on tiles: int4_tile_rows_route.
 KMAJOR_MIN_ROWS, KMAJOR_MAX_ROWS = 33, 512
 # from 17 rows on kernels at least this wide or this large (17 rows, groups of 128, us:
 # K=5120, N=13824: 26 against 36; K=13824, N=5120: 29 against 37; K=11008, N=4096: 25 against
@@ -140,9 +140,9 @@ def strip_rows_params(layer, dtype, input_dim, units, block_size):
 
 
 # Rows up to which the int4 tile kernel beats the GEMM on the de-quantised kernel (us, GEMM route / tiles).  Float32: grouped
-# K=N=4096 768 rows 107 / 82, 1024 147 / 100, 2048 241 / 199; K=4096, N=11008 2048 rows 701 / 488; 1024 rows of K=N=2048 53 /
-# 45, K=4096, N=1024 60.2 / 59.9; K=N=2048 4000 rows 132 / 180: small kernels up to 1024.  Per channel (two parts a weight fewer
-# for the GEMM) 700 rows 97 / 79, 1024 104 / 101, K=2048, N=8192 96 / 98.  Bfloat16: while the tiles are one turn of the chip,
+# K=N=4096 1024 rows 138 / 93, 2048 225 / 186; K=8192, N=4096 800 rows 249 / 146; K=4096, N=11008 2048 rows 688 / 462; 1024 rows of
+# K=N=2048 53 / 43, K=4096, N=1024 56.5 / 55.0; K=N=2048 4000 rows 132 / 180: small kernels up to 1024.  Per channel (two parts a
+# weight fewer for the GEMM) K=N=4096 700 rows 97 / 74, 1024 98 / 101.  Bfloat16: while the tiles are one turn of the chip,
 # and enough for it (weights without an offset, as the GEMM's): 1024 rows K=N=4096 55 / 41, K=14336, N=4096 153 / 128, K=N=2048
 # 36 / 19, 640 rows K=N=4096 51 / 38, K=4096, N=1024 28 / 24; with an offset K=4096, N=14336 138 / 143.
 TILE_ROWS_MAX_F32, TILE_ROWS_MAX_F32_LARGE, TILE_ROWS_MAX_F32_CHANNEL, TILE_LARGE_WEIGHTS = 1024, 2048, 768, 16 << 20
@@ -153,9 +153,9 @@ def int4_tile_rows_route(dtype, rows, input_dim, units, block_size):
     """Whether an int4 call of more rows than the decode kernels take goes to `ops.int4_matmul_tiles_rows`: shapes
     that neither the tile kernel's aligned entry (`ops.int4_kmajor_supported`) nor the GEMM on the de-quantised kernel takes
     (K % 128, N % 64), which went in passes of 32 bfloat16 or 8 float32 rows over the kernel (us, passes / tiles: K=1600,
-    N=6400 bfloat16 48 rows 25.6 / 15, 300 137 / 19; float32 17 rows 25 / 15, 300 307 / 30; one pass, up to 32 bfloat16 rows of a
+    N=6400 bfloat16 48 rows 25.6 / 13, 300 137 / 17; float32 17 rows 25 / 14, 300 307 / 24; one pass, up to 32 bfloat16 rows of a
     kernel this small, is as good), and rows of aligned shapes up to the limits above.  Where N % 8 or K % 16 leave only the
-    kernel of one output per thread (K=2048, N=5247: 480 us at 32 rows, 6.1 ms at 1200, against 15 and 82) every shape
+    kernel of one output per thread (K=2048, N=5247: 480 us at 32 rows, 6.1 ms at 1200, against 15 and 55) every shape
     goes here."""
     if not (dtype in (torch.float32, torch.bfloat16) and rows > kops.STRIP_MAX_ROWS
             and kops.int4_tiles_rows_supported(input_dim, units, block_size)):

@@ -52,8 +52,9 @@ def quantize_rows(quantizer, x2):
 
 
 def quantizes_alone(quantizer):
-    """Whether a layer's quantizer is the plain abs-max one, nobody shares its rows and nobody has put a function of their own
-    in the place of `quantizers.abs_max_quantize`: its forward may then quantise the rows in the call that multiplies them."""
+    """Whether a layer's forward may quantise its rows in the call that multiplies them: its quantizer is the plain abs-max one,
+    nobody shares its rows, and `quantizers.abs_max_quantize`, which that call goes round, is the package's own (a program
+    that wraps it, to count or to time, goes on seeing every call)."""
     return (type(quantizer) is quantizers.AbsMaxQuantizer and quantizer.output_dtype == "int8"
             and getattr(_state, "memo", None) is None and quantizers.abs_max_quantize is _abs_max_quantize)
 
