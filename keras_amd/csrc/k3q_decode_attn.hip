@@ -316,6 +316,9 @@ __global__ __launch_bounds__(256) void rope_cache_rows(RopeParams p) {
 constexpr int kPKeys = 64, kPRows = 64;             // cache rows per block, positions per workgroup
 constexpr int kPKPitch = kHd * 2 + 16;              // LDS bytes per key row
 constexpr int kPVPitch = kPKeys * 2 + 24;           // and per value column (of the transposed tile)
+// Scores below this leave float32's range when they are taken to base 2: closed, as in the library (a mask of the type's
+// lowest value closes a row whose keys it all names, and does not make it the mean of all values).
+constexpr float kPLowest = -2.3586498e38f;
 struct PromptParams {
     const uint16_t* q;      // [B, T, H, 128]
     const uint16_t *kc, *vc;  // [B, H, max_len, 128]
@@ -395,7 +398,8 @@ __device__ __forceinline__ void prompt_walk(const PromptParams& p, char* ks, cha
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const u32 w = mk[kt][e >> 1];
-                x[kt][e] = acc[e] * p.scale + __uint_as_float(e & 1 ? w & 0xffff0000u : w << 16);
+                const float v = acc[e] * p.scale + __uint_as_float(e & 1 ? w & 0xffff0000u : w << 16);
+                x[kt][e] = v < kPLowest ? -INFINITY : v;
                 top = fmaxf(top, x[kt][e]);
             }
         }

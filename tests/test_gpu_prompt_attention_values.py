@@ -49,3 +49,21 @@ def test_position_that_sees_nothing(dev):
     got, lib = kops.prompt_attention(q, k, v, mask), library(q, k, v, mask)
     assert not got[:, 3].any() and not got[:, 65:].any() and not lib[:, 3].any()
     assert bool(got.isfinite().all()) and bool(got[:, 4].any())
+
+
+@pytest.mark.parametrize("value", [torch.finfo(torch.bfloat16).min, -2.4e38, -2.3e38, -1e9, -30.0])
+def test_masks_of_low_finite_values(dev, value):
+    """A row that is low all over, and rows that are low in part."""
+    mk = lambda *s: torch.randn(*s, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(dev)
+    q, k, v = mk(1, 20, 2, 128), mk(1, 2, 128, 128), mk(1, 2, 128, 128)
+    mask = torch.zeros(20, 128, dtype=torch.bfloat16, device=dev)
+    mask[3] = value
+    mask[4, 64:], mask[5, :64], mask[6, ::2] = value, value, value
+    mask[7], mask[7, 100] = value, 0
+    got, lib = kops.prompt_attention(q, k, v, mask).double(), library(q, k, v, mask).double()
+    assert bool(got.isfinite().all())
+    assert torch.equal(got[:, 3] == 0, lib[:, 3] == 0)
+    # (either is a rounding of the result to bfloat16 and a few of its probabilities away from float64's)
+    assert float((got - lib).norm() / lib.norm()) < 2.0 ** -8
+    for row in (3, 4, 5, 6, 7):
+        assert float((got[:, row] - lib[:, row]).abs().max()) <= 2.0 ** -6 * max(1.0, float(lib[:, row].abs().max()))
