@@ -110,3 +110,32 @@ def test_splits_where_they_pay(rows, parts, K, N, plan):
     """Measured: the best plan of each, 6 to 33 % ahead of fewer splits (the last two: of more)."""
     out = (ctypes.c_int * 4)()
     assert _lib.load().k3qt_w4_tile_plan(rows, parts, K, N, out) == 0 and tuple(out)[:3] == plan
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block_size", [128, None])
+@pytest.mark.parametrize("M,K,N,plan", [
+    (65, 5120, 11008, (4, 256, 5)), (338, 5120, 2048, (4, 128, 5)), (64, 5120, 11008, (2, 128, 2)), (96, 14336, 2048, (2, 128, 8)),
+])
+def test_large_tiles_with_splits(dev, M, K, N, plan, block_size):
+    """Through the entry of the layers' own shapes: partial sums of every row, added by the second pass."""
+    out = (ctypes.c_int * 4)()
+    assert _lib.load().k3qt_w4_tile_plan(M, 1, K, N, out) == 0 and tuple(out)[:3] == plan
+    qk, bias = make_layer(K, N, block_size, seed=M, with_bias=True)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(K)).to(torch.bfloat16)
+    scale, kernel, b = qk["kernel_scale"].to(torch.bfloat16), qk["kernel"].to(dev), bias.to(torch.bfloat16)
+    zero = qk["kernel_zero"] if block_size else None
+    got = []
+    for fill in (0xFF, 0x7F):
+        kops._workspace(dev, 64 << 20).fill_(fill)
+        got.append(kops.int4_matmul_tiles_strip(
+            x.to(dev), kops.int4_strip_copy(kernel, N), N, scale.to(dev), kernel_zero=None if zero is None else zero.to(dev),
+            block_size=block_size, bias=b.to(dev)).cpu())
+    assert torch.equal(got[0], got[1])
+    rows = torch.tensor([0, 1, 31, 32, M // 2, M - 2, M - 1])
+    exact = c_w4_matmul_f64(x[rows], qk["kernel"], scale, zero, block_size, b, N)
+    mag = magnitude(x[rows], kernel, scale, zero, block_size, N)
+    # (the bound of test_tile_plans with an offset of 136)
+    bound = mag * 17 * 2.0 ** -24 * K ** 0.5 + (exact.abs() + 2 * b.double().abs()) * 3.05 * 2.0 ** -8
+    err = (got[0][rows].double() - exact).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
